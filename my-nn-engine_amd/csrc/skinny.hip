@@ -1,4 +1,4 @@
-// DequantMatMul for a few dozen activation rows (16 <= M <= 64: batched decode, short prefill
+// DequantMatMul for a few dozen activation rows (2 <= M <= 64: batched decode, short prefill
 // chunks): the int8 weight matrix is still the whole cost, so it is streamed ONCE, as int8, and turned
 // into matrix-core operands in registers -- unlike the large-M path, which multiplies by a 16-bit
 // copy of the weights (twice the bytes) in 256-row tiles that M rows would leave mostly empty.
@@ -431,7 +431,10 @@ __global__ __launch_bounds__(kReduceRopeThreads) void skinny_reduce_rope_kernel(
 // M <= 32): what bench.py --workload decode_batch --skinny-ablation times
 static int g_skinny_ablation = 0;
 
-bool skinny_gemm_supported(int M, int N, int K) { return M >= 16 && M <= 64 && K % kSkinnyK == 0 && K >= 2 * kSkinnyK && N >= 1; }
+// (from two rows on: a batch of 2 .. 15 leaves most columns of an MFMA tile empty, but the weights are the whole cost --
+// against row tiles of four on the vector units, each of which streams the matrix again, a batch-8 step of the
+// TinyLlama shape went from 4.20 to 1.16 ms)
+bool skinny_gemm_supported(int M, int N, int K) { return M >= 2 && M <= 64 && K % kSkinnyK == 0 && K >= 2 * kSkinnyK && N >= 1; }
 
 // K ranges: enough waves to keep ~1000 in flight, each with at least as many steps as it has stages
 static int skinny_ksplit(int N, int K) {
