@@ -195,6 +195,7 @@ struct Model {
     hipGraphExec_t graph_loop_exec = nullptr;
     bool qkv_attn = false;
     bool lm_argmax = false;       // ... and the lm_head launch finds the greedy token and moves the loop state on
+    uint64_t *argmax_scratch = nullptr;  // per-part candidates of the argmax launch (long rows)
     uint64_t *lm_cand = nullptr;  // its candidate words (all ~0 between launches)
     int spin_limit = 400000;      // polls a consumer role makes before it gives up and raises the error word
     int handover_failures = 0;    // steps whose hand-over gave up; the executor then rebuilt itself with one op per launch
@@ -600,15 +601,10 @@ static int enqueue_step(Model &m) {
     // greedy token of the last row of each sequence; for a batch-1 decode step the same launch
     // moves the device-side loop state on (token -> next input, position / past / active + 1)
     note(m, rows == 1 ? "argmax_advance" : "argmax_last", (double)B * V * eb);
-    if (S == 1) {
-        // the last (only) rows of all sequences are contiguous: one launch, one workgroup per sequence
-        AdvanceState adv{};
-        if (rows == 1) adv = AdvanceState{m.d_ids, m.d_pos, m.d_past, m.d_active, m.d_tokens, m.d_step, m.token_cap};
-        TRY(argmax_rows<T>(m.d_next, m.logits, B, V, adv, s));
-    } else {
-        for (int b = 0; b < B; b++)
-            TRY(argmax_rows<T>(m.d_next + b, (const T *)m.logits + ((size_t)b * S + (S - 1)) * V, 1, V, AdvanceState{}, s));
-    }
+    // one launch for all sequences: their last rows are S rows of logits apart
+    AdvanceState adv{};
+    if (rows == 1) adv = AdvanceState{m.d_ids, m.d_pos, m.d_past, m.d_active, m.d_tokens, m.d_step, m.token_cap};
+    TRY(argmax_rows<T>(m.d_next, (const T *)m.logits + (size_t)(S - 1) * V, B, V, (size_t)S * V, adv, s, m.argmax_scratch));
     launch_timer() = LaunchTimer{};
     m.launches = (int)m.record.size();
     return 0;
@@ -913,6 +909,8 @@ static int build(Model &m, void **init, void **state) {
     size_t o_sc = plan.take(32 + (size_t)c.batch * 4), o_tok = plan.take((size_t)m.token_cap * 4);
     size_t o_as = plan.take(attn_scratch_bytes(c.batch, c.n_heads, c.seq_q, c.head_dim, m.nsplit));
     size_t o_cand = plan.take(rows == 1 ? (size_t)kGemvArgmaxWords * 8 : 0);
+    const size_t amax_bytes = argmax_scratch_bytes(c.batch, V);
+    size_t o_amax = plan.take(amax_bytes);
     const bool strm = c.streaming_kv != 0;
     size_t o_kvpos = plan.take(strm ? (size_t)c.max_seq * 8 : 0);
     size_t o_qref = plan.take(strm ? (size_t)rows * QD * eb : 0), o_knew = plan.take(strm ? (size_t)rows * KD * eb : 0);
@@ -936,6 +934,7 @@ static int build(Model &m, void **init, void **state) {
     m.d_tokens = (int32_t *)(m.arena + o_tok);
     m.attn_scratch = m.arena + o_as;
     m.lm_cand = (uint64_t *)(m.arena + o_cand);
+    m.argmax_scratch = amax_bytes ? (uint64_t *)(m.arena + o_amax) : nullptr;
     m.d_kvpos = (int64_t *)(m.arena + o_kvpos);
     m.q_ref = m.arena + o_qref; m.k_new = m.arena + o_knew; m.v_new = m.arena + o_vnew; m.attn_ref = m.arena + o_aref;
     m.k_rot = m.arena + o_krot;
@@ -979,8 +978,8 @@ static int build(Model &m, void **init, void **state) {
     return capture_step(m);
 }
 
-// Captures the decode step once (one new token per sequence, any batch: every launch reads its positions and
-// lengths from device memory).  Called again when the executor changes its launch plan.
+// Captures the step once (any batch, decode or prefill: every launch reads its positions and lengths from device
+// memory).  Called again when the executor changes its launch plan.
 constexpr int kLoopSteps = 32;
 static int capture_step(Model &m) {
     if (m.graph_exec) (void)hipGraphExecDestroy(m.graph_exec);
@@ -990,7 +989,7 @@ static int capture_step(Model &m) {
     m.graph_exec = m.graph_loop_exec = nullptr;
     m.graph = m.graph_loop = nullptr;
     m.use_graph = false;
-    if (m.cfg.seq_q != 1 || m.cfg.streaming_kv) return 0;  // (the streaming operators take host scalars at launch time)
+    if (m.cfg.streaming_kv) return 0;  // (the streaming operators take host scalars at launch time)
     hipError_t e = hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) {
         int rc = enqueue(m);
@@ -1004,7 +1003,7 @@ static int capture_step(Model &m) {
     } else (void)hipGetLastError();
     // batch-1 decode: several steps in one graph for the device-resident loop (every step leaves the next one's token,
     // position and lengths on the device, so the steps of a graph chain like separate launches of the one-step graph)
-    if (m.use_graph && m.cfg.batch == 1 && hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+    if (m.use_graph && m.cfg.batch * m.cfg.seq_q == 1 && hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
         int rc = 0;
         for (int i = 0; i < kLoopSteps && rc == 0; i++) rc = enqueue(m);
         hipError_t e2 = hipStreamEndCapture(m.stream, &m.graph_loop);

@@ -179,6 +179,25 @@ __global__ void embed_dequant_kernel(T *out, const int8_t *table, const T *scale
     for (int i = threadIdx.x; i < hidden; i += blockDim.x)
         Elem<T>::st(out, (size_t)blockIdx.x * hidden + i, (float)table[(size_t)r * hidden + i] * s);
 }
+// the same 16 codes per thread (one 16-byte load, two 16-byte stores): the row is two dependent memory round trips
+// behind the id, not a loop of them
+template <typename T>
+__global__ void embed_dequant_vec_kernel(T *out, const int8_t *table, const T *scale, const int64_t *ids, int vocab,
+                                         int hidden) {
+    int64_t r = ids[blockIdx.x];
+    if (r < 0) r += vocab;
+    const float s = Elem<T>::ld(scale, (size_t)r);
+    for (int c = threadIdx.x; c < hidden >> 4; c += blockDim.x) {
+        float f[16];
+        widen16_i8(((const U4 *)(table + (size_t)r * hidden))[c], f);
+        uint32_t o[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) o[i] = pack2<T>(f[2 * i] * s, f[2 * i + 1] * s);
+        U4 *dst = (U4 *)(out + (size_t)blockIdx.x * hidden + (size_t)c * 16);
+        dst[0] = U4{o[0], o[1], o[2], o[3]};
+        dst[1] = U4{o[4], o[5], o[6], o[7]};
+    }
+}
 
 // ---- elementwise groups ------------------------------------------------------------------------
 template <typename T>
@@ -375,33 +394,21 @@ int interleave_row_groups(void *dst, const void *src, size_t rows, size_t row_by
 
 // ---- greedy argmax, last maximum wins (reference crates/llm/src/session.rs:683-690) -----------
 // one workgroup of 1024 threads per row, 16-byte loads; (value, index) ordered by value, then index
+constexpr int kArgmaxThreads = 1024;
+// this thread's best of entries [i0, i1) of a row (i0 a multiple of 8)
 template <typename T>
-__global__ __launch_bounds__(1024) void argmax_last_kernel(int32_t *out, const T *logits, int n, AdvanceState adv) {
-    __shared__ float sv[16];
-    __shared__ int si[16];
-    const T *row = logits + (size_t)blockIdx.x * n;
-    // the loop state this launch moves on: read now, so that the tail is stores only
-    int st_step = 0, st_past = 0, st_active = 0;
-    int64_t st_pos = 0;
-    if (adv.ids && threadIdx.x == 0) {
-        st_step = *adv.step;
-        st_pos = adv.pos[0];
-        st_past = *adv.past;
-        st_active = *adv.active;
-    }
-    float bv = -INFINITY;
-    int bi = -1;
+__device__ inline void argmax_scan(const T *row, int i0, int i1, float &bv, int &bi) {
     if constexpr (sizeof(T) == 2) {
-        const int nvec = (((uintptr_t)row & 15) == 0) ? n / 8 : 0;
+        const int v0 = i0 / 8, nvec = (((uintptr_t)row & 15) == 0) ? i1 / 8 : v0;
         // eight loads in flight per thread (one at a time, a 128256-entry row was sixteen dependent round trips: 17 us)
         constexpr int kAhead = 8;
-        for (int c0 = threadIdx.x; c0 < nvec; c0 += 1024 * kAhead) {
+        for (int c0 = v0 + threadIdx.x; c0 < nvec; c0 += kArgmaxThreads * kAhead) {
             U4 v[kAhead];
 #pragma unroll
-            for (int j = 0; j < kAhead; j++) v[j] = ((const U4 *)row)[min(c0 + j * 1024, nvec - 1)];
+            for (int j = 0; j < kAhead; j++) v[j] = ((const U4 *)row)[min(c0 + j * kArgmaxThreads, nvec - 1)];
 #pragma unroll
             for (int j = 0; j < kAhead; j++) {
-                const int c = c0 + j * 1024;
+                const int c = c0 + j * kArgmaxThreads;
                 if (c >= nvec) break;
                 float f[8];
                 widen8<T>(v[j], f);
@@ -409,46 +416,131 @@ __global__ __launch_bounds__(1024) void argmax_last_kernel(int32_t *out, const T
                 for (int e = 0; e < 8; e++) argmax_take(bv, bi, f[e], c * 8 + e);
             }
         }
-        for (int i = nvec * 8 + threadIdx.x; i < n; i += 1024) argmax_take(bv, bi, Elem<T>::ld(row, i), i);
+        for (int i = nvec * 8 + threadIdx.x; i < i1; i += kArgmaxThreads) argmax_take(bv, bi, Elem<T>::ld(row, i), i);
     } else {
-        for (int i = threadIdx.x; i < n; i += 1024) argmax_take(bv, bi, Elem<T>::ld(row, i), i);
+        for (int i = i0 + threadIdx.x; i < i1; i += kArgmaxThreads) argmax_take(bv, bi, Elem<T>::ld(row, i), i);
     }
+}
+__device__ inline void argmax_wave(float &bv, int &bi) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         float ov = __shfl_xor(bv, off, 64);
         int oi = __shfl_xor(bi, off, 64);
         if (oi >= 0) argmax_take(bv, bi, ov, oi);
     }
+}
+// best of the workgroup in thread 0 (sv, si: LDS of a value and an index per wave)
+__device__ inline void argmax_block(float *sv, int *si, float &bv, int &bi) {
+    argmax_wave(bv, bi);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; w++)
+    if (threadIdx.x == 0)
+        for (int w = 1; w < kArgmaxThreads / 64; w++)
             if (si[w] >= 0) argmax_take(bv, bi, sv[w], si[w]);
+}
+struct AdvanceLoaded {
+    int step = 0, past = 0, active = 0;
+    int64_t pos = 0;
+};
+// the loop state a launch moves on: read first, so that the tail is stores only
+__device__ inline AdvanceLoaded advance_load(const AdvanceState &adv) {
+    AdvanceLoaded st;
+    if (adv.ids && threadIdx.x == 0) {
+        st.step = *adv.step;
+        st.pos = adv.pos[0];
+        st.past = *adv.past;
+        st.active = *adv.active;
+    }
+    return st;
+}
+__device__ inline void advance_store(const AdvanceState &adv, const AdvanceLoaded &st, int token) {
+    if (!adv.ids) return;
+    if (st.step < adv.cap) adv.tokens[st.step] = token;
+    *adv.step = st.step + 1;
+    adv.ids[0] = token;
+    adv.pos[0] = st.pos + 1;
+    *adv.past = st.past + 1;
+    *adv.active = st.active + 1;
+}
+template <typename T>
+__global__ __launch_bounds__(kArgmaxThreads) void argmax_last_kernel(int32_t *out, const T *logits, int n, size_t row_stride,
+                                                                     AdvanceState adv) {
+    __shared__ float sv[kArgmaxThreads / 64];
+    __shared__ int si[kArgmaxThreads / 64];
+    const AdvanceLoaded st = advance_load(adv);
+    float bv = -INFINITY;
+    int bi = -1;
+    argmax_scan(logits + (size_t)blockIdx.x * row_stride, 0, n, bv, bi);
+    argmax_block(sv, si, bv, bi);
+    if (threadIdx.x == 0) {
         out[blockIdx.x] = bi;
-        if (adv.ids) {
-            if (st_step < adv.cap) adv.tokens[st_step] = bi;
-            *adv.step = st_step + 1;
-            adv.ids[0] = bi;
-            adv.pos[0] = st_pos + 1;
-            *adv.past = st_past + 1;
-            *adv.active = st_active + 1;
-        }
+        advance_store(adv, st, bi);
+    }
+}
+// Long rows: each row in gridDim.y parts, the best of a part as one word (index low, value bits high) in cand; the
+// second launch, one wave per row, takes the best of a row's words.  A 128256-entry row costs a single workgroup 16 us of
+// compares; in parts the two launches take 6.
+template <typename T>
+__global__ __launch_bounds__(kArgmaxThreads) void argmax_part_kernel(uint64_t *cand, const T *logits, int n, size_t row_stride, int part) {
+    __shared__ float sv[kArgmaxThreads / 64];
+    __shared__ int si[kArgmaxThreads / 64];
+    float bv = -INFINITY;
+    int bi = -1;
+    const int i0 = blockIdx.y * part;
+    argmax_scan(logits + (size_t)blockIdx.x * row_stride, i0, min(n, i0 + part), bv, bi);
+    argmax_block(sv, si, bv, bi);
+    if (threadIdx.x == 0)
+        cand[(size_t)blockIdx.x * gridDim.y + blockIdx.y] = (uint64_t)(uint32_t)bi | ((uint64_t)__builtin_bit_cast(uint32_t, bv) << 32);
+}
+__global__ __launch_bounds__(64) void argmax_pick_kernel(int32_t *out, const uint64_t *cand, int parts, AdvanceState adv) {
+    const AdvanceLoaded st = advance_load(adv);
+    float bv = -INFINITY;
+    int bi = -1;
+    for (int i = threadIdx.x; i < parts; i += 64) {
+        const uint64_t w = cand[(size_t)blockIdx.x * parts + i];
+        if ((int)(uint32_t)w >= 0) argmax_take(bv, bi, __builtin_bit_cast(float, (uint32_t)(w >> 32)), (int)(uint32_t)w);
+    }
+    argmax_wave(bv, bi);
+    if (threadIdx.x == 0) {
+        out[blockIdx.x] = bi;
+        advance_store(adv, st, bi);
     }
 }
 
+// parts of a row: at least 8192 entries each (one pass of a workgroup), none for rows a single workgroup takes in 7 us
+static int argmax_part_len(int n) { return n > 65536 ? 8192 : n; }
+size_t argmax_scratch_bytes(int rows, int n) {
+    const int part = argmax_part_len(n);
+    return part < n ? (size_t)rows * ((n + part - 1) / part) * sizeof(uint64_t) : 0;
+}
+
 template <typename T>
-int argmax_rows(int32_t *out, const void *logits, int rows, int n, AdvanceState adv, hipStream_t s) {
-    MYNN_LAUNCH(argmax_last_kernel<T>, dim3(rows), dim3(1024), 0, s, out, (const T *)logits, n, adv);
+int argmax_rows(int32_t *out, const void *logits, int rows, int n, size_t row_stride, AdvanceState adv, hipStream_t s, uint64_t *scratch) {
+    const int part = argmax_part_len(n);
+    if (scratch && part < n) {
+        const int parts = (n + part - 1) / part;
+        MYNN_LAUNCH(argmax_part_kernel<T>, dim3(rows, parts), dim3(kArgmaxThreads), 0, s, scratch, (const T *)logits, n, row_stride, part);
+        int rc = launch_status("argmax_part_kernel");
+        if (rc) return rc;
+        MYNN_LAUNCH(argmax_pick_kernel, dim3(rows), dim3(64), 0, s, out, scratch, parts, adv);
+        return launch_status("argmax_pick_kernel");
+    }
+    MYNN_LAUNCH(argmax_last_kernel<T>, dim3(rows), dim3(kArgmaxThreads), 0, s, out, (const T *)logits, n, row_stride, adv);
     return launch_status("argmax_last_kernel");
 }
-template int argmax_rows<bf16_t>(int32_t *, const void *, int, int, AdvanceState, hipStream_t);
-template int argmax_rows<f16_t>(int32_t *, const void *, int, int, AdvanceState, hipStream_t);
-template int argmax_rows<float>(int32_t *, const void *, int, int, AdvanceState, hipStream_t);
+template int argmax_rows<bf16_t>(int32_t *, const void *, int, int, size_t, AdvanceState, hipStream_t, uint64_t *);
+template int argmax_rows<f16_t>(int32_t *, const void *, int, int, size_t, AdvanceState, hipStream_t, uint64_t *);
+template int argmax_rows<float>(int32_t *, const void *, int, int, size_t, AdvanceState, hipStream_t, uint64_t *);
 
 template <typename T>
 int embed_dequant(void *out, const int8_t *table, const void *scale, const int64_t *ids, int n_ids, int vocab,
                   int hidden, hipStream_t s) {
+    if (hidden % 16 == 0 && aligned16(table) && aligned16(out)) {
+        MYNN_LAUNCH(embed_dequant_vec_kernel<T>, dim3(n_ids), dim3(hidden >= 4096 ? 256 : (hidden / 16 + 63) / 64 * 64), 0, s, (T *)out, table,
+                    (const T *)scale, ids, vocab, hidden);
+        return launch_status("embed_dequant_vec_kernel");
+    }
     MYNN_LAUNCH(embed_dequant_kernel<T>, dim3(n_ids), dim3(256), 0, s, (T *)out, table, (const T *)scale, ids,
                        vocab, hidden);
     return launch_status("embed_dequant_kernel");
@@ -628,6 +720,6 @@ extern "C" int mynn_argmax_last(int32_t *out_index, const void *logits, int n, i
     MYNN_REQUIRE(out_index && logits && n > 0, MYNN_ERR_INVALID, "argmax_last: bad operand");
     return dispatch_dtype(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
-        return argmax_rows<T>(out_index, logits, 1, n, AdvanceState{}, as_stream(s));
+        return argmax_rows<T>(out_index, logits, 1, n, (size_t)n, AdvanceState{}, as_stream(s), nullptr);
     });
 }

@@ -19,7 +19,7 @@ int dequant_gemv_dispatch(void *out, const void *act, const int8_t *wq, const vo
                           int act_dtype, int out_dtype, hipStream_t s);
 
 // gemm.hip -- matrix-core DequantMatMul, M >= 16, 16-bit types
-// skinny.hip -- 16 <= M <= 64 rows against int8 weights streamed once (scale after the sum); `scratch` holds
+// skinny.hip -- 2 <= M <= 64 rows against int8 weights streamed once (scale after the sum); `scratch` holds
 // skinny_scratch_bytes(M, N, K) of f32 partial sums; epi is one of GEMM_* (SWIGLU: interleaved gate/up rows)
 bool skinny_gemm_supported(int M, int N, int K);
 size_t skinny_scratch_bytes(int M, int N, int K);
@@ -140,10 +140,12 @@ template <typename T>
 int gemv_norm_argmax(void *out, const void *x, const void *norm_w, float eps, const int8_t *wq, const void *scale, int N, int K,
                      uint64_t *cand, int32_t *next, AdvanceState adv, int *err, int spin_limit, hipStream_t s);
 
-// out[r] = index of the LAST maximum of logits row r; when adv.ids != nullptr the launch also
-// records the token and moves the decode loop on by one position
+// out[r] = index of the LAST maximum of logits row r (rows row_stride elements apart); when adv.ids != nullptr the
+// launch also records the token and moves the decode loop on by one position.  scratch (argmax_scratch_bytes, may be
+// null): lets several workgroups share a long row
 template <typename T>
-int argmax_rows(int32_t *out, const void *logits, int rows, int n, AdvanceState adv, hipStream_t s);
+int argmax_rows(int32_t *out, const void *logits, int rows, int n, size_t row_stride, AdvanceState adv, hipStream_t s, uint64_t *scratch);
+size_t argmax_scratch_bytes(int rows, int n);
 template <typename T>
 int embed_dequant(void *out, const int8_t *table, const void *scale, const int64_t *ids, int n_ids, int vocab,
                   int hidden, hipStream_t s);
