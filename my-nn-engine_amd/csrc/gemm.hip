@@ -17,8 +17,8 @@
 #include <map>
 #include <mutex>
 
+#include "gemm_store.h"
 #include "kernels.h"
-#include "mfma.h"
 
 namespace mynn {
 
@@ -86,81 +86,6 @@ __device__ inline void tile_of(int b, int nblocks, int tiles_m, int tiles_n, int
     const int rows_here = min(BAND, tiles_m - band * BAND);
     tm = band * BAND + in_band % rows_here;
     tn = in_band / rows_here;
-}
-
-// ---- store of a workgroup tile.  The MFMAs take the weight fragment as their first operand, so an
-// accumulator tile is the transpose of the output tile: lane l holds output row l % 32 and, in elements
-// 4q..4q+3, the four neighbouring output columns 8q + 4*(l/32) + 0..3 -- one 8-byte piece of a row.  Each
-// wave turns one 32-row strip of its tile at a time into row-major 16-bit values in its own LDS patch (the
-// operand buffers are free by now) and writes it out, and reads the residual, 16 bytes per lane, rows
-// contiguous.
-// at(i, j, e): element e of the accumulator of MFMA tile (i, j), as f32 ready to be rounded.
-template <typename T, typename G, int EPI, typename AccAt>
-__device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const T *R, int M, int N, int m0,
-                                           int n0, int wrow, int wcol, int lane, int wave) {
-    constexpr int TI = G::TI, TJ = G::TJ;
-    constexpr int EST = G::EST;
-    static_assert(EPI != GEMM_SWIGLU || TJ % 2 == 0, "the SwiGLU store pairs neighbouring column tiles");
-    constexpr int OC = EPI == GEMM_SWIGLU ? TJ * 16 : TJ * 32;  // output columns of the wave tile
-    constexpr int CPR = OC / 8;                                 // 16-byte chunks per strip row
-    const int ldc = EPI == GEMM_SWIGLU ? N >> 1 : N;
-    const int c0 = EPI == GEMM_SWIGLU ? (n0 + wcol) >> 1 : n0 + wcol;
-    T *patch = (T *)lds + (size_t)wave * 32 * EST;
-    const bool vec_ok = (ldc & 7) == 0;
-#pragma unroll
-    for (int i = 0; i < TI; i++) {
-        T *prow = patch + (lane & 31) * EST + (lane >> 5) * 4;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            if (EPI == GEMM_SWIGLU) {
-#pragma unroll
-                for (int j = 0; j < TJ; j += 2) {
-                    float o[4];
-#pragma unroll
-                    for (int x = 0; x < 4; x++) {
-                        const float g = Elem<T>::rnd(at(i, j, 4 * q + x)), u = Elem<T>::rnd(at(i, j + 1, 4 * q + x));
-                        // hardware 2^x and reciprocal (about 1 ulp of f32 each, far below the 16-bit rounding that
-                        // follows); the exact expf and division cost ~35 instructions per element here
-                        const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
-                        o[x] = (g * sig) * u;
-                    }
-                    *(uint2 *)(prow + j * 16 + 8 * q) = uint2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < TJ; j++)
-                    *(uint2 *)(prow + j * 32 + 8 * q) = uint2{pack2<T>(at(i, j, 4 * q), at(i, j, 4 * q + 1)),
-                                                              pack2<T>(at(i, j, 4 * q + 2), at(i, j, 4 * q + 3))};
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        const int row0 = m0 + wrow + i * 32;
-#pragma unroll
-        for (int q = 0; q < 32 * CPR / 64; q++) {
-            const int ch = q * 64 + lane, r = ch / CPR, cc = (ch % CPR) * 8;
-            const int row = row0 + r, col = c0 + cc;
-            if (row >= M || col >= ldc) continue;
-            U4 v = *(const U4 *)&patch[r * EST + cc];
-            const size_t at = (size_t)row * ldc + col;
-            if (vec_ok && col + 8 <= ldc) {
-                if (EPI == GEMM_RESIDUAL) {
-                    float fv[8], fr8[8];
-                    widen8<T>(v, fv);
-                    widen8<T>(*(const U4 *)(R + at), fr8);
-                    v = U4{pack2<T>(fr8[0] + fv[0], fr8[1] + fv[1]), pack2<T>(fr8[2] + fv[2], fr8[3] + fv[3]),
-                           pack2<T>(fr8[4] + fv[4], fr8[5] + fv[5]), pack2<T>(fr8[6] + fv[6], fr8[7] + fv[7])};
-                }
-                *(U4 *)(C + at) = v;
-            } else {
-                for (int x = 0; x < 8 && col + x < ldc; x++) {
-                    const float f = Elem<T>::ld(patch, r * EST + cc + x);
-                    if (EPI == GEMM_RESIDUAL) Elem<T>::st(C, at + x, Elem<T>::ld(R, at + x) + f);
-                    else C[at + x] = patch[r * EST + cc + x];
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
 }
 
 // KTAIL: K is not a multiple of 2*BK, so the last steps mask the columns of A past K.
@@ -520,6 +445,12 @@ static int gemm_launch_dma(void *out, const void *act, const void *wt, const voi
 bool qgemm_dma_supported(int M, int N, int K) {
     return K % 128 == 0 && (long)((M + 255) / 256) * ((N + 255) / 256) >= 128;
 }
+// its time, microseconds: rounds over the 256 CUs, a last one that is half empty a little faster than a full one
+double qgemm_dma_us(int M, int N, int K) {
+    if (!qgemm_dma_supported(M, N, K)) return 1e30;
+    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256), rounds = (tiles + 255) / 256;
+    return 4.0 + K * 1e-3 * (tiles < 256 ? 9.5 + 6.0 * tiles / 256 : 15.5 * rounds);
+}
 int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_scale, const int8_t *rhs, const void *rhs_scale,
               const void *res, int M, int N, int K, int dtype, int epi, hipStream_t s) {
     MYNN_REQUIRE(qgemm_dma_supported(M, N, K), MYNN_ERR_UNSUPPORTED, "quantized_matmul (large tiles): M=%d N=%d K=%d", M, N, K);
@@ -582,32 +513,71 @@ int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, in
     });
 }
 
-// ---- library-owned workspaces of the stand-alone entry point: one per stream, so calls on different streams never
-// share a dequantised weight; the table is guarded by a mutex.  A workspace only ever grows, and growing waits for
-// the stream's earlier work before the old block is released.
+// The time of gemm_nt_mfma, microseconds: grids of at least one round of 256 x 256 tiles run at 1.0 - 1.1 PFLOP/s (fp16;
+// bf16 5 % above), smaller ones take as long as one tile does on its CU, which tile_gemm beats at every size measured.
+double gemm_nt_mfma_us(int M, int N, int K, int dtype) {
+    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
+    if (tiles < 256) return 1e30;
+    return 6.0 + 2.0 * 256 * 256 * K * (double)tiles / (dtype == MYNN_BF16 ? 1.10e9 : 1.03e9);
+}
+// ... and of dequant_weight_rows before it (3 bytes per weight)
+static double dequant_us(int N, int K) { return 2.0 + 3.0 * N * K / 5.6e6; }
+
+// ---- library-owned workspaces of the stand-alone entry points: one per stream, so calls on different streams never
+// share a dequantised weight or partial sums; the table is guarded by a mutex.  A workspace only ever grows, and growing
+// waits for the stream's earlier work before the old block is released.  Its first bytes are tile_gemm's arrival counters,
+// zero between calls.
 struct StreamWs {
-    void *ptr = nullptr;
+    char *ptr = nullptr;
     size_t bytes = 0;
 };
 static std::mutex g_ws_mu;
 static std::map<hipStream_t, StreamWs> g_ws;
+constexpr size_t kWsCounterBytes = (size_t)kTgCounters * 4;
 
-static int stream_workspace(hipStream_t s, size_t need, void **out) {
+// out->bytes: what there is behind the counters; less than `need` only while the stream is being captured
+static int stream_workspace(hipStream_t s, size_t need, StreamWs *out) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     StreamWs &w = g_ws[s];
-    if (need > w.bytes) {
+    if (need + kWsCounterBytes > w.bytes) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
-            return fail(MYNN_ERR_STATE, "dequant_matmul: the library workspace cannot grow while the stream is being captured; "
-                                        "pass a workspace (mynn_dequant_matmul_ws) or a prepared weight");
+        if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+            *out = StreamWs{w.ptr, w.ptr ? w.bytes - kWsCounterBytes : 0};
+            return 0;
+        }
         MYNN_HIP(hipStreamSynchronize(s));
         if (w.ptr) MYNN_HIP(hipFree(w.ptr));
         w = StreamWs{};
-        MYNN_HIP(hipMalloc(&w.ptr, need));
-        w.bytes = need;
+        MYNN_HIP(hipMalloc((void **)&w.ptr, need + kWsCounterBytes));
+        w.bytes = need + kWsCounterBytes;
+        MYNN_HIP(hipMemsetAsync(w.ptr, 0, kWsCounterBytes, s));
     }
-    *out = w.ptr;
+    *out = StreamWs{w.ptr, w.bytes - kWsCounterBytes};
     return 0;
+}
+
+__global__ void zero_words_kernel(uint32_t *p, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0u;
+}
+
+// The product from the int8 weights as they are stored (tile_gemm), or nothing when it is not the one to take: one or two
+// rows (the GEMV streams faster: two rows of a matrix below 64 MB 10 against 12 us), other types, K not a multiple of 16,
+// unaligned operands, or so many rows that dequantising once and multiplying by 16-bit weights is faster.
+static bool takes_tiles(const void *out, const void *act, const int8_t *wq, int M, int N, int K, int act_dtype, int out_dtype, int *kind) {
+    if (act_dtype == MYNN_F32 || act_dtype != out_dtype || !aligned16(out) || !aligned16(act) || !aligned16(wq)) return false;
+    *kind = M >= 16 ? TG_W8 : TG_W8S;
+    return M >= (2l * K * 4 > 65536 || (long)N * K >= (64l << 20) ? 2 : 3) && N > 0 && tile_gemm_supported(*kind, M, N, K);
+}
+// scratch: what both the library's workspace and a caller's (mynn_dequant_matmul_workspace_bytes) can hold, so that both
+// make the same choice
+static size_t tiles_scratch(int kind, int N, int K) {
+    if (kind == TG_W8S) return kTgScratchMax;
+    const size_t b = gemm_weight_bytes(N, K);
+    return b <= kWsCounterBytes ? 0 : b - kWsCounterBytes < kTgScratchMax ? b - kWsCounterBytes : kTgScratchMax;
+}
+static bool tiles_first(const TgPlan &plan, int kind, int M, int N, int K, int dtype) {
+    return kind == TG_W8S || plan.us <= gemm_nt_mfma_us(M, N, K, dtype) + dequant_us(N, K);
 }
 
 int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
@@ -615,6 +585,17 @@ int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *
     int rc = dequant_weight_rows(ws, wq, scale, N, K, dtype, 0, 0, s);
     if (rc) return rc;
     return gemm_nt_mfma(out, act, ws, nullptr, M, N, K, dtype, GEMM_PLAIN, s, tile);
+}
+
+// partial sums of quantized_matmul's K ranges (0 bytes under capture when there are none yet: one range then)
+int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters, size_t *bytes) {
+    StreamWs w;
+    int rc = stream_workspace(s, need, &w);
+    if (rc) return rc;
+    *counters = (int *)w.ptr;
+    *part = w.ptr + kWsCounterBytes;
+    *bytes = w.ptr ? w.bytes : 0;
+    return 0;
 }
 
 // the reference's kernel choice (cuda.rs:1518-1652): matrix cores for M >= 16 with 16-bit operands
@@ -641,6 +622,19 @@ extern "C" int mynn_dequant_matmul_ws(void *out, const void *act, const int8_t *
         MYNN_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= gemm_weight_bytes(N, K), MYNN_ERR_INVALID,
                      "dequant_matmul: the workspace must hold %zu bytes (mynn_dequant_matmul_workspace_bytes), 16-byte aligned",
                      gemm_weight_bytes(N, K));
+        int kind = 0;
+        if (gemm_tile == 0 && scale && takes_tiles(out, act, wq, M, N, K, act_dtype, out_dtype, &kind)) {
+            const TgPlan plan = tile_gemm_plan(kind, out_dtype, M, N, K, tiles_scratch(kind, N, K));
+            if (tiles_first(plan, kind, M, N, K, out_dtype)) {
+                if (plan.ks > 1) {  // (the caller's memory holds anything)
+                    MYNN_LAUNCH(zero_words_kernel, dim3(kTgCounters / 256), dim3(256), 0, as_stream(s), (uint32_t *)workspace, kTgCounters);
+                    int rc = launch_status("zero_words_kernel");
+                    if (rc) return rc;
+                }
+                return tile_gemm(kind, plan, out, nullptr, act, wq, nullptr, scale, nullptr, M, N, K, out_dtype, GEMM_PLAIN,
+                                 (char *)workspace + kWsCounterBytes, (int *)workspace, as_stream(s));
+            }
+        }
         return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, workspace, gemm_tile, as_stream(s));
     }
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));
@@ -649,12 +643,29 @@ extern "C" int mynn_dequant_matmul_ws(void *out, const void *act, const int8_t *
 extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N,
                                    int K, int act_dtype, int out_dtype, mynn_stream s) {
     MYNN_REQUIRE(M >= 1, MYNN_ERR_INVALID, "dequant_matmul: M=%d", M);
+    int kind = 0;
+    if (scale && takes_tiles(out, act, wq, M, N, K, act_dtype, out_dtype, &kind)) {
+        TgPlan plan = tile_gemm_plan(kind, out_dtype, M, N, K, tiles_scratch(kind, N, K));
+        if (tiles_first(plan, kind, M, N, K, out_dtype)) {
+            void *part = nullptr;
+            int *counters = nullptr;
+            size_t have = 0;
+            if (plan.ks > 1) {
+                int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters, &have);
+                if (rc) return rc;
+                if (have < plan.part_bytes) plan = tile_gemm_plan(kind, out_dtype, M, N, K, have);
+            }
+            return tile_gemm(kind, plan, out, nullptr, act, wq, nullptr, scale, nullptr, M, N, K, out_dtype, GEMM_PLAIN, part, counters, as_stream(s));
+        }
+    }
     if (takes_matrix_cores(act, wq, M, K, act_dtype, out_dtype)) {
         MYNN_REQUIRE(N > 0 && K > 0, MYNN_ERR_INVALID, "dequant_matmul: N=%d K=%d", N, K);
-        void *ws = nullptr;
+        StreamWs ws;
         int rc = stream_workspace(as_stream(s), gemm_weight_bytes(N, K), &ws);
         if (rc) return rc;
-        return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws, 0, as_stream(s));
+        MYNN_REQUIRE(ws.bytes >= gemm_weight_bytes(N, K), MYNN_ERR_STATE, "dequant_matmul: the library workspace cannot grow while the stream is being captured; "
+                                                                          "pass a workspace (mynn_dequant_matmul_ws) or a prepared weight");
+        return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s));
     }
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));
 }

@@ -59,7 +59,7 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
 // matrix-core GEMM pieces.  A dequantised weight is [N, Kp] of the 16-bit type, Kp = K rounded up to 64,
 // zero padded (gemm_weight_bytes); dequant_weight_rows writes one (group/which: see gemm.hip), and
 // gemm_nt_mfma multiplies by it: out = store(act . wt^T) with the store one of GEMM_*.
-enum { GEMM_PLAIN = 0, GEMM_RESIDUAL = 1, GEMM_SWIGLU = 2 };
+enum { GEMM_PLAIN = 0, GEMM_RESIDUAL = 1, GEMM_SWIGLU = 2, GEMM_SWIGLU_PAIRS = 3 };
 size_t gemm_weight_bytes(int N, int K);
 int dequant_weight_rows(void *dst, const int8_t *wq, const void *scale, int N, int K, int dtype, int group, int which,
                         hipStream_t s);
@@ -72,14 +72,34 @@ int interleave_row_groups(void *dst, const void *src, size_t rows, size_t row_by
 // QuantizedMatMul (int8 x int8 -> exact int32 -> two scales) with the large direct-to-LDS tiles of the
 // matrix-core GEMM; res (optional) is added to the rounded result and rounded again
 bool qgemm_dma_supported(int M, int N, int K);
+double qgemm_dma_us(int M, int N, int K);  // its time by measurement, for the choice against tile_gemm
 int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_scale, const int8_t *rhs, const void *rhs_scale,
               const void *res, int M, int N, int K, int dtype, int epi, hipStream_t s);
 // tile: 0 heuristic; 1 = 256x128, 2 = 256x256 (register staged); 3 = 256x256, 4 = 256x320 (direct to LDS)
 int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, int M, int N, int K, int dtype, int epi,
                  hipStream_t s, int tile = 0);
+double gemm_nt_mfma_us(int M, int N, int K, int dtype);  // its time by measurement, for the choice against tile_gemm
 // W_T = T(wq * scale) into `ws` (gemm_weight_bytes), then out = act . W_T^T
 int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
                       int tile, hipStream_t s);
+
+// tile_gemm.hip -- products of ordinary size with operand tiles of 32 .. 128 rows, K ranges where those do not fill the
+// device.  TG_W8 / TG_W8S: 16-bit activations, int8 weights scaled before / after the products; TG_I8: QuantizedMatMul.
+enum { TG_W8 = 0, TG_W8S = 1, TG_I8 = 2 };
+struct TgPlan {
+    int tile = 0, ks = 1;  // which tile, how many K ranges
+    double us = 0;         // the time the choice was made by
+    size_t part_bytes = 0; // partial sums of the ranges
+};
+constexpr int kTgCounters = 4096;             // arrival counters (ints) of a launch, zero between launches
+constexpr size_t kTgScratchMax = 32u << 20;   // no plan needs more partial sums than this
+bool tile_gemm_supported(int kind, int M, int N, int K);
+// the best choice whose partial sums fit scratch_bytes (0: one K range)
+TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes);
+// epi: GEMM_PLAIN, GEMM_RESIDUAL or GEMM_SWIGLU_PAIRS (gate and up rows alternate); part, counters: for plans with ranges
+int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters, size_t *bytes);  // the stream's (gemm.hip)
+int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
+              const void *res, int M, int N, int K, int dtype, int epi, void *part, int *counters, hipStream_t s);
 
 // elementwise.hip
 // device-side loop state of a batch-1 decode model; a null `ids` means "no bookkeeping"

@@ -1,0 +1,480 @@
+// Matrix products of ordinary size: too many activation rows for the kernels that stream the weights past a few rows
+// (gemv.hip, skinny.hip), too few tiles for one round of the 256-row kernel of gemm.hip.
+//
+//   TG_W8   out = act . T(wq * scale)^T   16-bit activations, int8 weights dequantised WITH the scale (one rounding, as the
+//                                         reference's matrix-core path: dequant_matmul_wmma.cuh:65-76)
+//   TG_W8S  out = T((act . wq^T) * scale) the same operands, scale after the f32 sum (fewer than 16 rows: dequant_gemv.cuh:12-59)
+//   TG_I8   out = T((acc * a_scale) * b_scale), acc = int8 x int8 in exact int32 (QuantizedMatMul)
+//
+// The weights are read once per row tile, as the int8 they are stored as: no dequantised copy is written or read (a pass of
+// 3 bytes per weight that cost more than the product itself below a few hundred rows).  Operand tiles go global -> LDS with
+// global_load_lds_dwordx4, NS stages deep: with this few workgroups per CU what bounds the product is the latency of the
+// weight stream, and the stages in flight are what hides it.  A K step is 128 bytes of an activation row (64 values of 16
+// bits, 128 int8).  16-byte chunks are placed so that the 128-bit fragment reads of 16 neighbouring rows fall into
+// different LDS banks: row r's chunk c at 8r + (c ^ (r/2 & 7)) for 128-byte rows, 4r + (c ^ (r/4 & 3)) for the 64-byte
+// rows of int8 weights against 16-bit activations.
+//
+// When the tiles do not fill the device the K range is split over workgroups.  Each leaves its partial sums in scratch
+// memory (agent-scope stores, which go past the XCD's L2) and counts itself in; the last to arrive adds them up in the
+// order of the ranges -- the result does not depend on who was last -- and stores the output.  Nobody waits for anybody.
+#include <type_traits>
+
+#include "gemm_store.h"
+#include "kernels.h"
+#include "mfma.h"
+
+namespace mynn {
+
+typedef int i4x_t __attribute__((ext_vector_type(4)));
+typedef int i16x_t __attribute__((ext_vector_type(16)));
+
+template <int KIND_, int BM_, int BN_, int WM_, int WN_, int NS_, int WPE_>
+struct TgTile {
+    static constexpr int KIND = KIND_, BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, WPE = WPE_;
+    static constexpr int THREADS = WM * WN * 64;
+    static constexpr int TI = BM / WM / 32, TJ = BN / WN / 32;
+    static constexpr int BROW = KIND == TG_I8 ? 128 : 64;  // bytes of a weight row per K step
+    static constexpr int STAGE = BM * 128 + BN * BROW;
+    static constexpr int CHA = BM * 8 / THREADS, CHB = BN * (BROW / 16) / THREADS;  // 16-byte chunks per thread
+    static constexpr int EST = BN / WN + 8;                                         // store staging row stride
+    static constexpr int STORE = WM * WN * 32 * EST * 2;
+    static constexpr int LDS = NS * STAGE > STORE + BN * 4 ? NS * STAGE : STORE + BN * 4;  // (column scales above the staging)
+    static_assert(BM * 8 % THREADS == 0 && BN * (BROW / 16) % THREADS == 0, "whole load instructions per wave");
+};
+
+__device__ U4 g_tg_zero;  // what the chunks past the end of a row are read from
+
+template <typename T> __device__ inline U4 scale_operand(const U4 &v, float sc);
+template <> __device__ inline U4 scale_operand<f16_t>(const U4 &v, float sc) {
+    // |w| <= 128 times a 16-bit scale is exact in f32, so this product's one rounding is the rounding of T(w * scale)
+    const h2_t s2 = {(_Float16)sc, (_Float16)sc};
+    auto m = [&](uint32_t x) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, x) * s2); };
+    return U4{m(v.x), m(v.y), m(v.z), m(v.w)};
+}
+template <> __device__ inline U4 scale_operand<bf16_t>(const U4 &v, float sc) { return v; }  // (see weight_operand)
+
+// 8 int8 weights -> an MFMA operand, scaled or not
+template <typename T, bool SCALED> __device__ inline U4 weight_operand(uint32_t w0, uint32_t w1, float sc) {
+    if constexpr (!SCALED) return i8x8_to_operand<T>(w0, w1);
+    else if constexpr (std::is_same<T, f16_t>::value) return scale_operand<T>(i8x8_to_operand<T>(w0, w1), sc);
+    else {
+        auto two = [&](uint32_t w, int sh) {
+            return pack2<T>((float)(int8_t)((w >> sh) & 0xFF) * sc, (float)(int8_t)((w >> (sh + 8)) & 0xFF) * sc);
+        };
+        return U4{two(w0, 0), two(w0, 16), two(w1, 0), two(w1, 16)};
+    }
+}
+
+// TAIL: the rows are not whole K steps, the last one reads zeros past their end
+template <typename T, typename G, int EPI, bool TAIL>
+__global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const void *A_, const int8_t *B, int M, int N, int K, int ks, T *C,
+                                                                      const T *R, const T *a_scale, const T *b_scale,
+                                                                      uint64_t *part, int *counter, int32_t *acc_out) {
+    constexpr int KIND = G::KIND, BM = G::BM, BN = G::BN, TI = G::TI, TJ = G::TJ, NS = G::NS, BROW = G::BROW;
+    constexpr bool I8 = KIND == TG_I8;
+    constexpr int EA = I8 ? 1 : 2;
+    constexpr int CHA = G::CHA, CHB = G::CHB;
+    extern __shared__ __align__(16) char lds[];
+    const char *A = (const char *)A_;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / G::WN, wn = wave % G::WN;
+    const int wrow = wm * TI * 32, wcol = wn * TJ * 32;
+
+    // Workgroup -> (row tile, K range, column tile).  Consecutive ids go round-robin over the 8 XCDs, so an id is first
+    // turned into an index that is contiguous inside an XCD; there the row tiles of a band share the weight tile they
+    // multiply by, then come the K ranges, then the columns.
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    int tm, tn, kz;
+    {
+        constexpr int XCD = 8, BAND = 8;
+        const int nb = gridDim.x, x = blockIdx.x % XCD, per = nb / XCD, rem = nb % XCD;
+        const int l = x * per + min(x, rem) + blockIdx.x / XCD;
+        const int band = l / (BAND * tiles_n * ks), in_band = l - band * BAND * tiles_n * ks;
+        const int rows_here = min(BAND, tiles_m - band * BAND);
+        tm = band * BAND + in_band % rows_here;
+        const int rest = in_band / rows_here;
+        kz = rest % ks;
+        tn = rest / ks;
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int a_bytes = K * EA;                    // bytes of an activation row; a weight row is K bytes
+    const int iters = (a_bytes + 127) / 128;
+    const int it0 = (int)((long)iters * kz / ks), it1 = (int)((long)iters * (kz + 1) / ks);
+    const int n_it = it1 - it0;
+
+    // this lane's chunks of each operand tile: LDS position P = (CH * wave + i) * 64 + lane.  Offsets are from the tile's
+    // first row, so that a step's address is a scalar base plus a 32-bit lane offset.
+    uint32_t aoff[CHA], boff[CHB];
+#pragma unroll
+    for (int i = 0; i < CHA; i++) {
+        const int P = (CHA * wave + i) * 64 + lane, r = P >> 3;
+        aoff[i] = (uint32_t)(min(r, M - 1 - m0) * a_bytes + ((P & 7) ^ ((r >> 1) & 7)) * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < CHB; i++) {
+        const int P = (CHB * wave + i) * 64 + lane;
+        const int r = BROW == 128 ? P >> 3 : P >> 2;
+        boff[i] = (uint32_t)(min(r, N - 1 - n0) * K + (BROW == 128 ? (P & 7) ^ ((r >> 1) & 7) : (P & 3) ^ ((r >> 2) & 3)) * 16);
+    }
+    const char *a_tile = A + (size_t)m0 * a_bytes, *b_tile = (const char *)B + (size_t)n0 * K;
+    auto dma = [&](const char *src, char *dst) {  // (dst is wave-uniform; the lane's 16 bytes are implicit)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src, (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+    };
+    auto issue = [&](int it, char *st) {
+        it = it0 + min(it, n_it - 1);  // (past the range: a repeat of the last step, never read; it keeps the counts)
+        const char *ab = a_tile + (size_t)it * 128, *bb = b_tile + (size_t)it * BROW;
+        char *ad = st + CHA * wave * 1024, *bd = st + BM * 128 + CHB * wave * 1024;
+        const char *zero = (const char *)&g_tg_zero;
+#pragma unroll
+        for (int i = 0; i < CHA; i++) {
+            const char *p = ab + aoff[i];
+            const int P = (CHA * wave + i) * 64 + lane;
+            if (TAIL && it * 128 + ((P & 7) ^ ((P >> 4) & 7)) * 16 >= a_bytes) p = zero;
+            dma(p, ad + i * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < CHB; i++) {
+            const char *p = bb + boff[i];
+            const int P = (CHB * wave + i) * 64 + lane, c = BROW == 128 ? (P & 7) ^ ((P >> 4) & 7) : (P & 3) ^ ((P >> 4) & 3);
+            if (TAIL && it * BROW + c * 16 >= K) p = zero;
+            dma(p, bd + i * 1024);
+        }
+    };
+
+    using acc_t = std::conditional_t<I8, i16x_t, f16x_t>;
+    using sum_t = std::conditional_t<I8, int32_t, float>;
+    acc_t acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
+
+    // fragment reads: lane l takes row l % 32 of a 32-row tile, and its half g = l / 32 one of two 16-byte chunks
+    const int fr = lane & 31, g = lane >> 5;
+    int abase[TI], aswz[TI], bbase[TJ], bswz[TJ];
+    float wsc[TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++) {
+        const int r = wrow + i * 32 + fr;
+        abase[i] = 128 * r;
+        aswz[i] = (r >> 1) & 7;
+    }
+#pragma unroll
+    for (int j = 0; j < TJ; j++) {
+        const int r = wcol + j * 32 + fr;
+        bbase[j] = BM * 128 + BROW * r;
+        bswz[j] = BROW == 128 ? (r >> 1) & 7 : (r >> 2) & 3;
+        wsc[j] = KIND == TG_W8 ? Elem<T>::ld(b_scale, min(n0 + r, N - 1)) : 0.f;
+    }
+    // The fragments of one K step: MFMA step s takes chunk 2s + g of the activation row and, of 16-bit kinds, the 8 weights
+    // at the same k, half of chunk s -- the order of the 256-row kernel of gemm.hip, so that with one K range a row's sums
+    // are the same bits whichever of the two kernels its number of neighbours selects.
+    using w_t = std::conditional_t<I8, U4, uint2>;
+    struct Frags {
+        w_t w[4][TJ];
+        U4 a[4][TI];
+    };
+    auto read = [&](const char *st, Frags &f) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+                f.w[s][j] = *(const w_t *)(st + bbase[j] + (((I8 ? 2 * s + g : s) ^ bswz[j]) << 4) + (I8 ? 0 : 8 * g));
+#pragma unroll
+            for (int i = 0; i < TI; i++) f.a[s][i] = *(const U4 *)(st + abase[i] + (((2 * s + g) ^ aswz[i]) << 4));
+        }
+    };
+    auto multiply = [&](const Frags &f) {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+                U4 fb;
+                if constexpr (I8) fb = f.w[s][j];
+                else fb = weight_operand<T, KIND == TG_W8>(f.w[s][j].x, f.w[s][j].y, wsc[j]);
+#pragma unroll
+                for (int i = 0; i < TI; i++) {
+                    if constexpr (I8)
+                        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i4x_t, fb), __builtin_bit_cast(i4x_t, f.a[s][i]), acc[i][j], 0, 0, 0);
+                    else acc[i][j] = Mfma<T>::run(fb, f.a[s][i], acc[i][j]);
+                }
+            }
+    };
+
+    // One barrier per K step: behind it the tile of this step is whole (every wave has waited for its own share of the
+    // loads) and the stage of the step before is free.  The fragments of a step are read while the step before multiplies,
+    // so that neither the barrier nor the LDS latency is in front of the MFMAs.
+#pragma unroll
+    for (int s = 0; s < NS - 1; s++) issue(s, lds + s * G::STAGE);
+    int cur = 0, fill = NS - 1, it = 0;
+    auto fetch = [&](Frags &f) {
+        constexpr int VM = (NS - 2) * (CHA + CHB);  // loads that may stay in flight: those of the later stages
+        static_assert(VM < 64, "a counter of six bits");
+        __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 0x70);  // vmcnt(VM) lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read(lds + cur * G::STAGE, f);
+        issue(it + NS - 1, lds + fill * G::STAGE);
+        cur = cur + 1 == NS ? 0 : cur + 1;
+        fill = fill + 1 == NS ? 0 : fill + 1;
+        ++it;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Frags f0, f1;
+    fetch(f0);
+    while (it + 1 < n_it) {
+        fetch(f1);
+        multiply(f0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(f0);
+        multiply(f1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (it < n_it) {
+        fetch(f1);
+        multiply(f0);
+        multiply(f1);
+    } else multiply(f0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeats of the last step too, before LDS is reused
+    __syncthreads();
+
+    if (ks > 1) {
+        // partial sums, two per word, [range][(i, j), pair][thread]
+        const size_t tile = (size_t)tn * tiles_m + tm;
+        constexpr int WORDS = TI * TJ * 8;
+        uint64_t *p0 = part + tile * ks * (WORDS * G::THREADS) + tid;
+        uint64_t *mine = p0 + (size_t)kz * (WORDS * G::THREADS);
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const sum_t lo = acc[i][j][2 * e], hi = acc[i][j][2 * e + 1];
+                    const uint64_t v = (uint64_t)__builtin_bit_cast(uint32_t, lo) | ((uint64_t)__builtin_bit_cast(uint32_t, hi) << 32);
+                    __hip_atomic_store(mine + ((i * TJ + j) * 8 + e) * G::THREADS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // written through before this workgroup counts itself in
+        __syncthreads();
+        int *flag = (int *)lds;
+        if (tid == 0) {
+            const int before = __hip_atomic_fetch_add(counter + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (before == ks - 1) __hip_atomic_store(counter + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+            *flag = before;
+        }
+        __syncthreads();
+        const bool last = *flag == ks - 1;
+        __syncthreads();
+        if (!last) return;
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+                uint64_t v[8];
+                auto fetch = [&](int s) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        v[e] = __hip_atomic_load(p0 + (size_t)s * (WORDS * G::THREADS) + ((i * TJ + j) * 8 + e) * G::THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                };
+                fetch(0);
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    acc[i][j][2 * e] = __builtin_bit_cast(sum_t, (uint32_t)v[e]);
+                    acc[i][j][2 * e + 1] = __builtin_bit_cast(sum_t, (uint32_t)(v[e] >> 32));
+                }
+                for (int s = 1; s < ks; s++) {
+                    fetch(s);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        acc[i][j][2 * e] += __builtin_bit_cast(sum_t, (uint32_t)v[e]);
+                        acc[i][j][2 * e + 1] += __builtin_bit_cast(sum_t, (uint32_t)(v[e] >> 32));
+                    }
+                }
+            }
+    }
+
+    if constexpr (I8) {
+        constexpr bool F32 = sizeof(T) == 4;  // (f32 scales and output: stored as they lie, like the integer sums)
+        if (acc_out || F32) {
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < TJ; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        const int row = m0 + wrow + i * 32 + fr, col = n0 + wcol + j * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
+                        if (row >= M || col >= N) continue;
+                        if (acc_out) acc_out[(size_t)row * N + col] = acc[i][j][e];
+                        if (F32 && C) Elem<T>::st(C, (size_t)row * N + col, ((float)acc[i][j][e] * Elem<T>::ld(a_scale, row)) * Elem<T>::ld(b_scale, col));
+                    }
+        }
+        if (F32 || !C) return;
+    }
+    if constexpr (sizeof(T) == 4) {
+    } else if constexpr (KIND == TG_W8) {
+        gemm_store<T, G, EPI>([&](int i, int j, int e) { return acc[i][j][e]; }, (uint16_t *)lds, C, R, M, N, m0, n0, wrow, wcol, lane, wave);
+    } else {
+        // the column scales of the tile as f32 in LDS above the store's patches, the row scales in registers
+        float *bs = (float *)(lds + G::STORE);
+        for (int c = tid; c < BN; c += G::THREADS) bs[c] = n0 + c < N ? Elem<T>::ld(b_scale, n0 + c) : 0.f;
+        float asc[TI];
+#pragma unroll
+        for (int i = 0; i < TI; i++) asc[i] = I8 ? Elem<T>::ld(a_scale, min(m0 + wrow + i * 32 + fr, M - 1)) : 1.f;
+        __syncthreads();
+        const float *bw = bs + wcol + 4 * g;
+        gemm_store<T, G, EPI>(
+            [&](int i, int j, int e) {
+                const float b = bw[j * 32 + 8 * (e >> 2) + (e & 3)];
+                if constexpr (I8) return ((float)acc[i][j][e] * asc[i]) * b;
+                else return acc[i][j][e] * b;
+            },
+            (uint16_t *)lds, C, R, M, N, m0, n0, wrow, wcol, lane, wave);
+    }
+}
+
+// ---- which tile, and over how many K ranges.
+// The time of a launch, in microseconds, as measured over some 300 shapes (16 <= M <= 4096, the linear layers of the
+// benchmark's models and others; every tile at 1 .. 12 ranges) and fitted per tile:
+//
+//   t = launch + steps per range * (a * rounds + b * workgroups on the fullest CU) + e * ranges + partial sums at 4 TB/s
+//
+// a: what a step costs a CU however few workgroups it holds (latency); b: what each resident workgroup adds (LDS, MFMA and
+// dequantisation work); rounds: how often a CU takes a new set of workgroups.  Never less than the weights' bytes at 4.6
+// TB/s.  Choosing by it is within 2 % of the best choice on average, 14 % at worst.  (Two fits where the conversion of the
+// weights costs differ: it is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
+struct TgCost {
+    int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
+    float launch[2], a[2], b[2], e[2];  // [0] fp16, [1] bf16
+};
+// (the order of the tiles in tg_launch)
+constexpr TgCost kTgW8[] = {
+    {32, 64, 3, {3.52f, 4.76f}, {0.327f, 0.289f}, {0.057f, 0.071f}, {0.41f, 0.23f}},
+    {32, 128, 3, {3.57f, 4.35f}, {0.259f, 0.233f}, {0.134f, 0.148f}, {0.61f, 0.41f}},
+    {64, 64, 2, {3.70f, 4.68f}, {0.283f, 0.233f}, {0.098f, 0.127f}, {0.58f, 0.43f}},
+    {64, 128, 2, {3.80f, 5.01f}, {0.290f, 0.285f}, {0.155f, 0.151f}, {0.97f, 0.76f}},
+    {128, 128, 1, {4.88f, 6.67f}, {0.314f, 0.316f}, {0.268f, 0.271f}, {0.92f, 0.65f}},
+    {128, 128, 2, {3.99f, 5.37f}, {0.337f, 0.389f}, {0.249f, 0.275f}, {1.68f, 1.49f}},
+};
+constexpr TgCost kTgW8S[] = {
+    {32, 32, 3, {2.42f, 2.26f}, {0.300f, 0.350f}, {0.049f, 0.024f}, {0.65f, 0.71f}},
+    {32, 64, 3, {2.26f, 2.02f}, {0.266f, 0.320f}, {0.101f, 0.067f}, {0.68f, 0.73f}},
+    {32, 128, 3, {1.92f, 1.71f}, {0.229f, 0.245f}, {0.177f, 0.166f}, {1.00f, 1.05f}},
+};
+constexpr TgCost kTgI8[] = {
+    {32, 64, 2, {3.29f, 3.29f}, {0.060f, 0.060f}, {0.150f, 0.150f}, {0.65f, 0.65f}},
+    {64, 64, 1, {2.82f, 2.82f}, {0.166f, 0.166f}, {0.116f, 0.116f}, {1.00f, 1.00f}},
+    {64, 128, 2, {3.34f, 3.34f}, {0.093f, 0.093f}, {0.293f, 0.293f}, {0.74f, 0.74f}},
+    {128, 128, 1, {4.36f, 4.36f}, {0.292f, 0.292f}, {0.246f, 0.246f}, {1.94f, 1.94f}},
+    {128, 128, 2, {2.59f, 2.59f}, {0.650f, 0.650f}, {0.125f, 0.125f}, {1.97f, 1.97f}},
+    {128, 256, 1, {6.10f, 6.10f}, {0.441f, 0.441f}, {0.400f, 0.400f}, {1.84f, 1.84f}},
+};
+
+bool tile_gemm_supported(int kind, int M, int N, int K) {
+    return M >= 1 && N >= 1 && K >= 16 && K % (kind == TG_I8 ? 32 : 16) == 0 && (long)K * 256 * 2 < (1l << 31);
+}
+
+TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes) {
+    const TgCost *tab = kind == TG_W8 ? kTgW8 : kind == TG_W8S ? kTgW8S : kTgI8;
+    const int n_tiles = kind == TG_W8S ? 3 : 6, d = dtype == MYNN_BF16 ? 1 : 0;
+    const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
+    const double weights_us = (double)N * K / 4.6e6;
+    TgPlan best;
+    best.us = 1e30;
+    for (int t = 0; t < n_tiles; t++) {
+        const TgCost &c = tab[t];
+        const long tiles = (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+        for (int ks = 1; ks <= 16; ks += ks < 4 ? 1 : ks < 8 ? 2 : 4) {
+            const size_t part = ks > 1 ? (size_t)tiles * ks * c.bm * c.bn * 4 : 0;
+            // (a range is at least three steps, from 256 rows on 2048 values: shorter ranges did not win there, and so a
+            // block of rows has the same sums whatever it is multiplied with when K < 4096; a launch that already has four workgroups per CU gains nothing by ranges)
+            if (ks > 1 && (ks * (M >= 256 && kind != TG_I8 ? 32 : 3) > iters || tiles * ks > 1024 || tiles > kTgCounters || part > scratch_bytes)) continue;
+            const long wgs = (tiles * ks + 255) / 256, rounds = (wgs + c.per_cu - 1) / c.per_cu;
+            const double steps = (double)((iters + ks - 1) / ks) * (c.a[d] * rounds + c.b[d] * wgs);
+            const double us = c.launch[d] + (steps + (ks > 1 ? c.e[d] * ks + part * 2e-6 / 4.0 : 0.0) > weights_us ? steps + (ks > 1 ? c.e[d] * ks + part * 2e-6 / 4.0 : 0.0) : weights_us);
+            if (us < best.us) best = TgPlan{t, ks, us, part};
+        }
+    }
+    return best;
+}
+
+struct TgArgs {
+    void *out;
+    int32_t *acc_out;
+    const void *act;
+    const int8_t *wq;
+    const void *a_scale, *w_scale, *res;
+    int M, N, K, ks;
+    uint64_t *part;
+    int *counters;
+    hipStream_t s;
+};
+
+template <typename T, typename G, int EPI, bool TAIL> static int tg_go(const TgArgs &p) {
+    static bool lds_set = false;
+    if (!lds_set && G::LDS > 64 * 1024) {
+        MYNN_HIP(hipFuncSetAttribute((const void *)tile_gemm_kernel<T, G, EPI, TAIL>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
+        lds_set = true;
+    }
+    const int tiles = ((p.M + G::BM - 1) / G::BM) * ((p.N + G::BN - 1) / G::BN);
+    MYNN_LAUNCH((tile_gemm_kernel<T, G, EPI, TAIL>), dim3(tiles * p.ks), dim3(G::THREADS), G::LDS, p.s, p.act, p.wq, p.M, p.N, p.K, p.ks, (T *)p.out,
+                (const T *)p.res, (const T *)p.a_scale, (const T *)p.w_scale, p.part, p.counters, p.acc_out);
+    return launch_status("tile_gemm_kernel");
+}
+template <typename T, typename G> static int tg_epi(const TgArgs &p, int epi) {
+    const bool tail = (size_t)p.K * (G::KIND == TG_I8 ? 1 : 2) % 128 != 0;
+    if constexpr (G::KIND == TG_W8S || sizeof(T) == 4)
+        return tail ? tg_go<T, G, GEMM_PLAIN, true>(p) : tg_go<T, G, GEMM_PLAIN, false>(p);
+    else {
+        if (epi == GEMM_RESIDUAL) return tail ? tg_go<T, G, GEMM_RESIDUAL, true>(p) : tg_go<T, G, GEMM_RESIDUAL, false>(p);
+        if (epi == GEMM_SWIGLU_PAIRS) return tail ? tg_go<T, G, GEMM_SWIGLU_PAIRS, true>(p) : tg_go<T, G, GEMM_SWIGLU_PAIRS, false>(p);
+        return tail ? tg_go<T, G, GEMM_PLAIN, true>(p) : tg_go<T, G, GEMM_PLAIN, false>(p);
+    }
+}
+template <typename T> static int tg_launch(int kind, int tile, const TgArgs &p, int epi) {
+    if constexpr (sizeof(T) == 2) {
+        if (kind == TG_W8) {
+            if (tile == 0) return tg_epi<T, TgTile<TG_W8, 32, 64, 1, 2, 6, 2>>(p, epi);
+            if (tile == 1) return tg_epi<T, TgTile<TG_W8, 32, 128, 1, 4, 4, 2>>(p, epi);
+            if (tile == 2) return tg_epi<T, TgTile<TG_W8, 64, 64, 2, 2, 6, 2>>(p, epi);
+            if (tile == 3) return tg_epi<T, TgTile<TG_W8, 64, 128, 1, 4, 4, 2>>(p, epi);
+            if (tile == 4) return tg_epi<T, TgTile<TG_W8, 128, 128, 2, 4, 6, 2>>(p, epi);
+            // fp16: every weight is converted by one wave only (128 x 32 per wave); bf16: that form spills, 64 x 64 per wave
+            if constexpr (std::is_same<T, f16_t>::value) return tg_epi<T, TgTile<TG_W8, 128, 128, 1, 4, 3, 2>>(p, epi);
+            else return tg_epi<T, TgTile<TG_W8, 128, 128, 2, 2, 3, 2>>(p, epi);
+        }
+        if (kind == TG_W8S) {
+            if (tile == 0) return tg_epi<T, TgTile<TG_W8S, 32, 32, 1, 1, 8, 1>>(p, epi);
+            if (tile == 1) return tg_epi<T, TgTile<TG_W8S, 32, 64, 1, 2, 6, 2>>(p, epi);
+            return tg_epi<T, TgTile<TG_W8S, 32, 128, 1, 4, 4, 2>>(p, epi);
+        }
+    }
+    if (tile == 0) return tg_epi<T, TgTile<TG_I8, 32, 64, 1, 2, 6, 1>>(p, epi);
+    if (tile == 1) return tg_epi<T, TgTile<TG_I8, 64, 64, 2, 2, 6, 2>>(p, epi);
+    if (tile == 2) return tg_epi<T, TgTile<TG_I8, 64, 128, 2, 4, 3, 2>>(p, epi);
+    if (tile == 3) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 4, 1>>(p, epi);
+    if (tile == 4) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 2, 2>>(p, epi);
+    return tg_epi<T, TgTile<TG_I8, 128, 256, 2, 4, 3, 2>>(p, epi);
+}
+
+int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
+              const void *res, int M, int N, int K, int dtype, int epi, void *part, int *counters, hipStream_t s) {
+    MYNN_REQUIRE((out || acc_out) && act && wq && (w_scale || !out) && (kind != TG_I8 || a_scale || !out), MYNN_ERR_INVALID, "tile_gemm: null operand");
+    MYNN_REQUIRE(tile_gemm_supported(kind, M, N, K), MYNN_ERR_UNSUPPORTED, "tile_gemm: M=%d N=%d K=%d", M, N, K);
+    MYNN_REQUIRE(aligned16(act) && aligned16(wq), MYNN_ERR_INVALID, "tile_gemm: operands must be 16-byte aligned");
+    MYNN_REQUIRE(!out || (aligned16(out) && (!res || aligned16(res))), MYNN_ERR_INVALID, "tile_gemm: output and residual must be 16-byte aligned");
+    MYNN_REQUIRE(epi != GEMM_RESIDUAL || res, MYNN_ERR_INVALID, "tile_gemm: residual store without a residual");
+    MYNN_REQUIRE(epi != GEMM_SWIGLU_PAIRS || (N % 2 == 0 && !acc_out), MYNN_ERR_INVALID, "tile_gemm: SwiGLU store needs row pairs, N=%d", N);
+    MYNN_REQUIRE(epi != GEMM_SWIGLU && (kind != TG_W8S || epi == GEMM_PLAIN), MYNN_ERR_INVALID, "tile_gemm: store %d", epi);
+    MYNN_REQUIRE(plan.ks >= 1 && (plan.ks == 1 || (part && counters && aligned16(part))), MYNN_ERR_INVALID, "tile_gemm: K ranges without scratch memory");
+    const TgArgs p{out, acc_out, act, wq, a_scale, w_scale, res, M, N, K, plan.ks, (uint64_t *)part, counters, s};
+    MYNN_REQUIRE(dtype != MYNN_F32 || (kind == TG_I8 && epi == GEMM_PLAIN), MYNN_ERR_UNSUPPORTED, "tile_gemm: f32 output of int8 products only");
+    return dispatch_dtype(dtype, [&](auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        return tg_launch<T>(kind, plan.tile, p, epi);
+    });
+}
+
+}  // namespace mynn
