@@ -80,6 +80,13 @@ struct Lin {
     int N = 0, K = 0;
 };
 
+// How an executor multiplies by one of its linears: tile_gemm from the int8 weights, or the 256-row kernels of gemm.hip
+// (which read a resident 16-bit copy, and of an int8 gate/up pair an interleaved copy)
+struct LinPlan {
+    bool tile = false;
+    TgPlan plan;
+};
+
 struct Layer {
     const void *norm1 = nullptr, *norm2 = nullptr;
     Lin qkv, o, gate, up, gu, down;  // qkv = rows of q,k,v concatenated; gu = gate/up rows interleaved
@@ -163,7 +170,10 @@ struct Model {
     WeightSet *wset = nullptr;  // the derived weight copies (shared with the session's other executors)
     bool w8a8_fused = false;  // W8A8 with the large int8 tiles: norm+quantise, residual and SwiGLU ride on the launches
     bool qgemv1 = false;      // W8A8 at batch 1: norm, quantiser, int8 GEMV and residual / SwiGLU of a linear in one launch
-    bool resident16 = false;  // the wt_* copies exist and the matrix-core path with fused stores is used
+    bool resident16 = false;  // the matrix-core path with fused stores: tiles of the int8 weights or the wt_* copies, by plan
+    LinPlan pl_qkv, pl_o, pl_gu, pl_down, pl_lm;
+    void *tg_part = nullptr;     // tile_gemm's partial sums and arrival counters
+    int *tg_counters = nullptr;
     bool skinny = false;      // 16..64 rows: int8 weights streamed once through the few-row matrix-core kernel
     float *skinny_scratch = nullptr;
     void *cos_t = nullptr, *sin_t = nullptr;
@@ -256,10 +266,16 @@ static void note(Model &m, const char *name, double bytes, double flops = 0.0) {
         if (rc__) return rc__; \
     } while (0)
 
-// one matrix-core GEMM against a resident dequantised weight
-static int gemm_rows(Model &m, void *out, const void *act, const void *wt, const void *res, int M, int N, int K, int epi,
+// one matrix-core GEMM: from the int8 weights, or against a resident dequantised copy, as planned
+static int gemm_rows(Model &m, const LinPlan &pl, void *out, const void *act, const Lin &l, const void *wt, const void *res, int M, int epi,
                      const char *name) {
+    const int N = l.N, K = l.K;
     const double eb = 2.0, n_out = epi == GEMM_SWIGLU ? N / 2 : N;
+    if (pl.tile) {
+        note(m, name, (double)N * K + N * eb + ((double)M * K + (double)M * n_out * (epi == GEMM_RESIDUAL ? 2 : 1)) * eb, 2.0 * M * N * K);
+        return tile_gemm(TG_W8, pl.plan, out, nullptr, act, (const int8_t *)l.w, nullptr, l.scale, res, M, N, K, m.cfg.dtype,
+                         epi == GEMM_SWIGLU ? GEMM_SWIGLU_PAIRS : epi, m.tg_part, m.tg_counters, m.stream);
+    }
     note(m, name, ((double)N * K + (double)M * K + (double)M * n_out * (epi == GEMM_RESIDUAL ? 2 : 1)) * eb, 2.0 * M * N * K);
     return gemm_nt_mfma(out, act, wt, res, M, N, K, m.cfg.dtype, epi, m.stream, m.cfg.gemm_tile);
 }
@@ -312,10 +328,11 @@ static int linear_w8a8(Model &m, void *out, const void *act, const Lin &l, int M
                                  m.stream);
 }
 
-// W8A8 with the large int8 tiles: (RMSNorm +) per-row quantisation of the input, then the product with the
+// W8A8 on the matrix cores: (RMSNorm +) per-row quantisation of the input, then the product with the
 // store that the layer needs (plain, + residual, SwiGLU over interleaved gate/up rows)
-static int qlinear_fused(Model &m, void *out, const void *act, const void *norm_w, const void *w, const void *scale, const void *res,
-                         int M, int N, int K, int epi, const char *name) {
+static int qlinear_fused(Model &m, const LinPlan &pl, void *out, const void *act, const void *norm_w, const Lin &l, const void *res, int M,
+                         int epi, const char *name, const void *w32 = nullptr, const void *scale32 = nullptr) {
+    const int N = l.N, K = l.K;
     const double eb = dtype_size(m.cfg.dtype);
     if (norm_w) {
         note(m, "rms_norm_quantize", (double)M * K * (eb + 1) + M * eb + K * eb);
@@ -326,7 +343,12 @@ static int qlinear_fused(Model &m, void *out, const void *act, const void *norm_
     }
     const int n_out = epi == GEMM_SWIGLU ? N / 2 : N;
     note(m, name, (double)N * K + (double)M * K + N * eb + (double)M * n_out * eb * (res ? 2 : 1), 2.0 * M * N * K);
-    return qgemm_dma(out, nullptr, m.a8, m.a8_scale, (const int8_t *)w, scale, res, M, N, K, m.cfg.dtype, epi, m.stream);
+    if (pl.tile)
+        return tile_gemm(TG_I8, pl.plan, out, nullptr, m.a8, (const int8_t *)l.w, m.a8_scale, l.scale, res, M, N, K, m.cfg.dtype,
+                         epi == GEMM_SWIGLU ? GEMM_SWIGLU_PAIRS : epi, m.tg_part, m.tg_counters, m.stream);
+    // (w32, scale32: the rows of gate and up in groups of 32, as the large tiles' SwiGLU store wants them)
+    return qgemm_dma(out, nullptr, m.a8, m.a8_scale, (const int8_t *)(w32 ? w32 : l.w), scale32 ? scale32 : l.scale, res, M, N, K, m.cfg.dtype, epi,
+                     m.stream);
 }
 
 // The attention block of the streaming-KV graph, op for op (decoder.rs:281-347, 472-487): RoPE(q); k and v un-rotated
@@ -438,7 +460,7 @@ static int enqueue_step(Model &m) {
         } else if (qfused) {
             TRY(qlinear1(m.qkv, m.x, L.norm1, L.qkv, nullptr, GEMM_PLAIN, "qgemv_norm_quant_qkv"));
         } else if (m.w8a8_fused) {
-            TRY(qlinear_fused(m, m.qkv, m.x, L.norm1, L.qkv.w, L.qkv.scale, nullptr, rows, L.qkv.N, H, GEMM_PLAIN, "qlinear_qkv"));
+            TRY(qlinear_fused(m, m.pl_qkv, m.qkv, m.x, L.norm1, L.qkv, nullptr, rows, GEMM_PLAIN, "qlinear_qkv"));
         } else {
             if (!nrm_ready) {
                 note(m, "rms_norm", 2.0 * rows * H * eb + H * eb);
@@ -453,7 +475,7 @@ static int enqueue_step(Model &m) {
                                 (kv8 && D != 64 && D != 128) || streaming || L.qkv_b || c.unfused_decode ? nullptr : &rp, &roped));
             }
             else if (w8a8) TRY(linear_w8a8(m, m.qkv, m.nrm, L.qkv, rows, true, "qlinear_qkv"));
-            else if (m.resident16) TRY(gemm_rows(m, m.qkv, m.nrm, L.wt_qkv, nullptr, rows, L.qkv.N, H, GEMM_PLAIN, "linear_qkv"));
+            else if (m.resident16) TRY(gemm_rows(m, m.pl_qkv, m.qkv, m.nrm, L.qkv, L.wt_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv"));
             else TRY(linear_rows<T>(m, m.qkv, m.nrm, L.qkv, rows, "linear_qkv"));
         }
         if (L.qkv_b) {
@@ -535,9 +557,9 @@ static int enqueue_step(Model &m) {
             TRY(qlinear1(m.hmid, m.x2, L.norm2, L.gu, nullptr, GEMM_SWIGLU, "qgemv_norm_quant_gateup_swiglu"));
             TRY(qlinear1(m.x, m.hmid, nullptr, L.down, m.x2, GEMM_RESIDUAL, "qgemv_quant_down_residual"));
         } else if (m.w8a8_fused) {
-            TRY(qlinear_fused(m, m.x2, m.attn, nullptr, L.o.w, L.o.scale, m.x, rows, H, QD, GEMM_RESIDUAL, "qlinear_o_residual"));
-            TRY(qlinear_fused(m, m.hmid, m.x2, L.norm2, L.q8_gu, L.q8_gu_scale, nullptr, rows, 2 * F, H, GEMM_SWIGLU, "qlinear_gateup_swiglu"));
-            TRY(qlinear_fused(m, m.x, m.hmid, nullptr, L.down.w, L.down.scale, m.x2, rows, H, F, GEMM_RESIDUAL, "qlinear_down_residual"));
+            TRY(qlinear_fused(m, m.pl_o, m.x2, m.attn, nullptr, L.o, m.x, rows, GEMM_RESIDUAL, "qlinear_o_residual"));
+            TRY(qlinear_fused(m, m.pl_gu, m.hmid, m.x2, L.norm2, L.gu, nullptr, rows, GEMM_SWIGLU, "qlinear_gateup_swiglu", L.q8_gu, L.q8_gu_scale));
+            TRY(qlinear_fused(m, m.pl_down, m.x, m.hmid, nullptr, L.down, m.x2, rows, GEMM_RESIDUAL, "qlinear_down_residual"));
         } else if (w8a8) {
             TRY(linear_w8a8(m, m.proj, m.attn, L.o, rows, true, "qlinear_o"));
             note(m, "add", 3.0 * rows * H * eb);
@@ -553,11 +575,11 @@ static int enqueue_step(Model &m) {
             TRY(mynn_add(m.x, m.x2, m.proj, (size_t)rows * H, c.dtype, s));
         } else if (m.resident16) {
             // residual adds and SwiGLU ride on the GEMM stores
-            TRY(gemm_rows(m, m.x2, m.attn, L.wt_o, m.x, rows, H, QD, GEMM_RESIDUAL, "linear_o_residual"));
+            TRY(gemm_rows(m, m.pl_o, m.x2, m.attn, L.o, L.wt_o, m.x, rows, GEMM_RESIDUAL, "linear_o_residual"));
             note(m, "rms_norm", 2.0 * rows * H * eb + H * eb);
             TRY(mynn_rms_norm(m.nrm, m.x2, L.norm2, rows, H, c.eps, c.dtype, s));
-            TRY(gemm_rows(m, m.hmid, m.nrm, L.wt_gu, nullptr, rows, 2 * F, H, GEMM_SWIGLU, "linear_gateup_swiglu"));
-            TRY(gemm_rows(m, m.x, m.hmid, L.wt_down, m.x2, rows, H, F, GEMM_RESIDUAL, "linear_down_residual"));
+            TRY(gemm_rows(m, m.pl_gu, m.hmid, m.nrm, L.gu, L.wt_gu, nullptr, rows, GEMM_SWIGLU, "linear_gateup_swiglu"));
+            TRY(gemm_rows(m, m.pl_down, m.x, m.hmid, L.down, L.wt_down, m.x2, rows, GEMM_RESIDUAL, "linear_down_residual"));
         } else {
             TRY(linear_rows<T>(m, m.proj, m.attn, L.o, rows, "linear_o"));
             note(m, "add", 3.0 * rows * H * eb);
@@ -587,7 +609,7 @@ static int enqueue_step(Model &m) {
     } else if (qfused) {
         TRY(qlinear1(m.logits, m.x, m.final_norm, m.lm_head, nullptr, GEMM_PLAIN, "qgemv_norm_quant_lm_head"));
     } else if (m.w8a8_fused) {
-        TRY(qlinear_fused(m, m.logits, m.x, m.final_norm, m.lm_head.w, m.lm_head.scale, nullptr, rows, V, H, GEMM_PLAIN, "qlinear_lm_head"));
+        TRY(qlinear_fused(m, m.pl_lm, m.logits, m.x, m.final_norm, m.lm_head, nullptr, rows, GEMM_PLAIN, "qlinear_lm_head"));
     } else {
         if (!nrm_ready) {
             note(m, "rms_norm", 2.0 * rows * H * eb + H * eb);
@@ -595,7 +617,7 @@ static int enqueue_step(Model &m) {
         }
         if (m.skinny) TRY(skinny_rows(m, m.logits, m.nrm, m.lm_head, m.pk_lm_head, nullptr, rows, GEMM_PLAIN, "linear_lm_head"));
         else if (w8a8) TRY(linear_w8a8(m, m.logits, m.nrm, m.lm_head, rows, true, "qlinear_lm_head"));
-        else if (m.resident16) TRY(gemm_rows(m, m.logits, m.nrm, m.wt_lm_head, nullptr, rows, V, H, GEMM_PLAIN, "linear_lm_head"));
+        else if (m.resident16) TRY(gemm_rows(m, m.pl_lm, m.logits, m.nrm, m.lm_head, m.wt_lm_head, nullptr, rows, GEMM_PLAIN, "linear_lm_head"));
         else TRY(linear_rows<T>(m, m.logits, m.nrm, m.lm_head, rows, "linear_lm_head"));
     }
     // greedy token of the last row of each sequence; for a batch-1 decode step the same launch
@@ -769,6 +791,32 @@ static int build(Model &m, void **init, void **state) {
                    skinny_gemm_supported(rows_, H, QD) && skinny_gemm_supported(rows_, 2 * F, H) &&
                    skinny_gemm_supported(rows_, H, F) && skinny_gemm_supported(rows_, V, H);
     }
+    // which linears of a matrix-core executor multiply by tiles of the int8 weights as they are: those too small for the
+    // 256-row kernels to be the faster ones (some 1500 rows for a 11264 x 2048 matrix, every int8 product below half a
+    // round of tiles); a model with none of the others never makes the resident copies.  (Up to 64 rows the few-row kernel
+    // streams a tiled copy; shapes that it does not take stay with the resident one.)
+    const int tile_kind = c.quantize_activations ? TG_I8 : TG_W8;
+    size_t tg_part_bytes = 0;
+    auto plan_linear = [&](LinPlan &pl, int N, int K, const void *first, const void *last) {
+        const int rows_ = c.batch * c.seq_q;
+        pl = LinPlan{};
+        if (c.gemm_tile || !tile_gemm_supported(tile_kind, rows_, N, K) || !aligned16(first) || !aligned16(last)) return;
+        pl.plan = tile_gemm_plan(tile_kind, c.dtype, rows_, N, K, kTgScratchMax);
+        pl.tile = pl.plan.us <= (tile_kind == TG_I8 ? qgemm_dma_us(rows_, N, K) : gemm_nt_mfma_us(rows_, N, K, c.dtype));
+        if (pl.tile) tg_part_bytes = std::max(tg_part_bytes, pl.plan.part_bytes);
+    };
+    bool all_tiles = false;
+    if (m.quant && !m.skinny && c.batch * c.seq_q >= (c.quantize_activations ? 2 : 65)) {
+        bool ok = true;
+        for (const Layer &L : m.layers) ok = ok && aligned16(L.o.w) && aligned16(L.down.w);
+        const void *odd = ok ? nullptr : (const void *)1;
+        plan_linear(m.pl_qkv, QD + 2 * KD, H, nullptr, nullptr);
+        plan_linear(m.pl_o, H, QD, odd, odd);
+        plan_linear(m.pl_gu, 2 * F, H, nullptr, nullptr);
+        plan_linear(m.pl_down, H, F, odd, odd);
+        plan_linear(m.pl_lm, V, H, m.lm_head.w, m.lm_head.w);
+        all_tiles = m.pl_qkv.tile && m.pl_o.tile && m.pl_gu.tile && m.pl_down.tile && m.pl_lm.tile;
+    }
     if (m.skinny) {
         // one more int8 copy of every linear weight, tiled for sequential streaming (1 byte per weight)
         if (!ws.packed8) {
@@ -798,8 +846,8 @@ static int build(Model &m, void **init, void **state) {
         }
         m.pk_lm_head = ws.pk_lm_head;
     }
-    if (m.quant && !m.skinny && !c.quantize_activations && c.batch * c.seq_q >= 16 && H % 8 == 0 && QD % 8 == 0 && F % 32 == 0) {
-        if (!ws.resident16) {
+    if (m.quant && !m.skinny && !c.quantize_activations && c.batch * c.seq_q >= 16 && H % 8 == 0 && QD % 8 == 0 && (F % 32 == 0 || all_tiles)) {
+        if (!ws.resident16 && !all_tiles) {
             ws.bytes_resident16 = 0;
             auto resident = [&](void **dst, const Lin &l) {
                 renew(dst);
@@ -842,32 +890,34 @@ static int build(Model &m, void **init, void **state) {
         if (need) MYNN_HIP(hipMalloc(&m.ws, need));
     }
 
-    // ---- W8A8 prefill executors: every linear is large enough for the 256-row int8 tiles; gate and up become one
-    // product whose store applies SwiGLU, so their rows (and scales) are interleaved in groups of 32 once
-    {
+    // ---- W8A8 executors of several rows: norm + quantiser, then the int8 product with its store in one launch.  Where the
+    // large tiles take the gate/up product, its rows (and scales) are interleaved in groups of 32 once
+    if (m.quant && c.quantize_activations && c.batch * c.seq_q >= 2 && c.dtype != MYNN_F32) {
         const int rows_ = c.batch * c.seq_q;
-        if (m.quant && c.quantize_activations && c.dtype != MYNN_F32 && F % 32 == 0 && qgemm_dma_supported(rows_, QD + 2 * KD, H) &&
-            qgemm_dma_supported(rows_, H, QD) && qgemm_dma_supported(rows_, 2 * F, H) && qgemm_dma_supported(rows_, H, F) &&
-            qgemm_dma_supported(rows_, V, H)) {
-            const size_t seb = dtype_size(c.dtype);
-            if (!ws.q8) ws.bytes_q8 = 0;
-            for (size_t li = 0; li < m.layers.size() && !ws.q8; li++) {
-                Layer &L = m.layers[li];
-                WeightLayer &W = ws.layers[li];
-                renew(&W.q8_gu); renew(&W.q8_gu_scale);
-                MYNN_HIP(hipMalloc(&W.q8_gu, (size_t)2 * F * H));
-                MYNN_HIP(hipMalloc(&W.q8_gu_scale, (size_t)2 * F * seb));
-                ws.bytes_q8 += (size_t)2 * F * H + (size_t)2 * F * seb;
-                TRY(interleave_row_groups(W.q8_gu, L.gate.w, F, (size_t)H, 32, 0, m.stream));
-                TRY(interleave_row_groups(W.q8_gu, L.up.w, F, (size_t)H, 32, 1, m.stream));
-                TRY(interleave_row_groups(W.q8_gu_scale, L.gate.scale, F, seb, 32, 0, m.stream));
-                TRY(interleave_row_groups(W.q8_gu_scale, L.up.scale, F, seb, 32, 1, m.stream));
-            }
-            MYNN_HIP(hipStreamSynchronize(m.stream));
-            ws.q8 = true;
-            for (size_t li = 0; li < m.layers.size(); li++) {
-                m.layers[li].q8_gu = ws.layers[li].q8_gu;
-                m.layers[li].q8_gu_scale = ws.layers[li].q8_gu_scale;
+        auto either = [&](const LinPlan &pl, int N, int K) { return pl.tile || qgemm_dma_supported(rows_, N, K); };
+        if ((m.pl_gu.tile || F % 32 == 0) && either(m.pl_qkv, QD + 2 * KD, H) && either(m.pl_o, H, QD) && either(m.pl_gu, 2 * F, H) &&
+            either(m.pl_down, H, F) && either(m.pl_lm, V, H)) {
+            if (!m.pl_gu.tile) {
+                const size_t seb = dtype_size(c.dtype);
+                if (!ws.q8) ws.bytes_q8 = 0;
+                for (size_t li = 0; li < m.layers.size() && !ws.q8; li++) {
+                    Layer &L = m.layers[li];
+                    WeightLayer &W = ws.layers[li];
+                    renew(&W.q8_gu); renew(&W.q8_gu_scale);
+                    MYNN_HIP(hipMalloc(&W.q8_gu, (size_t)2 * F * H));
+                    MYNN_HIP(hipMalloc(&W.q8_gu_scale, (size_t)2 * F * seb));
+                    ws.bytes_q8 += (size_t)2 * F * H + (size_t)2 * F * seb;
+                    TRY(interleave_row_groups(W.q8_gu, L.gate.w, F, (size_t)H, 32, 0, m.stream));
+                    TRY(interleave_row_groups(W.q8_gu, L.up.w, F, (size_t)H, 32, 1, m.stream));
+                    TRY(interleave_row_groups(W.q8_gu_scale, L.gate.scale, F, seb, 32, 0, m.stream));
+                    TRY(interleave_row_groups(W.q8_gu_scale, L.up.scale, F, seb, 32, 1, m.stream));
+                }
+                MYNN_HIP(hipStreamSynchronize(m.stream));
+                ws.q8 = true;
+                for (size_t li = 0; li < m.layers.size(); li++) {
+                    m.layers[li].q8_gu = ws.layers[li].q8_gu;
+                    m.layers[li].q8_gu_scale = ws.layers[li].q8_gu_scale;
+                }
             }
             m.w8a8_fused = true;
         }
@@ -909,6 +959,7 @@ static int build(Model &m, void **init, void **state) {
     size_t o_sc = plan.take(32 + (size_t)c.batch * 4), o_tok = plan.take((size_t)m.token_cap * 4);
     size_t o_as = plan.take(attn_scratch_bytes(c.batch, c.n_heads, c.seq_q, c.head_dim, m.nsplit));
     size_t o_cand = plan.take(rows == 1 ? (size_t)kGemvArgmaxWords * 8 : 0);
+    size_t o_tgp = plan.take(tg_part_bytes), o_tgc = plan.take(tg_part_bytes ? (size_t)kTgCounters * 4 : 0);
     const size_t amax_bytes = argmax_scratch_bytes(c.batch, V);
     size_t o_amax = plan.take(amax_bytes);
     const bool strm = c.streaming_kv != 0;
@@ -933,6 +984,8 @@ static int build(Model &m, void **init, void **state) {
     m.d_next = m.d_past + 8;  // one token per sequence after the scalars
     m.d_tokens = (int32_t *)(m.arena + o_tok);
     m.attn_scratch = m.arena + o_as;
+    m.tg_part = m.arena + o_tgp;
+    m.tg_counters = (int *)(m.arena + o_tgc);
     m.lm_cand = (uint64_t *)(m.arena + o_cand);
     m.argmax_scratch = amax_bytes ? (uint64_t *)(m.arena + o_amax) : nullptr;
     m.d_kvpos = (int64_t *)(m.arena + o_kvpos);

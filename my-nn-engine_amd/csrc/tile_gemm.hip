@@ -17,6 +17,7 @@
 // When the tiles do not fill the device the K range is split over workgroups.  Each leaves its partial sums in scratch
 // memory (agent-scope stores, which go past the XCD's L2) and counts itself in; the last to arrive adds them up in the
 // order of the ranges -- the result does not depend on who was last -- and stores the output.  Nobody waits for anybody.
+#include <algorithm>
 #include <type_traits>
 
 #include "gemm_store.h"
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 //
 // a: what a step costs a CU however few workgroups it holds (latency); b: what each resident workgroup adds (LDS, MFMA and
 // dequantisation work); rounds: how often a CU takes a new set of workgroups.  Never less than the weights' bytes at 4.6
-// TB/s.  Choosing by it is within 2 % of the best choice on average, 14 % at worst.  (Two fits where the conversion of the
+// TB/s or the tiles' operations at the rate that long launches reach (0.95 PFLOP/s fp16, 0.82 bf16, 1.75 int8).  Choosing by it is within 2 % of the best choice on average, 14 % at worst.  (Two fits where the conversion of the
 // weights costs differ: it is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
 struct TgCost {
     int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
@@ -380,6 +381,7 @@ TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_b
     const TgCost *tab = kind == TG_W8 ? kTgW8 : kind == TG_W8S ? kTgW8S : kTgI8;
     const int n_tiles = kind == TG_W8S ? 3 : 6, d = dtype == MYNN_BF16 ? 1 : 0;
     const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
+    const double rate = kind == TG_I8 ? 1.75e9 : d ? 0.82e9 : 0.95e9;  // per microsecond
     const double weights_us = (double)N * K / 4.6e6;
     TgPlan best;
     best.us = 1e30;
@@ -392,8 +394,9 @@ TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_b
             // block of rows has the same sums whatever it is multiplied with when K < 4096; a launch that already has four workgroups per CU gains nothing by ranges)
             if (ks > 1 && (ks * (M >= 256 && kind != TG_I8 ? 32 : 3) > iters || tiles * ks > 1024 || tiles > kTgCounters || part > scratch_bytes)) continue;
             const long wgs = (tiles * ks + 255) / 256, rounds = (wgs + c.per_cu - 1) / c.per_cu;
-            const double steps = (double)((iters + ks - 1) / ks) * (c.a[d] * rounds + c.b[d] * wgs);
-            const double us = c.launch[d] + (steps + (ks > 1 ? c.e[d] * ks + part * 2e-6 / 4.0 : 0.0) > weights_us ? steps + (ks > 1 ? c.e[d] * ks + part * 2e-6 / 4.0 : 0.0) : weights_us);
+            double us = (double)((iters + ks - 1) / ks) * (c.a[d] * rounds + c.b[d] * wgs);
+            if (ks > 1) us += c.e[d] * ks + part * 2e-6 / 4.0;
+            us = std::max(us, std::max(weights_us, 2.0 * tiles * c.bm * c.bn * K / rate)) + c.launch[d];
             if (us < best.us) best = TgPlan{t, ks, us, part};
         }
     }
