@@ -377,7 +377,7 @@ bool tile_gemm_supported(int kind, int M, int N, int K) {
     return M >= 1 && N >= 1 && K >= 16 && K % (kind == TG_I8 ? 32 : 16) == 0 && (long)K * 256 * 2 < (1l << 31);
 }
 
-TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes) {
+static TgPlan tg_choose(int kind, int dtype, int M, int N, int K, size_t scratch_bytes) {
     const TgCost *tab = kind == TG_W8 ? kTgW8 : kind == TG_W8S ? kTgW8S : kTgI8;
     const int n_tiles = kind == TG_W8S ? 3 : 6, d = dtype == MYNN_BF16 ? 1 : 0;
     const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
@@ -401,6 +401,20 @@ TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_b
         }
     }
     return best;
+}
+
+// (the search is some 50 evaluations, half a microsecond of an operator call: a thread remembers its last few)
+TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes) {
+    struct Entry {
+        int kind = -1, dtype, M, N, K;
+        size_t scratch;
+        TgPlan plan;
+    };
+    thread_local Entry table[32];
+    Entry &e = table[((unsigned)M * 31u + (unsigned)N * 17u + (unsigned)K * 7u + (unsigned)kind * 5u + (unsigned)dtype) % 32u];
+    if (e.kind != kind || e.dtype != dtype || e.M != M || e.N != N || e.K != K || e.scratch != scratch_bytes)
+        e = Entry{kind, dtype, M, N, K, scratch_bytes, tg_choose(kind, dtype, M, N, K, scratch_bytes)};
+    return e.plan;
 }
 
 struct TgArgs {
