@@ -1,6 +1,8 @@
 // The small memory-bound operators of the decoder: RMSNorm, RoPE, KV-cache updates (plain and
 // quantizing), DequantizeLinear, row gather, SwiGLU / Add groups, dynamic activation
 // quantisation and the greedy argmax.  All compute in f32 and round once at the store.
+#include <type_traits>
+
 #include "kernels.h"
 #include "mfma.h"
 
@@ -263,26 +265,35 @@ __global__ __launch_bounds__(kEwThreads) void dynquant_kernel(void *y_, T *y_sca
     }
 }
 
-// Symmetric per-row quantisation of 16-bit rows of at most 8 * 64 * NCH values (a multiple of 8): one wave
-// per row, the row read once with 128-bit loads and kept in registers, reductions inside the wave (no
-// workgroup barrier); same arithmetic as dynquant_kernel<T, true>.
+// Symmetric per-row quantisation of 16-bit rows of at most 8 * 64 * W * NCH values (a multiple of 8): the row read once
+// with 128-bit loads and kept in registers; same arithmetic as dynquant_kernel<T, true>.  W = 1: one wave per row,
+// reductions inside the wave.  W = 4: a workgroup per row, for few rows (a wave per row left most CUs without one: 97 rows
+// of 4096 took 6.4 us) and for rows that one wave cannot hold (500 of 14336 on the looping kernel: 28 us).
 // NORM: the row is first RMS-normalised exactly as rms_norm_vec_kernel does (rounded to the storage type)
 // and only the quantised form is written -- the normalised activations of a W8A8 layer have no other reader.
-template <typename T, bool NORM, int NCH>
+template <typename T, bool NORM, int NCH, int W>
 __global__ __launch_bounds__(kEwThreads) void dynquant_rows_vec_kernel(int8_t *y, T *y_scale, int8_t *y_zp, const T *x, const T *w,
                                                                        int rows, int dim, float eps) {
-    const int lane = threadIdx.x & 63, row = blockIdx.x * (kEwThreads / 64) + (threadIdx.x >> 6);
-    if (row >= rows) return;  // whole wave
+    __shared__ float red[2][W];
+    const int lane = W == 1 ? threadIdx.x & 63 : threadIdx.x;
+    const int row = W == 1 ? blockIdx.x * (kEwThreads / 64) + (threadIdx.x >> 6) : blockIdx.x;
+    if (W == 1 && row >= rows) return;  // whole wave
     const size_t base = (size_t)row * dim;
     const int chunks = dim >> 3;
-    U4 v[NCH];
+    U4 v[NCH], nw[NCH];
     float ss = 0.f;
 #pragma unroll
     for (int q = 0; q < NCH; q++) {
-        const int c = lane + q * 64;
+        const int c = lane + q * 64 * W;
         v[q] = U4{0u, 0u, 0u, 0u};
         if (c < chunks) {
             v[q] = *(const U4 *)(x + base + (size_t)c * 8);
+            if (NORM && W > 1) nw[q] = *(const U4 *)(w + (size_t)c * 8);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NCH; q++) {
+        if (lane + q * 64 * W < chunks) {
             if (NORM) {
                 float f[8];
                 widen8<T>(v[q], f);
@@ -292,15 +303,22 @@ __global__ __launch_bounds__(kEwThreads) void dynquant_rows_vec_kernel(int8_t *y
         }
     }
     if (NORM) {
-        const float tot = wave_sum(ss);
+        float tot = wave_sum(ss);
+        if constexpr (W > 1) {
+            if ((threadIdx.x & 63) == 0) red[0][threadIdx.x >> 6] = tot;
+            __syncthreads();
+            tot = red[0][0];
+#pragma unroll
+            for (int i = 1; i < W; i++) tot += red[0][i];
+        }
         const float inv = 1.0f / sqrtf(tot / (float)dim + eps);
 #pragma unroll
         for (int q = 0; q < NCH; q++) {
-            const int c = lane + q * 64;
+            const int c = lane + q * 64 * W;
             if (c < chunks) {
                 float f[8], g[8];
                 widen8<T>(v[q], f);
-                widen8<T>(*(const U4 *)(w + (size_t)c * 8), g);
+                widen8<T>(W > 1 ? nw[q] : *(const U4 *)(w + (size_t)c * 8), g);
                 v[q].x = pack2<T>((f[0] * inv) * g[0], (f[1] * inv) * g[1]);
                 v[q].y = pack2<T>((f[2] * inv) * g[2], (f[3] * inv) * g[3]);
                 v[q].z = pack2<T>((f[4] * inv) * g[4], (f[5] * inv) * g[5]);
@@ -317,11 +335,17 @@ __global__ __launch_bounds__(kEwThreads) void dynquant_rows_vec_kernel(int8_t *y
         for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(f[i]));
     }
     amax = wave_max(amax);
+    if constexpr (W > 1) {
+        if ((threadIdx.x & 63) == 0) red[1][threadIdx.x >> 6] = amax;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < W; i++) amax = fmaxf(amax, red[1][i]);
+    }
     const float sc = amax > 0.f ? amax / 127.0f : 1.0f;
     const float inv = 1.0f / sc;
 #pragma unroll
     for (int q = 0; q < NCH; q++) {
-        const int c = lane + q * 64;
+        const int c = lane + q * 64 * W;
         if (c < chunks) {
             float f[8];
             widen8<T>(v[q], f);
@@ -343,21 +367,30 @@ __global__ __launch_bounds__(kEwThreads) void dynquant_rows_vec_kernel(int8_t *y
 
 template <typename T, bool NORM>
 static int dynquant_rows_vec(int8_t *y, void *y_scale, int8_t *y_zp, const void *x, const void *w, int rows, int dim, float eps, hipStream_t s) {
-    const dim3 grid((rows + kEwThreads / 64 - 1) / (kEwThreads / 64)), block(kEwThreads);
+    const dim3 block(kEwThreads);
+    auto go = [&](auto nch, auto w_) {
+        constexpr int NCH = decltype(nch)::value, W = decltype(w_)::value;
+        const dim3 grid(W == 1 ? (rows + kEwThreads / 64 - 1) / (kEwThreads / 64) : rows);
+        MYNN_LAUNCH((dynquant_rows_vec_kernel<T, NORM, NCH, W>), grid, block, 0, s, y, (T *)y_scale, y_zp, (const T *)x, (const T *)w, rows, dim, eps);
+    };
+    using std::integral_constant;
     const int nch = (dim / 8 + 63) / 64;
-    if (nch <= 4)
-        MYNN_LAUNCH((dynquant_rows_vec_kernel<T, NORM, 4>), grid, block, 0, s, y, (T *)y_scale, y_zp, (const T *)x, (const T *)w, rows, dim, eps);
-    else if (nch <= 8)
-        MYNN_LAUNCH((dynquant_rows_vec_kernel<T, NORM, 8>), grid, block, 0, s, y, (T *)y_scale, y_zp, (const T *)x, (const T *)w, rows, dim, eps);
-    else if (nch <= 12)
-        MYNN_LAUNCH((dynquant_rows_vec_kernel<T, NORM, 12>), grid, block, 0, s, y, (T *)y_scale, y_zp, (const T *)x, (const T *)w, rows, dim, eps);
-    else
-        MYNN_LAUNCH((dynquant_rows_vec_kernel<T, NORM, 16>), grid, block, 0, s, y, (T *)y_scale, y_zp, (const T *)x, (const T *)w, rows, dim, eps);
+    // (a workgroup per row until the rows alone fill the device with waves)
+    if (rows < 2048 || nch > 16) {
+        const int n4 = (nch + 3) / 4;
+        if (n4 <= 1) go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+        else if (n4 <= 2) go(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+        else if (n4 <= 4) go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+        else go(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+    } else if (nch <= 4) go(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+    else if (nch <= 8) go(integral_constant<int, 8>{}, integral_constant<int, 1>{});
+    else if (nch <= 12) go(integral_constant<int, 12>{}, integral_constant<int, 1>{});
+    else go(integral_constant<int, 16>{}, integral_constant<int, 1>{});
     return launch_status("dynquant_rows_vec_kernel");
 }
 
 static bool dynquant_vec_ok(const void *y, const void *x, int dim) {
-    return dim % 8 == 0 && dim <= 8 * 64 * 16 && aligned16(x) && ((uintptr_t)y & 7) == 0;
+    return dim % 8 == 0 && dim <= 8 * 64 * 32 && aligned16(x) && ((uintptr_t)y & 7) == 0;
 }
 
 // RMSNorm followed by symmetric per-row quantisation (the pair RMSNormalization -> DynamicQuantizeLinear of a
