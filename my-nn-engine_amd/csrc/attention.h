@@ -4,6 +4,10 @@
 
 namespace mynn {
 
+// arrival counters of the streaming decode kernel, one per (sequence, kv head): more of those than this are never split
+// over so many key ranges that the merge launch would show
+constexpr int kAttnArrive = 1024;
+
 struct AttnParams {
     void *out;
     const void *q, *k, *v, *k_scale, *v_scale;
@@ -20,6 +24,7 @@ struct AttnParams {
     // K and V then are the caches the new row is appended to
     const void *qkv, *cos_t, *sin_t;
     const int64_t *d_pos;
+    int fuse_stream;          // ... the streaming kernel's fused form (else the latency kernel's)
     // additive mask (operator slot 3), storage type: element (b * Hq + h) * mask_os + sq * mask_rs + key
     const void *mask;
     long mask_os, mask_rs;
@@ -33,6 +38,7 @@ struct AttnParams {
     int page_shift, pages_per_seq;
     float *part_o;            // [B*Hq*Sq, nsplit, D]
     float *part_ml;           // [B*Hq*Sq, nsplit, 2]
+    int *arrive;              // streaming decode kernel: kAttnArrive counters, zero between launches (null: merged by a second launch)
     // element strides of Q and out: batch, head, row.  Reference layout [B,Hq,Sq,D] is
     // (Hq*Sq*D, Sq*D, D); token-major [B,Sq,Hq*D] is (Sq*Hq*D, D, Hq*D).
     long q_bs, q_hs, q_rs, o_bs, o_hs, o_rs;

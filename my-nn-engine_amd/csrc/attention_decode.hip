@@ -439,10 +439,10 @@ int attention_decode_launch(AttnParams p, int D, int dtype, int kv_int8, void *s
                  "fused decode attention: position, past_len and active length must be device scalars");
     // the plan (attn_plan, with the same kv_len) was made for the streaming kernel when it is eligible
     const int kv_len = p.d_active ? p.cache_len : (p.active < p.cache_len ? p.active : p.cache_len);
-    if (!fuse && !p.mask && attn_stream_eligible(p.B, p.Sq, p.Hq, p.Hkv, D, dtype, kv_int8, kv_len, p.cache_len))
+    if ((!fuse || p.fuse_stream) && !p.mask && attn_stream_eligible(p.B, p.Sq, p.Hq, p.Hkv, D, dtype, kv_int8, kv_len, p.cache_len))
         return attention_stream_launch(p, D, dtype, kv_int8, s);
     if (p.page_table) {  // (the plan is the streaming kernel's: that kernel has the paged form)
-        MYNN_REQUIRE(!fuse && !p.mask, MYNN_ERR_UNSUPPORTED, "paged attention: neither the fused decode form nor a mask");
+        MYNN_REQUIRE((!fuse || p.fuse_stream) && !p.mask, MYNN_ERR_UNSUPPORTED, "paged attention: neither the latency kernel's fused form nor a mask");
         return attention_stream_launch(p, D, dtype, kv_int8, s);
     }
     bool whole = false;  // the launch wrote the finished output: nothing to merge whatever the plan's split count
@@ -499,10 +499,11 @@ static std::map<hipStream_t, Grown> g_scratch;
 // process ends).  The array's name is only a handle on the host: the address kernels get is asked for once per device.
 constexpr size_t kStaticScratchBytes = 8u << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
+static __device__ int scratch_arrive[kAttnArrive];
 constexpr int kMaxDevices = 64;
-static void *g_static_ptr[kMaxDevices] = {};
+static void *g_static_ptr[kMaxDevices] = {}, *g_static_arrive[kMaxDevices] = {};
 static std::mutex g_static_mu;
-static int static_scratch(void **out) {
+static int static_scratch(void **out, int **arrive) {
     int dev = 0;
     MYNN_HIP(hipGetDevice(&dev));
     MYNN_REQUIRE(dev >= 0 && dev < kMaxDevices, MYNN_ERR_UNSUPPORTED, "attention_noalloc: device %d", dev);
@@ -511,9 +512,11 @@ static int static_scratch(void **out) {
         void *ptr = nullptr;
         MYNN_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
         MYNN_REQUIRE(ptr, MYNN_ERR_STATE, "attention_noalloc: the scratch array has no device address");
+        MYNN_HIP(hipGetSymbolAddress(&g_static_arrive[dev], HIP_SYMBOL(scratch_arrive)));
         g_static_ptr[dev] = ptr;
     }
     *out = g_static_ptr[dev];
+    *arrive = (int *)g_static_arrive[dev];
     return 0;
 }
 
@@ -557,14 +560,17 @@ static int attention_entry(void *out, const void *Q, const void *K, const void *
             MYNN_REQUIRE(need <= kStaticScratchBytes, MYNN_ERR_UNSUPPORTED,
                          "attention_noalloc: this shape needs %zu bytes of partial results, the library's fixed array holds %zu", need,
                          kStaticScratchBytes);
-            int rc = static_scratch(&scr);
+            int rc = static_scratch(&scr, &p.arrive);
             if (rc) return rc;
         } else {
             std::lock_guard<std::mutex> lk(g_scratch_mu);
             Grown &g = g_scratch[st];
-            int rc = ensure(g, need, false, st);
+            const size_t had = g.bytes;
+            int rc = ensure(g, need + kAttnArrive * 4, false, st);
             if (rc) return rc;
-            scr = g.ptr;
+            if (g.bytes != had) MYNN_HIP(hipMemsetAsync(g.ptr, 0, kAttnArrive * 4, st));  // the counters in front
+            p.arrive = (int *)g.ptr;
+            scr = (char *)g.ptr + kAttnArrive * 4;
         }
     }
     return attention_decode_launch(p, head_dim, dtype, kv_int8, scr, st);

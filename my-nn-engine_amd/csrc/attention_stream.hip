@@ -14,11 +14,13 @@
 //            in LDS (row stride 136 bytes: conflict-free) and read back two dims at a time, each pair of
 //            keys split into an "even dims" and an "odd dims" operand by one v_perm -- the 16 rows of
 //            an MFMA tile are dims 32c + 2r (+1),
-// then waves are combined through LDS and key ranges by a small second launch (attn_merge_kernel).
+// then waves are combined through LDS, and key ranges by the workgroup of a (sequence, kv head) that arrives last
+// (or by a second launch, attn_merge_kernel, where the caller's scratch memory has no arrival counters).
 // P enters the second product as a sum of two storage-type values.  Replaces the reference's attention_decode (attention.cuh:495-606) for these shapes.
 #include <type_traits>
 
 #include "attention.h"
+#include "kernels.h"
 #include "mfma.h"
 
 namespace mynn {
@@ -48,8 +50,23 @@ constexpr long kStreamMinKeys = 8192;
 // (pages hold a power of two >= 32 rows, tiles start at multiples of 32), so the page is a wave-uniform value per
 // tile: the workgroup's part of the table sits in one register (lane i = the i-th page of its key range, at most 64)
 // and a tile picks its entry with v_readlane -- no dependent load in the key loop.
-template <typename T, int D, int G, bool KVI8, bool PAGED>
-__global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(AttnParams p) {
+// FUSE: q is the raw q|k|v projection row of the sequence; the kernel rotates the queries itself, and the workgroup whose
+// key range holds row *d_past writes the new key (rotated) and value there before it walks its keys: the RoPE + append
+// launch in front of it disappears.
+// What the kernel needs of AttnParams (a launch pays for its argument bytes: 0.9 us of host time for 300 against 60).
+struct StreamParams {
+    void *out;
+    const void *q, *k, *v, *k_scale, *v_scale, *cos_t, *sin_t;
+    const int64_t *d_pos;
+    const int32_t *d_active, *d_past, *page_table;
+    float *part_o, *part_ml;
+    int *arrive;
+    long q_bs, q_hs, o_bs, o_hs;
+    float scale;
+    int Hq, Hkv, cache_len, active, nsplit, slice, page_shift, pages_per_seq;
+};
+template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE>
+__global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParams p) {
     constexpr int KB = D / 32;              // 32-dim blocks of a key row
     constexpr int LPK = D / 8;              // lanes per key row when a tile is loaded 16 bytes per lane
     constexpr int KPP = 64 / LPK;           // key rows per load pass of a wave
@@ -74,6 +91,11 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(AttnParams 
     const int active = p.d_active ? *p.d_active : p.active;
     const int bound = min(active, p.cache_len);
     const int k0 = split * p.slice, k1 = min(bound, k0 + p.slice);
+    // key ranges that hold a row; the launch is sized for the whole cache, the ranges past the context only leave
+    const int n_act = p.arrive ? max(1, min(p.nsplit, (bound + p.slice - 1) / p.slice)) : p.nsplit;
+    const int past = FUSE ? *p.d_past : 0;
+    const bool owner = FUSE && split == min(past / p.slice, p.nsplit - 1);
+    if (split >= n_act && !owner) return;
     const size_t kv_base = PAGED ? 0 : (size_t)bhkv * p.cache_len;
     using TKV = typename std::conditional<KVI8, int8_t, T>::type;
     using Chunk = typename std::conditional<KVI8, uint2, U4>::type;  // 8 elements of a cached row
@@ -89,6 +111,53 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(AttnParams 
         const int pg = __builtin_amdgcn_readlane(pg_reg, __builtin_amdgcn_readfirstlane((t0 >> psh) - pg0));
         return ((size_t)pg * p.Hkv + hkv) << psh;
     };
+    if constexpr (FUSE) {
+        if (owner) {
+            // wave 0 the key, wave 1 the value of the new row: lane i < D/2 has elements i and i + D/2
+            constexpr int half = D / 2;
+            const size_t tok = kv_cache_row(KvPaging{PAGED ? p.page_table : nullptr, p.page_shift, p.pages_per_seq}, b, hkv, past, p.Hkv, p.cache_len);
+            if (wave < 2) {
+                const bool on = lane < half, is_k = wave == 0;
+                const T *src = (const T *)p.q + (size_t)b * p.q_bs + (size_t)(p.Hq + (is_k ? 0 : p.Hkv) + hkv) * D;
+                float lo = 0.f, hi = 0.f;
+                if (on) {
+                    lo = Elem<T>::ld(src, lane);
+                    hi = Elem<T>::ld(src, lane + half);
+                    if (is_k) {
+                        const T *ct = (const T *)p.cos_t + (size_t)*p.d_pos * D, *st = (const T *)p.sin_t + (size_t)*p.d_pos * D;
+                        const float rl = Elem<T>::rnd(lo * Elem<T>::ld(ct, lane) - hi * Elem<T>::ld(st, lane));
+                        const float rh = Elem<T>::rnd(hi * Elem<T>::ld(ct, lane + half) + lo * Elem<T>::ld(st, lane + half));
+                        lo = rl;
+                        hi = rh;
+                    }
+                }
+                if constexpr (KVI8) {  // the rule of rope_quant_kv_append_kernel
+                    const float amax = wave_max(fmaxf(fabsf(lo), fabsf(hi)));
+                    const float inv = amax == 0.f ? 0.f : 127.0f / amax;
+                    auto code = [&](float x) -> int8_t {
+                        const float a = x * inv;
+                        const int q = (int)(a + (a >= 0.f ? 0.5f : -0.5f));
+                        return (int8_t)(q < -128 ? -128 : (q > 127 ? 127 : q));
+                    };
+                    if (lane == 0) Elem<T>::st((T *)(is_k ? p.k_scale : p.v_scale), tok, amax * (1.0f / 127.0f));
+                    int8_t *dst = (int8_t *)(is_k ? p.k : p.v) + tok * D;
+                    if (on) {
+                        dst[lane] = code(lo);
+                        dst[lane + half] = code(hi);
+                    }
+                } else if (on) {
+                    T *dst = (T *)(is_k ? p.k : p.v) + tok * D;
+                    Elem<T>::st(dst, lane, lo);
+                    Elem<T>::st(dst, lane + half, hi);
+                }
+            }
+            // the row is read back by this workgroup: written through, and no older copy of its line left in the L1
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (split >= n_act) return;
+        }
+    }
     auto operand = [](const Chunk &c) -> U4 {
         if constexpr (KVI8) return i8x8_to_operand<T>(c.x, c.y);
         else return c;
@@ -103,6 +172,26 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(AttnParams 
         for (int j = 0; j < KB; j++) {
             qf[j] = *(const U4 *)(qrow + j * 32 + quad * 8);
             if (col >= G) qf[j] = U4{0u, 0u, 0u, 0u};
+        }
+        if constexpr (FUSE) {  // dims d and d + D/2 of a rotation pair are blocks j and j + KB/2 of the same lane
+            const T *ct = (const T *)p.cos_t + (size_t)*p.d_pos * D + quad * 8, *st = (const T *)p.sin_t + (size_t)*p.d_pos * D + quad * 8;
+#pragma unroll
+            for (int j = 0; j < KB / 2; j++) {
+                float xl[8], xh[8], cl[8], ch[8], sl[8], sh[8], ol[8], oh[8];
+                widen8<T>(qf[j], xl);
+                widen8<T>(qf[j + KB / 2], xh);
+                widen8<T>(*(const U4 *)(ct + j * 32), cl);
+                widen8<T>(*(const U4 *)(ct + (j + KB / 2) * 32), ch);
+                widen8<T>(*(const U4 *)(st + j * 32), sl);
+                widen8<T>(*(const U4 *)(st + (j + KB / 2) * 32), sh);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    ol[i] = xl[i] * cl[i] - xh[i] * sl[i];
+                    oh[i] = xh[i] * ch[i] + xl[i] * sh[i];
+                }
+                qf[j] = U4{pack2<T>(ol[0], ol[1]), pack2<T>(ol[2], ol[3]), pack2<T>(ol[4], ol[5]), pack2<T>(ol[6], ol[7])};
+                qf[j + KB / 2] = U4{pack2<T>(oh[0], oh[1]), pack2<T>(oh[2], oh[3]), pack2<T>(oh[4], oh[5]), pack2<T>(oh[6], oh[7])};
+            }
         }
     }
 
@@ -286,38 +375,96 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(AttnParams 
     }
     __syncthreads();
 
-    // ---- combine the waves (a wave with no tile has m = -inf, l = 0, o = 0)
+    // ---- combine the waves (a wave with no tile has m = -inf, l = 0, o = 0), two dims per thread
     T *out = (T *)p.out;
-    for (int idx = tid; idx < G * D; idx += kStreamThreads) {
-        const int g = idx / D, d = idx % D;
+    for (int idx = tid; idx < G * D / 2; idx += kStreamThreads) {
+        const int g = idx / (D / 2), d = idx % (D / 2) * 2;
         float mt = -INFINITY;
 #pragma unroll
         for (int w = 0; w < kStreamWaves; w++) mt = fmaxf(mt, m_s[w][g]);
-        float lt = 0.f, ot = 0.f;
+        float lt = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
         for (int w = 0; w < kStreamWaves; w++) {
             const float c = m_s[w][g] == -INFINITY ? 0.f : fast_exp(m_s[w][g] - mt);
             lt = fmaf(l_s[w][g], c, lt);
-            ot = fmaf(o_s[w][g][d], c, ot);
+            o0 = fmaf(o_s[w][g][d], c, o0);
+            o1 = fmaf(o_s[w][g][d + 1], c, o1);
         }
-        const size_t row = (size_t)(b * p.Hq + head0 + g);
-        if (p.nsplit == 1) {
-            Elem<T>::st(out, (size_t)b * p.o_bs + (size_t)(head0 + g) * p.o_hs + d, ot / lt);
+        const size_t row = (size_t)(b * p.Hq + head0 + g), at = (size_t)b * p.o_bs + (size_t)(head0 + g) * p.o_hs + d;
+        if (n_act == 1) {
+            Elem<T>::st(out, at, o0 / lt);
+            Elem<T>::st(out, at + 1, o1 / lt);
+        } else if (p.arrive) {
+            // (past this XCD's L2: whoever arrives last reads them)
+            auto word = [](float lo, float hi) { return (uint64_t)__builtin_bit_cast(uint32_t, lo) | ((uint64_t)__builtin_bit_cast(uint32_t, hi) << 32); };
+            __hip_atomic_store((uint64_t *)(p.part_o + (row * p.nsplit + split) * D + d), word(o0, o1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == 0) __hip_atomic_store((uint64_t *)(p.part_ml + (row * p.nsplit + split) * 2), word(mt, lt), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
             // merged by attn_merge_kernel in the next launch
-            p.part_o[(row * p.nsplit + split) * D + d] = ot;
+            float *po = p.part_o + (row * p.nsplit + split) * D + d;
+            po[0] = o0;
+            po[1] = o1;
             if (d == 0) {
                 p.part_ml[(row * p.nsplit + split) * 2] = mt;
                 p.part_ml[(row * p.nsplit + split) * 2 + 1] = lt;
             }
         }
     }
+    if (n_act == 1 || !p.arrive) return;
+
+    // ---- the last key range to arrive merges them, in their order (the result does not depend on who was last)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this range's results are written through before it counts itself in
+    __syncthreads();
+    int *flag = (int *)&p_s[0][0];
+    if (tid == 0) {
+        const int before = __hip_atomic_fetch_add(p.arrive + bhkv, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before == n_act - 1) __hip_atomic_store(p.arrive + bhkv, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
+        *flag = before;
+    }
+    __syncthreads();
+    if (*flag != n_act - 1) return;
+    for (int idx = tid; idx < G * D / 2; idx += kStreamThreads) {
+        const int g = idx / (D / 2), d = idx % (D / 2) * 2;
+        const size_t row = (size_t)(b * p.Hq + head0 + g);
+        const uint64_t *ml = (const uint64_t *)(p.part_ml + row * p.nsplit * 2), *po = (const uint64_t *)(p.part_o + row * p.nsplit * D + d);
+        auto lo = [](uint64_t w) { return __builtin_bit_cast(float, (uint32_t)w); };
+        auto hi = [](uint64_t w) { return __builtin_bit_cast(float, (uint32_t)(w >> 32)); };
+        // eight ranges in flight; their maximum first, as attn_merge_kernel has it
+        constexpr int AH = 8;
+        float mt = -INFINITY;
+        for (int s0 = 0; s0 < n_act; s0 += AH) {
+            uint64_t w[AH];
+#pragma unroll
+            for (int i = 0; i < AH; i++) w[i] = __hip_atomic_load(ml + min(s0 + i, n_act - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int i = 0; i < AH; i++) mt = fmaxf(mt, lo(w[i]));
+        }
+        float lt = 0.f, o0 = 0.f, o1 = 0.f;
+        for (int s0 = 0; s0 < n_act; s0 += AH) {
+            uint64_t w[AH], o[AH];
+#pragma unroll
+            for (int i = 0; i < AH; i++) {
+                const int sp = min(s0 + i, n_act - 1);
+                w[i] = __hip_atomic_load(ml + sp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                o[i] = __hip_atomic_load(po + (size_t)sp * (D / 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (int i = 0; i < AH; i++) {
+                const float ms = lo(w[i]);
+                const float c = ms == -INFINITY || s0 + i >= n_act ? 0.f : fast_exp(ms - mt);
+                lt = fmaf(hi(w[i]), c, lt);
+                o0 = fmaf(lo(o[i]), c, o0);
+                o1 = fmaf(hi(o[i]), c, o1);
+            }
+        }
+        const size_t at = (size_t)b * p.o_bs + (size_t)(head0 + g) * p.o_hs + d;
+        Elem<T>::st(out, at, o0 / lt);
+        Elem<T>::st(out, at + 1, o1 / lt);
+    }
 }
 
 // ---- merge of key ranges: out[row, d] = sum_s o_s * exp(m_s - m) / sum_s l_s * exp(m_s - m).
-// A launch of its own: a kernel boundary is the cheap way to make the partial results of workgroups on
-// other XCDs visible (in-kernel hand-over needs either cache-wide fences, which slowed the whole
-// launch down 2-3x, or loads past the L2 at 1-2 us each).
+// A launch of its own, for callers whose scratch memory has no arrival counters and for the per-slice kernel.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnParams p, int D) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;  // (b, head, sq, d)
@@ -419,23 +566,23 @@ bool attn_stream_possible(int B, int Sq, int Hq, int Hkv, int D, int dtype, int 
            cache_len >= kStreamTile && (long)B * Hkv * cache_len >= kStreamMinKeys;
 }
 
-template <typename T, int D, bool KVI8, bool PAGED>
-static int stream_g(const AttnParams &p, hipStream_t s) {
-    dim3 grid(p.B * p.Hkv, p.nsplit), block(kStreamThreads);
+template <typename T, int D, bool KVI8, bool PAGED, bool FUSE>
+static int stream_g(const StreamParams &p, int B, hipStream_t s) {
+    dim3 grid(B * p.Hkv, p.nsplit), block(kStreamThreads);
     switch (p.Hq / p.Hkv) {
-    case 1: MYNN_LAUNCH((attn_stream_kernel<T, D, 1, KVI8, PAGED>), grid, block, 0, s, p); break;
-    case 2: MYNN_LAUNCH((attn_stream_kernel<T, D, 2, KVI8, PAGED>), grid, block, 0, s, p); break;
-    case 4: MYNN_LAUNCH((attn_stream_kernel<T, D, 4, KVI8, PAGED>), grid, block, 0, s, p); break;
-    case 8: MYNN_LAUNCH((attn_stream_kernel<T, D, 8, KVI8, PAGED>), grid, block, 0, s, p); break;
+    case 1: MYNN_LAUNCH((attn_stream_kernel<T, D, 1, KVI8, PAGED, FUSE>), grid, block, 0, s, p); break;
+    case 2: MYNN_LAUNCH((attn_stream_kernel<T, D, 2, KVI8, PAGED, FUSE>), grid, block, 0, s, p); break;
+    case 4: MYNN_LAUNCH((attn_stream_kernel<T, D, 4, KVI8, PAGED, FUSE>), grid, block, 0, s, p); break;
+    case 8: MYNN_LAUNCH((attn_stream_kernel<T, D, 8, KVI8, PAGED, FUSE>), grid, block, 0, s, p); break;
     default: return fail(MYNN_ERR_UNSUPPORTED, "streaming attention: %d query heads per kv head", p.Hq / p.Hkv);
     }
     return launch_status("attn_stream_kernel");
 }
 
-template <typename T, int D>
-static int stream_kv(const AttnParams &p, int kv_int8, hipStream_t s) {
-    if (p.page_table) return kv_int8 ? stream_g<T, D, true, true>(p, s) : stream_g<T, D, false, true>(p, s);
-    return kv_int8 ? stream_g<T, D, true, false>(p, s) : stream_g<T, D, false, false>(p, s);
+template <typename T, int D, bool FUSE>
+static int stream_kv(const StreamParams &p, int B, int kv_int8, hipStream_t s) {
+    if (p.page_table) return kv_int8 ? stream_g<T, D, true, true, FUSE>(p, B, s) : stream_g<T, D, false, true, FUSE>(p, B, s);
+    return kv_int8 ? stream_g<T, D, true, false, FUSE>(p, B, s) : stream_g<T, D, false, false, FUSE>(p, B, s);
 }
 
 // what the paged form needs whatever the sizes: one query row, a 16-bit type, head_dim 64 or 128, 1/2/4/8 query heads
@@ -449,7 +596,7 @@ bool attn_stream_paged_supported(int Sq, int Hq, int Hkv, int D, int dtype, int 
 int attention_stream_launch(const AttnParams &p, int D, int dtype, int kv_int8, hipStream_t s) {
     MYNN_REQUIRE(!kv_int8 || (p.k_scale && p.v_scale && p.cache_len % kStreamTile == 0), MYNN_ERR_INVALID,
                  "streaming attention: int8 KV needs scales and a cache length that is a multiple of %d", kStreamTile);
-    MYNN_REQUIRE(p.q_rs >= 0 && aligned16(p.q) && aligned16(p.k) && aligned16(p.v) && p.q_bs % 8 == 0 && p.q_hs % 8 == 0,
+    MYNN_REQUIRE(p.q_rs >= 0 && aligned16(p.qkv ? p.qkv : p.q) && aligned16(p.k) && aligned16(p.v) && p.q_bs % 8 == 0 && p.q_hs % 8 == 0,
                  MYNN_ERR_INVALID, "streaming attention: q, k, v must be 16-byte aligned");
     MYNN_REQUIRE(p.nsplit == 1 || (p.part_o && p.part_ml), MYNN_ERR_INVALID,
                  "streaming attention: no scratch for %d key ranges", p.nsplit);
@@ -465,9 +612,20 @@ int attention_stream_launch(const AttnParams &p, int D, int dtype, int kv_int8, 
         MYNN_REQUIRE((p.slice >> p.page_shift) + 2 <= 64, MYNN_ERR_UNSUPPORTED,
                      "paged attention: a key range of %d rows spans more than 62 pages of %d rows", p.slice, 1 << p.page_shift);
     }
+    const bool fuse = p.qkv != nullptr;
+    MYNN_REQUIRE(!fuse || (p.nsplit == 1 || p.arrive), MYNN_ERR_INVALID, "streaming attention: the fused form merges its own key ranges");
+    const StreamParams sp{p.out, fuse ? p.qkv : p.q, p.k, p.v, p.k_scale, p.v_scale, p.cos_t, p.sin_t, p.d_pos, p.d_active, p.d_past, p.page_table, p.part_o,
+                          p.part_ml, p.nsplit > 1 && p.B * p.Hkv <= kAttnArrive ? p.arrive : nullptr, fuse ? (long)(p.Hq + 2 * p.Hkv) * D : p.q_bs,
+                          fuse ? (long)D : p.q_hs, p.o_bs, p.o_hs, p.scale, p.Hq, p.Hkv, p.cache_len, p.active, p.nsplit, p.slice, p.page_shift,
+                          p.pages_per_seq};
     int rc;
-    if (dtype == MYNN_F16) rc = D == 64 ? stream_kv<f16_t, 64>(p, kv_int8, s) : stream_kv<f16_t, 128>(p, kv_int8, s);
-    else rc = D == 64 ? stream_kv<bf16_t, 64>(p, kv_int8, s) : stream_kv<bf16_t, 128>(p, kv_int8, s);
+    auto go = [&](auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        if (fuse) return D == 64 ? stream_kv<T, 64, true>(sp, p.B, kv_int8, s) : stream_kv<T, 128, true>(sp, p.B, kv_int8, s);
+        return D == 64 ? stream_kv<T, 64, false>(sp, p.B, kv_int8, s) : stream_kv<T, 128, false>(sp, p.B, kv_int8, s);
+    };
+    rc = dtype == MYNN_F16 ? go((f16_t *)nullptr) : go((bf16_t *)nullptr);
+    if (sp.arrive) return rc;
     if (rc || p.nsplit == 1) return rc;
     return attention_merge_launch(p, D, dtype, s);
 }

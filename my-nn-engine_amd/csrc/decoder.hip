@@ -188,6 +188,8 @@ struct Model {
     int32_t *d_past = nullptr, *d_active = nullptr, *d_next = nullptr, *d_tokens = nullptr, *d_step = nullptr;
     void *attn_scratch = nullptr;
     int nsplit = 1, slice = 0, heads_per_wg = 1;
+    int *attn_arrive = nullptr;      // arrival counters of the streaming decode kernel's key ranges
+    bool attn_stream_fuse = false;   // that kernel rotates, appends and attends in one launch
     int token_cap = 0;
     // host staging (pinned)
     char *h_stage = nullptr;
@@ -493,13 +495,15 @@ static int enqueue_step(Model &m) {
             p.d_active = m.d_active; p.nsplit = m.nsplit; p.slice = m.slice; p.heads_per_wg = m.heads_per_wg;
             attn_token_major_layout(p, D);
             p.page_table = m.paging.table; p.page_shift = m.paging.shift; p.pages_per_seq = m.paging.pages_per_seq;
+            p.arrive = m.attn_arrive;
             // (an int8 cache: the form for a cache one workgroup covers quantises the new row itself)
-            const bool fuse_attn = (fused || qfused) && !m.pages &&
-                                   (kv8 ? attention_fused_kv8_supported(D, c.max_seq) : attention_fused_supported(D, Hq / Hkv));
+            p.fuse_stream = m.attn_stream_fuse && !roped;
+            const bool fuse_attn = p.fuse_stream || ((fused || qfused) && !m.pages &&
+                                   (kv8 ? attention_fused_kv8_supported(D, c.max_seq) : attention_fused_supported(D, Hq / Hkv)));
             if (fuse_attn) {
                 // RoPE(q), RoPE(k), both cache appends and the attention in one launch
                 p.qkv = m.qkv; p.cos_t = m.cos_t; p.sin_t = m.sin_t; p.d_pos = m.d_pos; p.d_past = m.d_past;
-                note(m, kv8 ? "attention_rope_quant_append" : "attention_rope_append", (double)(QD + 2 * KD) * eb + 2.0 * KD * (kv8 ? 1 + eb / D : eb) + QD * eb);
+                note(m, kv8 ? "attention_rope_quant_append" : "attention_rope_append", ((double)(QD + 2 * KD) * eb + 2.0 * KD * (kv8 ? 1 + eb / D : eb) + QD * eb) * B);
                 TRY(attention_decode_launch(p, D, c.dtype, kv8 ? 1 : 0, m.attn_scratch, s));
             } else {
                 // prefill on the matrix cores: the attention kernel rotates the queries itself, reading them from the
@@ -926,7 +930,12 @@ static int build(Model &m, void **init, void **state) {
     // ---- arena: every activation of one step, the device scalars, attention split scratch
     const int rows = c.batch * c.seq_q;
     {
-        const bool fused_attn = m.quant && rows == 1 && !c.quantize_activations && !c.quant_kv_cache && !m.pages &&
+        // decode over a cache longer than the short form takes: the streaming kernel with RoPE and the appends inside
+        m.attn_stream_fuse = c.seq_q == 1 && !c.streaming_kv && !(c.unfused_decode && c.batch > 1) && c.batch * c.n_kv_heads <= kAttnArrive &&
+                             (m.pages ? attn_stream_paged_supported(1, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, 1 << m.paging.shift)
+                                      : attn_stream_eligible(c.batch, 1, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, c.quant_kv_cache, c.max_seq, c.max_seq)) &&
+                             !(rows == 1 && !m.pages && attention_fused_kv8_supported(c.head_dim, c.max_seq));
+        const bool fused_attn = m.quant && rows == 1 && !c.quantize_activations && !c.quant_kv_cache && !m.pages && !m.attn_stream_fuse &&
                                 attention_fused_supported(c.head_dim, c.n_heads / c.n_kv_heads);
         attn_plan(c.batch, c.seq_q, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, c.quant_kv_cache, c.max_seq, c.max_seq, fused_attn,
                   &m.slice, &m.nsplit, &m.heads_per_wg);
@@ -958,6 +967,7 @@ static int build(Model &m, void **init, void **state) {
     size_t o_ids = plan.take((size_t)rows * 8), o_pos = plan.take((size_t)c.seq_q * 8);
     size_t o_sc = plan.take(32 + (size_t)c.batch * 4), o_tok = plan.take((size_t)m.token_cap * 4);
     size_t o_as = plan.take(attn_scratch_bytes(c.batch, c.n_heads, c.seq_q, c.head_dim, m.nsplit));
+    size_t o_arr = plan.take(c.seq_q == 1 ? (size_t)kAttnArrive * 4 : 0);
     size_t o_cand = plan.take(rows == 1 ? (size_t)kGemvArgmaxWords * 8 : 0);
     size_t o_tgp = plan.take(tg_part_bytes), o_tgc = plan.take(tg_part_bytes ? (size_t)kTgCounters * 4 : 0);
     const size_t amax_bytes = argmax_scratch_bytes(c.batch, V);
@@ -984,6 +994,7 @@ static int build(Model &m, void **init, void **state) {
     m.d_next = m.d_past + 8;  // one token per sequence after the scalars
     m.d_tokens = (int32_t *)(m.arena + o_tok);
     m.attn_scratch = m.arena + o_as;
+    m.attn_arrive = c.seq_q == 1 ? (int *)(m.arena + o_arr) : nullptr;
     m.tg_part = m.arena + o_tgp;
     m.tg_counters = (int *)(m.arena + o_tgc);
     m.lm_cand = (uint64_t *)(m.arena + o_cand);
