@@ -439,10 +439,11 @@ int attention_decode_launch(AttnParams p, int D, int dtype, int kv_int8, void *s
                  "fused decode attention: position, past_len and active length must be device scalars");
     // the plan (attn_plan, with the same kv_len) was made for the streaming kernel when it is eligible
     const int kv_len = p.d_active ? p.cache_len : (p.active < p.cache_len ? p.active : p.cache_len);
-    if ((!fuse || p.fuse_stream) && !p.mask && attn_stream_eligible(p.B, p.Sq, p.Hq, p.Hkv, D, dtype, kv_int8, kv_len, p.cache_len))
+    if (fuse && p.fuse_stream) return attention_stream_launch(p, D, dtype, kv_int8, s);
+    if (!fuse && !p.mask && attn_stream_eligible(p.B, p.Sq, p.Hq, p.Hkv, D, dtype, kv_int8, kv_len, p.cache_len))
         return attention_stream_launch(p, D, dtype, kv_int8, s);
     if (p.page_table) {  // (the plan is the streaming kernel's: that kernel has the paged form)
-        MYNN_REQUIRE((!fuse || p.fuse_stream) && !p.mask, MYNN_ERR_UNSUPPORTED, "paged attention: neither the latency kernel's fused form nor a mask");
+        MYNN_REQUIRE(!fuse && !p.mask, MYNN_ERR_UNSUPPORTED, "paged attention: neither the latency kernel's fused form nor a mask");
         return attention_stream_launch(p, D, dtype, kv_int8, s);
     }
     bool whole = false;  // the launch wrote the finished output: nothing to merge whatever the plan's split count

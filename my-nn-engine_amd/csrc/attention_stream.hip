@@ -50,9 +50,10 @@ constexpr long kStreamMinKeys = 8192;
 // (pages hold a power of two >= 32 rows, tiles start at multiples of 32), so the page is a wave-uniform value per
 // tile: the workgroup's part of the table sits in one register (lane i = the i-th page of its key range, at most 64)
 // and a tile picks its entry with v_readlane -- no dependent load in the key loop.
-// FUSE: q is the raw q|k|v projection row of the sequence; the kernel rotates the queries itself, and the workgroup whose
-// key range holds row *d_past writes the new key (rotated) and value there before it walks its keys: the RoPE + append
-// launch in front of it disappears.
+// FUSE: q is the raw q|k|v projection row of the sequence; the kernel rotates the queries itself, and the wave whose tiles
+// hold row *d_past makes the new key (rotated) and value, writes them to the cache and keeps them in LDS, where it takes
+// them from when it comes to their tile: the RoPE + append launch in front of it disappears and nobody waits for a store.
+// (Written first and read back like any other row, behind a barrier: 8 us more at 32 sequences x 2048 keys.)
 // What the kernel needs of AttnParams (a launch pays for its argument bytes: 0.9 us of host time for 300 against 60).
 struct StreamParams {
     void *out;
@@ -111,51 +112,72 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
         const int pg = __builtin_amdgcn_readlane(pg_reg, __builtin_amdgcn_readfirstlane((t0 >> psh) - pg0));
         return ((size_t)pg * p.Hkv + hkv) << psh;
     };
-    if constexpr (FUSE) {
-        if (owner) {
-            // wave 0 the key, wave 1 the value of the new row: lane i < D/2 has elements i and i + D/2
-            constexpr int half = D / 2;
-            const size_t tok = kv_cache_row(KvPaging{PAGED ? p.page_table : nullptr, p.page_shift, p.pages_per_seq}, b, hkv, past, p.Hkv, p.cache_len);
-            if (wave < 2) {
-                const bool on = lane < half, is_k = wave == 0;
-                const T *src = (const T *)p.q + (size_t)b * p.q_bs + (size_t)(p.Hq + (is_k ? 0 : p.Hkv) + hkv) * D;
-                float lo = 0.f, hi = 0.f;
-                if (on) {
-                    lo = Elem<T>::ld(src, lane);
-                    hi = Elem<T>::ld(src, lane + half);
-                    if (is_k) {
-                        const T *ct = (const T *)p.cos_t + (size_t)*p.d_pos * D, *st = (const T *)p.sin_t + (size_t)*p.d_pos * D;
-                        const float rl = Elem<T>::rnd(lo * Elem<T>::ld(ct, lane) - hi * Elem<T>::ld(st, lane));
-                        const float rh = Elem<T>::rnd(hi * Elem<T>::ld(ct, lane + half) + lo * Elem<T>::ld(st, lane + half));
-                        lo = rl;
-                        hi = rh;
-                    }
-                }
-                if constexpr (KVI8) {  // the rule of rope_quant_kv_append_kernel
-                    const float amax = wave_max(fmaxf(fabsf(lo), fabsf(hi)));
-                    const float inv = amax == 0.f ? 0.f : 127.0f / amax;
-                    auto code = [&](float x) -> int8_t {
-                        const float a = x * inv;
-                        const int q = (int)(a + (a >= 0.f ? 0.5f : -0.5f));
-                        return (int8_t)(q < -128 ? -128 : (q > 127 ? 127 : q));
-                    };
-                    if (lane == 0) Elem<T>::st((T *)(is_k ? p.k_scale : p.v_scale), tok, amax * (1.0f / 127.0f));
-                    int8_t *dst = (int8_t *)(is_k ? p.k : p.v) + tok * D;
-                    if (on) {
-                        dst[lane] = code(lo);
-                        dst[lane + half] = code(hi);
-                    }
-                } else if (on) {
-                    T *dst = (T *)(is_k ? p.k : p.v) + tok * D;
-                    Elem<T>::st(dst, lane, lo);
-                    Elem<T>::st(dst, lane + half, hi);
-                }
+    // FUSE: the new row as the cache holds it, and its scales (KVI8)
+    __shared__ __align__(16) TKV new_row[2][FUSE ? D : 1];
+    __shared__ T new_scale[2];
+    const bool new_here = FUSE && past >= k0 && past < k1;  // ... is one of this key range's
+    const bool new_mine = owner && wave == (new_here ? ((past - k0) / kStreamTile) % kStreamWaves : 0);
+    struct NewRow {
+        T lo[2], hi[2], cl, ch, sl, sh;  // as loaded: k and v, cos and sin of this lane's pair (elements i and i + D/2)
+    };
+    auto request = [&](NewRow &r) {  // (in front of the first tile's loads: loads return in order)
+        constexpr int half = D / 2;
+        const T *src = (const T *)p.q + (size_t)b * p.q_bs + (size_t)(p.Hq + hkv) * D;
+        const T *ct = (const T *)p.cos_t + (size_t)*p.d_pos * D, *st = (const T *)p.sin_t + (size_t)*p.d_pos * D;
+        const int i = min(lane, half - 1);
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            r.lo[v] = src[(size_t)v * p.Hkv * D + i];
+            r.hi[v] = src[(size_t)v * p.Hkv * D + i + half];
+        }
+        r.cl = ct[i];
+        r.ch = ct[i + half];
+        r.sl = st[i];
+        r.sh = st[i + half];
+    };
+    auto append = [&](const NewRow &r) {
+        constexpr int half = D / 2;
+        const size_t tok = kv_cache_row(KvPaging{PAGED ? p.page_table : nullptr, p.page_shift, p.pages_per_seq}, b, hkv, past, p.Hkv, p.cache_len);
+        const int i = min(lane, half - 1);
+        auto f = [](const T &x) { return Elem<T>::ld(&x, 0); };
+        float lo[2] = {f(r.lo[0]), f(r.lo[1])}, hi[2] = {f(r.hi[0]), f(r.hi[1])};
+        const float rl = Elem<T>::rnd(lo[0] * f(r.cl) - hi[0] * f(r.sl));
+        const float rh = Elem<T>::rnd(hi[0] * f(r.ch) + lo[0] * f(r.sh));
+        lo[0] = rl;
+        hi[0] = rh;
+#pragma unroll
+        for (int v = 0; v < 2; v++) {
+            TKV *dst = (TKV *)(v ? p.v : p.k) + tok * D;
+            if constexpr (KVI8) {  // the rule of rope_quant_kv_append_kernel
+                const float amax = wave_max(fmaxf(fabsf(lo[v]), fabsf(hi[v])));
+                const float inv = amax == 0.f ? 0.f : 127.0f / amax;
+                auto code = [&](float x) -> int8_t {
+                    const float a = x * inv;
+                    const int q = (int)(a + (a >= 0.f ? 0.5f : -0.5f));
+                    return (int8_t)(q < -128 ? -128 : (q > 127 ? 127 : q));
+                };
+                Elem<T>::st(&new_scale[v], 0, amax * (1.0f / 127.0f));
+                if (lane == 0) Elem<T>::st((T *)(v ? p.v_scale : p.k_scale), tok, amax * (1.0f / 127.0f));
+                new_row[v][i] = code(lo[v]);
+                new_row[v][i + half] = code(hi[v]);
+            } else {
+                Elem<T>::st(new_row[v], i, lo[v]);
+                Elem<T>::st(new_row[v], i + half, hi[v]);
             }
-            // the row is read back by this workgroup: written through, and no older copy of its line left in the L1
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            if (split >= n_act) return;
+            if (lane < half) {
+                dst[lane] = new_row[v][lane];
+                dst[lane + half] = new_row[v][lane + half];
+            }
+        }
+    };
+    if constexpr (FUSE) {
+        if (split >= n_act) {  // a range without rows that the new one is appended behind
+            if (new_mine) {
+                NewRow r;
+                request(r);
+                append(r);
+            }
+            return;
         }
     }
     auto operand = [](const Chunk &c) -> U4 {
@@ -165,32 +187,16 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
     const int col = lane & 15, quad = lane >> 4;  // MFMA column (head) and row/k group of this lane
 
     // Q^T as the B operand of the score product: column = head, k = dims 8*quad..+7 of each block
-    U4 qf[KB];
+    U4 qf[KB], cs[2][FUSE ? KB : 1];
     {
         const T *qrow = (const T *)p.q + (size_t)b * p.q_bs + (size_t)(head0 + (col < G ? col : 0)) * p.q_hs;
 #pragma unroll
         for (int j = 0; j < KB; j++) {
             qf[j] = *(const U4 *)(qrow + j * 32 + quad * 8);
             if (col >= G) qf[j] = U4{0u, 0u, 0u, 0u};
-        }
-        if constexpr (FUSE) {  // dims d and d + D/2 of a rotation pair are blocks j and j + KB/2 of the same lane
-            const T *ct = (const T *)p.cos_t + (size_t)*p.d_pos * D + quad * 8, *st = (const T *)p.sin_t + (size_t)*p.d_pos * D + quad * 8;
-#pragma unroll
-            for (int j = 0; j < KB / 2; j++) {
-                float xl[8], xh[8], cl[8], ch[8], sl[8], sh[8], ol[8], oh[8];
-                widen8<T>(qf[j], xl);
-                widen8<T>(qf[j + KB / 2], xh);
-                widen8<T>(*(const U4 *)(ct + j * 32), cl);
-                widen8<T>(*(const U4 *)(ct + (j + KB / 2) * 32), ch);
-                widen8<T>(*(const U4 *)(st + j * 32), sl);
-                widen8<T>(*(const U4 *)(st + (j + KB / 2) * 32), sh);
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    ol[i] = xl[i] * cl[i] - xh[i] * sl[i];
-                    oh[i] = xh[i] * ch[i] + xl[i] * sh[i];
-                }
-                qf[j] = U4{pack2<T>(ol[0], ol[1]), pack2<T>(ol[2], ol[3]), pack2<T>(ol[4], ol[5]), pack2<T>(ol[6], ol[7])};
-                qf[j + KB / 2] = U4{pack2<T>(oh[0], oh[1]), pack2<T>(oh[2], oh[3]), pack2<T>(oh[4], oh[5]), pack2<T>(oh[6], oh[7])};
+            if constexpr (FUSE) {
+                cs[0][j] = *(const U4 *)((const T *)p.cos_t + (size_t)*p.d_pos * D + j * 32 + quad * 8);
+                cs[1][j] = *(const U4 *)((const T *)p.sin_t + (size_t)*p.d_pos * D + j * 32 + quad * 8);
             }
         }
     }
@@ -242,7 +248,36 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
         T v = __builtin_bit_cast(T, b);
         return Elem<T>::ld(&v, 0);
     };
-    auto process = [&](int t, const Chunk (*kr)[KB], const Chunk *vr, const uint2 *sr) {
+    auto process = [&](int t, Chunk (*kr)[KB], Chunk *vr, uint2 *sr) {
+        if constexpr (FUSE) {
+            if (new_here && new_mine && past >= t && past < t + kStreamTile) {
+                // (rows past the range stand for its last one, which may be the new row: no old content of it is used)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+                    if (min(t + a * 16 + col, k1 - 1) == past) {
+#pragma unroll
+                        for (int j = 0; j < KB; j++) kr[a][j] = *(const Chunk *)&new_row[0][j * 32 + quad * 8];
+                    }
+#pragma unroll
+                for (int q = 0; q < NP; q++)
+                    if (min(t + q * KPP + vk, k1 - 1) == past) vr[q] = *(const Chunk *)&new_row[1][vd];
+                if constexpr (KVI8) {
+#pragma unroll
+                    for (int a = 0; a < 2; a++) {
+                        const int e = past - (t + a * 16 + quad * 4);
+                        if (e >= 0 && e < 4) {
+                            auto put = [&](uint2 &four, T v) {
+                                const uint32_t bits = __builtin_bit_cast(uint16_t, v), keep = e & 1 ? 0xFFFFu : 0xFFFF0000u, sh = e & 1 ? 16 : 0;
+                                if (e < 2) four.x = (four.x & keep) | bits << sh;
+                                else four.y = (four.y & keep) | bits << sh;
+                            };
+                            put(sr[a], new_scale[0]);
+                            put(sr[2 + a], new_scale[1]);
+                        }
+                    }
+                }
+            }
+        }
         // ---- park V: [key][dim], two 8-byte stores per lane and pass
 #pragma unroll
         for (int q = 0; q < NP; q++) {
@@ -338,6 +373,11 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
     // order of the tiles changes nothing but the rounding of the online softmax, and it is a fixed function of the
     // grid.
     const int nt = (k1 - k0 - wave * kStreamTile + tstep - 1) / tstep;
+    NewRow fresh;
+    if constexpr (FUSE) {
+        if (new_mine) request(fresh);
+        if (nt <= 0 && new_mine) append(fresh);
+    }
     if (nt > 0) {
         const int rot = (int)((unsigned)(b + split) % (unsigned)nt);
         auto tile_at = [&](int n) {
@@ -347,6 +387,28 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
         };
         int n = 0;
         load_tile(tile_at(0), kA, vA, sA);
+        if constexpr (FUSE) {
+            // rotate the queries: dims d and d + D/2 of a pair are blocks j and j + KB/2 of the same lane
+#pragma unroll
+            for (int j = 0; j < KB / 2; j++) {
+                float xl[8], xh[8], cl[8], ch[8], sl[8], sh[8], ol[8], oh[8];
+                widen8<T>(qf[j], xl);
+                widen8<T>(qf[j + KB / 2], xh);
+                widen8<T>(cs[0][j], cl);
+                widen8<T>(cs[0][j + KB / 2], ch);
+                widen8<T>(cs[1][j], sl);
+                widen8<T>(cs[1][j + KB / 2], sh);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    ol[i] = xl[i] * cl[i] - xh[i] * sl[i];
+                    oh[i] = xh[i] * ch[i] + xl[i] * sh[i];
+                }
+                qf[j] = U4{pack2<T>(ol[0], ol[1]), pack2<T>(ol[2], ol[3]), pack2<T>(ol[4], ol[5]), pack2<T>(ol[6], ol[7])};
+                qf[j + KB / 2] = U4{pack2<T>(oh[0], oh[1]), pack2<T>(oh[2], oh[3]), pack2<T>(oh[4], oh[5]), pack2<T>(oh[6], oh[7])};
+            }
+            if (new_mine) append(fresh);
+            __builtin_amdgcn_wave_barrier();
+        }
         while (true) {
             load_tile(tile_at(n + 1), kB, vB, sB);
             process(tile_at(n), kA, vA, sA);

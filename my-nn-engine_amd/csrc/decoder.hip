@@ -175,6 +175,7 @@ struct Model {
     void *tg_part = nullptr;     // tile_gemm's partial sums and arrival counters
     int *tg_counters = nullptr;
     bool skinny = false;      // 16..64 rows: int8 weights streamed once through the few-row matrix-core kernel
+    bool rowblock = false;    // ... up to 32 rows: a linear is one launch (rowblock.hip), with the norm in front up to 16
     float *skinny_scratch = nullptr;
     void *cos_t = nullptr, *sin_t = nullptr;
     // arena
@@ -314,6 +315,21 @@ static int skinny_rows(Model &m, void *out, const void *act, const Lin &l, const
          2.0 * M * l.N * l.K);
     return dequant_gemm_skinny(out, act, (const int8_t *)(packed ? packed : l.w), packed != nullptr, l.scale, res, M, l.N, l.K,
                                m.cfg.dtype, epi, m.skinny_scratch, m.stream, next_norm, m.cfg.eps, m.nrm, normed, rope, roped);
+}
+
+// a linear of a rowblock executor on x, or on its RMSNorm: one launch where the kernel has the form, else norm + product
+static int rowblock_rows(Model &m, void *out, const void *x, const void *norm_w, const Lin &l, const void *packed, const void *res, int M, int epi,
+                         const char *name) {
+    const double eb = dtype_size(m.cfg.dtype), n_out = epi == GEMM_SWIGLU ? l.N / 2 : l.N;
+    const bool norm_in = norm_w && rowblock_supported(M, l.N, l.K, true);
+    if (norm_w && !norm_in) {
+        note(m, "rms_norm", 2.0 * M * l.K * eb + l.K * eb);
+        TRY(mynn_rms_norm(m.nrm, x, norm_w, M, l.K, m.cfg.eps, m.cfg.dtype, m.stream));
+        x = m.nrm;
+    }
+    if (!rowblock_supported(M, l.N, l.K, norm_in)) return skinny_rows(m, out, x, l, packed, res, M, epi, name);
+    note(m, name, (double)l.N * l.K + l.N * eb + (double)M * l.K * eb + (double)M * n_out * eb * (epi == GEMM_RESIDUAL ? 2 : 1), 2.0 * M * l.N * l.K);
+    return rowblock_gemm(out, x, packed, l.scale, res, norm_in ? norm_w : nullptr, m.cfg.eps, M, l.N, l.K, m.cfg.dtype, epi, m.stream);
 }
 
 // Options::quantize_activations: DynamicQuantizeLinear (per row, symmetric) then QuantizedMatMul.
@@ -461,6 +477,8 @@ static int enqueue_step(Model &m) {
             TRY(gemv_norm<T>(m.qkv, m.x, L.norm1, c.eps, (const int8_t *)L.qkv.w, L.qkv.scale, L.qkv.N, H, s));
         } else if (qfused) {
             TRY(qlinear1(m.qkv, m.x, L.norm1, L.qkv, nullptr, GEMM_PLAIN, "qgemv_norm_quant_qkv"));
+        } else if (m.rowblock) {
+            TRY(rowblock_rows(m, m.qkv, m.x, L.norm1, L.qkv, L.pk_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv"));
         } else if (m.w8a8_fused) {
             TRY(qlinear_fused(m, m.pl_qkv, m.qkv, m.x, L.norm1, L.qkv, nullptr, rows, GEMM_PLAIN, "qlinear_qkv"));
         } else {
@@ -546,6 +564,10 @@ static int enqueue_step(Model &m) {
             TRY(gemv_norm_swiglu<T>(m.hmid, m.x2, L.norm2, c.eps, (const int8_t *)L.gu.w, L.gu.scale, L.gu.N, H, s, fill, fill_words));
             note(m, "gemv_down_residual", (double)H * F + H * eb + F * eb + 2 * H * eb);
             TRY(gemv_residual<T>(m.x, m.hmid, (const int8_t *)L.down.w, L.down.scale, m.x2, H, F, s));
+        } else if (m.rowblock) {
+            TRY(rowblock_rows(m, m.x2, m.attn, nullptr, L.o, L.pk_o, m.x, rows, GEMM_RESIDUAL, "linear_o_residual"));
+            TRY(rowblock_rows(m, m.hmid, m.x2, L.norm2, L.gu, L.pk_gu, nullptr, rows, GEMM_SWIGLU, "linear_gateup_swiglu"));
+            TRY(rowblock_rows(m, m.x, m.hmid, nullptr, L.down, L.pk_down, m.x2, rows, GEMM_RESIDUAL, "linear_down_residual"));
         } else if (m.skinny) {
             bool normed = false;
             TRY(skinny_rows(m, m.x2, m.attn, L.o, L.pk_o, m.x, rows, GEMM_RESIDUAL, "linear_o_residual", L.norm2, &normed));
@@ -612,6 +634,8 @@ static int enqueue_step(Model &m) {
         TRY(gemv_norm<T>(m.logits, m.x, m.final_norm, c.eps, (const int8_t *)m.lm_head.w, m.lm_head.scale, V, H, s));
     } else if (qfused) {
         TRY(qlinear1(m.logits, m.x, m.final_norm, m.lm_head, nullptr, GEMM_PLAIN, "qgemv_norm_quant_lm_head"));
+    } else if (m.rowblock) {
+        TRY(rowblock_rows(m, m.logits, m.x, m.final_norm, m.lm_head, m.pk_lm_head, nullptr, rows, GEMM_PLAIN, "linear_lm_head"));
     } else if (m.w8a8_fused) {
         TRY(qlinear_fused(m, m.pl_lm, m.logits, m.x, m.final_norm, m.lm_head, nullptr, rows, GEMM_PLAIN, "qlinear_lm_head"));
     } else {
@@ -794,6 +818,8 @@ static int build(Model &m, void **init, void **state) {
         m.skinny = m.quant && !c.quantize_activations && skinny_gemm_supported(rows_, QD + 2 * KD, H) &&
                    skinny_gemm_supported(rows_, H, QD) && skinny_gemm_supported(rows_, 2 * F, H) &&
                    skinny_gemm_supported(rows_, H, F) && skinny_gemm_supported(rows_, V, H);
+        m.rowblock = m.skinny && c.seq_q == 1 && rowblock_supported(rows_, QD + 2 * KD, H, false) && rowblock_supported(rows_, H, QD, false) &&
+                     rowblock_supported(rows_, H, F, false);
     }
     // which linears of a matrix-core executor multiply by tiles of the int8 weights as they are: those too small for the
     // 256-row kernels to be the faster ones (some 1500 rows for a 11264 x 2048 matrix, every int8 product below half a
@@ -932,13 +958,19 @@ static int build(Model &m, void **init, void **state) {
     {
         // decode over a cache longer than the short form takes: the streaming kernel with RoPE and the appends inside
         m.attn_stream_fuse = c.seq_q == 1 && !c.streaming_kv && !(c.unfused_decode && c.batch > 1) && c.batch * c.n_kv_heads <= kAttnArrive &&
-                             (m.pages ? attn_stream_paged_supported(1, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, 1 << m.paging.shift)
-                                      : attn_stream_eligible(c.batch, 1, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, c.quant_kv_cache, c.max_seq, c.max_seq)) &&
+                             attn_stream_paged_supported(1, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, 32) &&
+                             (m.pages || (c.max_seq >= 32 && (!c.quant_kv_cache || c.max_seq % 32 == 0))) &&
+                             (m.pages || c.batch > 1 ||
+                              attn_stream_eligible(c.batch, 1, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, c.quant_kv_cache, c.max_seq, c.max_seq)) &&
                              !(rows == 1 && !m.pages && attention_fused_kv8_supported(c.head_dim, c.max_seq));
         const bool fused_attn = m.quant && rows == 1 && !c.quantize_activations && !c.quant_kv_cache && !m.pages && !m.attn_stream_fuse &&
                                 attention_fused_supported(c.head_dim, c.n_heads / c.n_kv_heads);
         attn_plan(c.batch, c.seq_q, c.n_heads, c.n_kv_heads, c.head_dim, c.dtype, c.quant_kv_cache, c.max_seq, c.max_seq, fused_attn,
                   &m.slice, &m.nsplit, &m.heads_per_wg);
+        if (m.attn_stream_fuse && !m.pages) {
+            m.heads_per_wg = c.n_heads / c.n_kv_heads;
+            attn_stream_plan(c.batch, c.n_kv_heads, c.max_seq, &m.slice, &m.nsplit);
+        }
         if (m.pages) {  // decode: the streaming kernel whatever the sizes; prefill: the matrix-core kernel, no key ranges
             m.slice = 0;
             m.nsplit = 1;

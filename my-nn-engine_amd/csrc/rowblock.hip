@@ -1,0 +1,254 @@
+// DequantMatMul for a handful of activation rows (2 <= M <= 32: small decode batches), one launch per linear.
+//
+// At this size a linear is a few microseconds, of which skinny.hip's form -- K ranges over workgroups, partial sums through
+// memory, a second launch that adds them up -- spends more on the second launch than on the weights.  Here one workgroup
+// owns 32 weight rows (RB row blocks) over the WHOLE K range: its waves split K among themselves, every wave has its share of
+// the weights in flight before the first product, and the partial sums meet in LDS, so the workgroup stores finished
+// output: scale, residual or SwiGLU, and in front the RMSNorm of the activation rows while they are staged (NORM).
+//
+//   out[m,n] = T(scale[n] * sum_k act[m,k] * wq[n,k])   (scale after the f32 sum, as skinny.hip)
+//
+// The weights are skinny.hip's tiled copy: a wave's step of 32 rows x 128 k is 4 KB, read by four sequential loads, and
+// turned exactly into the A operand of v_mfma_f32_32x32x16; the activation rows are the B operand's columns, read from LDS.
+#include <type_traits>
+
+#include "kernels.h"
+#include "mfma.h"
+
+namespace mynn {
+
+// WAVES waves of a workgroup: RB row blocks times WK shares of a slab of WK * 128 k (a step per wave).  DEPTH slabs of
+// weights are in flight per wave.  Activations, plain form: panels of SPP slabs, [M] rows, copied global -> LDS by the load
+// unit, the next panel while one is multiplied; NORM > 0: whole rows at once, NORM 16-byte pieces per lane.
+constexpr int kRbMaxRows = 32, kRbWaves = 8, kRbDepth = 4, kRbRed = 36;  // (floats per row of partial sums)
+template <int RB, int SPP> constexpr int rb_panel_k() { return kRbWaves / RB * 128 * SPP; }
+template <int RB, int SPP> constexpr int rb_row_bytes() { return (rb_panel_k<RB, SPP>() + 511) / 512 * 1024 + 16; }
+
+template <typename T, int RB, int SPP, int EPI, int NORM>
+__global__ __launch_bounds__(kRbWaves * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, const T *scale, const T *res, const T *norm_w, T *out,
+                                                                      int M, int N, int K, float eps) {
+    constexpr int WAVES = kRbWaves, WK = WAVES / RB, DEPTH = kRbDepth, RS = kRbRed;
+    extern __shared__ __align__(16) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 31, h = lane >> 5, rb = wave / WK, kw = wave % WK;
+    const int row_blocks = (N + 31) / 32, iters = K / 128, slabs = (iters + WK - 1) / WK;
+    const size_t pitch = (size_t)row_blocks * 256;  // 16-byte pieces of one step over all row blocks
+    const U4 *wsrc = pk + (size_t)min((int)blockIdx.x * RB + rb, row_blocks - 1) * 256 + lane;
+    U4 w[DEPTH][4];
+    auto load_w = [&](int sl, U4 *dst) {
+        const U4 *p = wsrc + (size_t)min(sl * WK + kw, iters - 1) * pitch;
+#pragma unroll
+        for (int j = 0; j < 4; j++) dst[j] = __builtin_nontemporal_load(p + j * 64);
+    };
+    // what the store of this thread's first output needs (mostly its only one), fetched in front of everything else
+    constexpr int PR = EPI == GEMM_SWIGLU ? 16 : 32;  // outputs per row block and activation row
+    T sc0, sc1, rs0;
+    {
+        const int o = min(tid, RB * M * PR - 1), c = o % PR, m = (o / PR) % M, n = min((((int)blockIdx.x * RB + o / (PR * M)) * 32) + (EPI == GEMM_SWIGLU ? 2 * c : c), N - 1);
+        sc0 = scale[n];
+        if constexpr (EPI == GEMM_SWIGLU) sc1 = scale[min(n + 1, N - 1)];
+        if constexpr (EPI == GEMM_RESIDUAL) rs0 = res[(size_t)m * N + n];
+    }
+    f16x_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+    const int mrow = min(r, M - 1);  // (columns past M repeat the last row and are not stored)
+    auto multiply = [&](const U4 *q, const char *arow) {  // arow: this lane's activation row at the step's first k
+        U4 b[8];
+#pragma unroll
+        for (int s = 0; s < 8; s++) b[s] = *(const U4 *)(arow + 128 * h + 16 * s);
+#pragma unroll
+        for (int s = 0; s < 8; s += 2) {
+            U4 c = q[s >> 1];
+            pin(c);  // (converted here, not when they were loaded)
+            acc = Mfma<T>::run(i8x8_to_operand<T>(c.x, c.y), b[s], acc);
+            acc = Mfma<T>::run(i8x8_to_operand<T>(c.z, c.w), b[s + 1], acc);
+        }
+    };
+    if constexpr (NORM > 0) {
+        // whole rows, a wave each: requested before the weights, as loads return in order
+        const int AS = K * 2 + 16, pieces = K >> 3;
+        for (int m = wave; m < M || m == wave; m += WAVES) {
+            U4 v[NORM], nw[NORM];
+            const int ml = min(m, M - 1);
+#pragma unroll
+            for (int q = 0; q < NORM; q++) {
+                const int c = min(lane + q * 64, pieces - 1);
+                v[q] = *(const U4 *)(act + (size_t)ml * K + c * 8);
+                nw[q] = *(const U4 *)(norm_w + c * 8);
+            }
+            if (m == wave) {
+#pragma unroll
+                for (int d = 0; d < DEPTH; d++) load_w(d, w[d]);
+            }
+            if (m >= M) break;
+            float ss = 0.f;
+#pragma unroll
+            for (int q = 0; q < NORM; q++) {
+                float f[8];
+                widen8<T>(v[q], f);
+                if (lane + q * 64 < pieces) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) ss += f[i] * f[i];
+                }
+            }
+            const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)K + eps);
+#pragma unroll
+            for (int q = 0; q < NORM; q++) {
+                const int c = lane + q * 64;
+                float f[8], g[8];
+                widen8<T>(v[q], f);
+                widen8<T>(nw[q], g);
+                if (c < pieces)
+                    *(U4 *)(lds + (size_t)m * AS + c * 16) = U4{pack2<T>((f[0] * inv) * g[0], (f[1] * inv) * g[1]), pack2<T>((f[2] * inv) * g[2], (f[3] * inv) * g[3]),
+                                                               pack2<T>((f[4] * inv) * g[4], (f[5] * inv) * g[5]), pack2<T>((f[6] * inv) * g[6], (f[7] * inv) * g[7])};
+            }
+        }
+        __syncthreads();
+        const char *arow = lds + (size_t)mrow * AS + kw * 256;
+        for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; d++) {
+                const int sl = s0 + d;
+                if (sl * WK + kw < iters) multiply(w[d], arow + (size_t)sl * WK * 256);
+                if (s0 + DEPTH < slabs) load_w(sl + DEPTH, w[d]);
+            }
+        }
+    } else {
+        constexpr int PK = rb_panel_k<RB, SPP>(), AS = rb_row_bytes<RB, SPP>(), CPR = (PK + 511) / 512;  // 1 KB copies per row
+        const int panels = (slabs + SPP - 1) / SPP;
+        auto issue_panel = [&](int p) {
+            char *dst = lds + (size_t)(p & 1) * M * AS;
+            for (int c = wave; c < M * CPR; c += WAVES) {
+                const int m = c / CPR, k = p * PK + (c % CPR) * 512 + lane * 8;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(act + (size_t)m * K + min(k, K - 8)),
+                                                 (__attribute__((address_space(3))) void *)(dst + (size_t)m * AS + (c % CPR) * 1024), 16, 0, 0);
+            }
+        };
+        issue_panel(0);
+        asm volatile("" ::: "memory");  // (the counts below rely on the order of the requests)
+#pragma unroll
+        for (int d = 0; d < DEPTH; d++) load_w(d, w[d]);
+        const char *arow = lds + (size_t)mrow * AS + kw * 256;
+        constexpr int AGE = (SPP < DEPTH ? SPP : DEPTH) * 4;  // weight loads younger than the panel that is waited for, at least
+        for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; d++) {
+                const int sl = s0 + d;
+                if (sl < slabs) {
+                    if (sl % SPP == 0) {
+                        // this panel is here, everyone is done with the one before it: its buffer takes the next
+                        __builtin_amdgcn_s_waitcnt((AGE & 15) | (AGE >> 4) << 14 | 0x70);
+                        asm volatile("" ::: "memory");
+                        __builtin_amdgcn_s_barrier();
+                        asm volatile("" ::: "memory");
+                        if (sl / SPP + 1 < panels) issue_panel(sl / SPP + 1);
+                        asm volatile("" ::: "memory");
+                    }
+                    if (sl * WK + kw < iters) multiply(w[d], arow + (size_t)((sl / SPP) & 1) * M * AS + (size_t)(sl % SPP) * WK * 256);
+                }
+                load_w(sl + DEPTH, w[d]);  // (past the end: the last step once more, unused; it keeps the counts)
+            }
+        }
+    }
+    __syncthreads();  // the activations are done with: their memory takes the partial sums
+
+    // D[n][m]: lane holds column m = lane % 32 and rows n = 8*(e/4) + 4*(lane/32) + e%4
+    float *red = (float *)lds;
+    if (r < M) {
+        float *dst = red + ((size_t)(kw * RB + rb) * M + r) * RS + 4 * h;
+#pragma unroll
+        for (int e4 = 0; e4 < 4; e4++) *(float4 *)(dst + e4 * 8) = float4{acc[e4 * 4], acc[e4 * 4 + 1], acc[e4 * 4 + 2], acc[e4 * 4 + 3]};
+    }
+    __syncthreads();
+    for (int o = tid; o < RB * M * PR; o += WAVES * 64) {
+        const int c = o % PR, m = (o / PR) % M, b = o / (PR * M);
+        const int n0 = ((int)blockIdx.x * RB + b) * 32;
+        const bool first = o == tid;
+        auto total = [&](int n) {
+            float t = 0.f;
+#pragma unroll
+            for (int k = 0; k < WK; k++) t += red[((size_t)(k * RB + b) * M + m) * RS + n];
+            return t;
+        };
+        if constexpr (EPI == GEMM_SWIGLU) {  // rows 2i / 2i+1 of the weight are gate_i / up_i
+            const int n = n0 + 2 * c;
+            if (n + 1 < N) {
+                const T sg = first ? sc0 : scale[n], su = first ? sc1 : scale[n + 1];
+                const float g = Elem<T>::rnd(total(2 * c) * Elem<T>::ld(&sg, 0)), u = Elem<T>::rnd(total(2 * c + 1) * Elem<T>::ld(&su, 0));
+                const float sig = 1.0f / (1.0f + expf(-g));
+                Elem<T>::st(out, (size_t)m * (N >> 1) + (n >> 1), (g * sig) * u);
+            }
+        } else {
+            const int n = n0 + c;
+            if (n < N) {
+                const T sn = first ? sc0 : scale[n];
+                float y = total(c) * Elem<T>::ld(&sn, 0);
+                if constexpr (EPI == GEMM_RESIDUAL) {
+                    const T rn = first ? rs0 : res[(size_t)m * N + n];
+                    y = Elem<T>::rnd(y) + Elem<T>::ld(&rn, 0);
+                }
+                Elem<T>::st(out, (size_t)m * N + n, y);
+            }
+        }
+    }
+}
+
+// ---- which form.  One row block per workgroup while that is at most one workgroup per CU (its eight waves split K), two
+// beyond; from 768 row blocks on skinny.hip's one-launch form streams the weights just as fast (28672 x 4096, 8 rows: 23
+// us) and this one is not taken.  The norm rides along up to 16 rows (8 rows x 2560 x 2048: 7.3 us with it against 6.0 +
+// a launch of 2.5; every workgroup normalises all rows for itself, at 32 rows that costs 3.7 us).
+static size_t rb_lds(int M, int N, int K, bool norm) {
+    const int blocks = (N + 31) / 32;
+    size_t act;
+    if (norm) act = (size_t)M * (K * 2 + 16);
+    else if (blocks <= 256) act = (size_t)(K > rb_panel_k<1, 1>() ? 2 : 1) * M * rb_row_bytes<1, 1>();
+    else act = (size_t)(K > rb_panel_k<2, 2>() ? 2 : 1) * M * rb_row_bytes<2, 2>();
+    const size_t red = (size_t)kRbWaves * M * kRbRed * sizeof(float);
+    return act > red ? act : red;
+}
+bool rowblock_supported(int M, int N, int K, bool norm) {
+    return M >= 1 && M <= kRbMaxRows && (M <= 16 || (long)N * K <= (12l << 20) || (N + 31) / 32 > 256) && K % 128 == 0 && N >= 1 && (N + 31) / 32 < 768 && (!norm || (M <= 16 && K <= 4096)) &&
+           rb_lds(M, N, K, norm) <= 160 * 1024;
+}
+
+template <typename T, int RB, int SPP, int EPI, int NORM>
+static int rb_go(const void *act, const void *pk, const void *scale, const void *res, const void *norm_w, void *out, int M, int N, int K, float eps,
+                 size_t lds, hipStream_t s) {
+    static size_t lds_set = 64 * 1024;
+    if (lds > lds_set) {
+        MYNN_HIP(hipFuncSetAttribute((const void *)rowblock_gemm_kernel<T, RB, SPP, EPI, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        lds_set = 160 * 1024;
+    }
+    MYNN_LAUNCH((rowblock_gemm_kernel<T, RB, SPP, EPI, NORM>), dim3((N + 32 * RB - 1) / (32 * RB)), dim3(kRbWaves * 64), lds, s, (const T *)act,
+                (const U4 *)pk, (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, M, N, K, eps);
+    return launch_status("rowblock_gemm_kernel");
+}
+
+int rowblock_gemm(void *out, const void *act, const void *packed, const void *scale, const void *res, const void *norm_w, float eps, int M, int N,
+                  int K, int dtype, int epi, hipStream_t s) {
+    MYNN_REQUIRE(out && act && packed && scale && (epi != GEMM_RESIDUAL || res), MYNN_ERR_INVALID, "rowblock_gemm: null operand");
+    MYNN_REQUIRE(rowblock_supported(M, N, K, norm_w != nullptr) && (epi != GEMM_SWIGLU || N % 2 == 0), MYNN_ERR_UNSUPPORTED, "rowblock_gemm: M=%d N=%d K=%d", M, N, K);
+    MYNN_REQUIRE(aligned16(act) && aligned16(packed) && (!norm_w || aligned16(norm_w)), MYNN_ERR_INVALID, "rowblock_gemm: operands must be 16-byte aligned");
+    const size_t lds = rb_lds(M, N, K, norm_w != nullptr);
+    const bool one = (N + 31) / 32 <= 256;
+    return dispatch_dtype16(dtype, [&](auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        auto go = [&](auto e) {
+            constexpr int EPI = decltype(e)::value;
+            if (norm_w && K <= 2048)
+                return one ? rb_go<T, 1, 1, EPI, 4>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
+                           : rb_go<T, 2, 2, EPI, 4>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s);
+            if (norm_w)
+                return one ? rb_go<T, 1, 1, EPI, 8>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
+                           : rb_go<T, 2, 2, EPI, 8>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s);
+            return one ? rb_go<T, 1, 1, EPI, 0>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
+                       : rb_go<T, 2, 2, EPI, 0>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s);
+        };
+        if (epi == GEMM_RESIDUAL) return go(std::integral_constant<int, GEMM_RESIDUAL>{});
+        if (epi == GEMM_SWIGLU) return go(std::integral_constant<int, GEMM_SWIGLU>{});
+        return go(std::integral_constant<int, GEMM_PLAIN>{});
+    });
+}
+
+}  // namespace mynn
