@@ -514,10 +514,12 @@ int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, in
 }
 
 // The time of gemm_nt_mfma, microseconds: grids of at least one round of 256 x 256 tiles run at 1.0 - 1.1 PFLOP/s (fp16;
-// bf16 5 % above), smaller ones take as long as one tile does on its CU, which tile_gemm beats at every size measured.
+// bf16 5 % above) of whole tiles, those that take 320 columns at a time (gemm_launch) at 1.13; smaller ones take as long as
+// one tile does on its CU, which tile_gemm beats at every size measured.
 double gemm_nt_mfma_us(int M, int N, int K, int dtype) {
-    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
+    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256), wide = (long)((M + 255) / 256) * ((N + 319) / 320);
     if (tiles < 256) return 1e30;
+    if (K % 64 == 0 && (wide + 255) / 256 * 320 < (tiles + 255) / 256 * 256) return 6.0 + 2.0 * 256 * 320 * K * (double)wide / 1.13e9;
     return 6.0 + 2.0 * 256 * 256 * K * (double)tiles / (dtype == MYNN_BF16 ? 1.10e9 : 1.03e9);
 }
 // ... and of dequant_weight_rows before it (3 bytes per weight)

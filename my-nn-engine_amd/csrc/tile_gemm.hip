@@ -10,7 +10,9 @@
 // 3 bytes per weight that cost more than the product itself below a few hundred rows).  Operand tiles go global -> LDS with
 // global_load_lds_dwordx4, NS stages deep: with this few workgroups per CU what bounds the product is the latency of the
 // weight stream, and the stages in flight are what hides it.  A K step is 128 bytes of an activation row (64 values of 16
-// bits, 128 int8).  16-byte chunks are placed so that the 128-bit fragment reads of 16 neighbouring rows fall into
+// bits, 128 int8); the waves meet at a barrier every KM steps.  KM = 2 where a step is long enough that the meeting, not
+// the load, is what it waits for: 64 x 128 (500 x 11264 x 2048 30.5 -> 29.9 us fp16, 300 rows bf16 26.4 -> 24.3) and the
+// eight waves of 128 x 128 (1000 rows 44.5 -> 43.4); smaller tiles do not change, 128 x 128 of int8 loses 14 %.  16-byte chunks are placed so that the 128-bit fragment reads of 16 neighbouring rows fall into
 // different LDS banks: row r's chunk c at 8r + (c ^ (r/2 & 7)) for 128-byte rows, 4r + (c ^ (r/4 & 3)) for the 64-byte
 // rows of int8 weights against 16-bit activations.
 //
@@ -29,9 +31,9 @@ namespace mynn {
 typedef int i4x_t __attribute__((ext_vector_type(4)));
 typedef int i16x_t __attribute__((ext_vector_type(16)));
 
-template <int KIND_, int BM_, int BN_, int WM_, int WN_, int NS_, int WPE_>
+template <int KIND_, int BM_, int BN_, int WM_, int WN_, int NS_, int WPE_, int KM_>
 struct TgTile {
-    static constexpr int KIND = KIND_, BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, WPE = WPE_;
+    static constexpr int KIND = KIND_, BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, WPE = WPE_, KM = KM_;
     static constexpr int THREADS = WM * WN * 64;
     static constexpr int TI = BM / WM / 32, TJ = BN / WN / 32;
     static constexpr int BROW = KIND == TG_I8 ? 128 : 64;  // bytes of a weight row per K step
@@ -73,6 +75,8 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
                                                                       uint64_t *part, int *counter, int32_t *acc_out) {
     constexpr int KIND = G::KIND, BM = G::BM, BN = G::BN, TI = G::TI, TJ = G::TJ, NS = G::NS, BROW = G::BROW;
     constexpr bool I8 = KIND == TG_I8;
+    // (pinned by hand for int8, 10 - 15 % at 128 x 256, and for the eight-wave fp tile, 4 - 7 %; the others lose by it)
+    constexpr bool MIX = I8 || (TI == 2 && TJ == 1 && G::THREADS == 512);
     constexpr int EA = I8 ? 1 : 2;
     constexpr int CHA = G::CHA, CHB = G::CHB;
     extern __shared__ __align__(16) char lds[];
@@ -204,38 +208,59 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
             }
     };
 
-    // One barrier per K step: behind it the tile of this step is whole (every wave has waited for its own share of the
-    // loads) and the stage of the step before is free.  The fragments of a step are read while the step before multiplies,
-    // so that neither the barrier nor the LDS latency is in front of the MFMAs.
+    // One barrier per KM K steps: behind it the tiles of these steps are whole (every wave has waited for its own share of
+    // the loads) and the stages of the KM steps before are free.  The fragments of a step are read while the step before
+    // multiplies, so that neither the barrier nor the LDS latency is in front of the MFMAs.
+    constexpr int KM = G::KM, AHEAD = NS - KM;  // steps whose loads are in flight ahead of the one that is read
+    static_assert(NS % KM == 0 && AHEAD >= KM, "whole groups of stages");
 #pragma unroll
-    for (int s = 0; s < NS - 1; s++) issue(s, lds + s * G::STAGE);
-    int cur = 0, fill = NS - 1, it = 0;
-    auto fetch = [&](Frags &f) {
-        constexpr int VM = (NS - 2) * (CHA + CHB);  // loads that may stay in flight: those of the later stages
-        static_assert(VM < 64, "a counter of six bits");
-        __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 0x70);  // vmcnt(VM) lgkmcnt(0)
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+    for (int s = 0; s < AHEAD; s++) issue(s, lds + s * G::STAGE);
+    int cur = 0, fill = AHEAD, it = 0;
+    auto fetch = [&](Frags &f, auto first) {
+        if constexpr (decltype(first)::value) {
+            constexpr int VM = (AHEAD - KM) * (CHA + CHB);  // loads that may stay in flight: those of the later stages
+            static_assert(VM < 64, "a counter of six bits");
+            __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 0x70);  // vmcnt(VM) lgkmcnt(0)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
         read(lds + cur * G::STAGE, f);
-        issue(it + NS - 1, lds + fill * G::STAGE);
+        issue(it + AHEAD, lds + fill * G::STAGE);
         cur = cur + 1 == NS ? 0 : cur + 1;
         fill = fill + 1 == NS ? 0 : fill + 1;
         ++it;
+        if constexpr (!MIX) __builtin_amdgcn_sched_barrier(0);
+    };
+    // the order inside a step where it is pinned: reads, copies and conversions between the MFMAs
+    auto end_of_step = [&]() {
+        if constexpr (MIX) {
+            constexpr int NM = 4 * TI * TJ, RPM = (4 * (TI + TJ) + NM - 1) / NM, DPM = (CHA + CHB + NM - 1) / NM;
+#pragma unroll
+            for (int n = 0; n < NM; n++) {
+                __builtin_amdgcn_sched_group_barrier(0x100, RPM, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, I8 ? 1 : 4, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x010, DPM, 0);
+            }
+        }
         __builtin_amdgcn_sched_barrier(0);
     };
+    constexpr std::true_type whole;
+    constexpr std::integral_constant<bool, KM == 1> second;
     Frags f0, f1;
-    fetch(f0);
+    fetch(f0, whole);
+    __builtin_amdgcn_sched_barrier(0);
     while (it + 1 < n_it) {
-        fetch(f1);
+        fetch(f1, second);
         multiply(f0);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch(f0);
+        end_of_step();
+        fetch(f0, whole);
         multiply(f1);
-        __builtin_amdgcn_sched_barrier(0);
+        end_of_step();
     }
     if (it < n_it) {
-        fetch(f1);
+        fetch(f1, second);
         multiply(f0);
         multiply(f1);
     } else multiply(f0);
@@ -344,20 +369,21 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 //
 // a: what a step costs a CU however few workgroups it holds (latency); b: what each resident workgroup adds (LDS, MFMA and
 // dequantisation work); rounds: how often a CU takes a new set of workgroups.  Never less than the weights' bytes at 4.6
-// TB/s or the tiles' operations at the rate that long launches reach (0.95 PFLOP/s fp16, 0.82 bf16, 1.75 int8).  Choosing by it is within 2 % of the best choice on average, 14 % at worst.  (Two fits where the conversion of the
-// weights costs differ: it is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
+// TB/s or the tiles' operations at the rate that long launches reach (0.93 PFLOP/s fp16, 0.88 bf16, 1.85 int8).  Choosing by it
+// is within 2 % of the best choice on average, 22 % at worst.  (Two fits where the conversion of the weights costs differ: it
+// is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
 struct TgCost {
     int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
     float launch[2], a[2], b[2], e[2];  // [0] fp16, [1] bf16
 };
 // (the order of the tiles in tg_launch)
 constexpr TgCost kTgW8[] = {
-    {32, 64, 3, {3.52f, 4.76f}, {0.327f, 0.289f}, {0.057f, 0.071f}, {0.41f, 0.23f}},
-    {32, 128, 3, {3.57f, 4.35f}, {0.259f, 0.233f}, {0.134f, 0.148f}, {0.61f, 0.41f}},
-    {64, 64, 2, {3.70f, 4.68f}, {0.283f, 0.233f}, {0.098f, 0.127f}, {0.58f, 0.43f}},
-    {64, 128, 2, {3.80f, 5.01f}, {0.290f, 0.285f}, {0.155f, 0.151f}, {0.97f, 0.76f}},
-    {128, 128, 1, {4.88f, 6.67f}, {0.314f, 0.316f}, {0.268f, 0.271f}, {0.92f, 0.65f}},
-    {128, 128, 2, {3.99f, 5.37f}, {0.337f, 0.389f}, {0.249f, 0.275f}, {1.68f, 1.49f}},
+    {32, 64, 3, {2.85f, 3.26f}, {0.308f, 0.311f}, {0.070f, 0.076f}, {0.53f, 0.47f}},
+    {32, 128, 3, {2.95f, 3.26f}, {0.241f, 0.254f}, {0.150f, 0.145f}, {0.67f, 0.66f}},
+    {64, 64, 2, {3.24f, 3.67f}, {0.237f, 0.236f}, {0.131f, 0.141f}, {0.62f, 0.60f}},
+    {64, 128, 2, {2.87f, 3.61f}, {0.296f, 0.313f}, {0.165f, 0.147f}, {1.07f, 1.06f}},
+    {128, 128, 1, {4.17f, 5.17f}, {0.281f, 0.312f}, {0.234f, 0.267f}, {0.95f, 0.90f}},
+    {128, 128, 2, {4.51f, 5.83f}, {0.231f, 0.319f}, {0.323f, 0.316f}, {1.65f, 1.65f}},
 };
 constexpr TgCost kTgW8S[] = {
     {32, 32, 3, {2.42f, 2.26f}, {0.300f, 0.350f}, {0.049f, 0.024f}, {0.65f, 0.71f}},
@@ -365,12 +391,12 @@ constexpr TgCost kTgW8S[] = {
     {32, 128, 3, {1.92f, 1.71f}, {0.229f, 0.245f}, {0.177f, 0.166f}, {1.00f, 1.05f}},
 };
 constexpr TgCost kTgI8[] = {
-    {32, 64, 2, {3.29f, 3.29f}, {0.060f, 0.060f}, {0.150f, 0.150f}, {0.65f, 0.65f}},
-    {64, 64, 1, {2.82f, 2.82f}, {0.166f, 0.166f}, {0.116f, 0.116f}, {1.00f, 1.00f}},
-    {64, 128, 2, {3.34f, 3.34f}, {0.093f, 0.093f}, {0.293f, 0.293f}, {0.74f, 0.74f}},
-    {128, 128, 1, {4.36f, 4.36f}, {0.292f, 0.292f}, {0.246f, 0.246f}, {1.94f, 1.94f}},
-    {128, 128, 2, {2.59f, 2.59f}, {0.650f, 0.650f}, {0.125f, 0.125f}, {1.97f, 1.97f}},
-    {128, 256, 1, {6.10f, 6.10f}, {0.441f, 0.441f}, {0.400f, 0.400f}, {1.84f, 1.84f}},
+    {32, 64, 2, {3.51f, 3.51f}, {0.000f, 0.000f}, {0.190f, 0.190f}, {0.69f, 0.69f}},
+    {64, 64, 1, {3.03f, 3.03f}, {0.159f, 0.159f}, {0.109f, 0.109f}, {0.99f, 0.99f}},
+    {64, 128, 2, {3.88f, 3.88f}, {0.000f, 0.000f}, {0.350f, 0.350f}, {0.66f, 0.66f}},
+    {128, 128, 1, {4.77f, 4.77f}, {0.276f, 0.276f}, {0.230f, 0.230f}, {1.78f, 1.78f}},
+    {128, 128, 2, {4.41f, 4.41f}, {0.607f, 0.607f}, {0.172f, 0.172f}, {1.55f, 1.55f}},
+    {128, 256, 1, {6.52f, 6.52f}, {0.383f, 0.383f}, {0.339f, 0.339f}, {1.61f, 1.61f}},
 };
 
 bool tile_gemm_supported(int kind, int M, int N, int K) {
@@ -381,7 +407,7 @@ static TgPlan tg_choose(int kind, int dtype, int M, int N, int K, size_t scratch
     const TgCost *tab = kind == TG_W8 ? kTgW8 : kind == TG_W8S ? kTgW8S : kTgI8;
     const int n_tiles = kind == TG_W8S ? 3 : 6, d = dtype == MYNN_BF16 ? 1 : 0;
     const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
-    const double rate = kind == TG_I8 ? 1.75e9 : d ? 0.82e9 : 0.95e9;  // per microsecond
+    const double rate = kind == TG_I8 ? 1.85e9 : d ? 0.88e9 : 0.93e9;  // per microsecond
     const double weights_us = (double)N * K / 4.6e6;
     TgPlan best;
     best.us = 1e30;
@@ -453,27 +479,27 @@ template <typename T, typename G> static int tg_epi(const TgArgs &p, int epi) {
 template <typename T> static int tg_launch(int kind, int tile, const TgArgs &p, int epi) {
     if constexpr (sizeof(T) == 2) {
         if (kind == TG_W8) {
-            if (tile == 0) return tg_epi<T, TgTile<TG_W8, 32, 64, 1, 2, 6, 2>>(p, epi);
-            if (tile == 1) return tg_epi<T, TgTile<TG_W8, 32, 128, 1, 4, 4, 2>>(p, epi);
-            if (tile == 2) return tg_epi<T, TgTile<TG_W8, 64, 64, 2, 2, 6, 2>>(p, epi);
-            if (tile == 3) return tg_epi<T, TgTile<TG_W8, 64, 128, 1, 4, 4, 2>>(p, epi);
-            if (tile == 4) return tg_epi<T, TgTile<TG_W8, 128, 128, 2, 4, 6, 2>>(p, epi);
+            if (tile == 0) return tg_epi<T, TgTile<TG_W8, 32, 64, 1, 2, 6, 2, 1>>(p, epi);
+            if (tile == 1) return tg_epi<T, TgTile<TG_W8, 32, 128, 1, 4, 4, 2, 1>>(p, epi);
+            if (tile == 2) return tg_epi<T, TgTile<TG_W8, 64, 64, 2, 2, 6, 2, 1>>(p, epi);
+            if (tile == 3) return tg_epi<T, TgTile<TG_W8, 64, 128, 1, 4, 4, 2, 2>>(p, epi);
+            if (tile == 4) return tg_epi<T, TgTile<TG_W8, 128, 128, 2, 4, 6, 2, 2>>(p, epi);
             // fp16: every weight is converted by one wave only (128 x 32 per wave); bf16: that form spills, 64 x 64 per wave
-            if constexpr (std::is_same<T, f16_t>::value) return tg_epi<T, TgTile<TG_W8, 128, 128, 1, 4, 3, 2>>(p, epi);
-            else return tg_epi<T, TgTile<TG_W8, 128, 128, 2, 2, 3, 2>>(p, epi);
+            if constexpr (std::is_same<T, f16_t>::value) return tg_epi<T, TgTile<TG_W8, 128, 128, 1, 4, 3, 2, 1>>(p, epi);
+            else return tg_epi<T, TgTile<TG_W8, 128, 128, 2, 2, 3, 2, 1>>(p, epi);
         }
         if (kind == TG_W8S) {
-            if (tile == 0) return tg_epi<T, TgTile<TG_W8S, 32, 32, 1, 1, 8, 1>>(p, epi);
-            if (tile == 1) return tg_epi<T, TgTile<TG_W8S, 32, 64, 1, 2, 6, 2>>(p, epi);
-            return tg_epi<T, TgTile<TG_W8S, 32, 128, 1, 4, 4, 2>>(p, epi);
+            if (tile == 0) return tg_epi<T, TgTile<TG_W8S, 32, 32, 1, 1, 8, 1, 1>>(p, epi);
+            if (tile == 1) return tg_epi<T, TgTile<TG_W8S, 32, 64, 1, 2, 6, 2, 1>>(p, epi);
+            return tg_epi<T, TgTile<TG_W8S, 32, 128, 1, 4, 4, 2, 1>>(p, epi);
         }
     }
-    if (tile == 0) return tg_epi<T, TgTile<TG_I8, 32, 64, 1, 2, 6, 1>>(p, epi);
-    if (tile == 1) return tg_epi<T, TgTile<TG_I8, 64, 64, 2, 2, 6, 2>>(p, epi);
-    if (tile == 2) return tg_epi<T, TgTile<TG_I8, 64, 128, 2, 4, 3, 2>>(p, epi);
-    if (tile == 3) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 4, 1>>(p, epi);
-    if (tile == 4) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 2, 2>>(p, epi);
-    return tg_epi<T, TgTile<TG_I8, 128, 256, 2, 4, 3, 2>>(p, epi);
+    if (tile == 0) return tg_epi<T, TgTile<TG_I8, 32, 64, 1, 2, 6, 1, 1>>(p, epi);
+    if (tile == 1) return tg_epi<T, TgTile<TG_I8, 64, 64, 2, 2, 6, 2, 1>>(p, epi);
+    if (tile == 2) return tg_epi<T, TgTile<TG_I8, 64, 128, 2, 4, 3, 2, 1>>(p, epi);
+    if (tile == 3) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 4, 1, 1>>(p, epi);
+    if (tile == 4) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 2, 2, 1>>(p, epi);
+    return tg_epi<T, TgTile<TG_I8, 128, 256, 2, 4, 3, 2, 1>>(p, epi);
 }
 
 int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
