@@ -61,7 +61,7 @@ bool attention_fused_supported(int D, int G);
 bool attention_fused_kv8_supported(int D, int cache_len);
 size_t attn_scratch_bytes(int B, int Hq, int Sq, int D, int nsplit);
 int attention_decode_launch(AttnParams p, int D, int dtype, int kv_int8, void *scratch, hipStream_t s);
-int attention_prefill_launch(const AttnParams &p, int D, int dtype, hipStream_t s);
+int attention_prefill_launch(const AttnParams &p, int D, int dtype, int kv_int8, hipStream_t s);
 bool attention_prefill_supported(const AttnParams &p, int D, int dtype, int kv_int8);
 // streaming decode kernel (attention_stream.hip): taken when eligible; attn_plan then returns its plan
 bool attn_stream_eligible(int B, int Sq, int Hq, int Hkv, int D, int dtype, int kv_int8, int kv_len, int cache_len);

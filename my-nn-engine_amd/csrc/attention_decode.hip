@@ -545,7 +545,7 @@ static int attention_entry(void *out, const void *Q, const void *K, const void *
     p.mask = mask; p.mask_os = mask_os; p.mask_rs = mask_rs;
     attn_reference_layout(p, head_dim);
     if (!mask && Sq > 1 && attention_prefill_supported(p, head_dim, dtype, kv_int8))
-        return attention_prefill_launch(p, head_dim, dtype, st);
+        return attention_prefill_launch(p, head_dim, dtype, kv_int8, st);
     int kv_len = d_active ? cache_seq_len : (active_seq_kv < cache_seq_len ? active_seq_kv : cache_seq_len);
     attn_plan(B, Sq, num_q_heads, num_kv_heads, head_dim, dtype, kv_int8, kv_len, cache_seq_len, mask != nullptr, &p.slice, &p.nsplit,
               &p.heads_per_wg);
@@ -658,7 +658,7 @@ extern "C" int mynn_attention_paged(void *out, const void *Q, const void *K_pool
         MYNN_REQUIRE(!kv_int8 && (head_dim == 64 || head_dim == 128) && scale > 0.f && aligned16(Q) && aligned16(out) && aligned16(K_pool) &&
                          aligned16(V_pool),
                      MYNN_ERR_UNSUPPORTED, "attention_paged: several query rows need a 16-bit cache, head_dim 64 or 128, a positive scale and 16-byte aligned operands");
-        return attention_prefill_launch(p, head_dim, dtype, as_stream(s));
+        return attention_prefill_launch(p, head_dim, dtype, 0, as_stream(s));
     }
     const int kv_len = d_active ? p.cache_len : (active_seq_kv < p.cache_len ? active_seq_kv : p.cache_len);
     paged_plan(B, Sq, num_kv_heads, kv_len, p.page_shift, &p.slice, &p.nsplit);

@@ -547,7 +547,7 @@ static int enqueue_step(Model &m) {
                 // know under replay -- callers add 2*KD*eb per cached row when they report
                 // flops: the causal half of QK^T and PV over the new rows alone (exact when past_len is 0)
                 note(m, "attention", (double)rows * 2.0 * QD * eb, S > 1 ? 2.0 * B * Hq * D * (double)S * (S + 1) : 0.0);
-                if (pf_kernel) TRY(attention_prefill_launch(p, D, c.dtype, s));
+                if (pf_kernel) TRY(attention_prefill_launch(p, D, c.dtype, kv8, s));
                 else TRY(attention_decode_launch(p, D, c.dtype, kv8, m.attn_scratch, s));
             }
         }
