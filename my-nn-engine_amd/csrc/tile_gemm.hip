@@ -12,7 +12,9 @@
 // weight stream, and the stages in flight are what hides it.  A K step is 128 bytes of an activation row (64 values of 16
 // bits, 128 int8); the waves meet at a barrier every KM steps.  KM = 2 where a step is long enough that the meeting, not
 // the load, is what it waits for: 64 x 128 (500 x 11264 x 2048 30.5 -> 29.9 us fp16, 300 rows bf16 26.4 -> 24.3) and the
-// eight waves of 128 x 128 (1000 rows 44.5 -> 43.4); smaller tiles do not change, 128 x 128 of int8 loses 14 %.  16-byte chunks are placed so that the 128-bit fragment reads of 16 neighbouring rows fall into
+// eight waves of 128 x 128 (1000 rows 44.5 -> 43.4); smaller tiles do not change, 128 x 128 of int8 does not either.
+// int8 takes eight waves and six stages where a CU gets one workgroup (64 x 128, 500 x 4096 x 14336: 55.5 -> 50.6 us against
+// three stages; 128 x 128 in two K ranges 46.2 -> 43.8 against four waves), four waves and two workgroups otherwise.  16-byte chunks are placed so that the 128-bit fragment reads of 16 neighbouring rows fall into
 // different LDS banks: row r's chunk c at 8r + (c ^ (r/2 & 7)) for 128-byte rows, 4r + (c ^ (r/4 & 3)) for the 64-byte
 // rows of int8 weights against 16-bit activations.
 //
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 // a: what a step costs a CU however few workgroups it holds (latency); b: what each resident workgroup adds (LDS, MFMA and
 // dequantisation work); rounds: how often a CU takes a new set of workgroups.  Never less than the weights' bytes at 4.6
 // TB/s or the tiles' operations at the rate that long launches reach (0.93 PFLOP/s fp16, 0.88 bf16, 1.85 int8).  Choosing by it
-// is within 2 % of the best choice on average, 22 % at worst.  (Two fits where the conversion of the weights costs differ: it
+// is within 2 % of the best choice on average, 27 % at worst.  (Two fits where the conversion of the weights costs differ: it
 // is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
 struct TgCost {
     int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
@@ -391,12 +393,12 @@ constexpr TgCost kTgW8S[] = {
     {32, 128, 3, {1.92f, 1.71f}, {0.229f, 0.245f}, {0.177f, 0.166f}, {1.00f, 1.05f}},
 };
 constexpr TgCost kTgI8[] = {
-    {32, 64, 2, {3.51f, 3.51f}, {0.000f, 0.000f}, {0.190f, 0.190f}, {0.69f, 0.69f}},
-    {64, 64, 1, {3.03f, 3.03f}, {0.159f, 0.159f}, {0.109f, 0.109f}, {0.99f, 0.99f}},
-    {64, 128, 2, {3.88f, 3.88f}, {0.000f, 0.000f}, {0.350f, 0.350f}, {0.66f, 0.66f}},
-    {128, 128, 1, {4.77f, 4.77f}, {0.276f, 0.276f}, {0.230f, 0.230f}, {1.78f, 1.78f}},
-    {128, 128, 2, {4.41f, 4.41f}, {0.607f, 0.607f}, {0.172f, 0.172f}, {1.55f, 1.55f}},
-    {128, 256, 1, {6.52f, 6.52f}, {0.383f, 0.383f}, {0.339f, 0.339f}, {1.61f, 1.61f}},
+    {32, 64, 2, {3.61f, 3.61f}, {0.001f, 0.001f}, {0.179f, 0.179f}, {0.63f, 0.63f}},
+    {64, 64, 1, {3.28f, 3.28f}, {0.146f, 0.146f}, {0.096f, 0.096f}, {0.93f, 0.93f}},
+    {64, 128, 1, {3.54f, 3.54f}, {0.190f, 0.190f}, {0.141f, 0.141f}, {0.80f, 0.80f}},
+    {64, 128, 2, {3.47f, 3.47f}, {0.101f, 0.101f}, {0.271f, 0.271f}, {1.12f, 1.12f}},
+    {128, 128, 1, {4.44f, 4.44f}, {0.244f, 0.244f}, {0.197f, 0.197f}, {0.92f, 0.92f}},
+    {128, 256, 1, {6.13f, 6.13f}, {0.377f, 0.377f}, {0.334f, 0.334f}, {1.76f, 1.76f}},
 };
 
 bool tile_gemm_supported(int kind, int M, int N, int K) {
@@ -496,9 +498,9 @@ template <typename T> static int tg_launch(int kind, int tile, const TgArgs &p, 
     }
     if (tile == 0) return tg_epi<T, TgTile<TG_I8, 32, 64, 1, 2, 6, 1, 1>>(p, epi);
     if (tile == 1) return tg_epi<T, TgTile<TG_I8, 64, 64, 2, 2, 6, 2, 1>>(p, epi);
-    if (tile == 2) return tg_epi<T, TgTile<TG_I8, 64, 128, 2, 4, 3, 2, 1>>(p, epi);
-    if (tile == 3) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 4, 1, 1>>(p, epi);
-    if (tile == 4) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 2, 2, 2, 1>>(p, epi);
+    if (tile == 2) return tg_epi<T, TgTile<TG_I8, 64, 128, 2, 4, 6, 2, 2>>(p, epi);
+    if (tile == 3) return tg_epi<T, TgTile<TG_I8, 64, 128, 2, 2, 3, 2, 1>>(p, epi);
+    if (tile == 4) return tg_epi<T, TgTile<TG_I8, 128, 128, 2, 4, 4, 2, 1>>(p, epi);
     return tg_epi<T, TgTile<TG_I8, 128, 256, 2, 4, 3, 2, 1>>(p, epi);
 }
 
