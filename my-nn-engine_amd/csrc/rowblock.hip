@@ -2,14 +2,15 @@
 //
 // At this size a linear is a few microseconds, of which skinny.hip's form -- K ranges over workgroups, partial sums through
 // memory, a second launch that adds them up -- spends more on the second launch than on the weights.  Here one workgroup
-// owns 32 weight rows (RB row blocks) over the WHOLE K range: its waves split K among themselves, every wave has its share of
-// the weights in flight before the first product, and the partial sums meet in LDS, so the workgroup stores finished
-// output: scale, residual or SwiGLU, and in front the RMSNorm of the activation rows while they are staged (NORM).
+// owns 16 .. 64 weight rows (RB row blocks of RH) over the WHOLE K range: its waves split K among themselves, every wave has
+// its share of the weights in flight before the first product, and the partial sums meet in LDS, so the workgroup stores
+// finished output: scale, residual or SwiGLU, and in front the RMSNorm of the activation rows while they are staged (NORM).
 //
 //   out[m,n] = T(scale[n] * sum_k act[m,k] * wq[n,k])   (scale after the f32 sum, as skinny.hip)
 //
 // The weights are skinny.hip's tiled copy: a wave's step of 32 rows x 128 k is 4 KB, read by four sequential loads, and
-// turned exactly into the A operand of v_mfma_f32_32x32x16; the activation rows are the B operand's columns, read from LDS.
+// turned exactly into the A operand of v_mfma_f32_32x32x16 (or half of it into that of 16x16x32); the activation rows are the
+// B operand's columns, read from LDS.
 #include <type_traits>
 
 #include "kernels.h"
@@ -20,49 +21,61 @@ namespace mynn {
 // WAVES waves of a workgroup: RB row blocks times WK shares of a slab of WK * 128 k (a step per wave).  DEPTH slabs of
 // weights are in flight per wave.  Activations, plain form: panels of SPP slabs, [M] rows, copied global -> LDS by the load
 // unit, the next panel while one is multiplied; NORM > 0: whole rows at once, NORM 16-byte pieces per lane.
-constexpr int kRbMaxRows = 32, kRbWaves = 8, kRbDepth = 4, kRbRed = 36;  // (floats per row of partial sums)
-template <int RB, int SPP> constexpr int rb_panel_k() { return kRbWaves / RB * 128 * SPP; }
+constexpr int kRbMaxRows = 32, kRbDepth = 4, kRbRed = 36;  // (floats per row of partial sums)
+template <int RB> constexpr int rb_waves() { return RB == 3 ? 12 : 8; }
+template <int RB, int SPP> constexpr int rb_panel_k() { return rb_waves<RB>() / RB * 128 * SPP; }
 template <int RB, int SPP> constexpr int rb_row_bytes() { return (rb_panel_k<RB, SPP>() + 511) / 512 * 1024 + 16; }
 
-template <typename T, int RB, int SPP, int EPI, int NORM>
-__global__ __launch_bounds__(kRbWaves * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, const T *scale, const T *res, const T *norm_w, T *out,
+typedef float f4x_t __attribute__((ext_vector_type(4)));
+template <typename T> __device__ inline f16x_t rb_mfma(const U4 &a, const U4 &b, f16x_t c) { return Mfma<T>::run(a, b, c); }
+template <typename T> __device__ inline f4x_t rb_mfma(const U4 &a, const U4 &b, f4x_t c) {
+    if constexpr (std::is_same<T, f16_t>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, a), __builtin_bit_cast(h8_t, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8_t, a), __builtin_bit_cast(b8_t, b), c, 0, 0, 0);
+}
+
+template <typename T, int RB, int RH, int SPP, int EPI, int NORM>
+__global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, const T *scale, const T *res, const T *norm_w, T *out,
                                                                       int M, int N, int K, float eps) {
-    constexpr int WAVES = kRbWaves, WK = WAVES / RB, DEPTH = kRbDepth, RS = kRbRed;
+    constexpr int WAVES = rb_waves<RB>(), WK = WAVES / RB, DEPTH = kRbDepth, RS = kRbRed;
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 31, h = lane >> 5, rb = wave / WK, kw = wave % WK;
+    const int r = lane % RH, h = lane / RH, rb = wave / WK, kw = wave % WK;
     const int row_blocks = (N + 31) / 32, iters = K / 128, slabs = (iters + WK - 1) / WK;
     const size_t pitch = (size_t)row_blocks * 256;  // 16-byte pieces of one step over all row blocks
-    const U4 *wsrc = pk + (size_t)min((int)blockIdx.x * RB + rb, row_blocks - 1) * 256 + lane;
-    U4 w[DEPTH][4];
+    // The copy's 16-byte piece of k 64 * a + 16 * j, row i of a block is number 64 * j + 32 * a + i of its step.  A lane of
+    // the 32-row form reads pieces (h, 0 .. 3), of the 16-row form (h % 2, h / 2) and (h % 2, 2 + h / 2).
+    const int block = min((int)blockIdx.x * RB + rb, row_blocks * (32 / RH) - 1);
+    constexpr int LPW = RH / 8;  // loads of a step
+    const U4 *wsrc = pk + (size_t)(block / (32 / RH)) * 256 + (RH == 32 ? lane : (h >> 1) * 64 + (h & 1) * 32 + (block & 1) * 16 + r);
+    U4 w[DEPTH][LPW];
     auto load_w = [&](int sl, U4 *dst) {
         const U4 *p = wsrc + (size_t)min(sl * WK + kw, iters - 1) * pitch;
 #pragma unroll
-        for (int j = 0; j < 4; j++) dst[j] = __builtin_nontemporal_load(p + j * 64);
+        for (int j = 0; j < LPW; j++) dst[j] = __builtin_nontemporal_load(p + j * (RH == 32 ? 64 : 128));
     };
     // what the store of this thread's first output needs (mostly its only one), fetched in front of everything else
-    constexpr int PR = EPI == GEMM_SWIGLU ? 16 : 32;  // outputs per row block and activation row
+    constexpr int PR = EPI == GEMM_SWIGLU ? RH / 2 : RH;  // outputs per row block and activation row
     T sc0, sc1, rs0;
     {
-        const int o = min(tid, RB * M * PR - 1), c = o % PR, m = (o / PR) % M, n = min((((int)blockIdx.x * RB + o / (PR * M)) * 32) + (EPI == GEMM_SWIGLU ? 2 * c : c), N - 1);
+        const int o = min(tid, RB * M * PR - 1), c = o % PR, m = (o / PR) % M, n = min((((int)blockIdx.x * RB + o / (PR * M)) * RH) + (EPI == GEMM_SWIGLU ? 2 * c : c), N - 1);
         sc0 = scale[n];
         if constexpr (EPI == GEMM_SWIGLU) sc1 = scale[min(n + 1, N - 1)];
         if constexpr (EPI == GEMM_RESIDUAL) rs0 = res[(size_t)m * N + n];
     }
-    f16x_t acc;
+    std::conditional_t<RH == 32, f16x_t, f4x_t> acc;
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = 0.f;
+    for (int e = 0; e < RH * RH / 64; e++) acc[e] = 0.f;
     const int mrow = min(r, M - 1);  // (columns past M repeat the last row and are not stored)
     auto multiply = [&](const U4 *q, const char *arow) {  // arow: this lane's activation row at the step's first k
-        U4 b[8];
+        U4 b[2 * LPW];
 #pragma unroll
-        for (int s = 0; s < 8; s++) b[s] = *(const U4 *)(arow + 128 * h + 16 * s);
+        for (int i = 0; i < 2 * LPW; i++) b[i] = *(const U4 *)(arow + (RH == 32 ? 128 * h + 16 * i : 128 * (h & 1) + 32 * (h >> 1) + 64 * (i >> 1) + 16 * (i & 1)));
 #pragma unroll
-        for (int s = 0; s < 8; s += 2) {
-            U4 c = q[s >> 1];
+        for (int i = 0; i < LPW; i++) {
+            U4 c = q[i];
             pin(c);  // (converted here, not when they were loaded)
-            acc = Mfma<T>::run(i8x8_to_operand<T>(c.x, c.y), b[s], acc);
-            acc = Mfma<T>::run(i8x8_to_operand<T>(c.z, c.w), b[s + 1], acc);
+            acc = rb_mfma<T>(i8x8_to_operand<T>(c.x, c.y), b[2 * i], acc);
+            acc = rb_mfma<T>(i8x8_to_operand<T>(c.z, c.w), b[2 * i + 1], acc);
         }
     };
     if constexpr (NORM > 0) {
@@ -121,6 +134,7 @@ __global__ __launch_bounds__(kRbWaves * 64) void rowblock_gemm_kernel(const T *a
             char *dst = lds + (size_t)(p & 1) * M * AS;
             for (int c = wave; c < M * CPR; c += WAVES) {
                 const int m = c / CPR, k = p * PK + (c % CPR) * 512 + lane * 8;
+                if (k - lane * 8 >= K) continue;
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(act + (size_t)m * K + min(k, K - 8)),
                                                  (__attribute__((address_space(3))) void *)(dst + (size_t)m * AS + (c % CPR) * 1024), 16, 0, 0);
             }
@@ -130,7 +144,7 @@ __global__ __launch_bounds__(kRbWaves * 64) void rowblock_gemm_kernel(const T *a
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) load_w(d, w[d]);
         const char *arow = lds + (size_t)mrow * AS + kw * 256;
-        constexpr int AGE = (SPP < DEPTH ? SPP : DEPTH) * 4;  // weight loads younger than the panel that is waited for, at least
+        constexpr int AGE = (SPP < DEPTH ? SPP : DEPTH) * LPW;  // weight loads younger than the panel that is waited for, at least
         for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
 #pragma unroll
             for (int d = 0; d < DEPTH; d++) {
@@ -153,17 +167,17 @@ __global__ __launch_bounds__(kRbWaves * 64) void rowblock_gemm_kernel(const T *a
     }
     __syncthreads();  // the activations are done with: their memory takes the partial sums
 
-    // D[n][m]: lane holds column m = lane % 32 and rows n = 8*(e/4) + 4*(lane/32) + e%4
+    // D[n][m]: lane holds column m = lane % RH and rows n = 4 * (lane / RH) + e % 4, + 8 * (e / 4) in the 32-row form
     float *red = (float *)lds;
     if (r < M) {
         float *dst = red + ((size_t)(kw * RB + rb) * M + r) * RS + 4 * h;
 #pragma unroll
-        for (int e4 = 0; e4 < 4; e4++) *(float4 *)(dst + e4 * 8) = float4{acc[e4 * 4], acc[e4 * 4 + 1], acc[e4 * 4 + 2], acc[e4 * 4 + 3]};
+        for (int e4 = 0; e4 < RH * RH / 256; e4++) *(float4 *)(dst + e4 * 8) = float4{acc[e4 * 4], acc[e4 * 4 + 1], acc[e4 * 4 + 2], acc[e4 * 4 + 3]};
     }
     __syncthreads();
     for (int o = tid; o < RB * M * PR; o += WAVES * 64) {
         const int c = o % PR, m = (o / PR) % M, b = o / (PR * M);
-        const int n0 = ((int)blockIdx.x * RB + b) * 32;
+        const int n0 = ((int)blockIdx.x * RB + b) * RH;
         const bool first = o == tid;
         auto total = [&](int n) {
             float t = 0.f;
@@ -194,17 +208,36 @@ __global__ __launch_bounds__(kRbWaves * 64) void rowblock_gemm_kernel(const T *a
     }
 }
 
-// ---- which form.  One row block per workgroup while that is at most one workgroup per CU (its eight waves split K), two
-// beyond; from 768 row blocks on skinny.hip's one-launch form streams the weights just as fast (28672 x 4096, 8 rows: 23
-// us) and this one is not taken.  The norm rides along up to 16 rows (8 rows x 2560 x 2048: 7.3 us with it against 6.0 +
-// a launch of 2.5; every workgroup normalises all rows for itself, at 32 rows that costs 3.7 us).
+// ---- which form: as many workgroups as there are CUs and no more, each with whole row blocks.
+// HALF   up to 256 blocks of 16 rows (and 16 activation rows: the columns of the 16 x 16 product)
+// ONE    one block of 32 rows per workgroup while that is at most one per CU
+// THREE  three blocks of 16 rows, twelve waves, up to 256 such workgroups (with a norm over more than 2048 values its rows
+//        do not fit the registers of twelve waves)
+// TWO    two blocks of 32 rows; from 768 row blocks on skinny.hip's one-launch form streams the weights just as fast
+//        (28672 x 4096, 8 rows: 23 us) and this kernel is not taken
+// 8 rows, us, 32-row forms / HALF or THREE: 2560 x 2048 with norm 7.2 / 6.1, 2048 x 2048 6.3 / 4.9, 2048 x 5632 9.4 / 7.2, 4096 x
+// 14336 18.6 / 14.5, 11264 x 2048 with norm 9.5 / 7.9, 10000 x 4096 12.6 / 11.2; but 6144 x 4096 9.1 / 9.7, 10000 x 4096 with norm
+// 14.1 / 15.9.  What a workgroup reads of its activations (as much as of 16 weight rows) is what keeps it from splitting further.
+// The norm rides along up to 16 rows (8 rows x 2560 x 2048: 7.2 us with it in the ONE form against 6.0 + a launch of 2.5;
+// every workgroup normalises all rows for itself, at 32 rows that costs 3.7 us).
+enum RbForm { RB_HALF, RB_ONE, RB_THREE, RB_TWO };
+static RbForm rb_form(int M, int N, int K, bool norm) {
+    if (M <= 16 && N <= 256 * 16) return RB_HALF;
+    if (N <= 256 * 32) return RB_ONE;
+    if (M <= 16 && N <= 256 * 48 && (!norm || K <= 2048)) return RB_THREE;
+    return RB_TWO;
+}
+// (K > 8192: half the panel per step, 4096 x 14336 14.5 us against 15.4)
 static size_t rb_lds(int M, int N, int K, bool norm) {
-    const int blocks = (N + 31) / 32;
+    auto panels = [&](int pk, int row) { return (size_t)(K > pk ? 2 : 1) * M * row; };
+    const RbForm f = rb_form(M, N, K, norm);
     size_t act;
     if (norm) act = (size_t)M * (K * 2 + 16);
-    else if (blocks <= 256) act = (size_t)(K > rb_panel_k<1, 1>() ? 2 : 1) * M * rb_row_bytes<1, 1>();
-    else act = (size_t)(K > rb_panel_k<2, 2>() ? 2 : 1) * M * rb_row_bytes<2, 2>();
-    const size_t red = (size_t)kRbWaves * M * kRbRed * sizeof(float);
+    else if (f == RB_HALF && K <= 8192) act = panels(rb_panel_k<1, 2>(), rb_row_bytes<1, 2>());
+    else if (f == RB_HALF || f == RB_ONE) act = panels(rb_panel_k<1, 1>(), rb_row_bytes<1, 1>());
+    else if (f == RB_THREE) act = panels(rb_panel_k<3, 2>(), rb_row_bytes<3, 2>());
+    else act = panels(rb_panel_k<2, 2>(), rb_row_bytes<2, 2>());
+    const size_t red = (size_t)(f == RB_THREE ? rb_waves<3>() : rb_waves<1>()) * M * kRbRed * sizeof(float);
     return act > red ? act : red;
 }
 bool rowblock_supported(int M, int N, int K, bool norm) {
@@ -212,15 +245,15 @@ bool rowblock_supported(int M, int N, int K, bool norm) {
            rb_lds(M, N, K, norm) <= 160 * 1024;
 }
 
-template <typename T, int RB, int SPP, int EPI, int NORM>
+template <typename T, int RB, int RH, int SPP, int EPI, int NORM>
 static int rb_go(const void *act, const void *pk, const void *scale, const void *res, const void *norm_w, void *out, int M, int N, int K, float eps,
                  size_t lds, hipStream_t s) {
     static size_t lds_set = 64 * 1024;
     if (lds > lds_set) {
-        MYNN_HIP(hipFuncSetAttribute((const void *)rowblock_gemm_kernel<T, RB, SPP, EPI, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        MYNN_HIP(hipFuncSetAttribute((const void *)rowblock_gemm_kernel<T, RB, RH, SPP, EPI, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         lds_set = 160 * 1024;
     }
-    MYNN_LAUNCH((rowblock_gemm_kernel<T, RB, SPP, EPI, NORM>), dim3((N + 32 * RB - 1) / (32 * RB)), dim3(kRbWaves * 64), lds, s, (const T *)act,
+    MYNN_LAUNCH((rowblock_gemm_kernel<T, RB, RH, SPP, EPI, NORM>), dim3((N + RH * RB - 1) / (RH * RB)), dim3(rb_waves<RB>() * 64), lds, s, (const T *)act,
                 (const U4 *)pk, (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, M, N, K, eps);
     return launch_status("rowblock_gemm_kernel");
 }
@@ -231,19 +264,18 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
     MYNN_REQUIRE(rowblock_supported(M, N, K, norm_w != nullptr) && (epi != GEMM_SWIGLU || N % 2 == 0), MYNN_ERR_UNSUPPORTED, "rowblock_gemm: M=%d N=%d K=%d", M, N, K);
     MYNN_REQUIRE(aligned16(act) && aligned16(packed) && (!norm_w || aligned16(norm_w)), MYNN_ERR_INVALID, "rowblock_gemm: operands must be 16-byte aligned");
     const size_t lds = rb_lds(M, N, K, norm_w != nullptr);
-    const bool one = (N + 31) / 32 <= 256;
+    const RbForm f = rb_form(M, N, K, norm_w != nullptr);
     return dispatch_dtype16(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
         auto go = [&](auto e) {
             constexpr int EPI = decltype(e)::value;
+#define RB_GO(RB, RH, SPP, NORM) rb_go<T, RB, RH, SPP, EPI, NORM>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
             if (norm_w && K <= 2048)
-                return one ? rb_go<T, 1, 1, EPI, 4>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
-                           : rb_go<T, 2, 2, EPI, 4>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s);
-            if (norm_w)
-                return one ? rb_go<T, 1, 1, EPI, 8>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
-                           : rb_go<T, 2, 2, EPI, 8>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s);
-            return one ? rb_go<T, 1, 1, EPI, 0>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
-                       : rb_go<T, 2, 2, EPI, 0>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s);
+                return f == RB_HALF ? RB_GO(1, 16, 1, 4) : f == RB_ONE ? RB_GO(1, 32, 1, 4) : f == RB_THREE ? RB_GO(3, 16, 2, 4) : RB_GO(2, 32, 2, 4);
+            if (norm_w) return f == RB_HALF ? RB_GO(1, 16, 1, 8) : f == RB_ONE ? RB_GO(1, 32, 1, 8) : RB_GO(2, 32, 2, 8);
+            if (f == RB_HALF) return K > 8192 ? RB_GO(1, 16, 1, 0) : RB_GO(1, 16, 2, 0);
+            return f == RB_ONE ? RB_GO(1, 32, 1, 0) : f == RB_THREE ? RB_GO(3, 16, 2, 0) : RB_GO(2, 32, 2, 0);
+#undef RB_GO
         };
         if (epi == GEMM_RESIDUAL) return go(std::integral_constant<int, GEMM_RESIDUAL>{});
         if (epi == GEMM_SWIGLU) return go(std::integral_constant<int, GEMM_SWIGLU>{});
