@@ -175,7 +175,7 @@ struct Model {
     void *tg_part = nullptr;     // tile_gemm's partial sums and arrival counters
     int *tg_counters = nullptr;
     bool skinny = false;      // 16..64 rows: int8 weights streamed once through the few-row matrix-core kernel
-    bool rowblock = false;    // ... up to 32 rows: a linear is one launch (rowblock.hip), with the norm in front up to 16
+    bool rowblock = false;    // ... one launch per linear (rowblock.hip), with the norm in front up to 16 rows
     float *skinny_scratch = nullptr;
     void *cos_t = nullptr, *sin_t = nullptr;
     // arena
@@ -478,7 +478,8 @@ static int enqueue_step(Model &m) {
         } else if (qfused) {
             TRY(qlinear1(m.qkv, m.x, L.norm1, L.qkv, nullptr, GEMM_PLAIN, "qgemv_norm_quant_qkv"));
         } else if (m.rowblock) {
-            TRY(rowblock_rows(m, m.qkv, m.x, L.norm1, L.qkv, L.pk_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv"));
+            TRY(rowblock_rows(m, m.qkv, nrm_ready ? m.nrm : m.x, nrm_ready ? nullptr : L.norm1, L.qkv, L.pk_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv"));
+            nrm_ready = false;
         } else if (m.w8a8_fused) {
             TRY(qlinear_fused(m, m.pl_qkv, m.qkv, m.x, L.norm1, L.qkv, nullptr, rows, GEMM_PLAIN, "qlinear_qkv"));
         } else {
@@ -567,7 +568,11 @@ static int enqueue_step(Model &m) {
         } else if (m.rowblock) {
             TRY(rowblock_rows(m, m.x2, m.attn, nullptr, L.o, L.pk_o, m.x, rows, GEMM_RESIDUAL, "linear_o_residual"));
             TRY(rowblock_rows(m, m.hmid, m.x2, L.norm2, L.gu, L.pk_gu, nullptr, rows, GEMM_SWIGLU, "linear_gateup_swiglu"));
-            TRY(rowblock_rows(m, m.x, m.hmid, nullptr, L.down, L.pk_down, m.x2, rows, GEMM_RESIDUAL, "linear_down_residual"));
+            if (rows <= 32) TRY(rowblock_rows(m, m.x, m.hmid, nullptr, L.down, L.pk_down, m.x2, rows, GEMM_RESIDUAL, "linear_down_residual"));
+            else {  // (K is long: the few-row kernel with the next norm in its second launch, 12.6 us at 48 rows x 2048 x 5632 against 13.1 + a norm)
+                const void *next_norm = li + 1 < m.layers.size() ? m.layers[li + 1].norm1 : m.final_norm;
+                TRY(skinny_rows(m, m.x, m.hmid, L.down, L.pk_down, m.x2, rows, GEMM_RESIDUAL, "linear_down_residual", next_norm, &nrm_ready));
+            }
         } else if (m.skinny) {
             bool normed = false;
             TRY(skinny_rows(m, m.x2, m.attn, L.o, L.pk_o, m.x, rows, GEMM_RESIDUAL, "linear_o_residual", L.norm2, &normed));
@@ -575,7 +580,8 @@ static int enqueue_step(Model &m) {
                 note(m, "rms_norm", 2.0 * rows * H * eb + H * eb);
                 TRY(mynn_rms_norm(m.nrm, m.x2, L.norm2, rows, H, c.eps, c.dtype, s));
             }
-            TRY(skinny_rows(m, m.hmid, m.nrm, L.gu, L.pk_gu, nullptr, rows, GEMM_SWIGLU, "linear_gateup_swiglu"));
+            if (L.pk_gu) TRY(rowblock_rows(m, m.hmid, m.nrm, nullptr, L.gu, L.pk_gu, nullptr, rows, GEMM_SWIGLU, "linear_gateup_swiglu"));
+            else TRY(skinny_rows(m, m.hmid, m.nrm, L.gu, L.pk_gu, nullptr, rows, GEMM_SWIGLU, "linear_gateup_swiglu"));
             const void *next_norm = li + 1 < m.layers.size() ? m.layers[li + 1].norm1 : m.final_norm;
             TRY(skinny_rows(m, m.x, m.hmid, L.down, L.pk_down, m.x2, rows, GEMM_RESIDUAL, "linear_down_residual", next_norm, &nrm_ready));
         } else if (qfused) {
@@ -635,7 +641,7 @@ static int enqueue_step(Model &m) {
     } else if (qfused) {
         TRY(qlinear1(m.logits, m.x, m.final_norm, m.lm_head, nullptr, GEMM_PLAIN, "qgemv_norm_quant_lm_head"));
     } else if (m.rowblock) {
-        TRY(rowblock_rows(m, m.logits, m.x, m.final_norm, m.lm_head, m.pk_lm_head, nullptr, rows, GEMM_PLAIN, "linear_lm_head"));
+        TRY(rowblock_rows(m, m.logits, nrm_ready ? m.nrm : m.x, nrm_ready ? nullptr : m.final_norm, m.lm_head, m.pk_lm_head, nullptr, rows, GEMM_PLAIN, "linear_lm_head"));
     } else if (m.w8a8_fused) {
         TRY(qlinear_fused(m, m.pl_lm, m.logits, m.x, m.final_norm, m.lm_head, nullptr, rows, GEMM_PLAIN, "qlinear_lm_head"));
     } else {

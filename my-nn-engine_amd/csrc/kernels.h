@@ -56,7 +56,7 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
                         float eps = 0.f, void *nrm_out = nullptr, bool *normed = nullptr, const SkinnyRope *rope = nullptr,
                         bool *roped = nullptr);
 
-// rowblock.hip -- the same product for up to 32 rows in one launch (packed: skinny_pack_weight's copy); norm_w: of the
+// rowblock.hip -- the same product in one launch, where that is the faster form (packed: skinny_pack_weight's copy); norm_w: of the
 // RMS-normalised rows.  epi: GEMM_PLAIN, GEMM_RESIDUAL, GEMM_SWIGLU (interleaved gate/up rows)
 bool rowblock_supported(int M, int N, int K, bool norm);
 int rowblock_gemm(void *out, const void *act, const void *packed, const void *scale, const void *res, const void *norm_w, float eps, int M, int N,

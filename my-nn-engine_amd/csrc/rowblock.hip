@@ -1,4 +1,4 @@
-// DequantMatMul for a handful of activation rows (2 <= M <= 32: small decode batches), one launch per linear.
+// DequantMatMul for a handful of activation rows (2 <= M <= 64: decode batches), one launch per linear.
 //
 // At this size a linear is a few microseconds, of which skinny.hip's form -- K ranges over workgroups, partial sums through
 // memory, a second launch that adds them up -- spends more on the second launch than on the weights.  Here one workgroup
@@ -18,13 +18,21 @@
 
 namespace mynn {
 
-// WAVES waves of a workgroup: RB row blocks times WK shares of a slab of WK * 128 k (a step per wave).  DEPTH slabs of
+// The waves of a workgroup: row blocks times shares of a slab of WK * 128 k (a step per wave) times groups of activation rows.  DEPTH slabs of
 // weights are in flight per wave.  Activations, plain form: panels of SPP slabs, [M] rows, copied global -> LDS by the load
 // unit, the next panel while one is multiplied; NORM > 0: whole rows at once, NORM 16-byte pieces per lane.
-constexpr int kRbMaxRows = 32, kRbDepth = 4, kRbRed = 36;  // (floats per row of partial sums)
-template <int RB> constexpr int rb_waves() { return RB == 3 ? 12 : 8; }
-template <int RB, int SPP> constexpr int rb_panel_k() { return rb_waves<RB>() / RB * 128 * SPP; }
-template <int RB, int SPP> constexpr int rb_row_bytes() { return (rb_panel_k<RB, SPP>() + 511) / 512 * 1024 + 16; }
+constexpr int kRbMaxRows = 64, kRbDepth = 4;
+// RB row blocks of RH weight rows per workgroup, WK waves that share a slab's K, CG groups of waves with MC tiles of RH
+// activation rows each
+template <int RB_, int RH_, int WK_, int CG_, int MC_, int SPP_> struct RbShape {
+    static constexpr int RB = RB_, RH = RH_, WK = WK_, CG = CG_, MC = MC_, SPP = SPP_, WAVES = RB * WK * CG, ROWS = CG * MC * RH;
+    static constexpr int PANEL = WK * 128 * SPP, ROW_BYTES = (PANEL + 511) / 512 * 1024 + 16;
+    static constexpr int RED = RH + 4;  // floats per row of partial sums
+    static size_t lds(int M, int K, bool norm) {
+        const size_t act = norm ? (size_t)M * (K * 2 + 16) : (size_t)(K > PANEL ? 2 : 1) * M * ROW_BYTES, red = (size_t)WK * RB * M * RED * sizeof(float);
+        return act > red ? act : red;
+    }
+};
 
 typedef float f4x_t __attribute__((ext_vector_type(4)));
 template <typename T> __device__ inline f16x_t rb_mfma(const U4 &a, const U4 &b, f16x_t c) { return Mfma<T>::run(a, b, c); }
@@ -33,13 +41,13 @@ template <typename T> __device__ inline f4x_t rb_mfma(const U4 &a, const U4 &b, 
     else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8_t, a), __builtin_bit_cast(b8_t, b), c, 0, 0, 0);
 }
 
-template <typename T, int RB, int RH, int SPP, int EPI, int NORM>
-__global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, const T *scale, const T *res, const T *norm_w, T *out,
+template <typename T, typename S, int EPI, int NORM>
+__global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, const T *scale, const T *res, const T *norm_w, T *out,
                                                                       int M, int N, int K, float eps) {
-    constexpr int WAVES = rb_waves<RB>(), WK = WAVES / RB, DEPTH = kRbDepth, RS = kRbRed;
+    constexpr int RB = S::RB, RH = S::RH, WK = S::WK, MC = S::MC, SPP = S::SPP, WAVES = S::WAVES, DEPTH = kRbDepth, RS = S::RED;
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane % RH, h = lane / RH, rb = wave / WK, kw = wave % WK;
+    const int r = lane % RH, h = lane / RH, cg = wave / (RB * WK), rb = wave / WK % RB, kw = wave % WK;
     const int row_blocks = (N + 31) / 32, iters = K / 128, slabs = (iters + WK - 1) / WK;
     const size_t pitch = (size_t)row_blocks * 256;  // 16-byte pieces of one step over all row blocks
     // The copy's 16-byte piece of k 64 * a + 16 * j, row i of a block is number 64 * j + 32 * a + i of its step.  A lane of
@@ -62,20 +70,31 @@ __global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(cons
         if constexpr (EPI == GEMM_SWIGLU) sc1 = scale[min(n + 1, N - 1)];
         if constexpr (EPI == GEMM_RESIDUAL) rs0 = res[(size_t)m * N + n];
     }
-    std::conditional_t<RH == 32, f16x_t, f4x_t> acc;
+    std::conditional_t<RH == 32, f16x_t, f4x_t> acc[MC];
+    int arow0[MC];  // this lane's activation row of each tile (rows past M repeat the last one and are not stored)
 #pragma unroll
-    for (int e = 0; e < RH * RH / 64; e++) acc[e] = 0.f;
-    const int mrow = min(r, M - 1);  // (columns past M repeat the last row and are not stored)
-    auto multiply = [&](const U4 *q, const char *arow) {  // arow: this lane's activation row at the step's first k
-        U4 b[2 * LPW];
+    for (int mc = 0; mc < MC; mc++) {
 #pragma unroll
-        for (int i = 0; i < 2 * LPW; i++) b[i] = *(const U4 *)(arow + (RH == 32 ? 128 * h + 16 * i : 128 * (h & 1) + 32 * (h >> 1) + 64 * (i >> 1) + 16 * (i & 1)));
+        for (int e = 0; e < RH * RH / 64; e++) acc[mc][e] = 0.f;
+        arow0[mc] = min((cg * MC + mc) * RH + r, M - 1);
+    }
+    auto multiply = [&](const U4 *q, const char *a0, int pitch) {  // a0: the activations at the step's first k
+        U4 b[MC][2 * LPW];
+#pragma unroll
+        for (int mc = 0; mc < MC; mc++)
+#pragma unroll
+            for (int i = 0; i < 2 * LPW; i++)
+                b[mc][i] = *(const U4 *)(a0 + (size_t)arow0[mc] * pitch + (RH == 32 ? 128 * h + 16 * i : 128 * (h & 1) + 32 * (h >> 1) + 64 * (i >> 1) + 16 * (i & 1)));
 #pragma unroll
         for (int i = 0; i < LPW; i++) {
             U4 c = q[i];
             pin(c);  // (converted here, not when they were loaded)
-            acc = rb_mfma<T>(i8x8_to_operand<T>(c.x, c.y), b[2 * i], acc);
-            acc = rb_mfma<T>(i8x8_to_operand<T>(c.z, c.w), b[2 * i + 1], acc);
+            const U4 lo = i8x8_to_operand<T>(c.x, c.y), hi = i8x8_to_operand<T>(c.z, c.w);
+#pragma unroll
+            for (int mc = 0; mc < MC; mc++) {
+                acc[mc] = rb_mfma<T>(lo, b[mc][2 * i], acc[mc]);
+                acc[mc] = rb_mfma<T>(hi, b[mc][2 * i + 1], acc[mc]);
+            }
         }
     };
     if constexpr (NORM > 0) {
@@ -118,17 +137,16 @@ __global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(cons
             }
         }
         __syncthreads();
-        const char *arow = lds + (size_t)mrow * AS + kw * 256;
         for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
 #pragma unroll
             for (int d = 0; d < DEPTH; d++) {
                 const int sl = s0 + d;
-                if (sl * WK + kw < iters) multiply(w[d], arow + (size_t)sl * WK * 256);
+                if (sl * WK + kw < iters) multiply(w[d], lds + (size_t)(sl * WK + kw) * 256, AS);
                 if (s0 + DEPTH < slabs) load_w(sl + DEPTH, w[d]);
             }
         }
     } else {
-        constexpr int PK = rb_panel_k<RB, SPP>(), AS = rb_row_bytes<RB, SPP>(), CPR = (PK + 511) / 512;  // 1 KB copies per row
+        constexpr int PK = S::PANEL, AS = S::ROW_BYTES, CPR = (PK + 511) / 512;  // 1 KB copies per row
         const int panels = (slabs + SPP - 1) / SPP;
         auto issue_panel = [&](int p) {
             char *dst = lds + (size_t)(p & 1) * M * AS;
@@ -143,7 +161,6 @@ __global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(cons
         asm volatile("" ::: "memory");  // (the counts below rely on the order of the requests)
 #pragma unroll
         for (int d = 0; d < DEPTH; d++) load_w(d, w[d]);
-        const char *arow = lds + (size_t)mrow * AS + kw * 256;
         constexpr int AGE = (SPP < DEPTH ? SPP : DEPTH) * LPW;  // weight loads younger than the panel that is waited for, at least
         for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
 #pragma unroll
@@ -159,7 +176,7 @@ __global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(cons
                         if (sl / SPP + 1 < panels) issue_panel(sl / SPP + 1);
                         asm volatile("" ::: "memory");
                     }
-                    if (sl * WK + kw < iters) multiply(w[d], arow + (size_t)((sl / SPP) & 1) * M * AS + (size_t)(sl % SPP) * WK * 256);
+                    if (sl * WK + kw < iters) multiply(w[d], lds + (size_t)((sl / SPP) & 1) * M * AS + (size_t)((sl % SPP) * WK + kw) * 256, AS);
                 }
                 load_w(sl + DEPTH, w[d]);  // (past the end: the last step once more, unused; it keeps the counts)
             }
@@ -169,10 +186,13 @@ __global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(cons
 
     // D[n][m]: lane holds column m = lane % RH and rows n = 4 * (lane / RH) + e % 4, + 8 * (e / 4) in the 32-row form
     float *red = (float *)lds;
-    if (r < M) {
-        float *dst = red + ((size_t)(kw * RB + rb) * M + r) * RS + 4 * h;
 #pragma unroll
-        for (int e4 = 0; e4 < RH * RH / 256; e4++) *(float4 *)(dst + e4 * 8) = float4{acc[e4 * 4], acc[e4 * 4 + 1], acc[e4 * 4 + 2], acc[e4 * 4 + 3]};
+    for (int mc = 0; mc < MC; mc++) {
+        const int m = (cg * MC + mc) * RH + r;
+        if (m >= M) continue;
+        float *dst = red + ((size_t)(kw * RB + rb) * M + m) * RS + 4 * h;
+#pragma unroll
+        for (int e4 = 0; e4 < RH * RH / 256; e4++) *(float4 *)(dst + e4 * 8) = float4{acc[mc][e4 * 4], acc[mc][e4 * 4 + 1], acc[mc][e4 * 4 + 2], acc[mc][e4 * 4 + 3]};
     }
     __syncthreads();
     for (int o = tid; o < RB * M * PR; o += WAVES * 64) {
@@ -209,51 +229,47 @@ __global__ __launch_bounds__(rb_waves<RB>() * 64) void rowblock_gemm_kernel(cons
 }
 
 // ---- which form: as many workgroups as there are CUs and no more, each with whole row blocks.
-// HALF   up to 256 blocks of 16 rows (and 16 activation rows: the columns of the 16 x 16 product)
-// ONE    one block of 32 rows per workgroup while that is at most one per CU
-// THREE  three blocks of 16 rows, twelve waves, up to 256 such workgroups (with a norm over more than 2048 values its rows
-//        do not fit the registers of twelve waves)
+// HALF   up to 256 blocks of 16 rows
+// ONE    one block of 32 rows per workgroup while that is at most one per CU (more than 32 activation rows: two of 16)
+// THREE  three blocks of 16 rows, twelve waves, up to 256 such workgroups (16 activation rows; with a norm over more than 2048
+//        values its rows do not fit the registers of twelve waves)
 // TWO    two blocks of 32 rows; from 768 row blocks on skinny.hip's one-launch form streams the weights just as fast
 //        (28672 x 4096, 8 rows: 23 us) and this kernel is not taken
 // 8 rows, us, 32-row forms / HALF or THREE: 2560 x 2048 with norm 7.2 / 6.1, 2048 x 2048 6.3 / 4.9, 2048 x 5632 9.4 / 7.2, 4096 x
 // 14336 18.6 / 14.5, 11264 x 2048 with norm 9.5 / 7.9, 10000 x 4096 12.6 / 11.2; but 6144 x 4096 9.1 / 9.7, 10000 x 4096 with norm
-// 14.1 / 15.9.  What a workgroup reads of its activations (as much as of 16 weight rows) is what keeps it from splitting further.
+// 14.1 / 15.9.  24 rows, ONE or TWO / HALF with two tiles of activation rows: 2048 x 2048 6.9 / 5.7, 2048 x 5632 11.0 / 9.0.  48 rows,
+// here / two launches of skinny.hip: 2560 x 2048 7.4 / 12, 2048 x 2048 7.0 / 12, 11264 x 2048 11.5 / 18, 2048 x 5632 13.1 / 12.6.
+// A CU gets some 50 GB/s of weights and 180 GB/s of activations, which every workgroup reads in full: that is what keeps
+// large K with many rows out of this kernel (rowblock_supported).
 // The norm rides along up to 16 rows (8 rows x 2560 x 2048: 7.2 us with it in the ONE form against 6.0 + a launch of 2.5;
 // every workgroup normalises all rows for itself, at 32 rows that costs 3.7 us).
-enum RbForm { RB_HALF, RB_ONE, RB_THREE, RB_TWO };
-static RbForm rb_form(int M, int N, int K, bool norm) {
-    if (M <= 16 && N <= 256 * 16) return RB_HALF;
-    if (N <= 256 * 32) return RB_ONE;
-    if (M <= 16 && N <= 256 * 48 && (!norm || K <= 2048)) return RB_THREE;
-    return RB_TWO;
-}
-// (K > 8192: half the panel per step, 4096 x 14336 14.5 us against 15.4)
-static size_t rb_lds(int M, int N, int K, bool norm) {
-    auto panels = [&](int pk, int row) { return (size_t)(K > pk ? 2 : 1) * M * row; };
-    const RbForm f = rb_form(M, N, K, norm);
-    size_t act;
-    if (norm) act = (size_t)M * (K * 2 + 16);
-    else if (f == RB_HALF && K <= 8192) act = panels(rb_panel_k<1, 2>(), rb_row_bytes<1, 2>());
-    else if (f == RB_HALF || f == RB_ONE) act = panels(rb_panel_k<1, 1>(), rb_row_bytes<1, 1>());
-    else if (f == RB_THREE) act = panels(rb_panel_k<3, 2>(), rb_row_bytes<3, 2>());
-    else act = panels(rb_panel_k<2, 2>(), rb_row_bytes<2, 2>());
-    const size_t red = (size_t)(f == RB_THREE ? rb_waves<3>() : rb_waves<1>()) * M * kRbRed * sizeof(float);
-    return act > red ? act : red;
+template <typename F> static auto rb_shape(int M, int N, int K, bool norm, F &&f) {
+    if (N <= 256 * 16) {
+        if (M > 32) return f(RbShape<1, 16, 4, 2, 2, 1>{});
+        if (M > 16) return f(RbShape<1, 16, 8, 1, 2, 1>{});
+        if (norm || K > 8192) return f(RbShape<1, 16, 8, 1, 1, 1>{});  // (4096 x 14336: 14.5 us against 15.4 with two slabs per panel)
+        return f(RbShape<1, 16, 8, 1, 1, 2>{});
+    }
+    if (N <= 256 * 32) return M > 32 ? f(RbShape<2, 16, 4, 1, 4, 1>{}) : f(RbShape<1, 32, 8, 1, 1, 1>{});
+    if (M <= 16 && N <= 256 * 48 && (!norm || K <= 2048)) return f(RbShape<3, 16, 4, 1, 1, 2>{});
+    return M > 32 ? f(RbShape<2, 32, 4, 1, 2, 1>{}) : f(RbShape<2, 32, 4, 1, 1, 2>{});
 }
 bool rowblock_supported(int M, int N, int K, bool norm) {
     return M >= 1 && M <= kRbMaxRows && (M <= 16 || (long)N * K <= (12l << 20) || (N + 31) / 32 > 256) && K % 128 == 0 && N >= 1 && (N + 31) / 32 < 768 && (!norm || (M <= 16 && K <= 4096)) &&
-           rb_lds(M, N, K, norm) <= 160 * 1024;
+           rb_shape(M, N, K, norm, [&](auto s) { return decltype(s)::lds(M, K, norm); }) <= 160 * 1024;
 }
 
-template <typename T, int RB, int RH, int SPP, int EPI, int NORM>
+template <typename T, typename S, int EPI, int NORM>
 static int rb_go(const void *act, const void *pk, const void *scale, const void *res, const void *norm_w, void *out, int M, int N, int K, float eps,
-                 size_t lds, hipStream_t s) {
+                 hipStream_t s) {
     static size_t lds_set = 64 * 1024;
+    const size_t lds = S::lds(M, K, NORM > 0);
     if (lds > lds_set) {
-        MYNN_HIP(hipFuncSetAttribute((const void *)rowblock_gemm_kernel<T, RB, RH, SPP, EPI, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        MYNN_HIP(hipFuncSetAttribute((const void *)rowblock_gemm_kernel<T, S, EPI, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         lds_set = 160 * 1024;
     }
-    MYNN_LAUNCH((rowblock_gemm_kernel<T, RB, RH, SPP, EPI, NORM>), dim3((N + RH * RB - 1) / (RH * RB)), dim3(rb_waves<RB>() * 64), lds, s, (const T *)act,
+    constexpr int rows = S::RB * S::RH;
+    MYNN_LAUNCH((rowblock_gemm_kernel<T, S, EPI, NORM>), dim3((N + rows - 1) / rows), dim3(S::WAVES * 64), lds, s, (const T *)act,
                 (const U4 *)pk, (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, M, N, K, eps);
     return launch_status("rowblock_gemm_kernel");
 }
@@ -263,23 +279,23 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
     MYNN_REQUIRE(out && act && packed && scale && (epi != GEMM_RESIDUAL || res), MYNN_ERR_INVALID, "rowblock_gemm: null operand");
     MYNN_REQUIRE(rowblock_supported(M, N, K, norm_w != nullptr) && (epi != GEMM_SWIGLU || N % 2 == 0), MYNN_ERR_UNSUPPORTED, "rowblock_gemm: M=%d N=%d K=%d", M, N, K);
     MYNN_REQUIRE(aligned16(act) && aligned16(packed) && (!norm_w || aligned16(norm_w)), MYNN_ERR_INVALID, "rowblock_gemm: operands must be 16-byte aligned");
-    const size_t lds = rb_lds(M, N, K, norm_w != nullptr);
-    const RbForm f = rb_form(M, N, K, norm_w != nullptr);
     return dispatch_dtype16(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
-        auto go = [&](auto e) {
-            constexpr int EPI = decltype(e)::value;
-#define RB_GO(RB, RH, SPP, NORM) rb_go<T, RB, RH, SPP, EPI, NORM>(act, packed, scale, res, norm_w, out, M, N, K, eps, lds, s)
-            if (norm_w && K <= 2048)
-                return f == RB_HALF ? RB_GO(1, 16, 1, 4) : f == RB_ONE ? RB_GO(1, 32, 1, 4) : f == RB_THREE ? RB_GO(3, 16, 2, 4) : RB_GO(2, 32, 2, 4);
-            if (norm_w) return f == RB_HALF ? RB_GO(1, 16, 1, 8) : f == RB_ONE ? RB_GO(1, 32, 1, 8) : RB_GO(2, 32, 2, 8);
-            if (f == RB_HALF) return K > 8192 ? RB_GO(1, 16, 1, 0) : RB_GO(1, 16, 2, 0);
-            return f == RB_ONE ? RB_GO(1, 32, 1, 0) : f == RB_THREE ? RB_GO(3, 16, 2, 0) : RB_GO(2, 32, 2, 0);
-#undef RB_GO
-        };
-        if (epi == GEMM_RESIDUAL) return go(std::integral_constant<int, GEMM_RESIDUAL>{});
-        if (epi == GEMM_SWIGLU) return go(std::integral_constant<int, GEMM_SWIGLU>{});
-        return go(std::integral_constant<int, GEMM_PLAIN>{});
+        return rb_shape(M, N, K, norm_w != nullptr, [&](auto shape) {
+            using S = decltype(shape);
+            auto go = [&](auto e) {
+                constexpr int EPI = decltype(e)::value;
+                if constexpr (S::ROWS <= 32 && !(S::ROWS == 32 && S::RH == 16)) {  // (the shapes of up to 16 rows)
+                    if (norm_w && K <= 2048) return rb_go<T, S, EPI, 4>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
+                    if constexpr (S::RB != 3)
+                        if (norm_w) return rb_go<T, S, EPI, 8>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
+                }
+                return rb_go<T, S, EPI, 0>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
+            };
+            if (epi == GEMM_RESIDUAL) return go(std::integral_constant<int, GEMM_RESIDUAL>{});
+            if (epi == GEMM_SWIGLU) return go(std::integral_constant<int, GEMM_SWIGLU>{});
+            return go(std::integral_constant<int, GEMM_PLAIN>{});
+        });
     });
 }
 

@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(T *out, const float 
 // the MLP's norm, the down projection before the next layer's): one workgroup per output row, four columns per
 // thread, every load issued before the first sum; x_out = T(T(sum * scale) + res), nrm_out = T((x * inv) * w)
 // with inv = 1 / sqrt(mean(x^2) + eps) over the stored (rounded) x, as the separate operators compute them.
-constexpr int kReduceNormThreads = 1024, kReduceNormMaxSplit = 8;
+constexpr int kReduceNormThreads = 1024, kReduceNormMaxSplit = 12;  // (2048 x 5632: 11 ranges)
 template <typename T>
 __global__ __launch_bounds__(kReduceNormThreads) void skinny_reduce_norm_kernel(T *x_out, T *nrm_out, const float *part, const T *scale,
                                                                               const T *res, const T *norm_w, int M, int N, int ksplit,
