@@ -75,7 +75,11 @@ int mynn_dequant_gemv(void *out, const void *act, const int8_t *wq, const void *
  *   M >= 16, 16-bit act+scale, K % 8 == 0 -> matrix-core GEMM with W dequantised to the 16-bit
  *        type (scale folded in, one rounding) before the MMA (dequant_matmul_wmma.cuh:87-192);
  *   otherwise scale-after-sum per (m,n) (dequant_gemv.cuh / dequant_matmul.cuh:12-51).
- * act [M,K], out [M,N]. */
+ * act [M,K], out [M,N].
+ * For M >= 16 the f32 sum of an output may run over several ranges of K, each summed up from zero and added in their
+ * order.  Their number is a function of M, N, K and the type alone: this call, the same call captured into a graph,
+ * mynn_dequant_matmul_ws with any tile and mynn_dequant_matmul_prepared give the same bits.  (Another M may be summed up
+ * in another number of ranges, so a row's last bits can depend on how many rows it is multiplied with.) */
 int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq, const void *scale,
                         int M, int N, int K, int act_dtype, int out_dtype, mynn_stream s);
 
@@ -84,7 +88,8 @@ int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq, const void
  * call; nothing global is touched, so the call can be captured into a graph and calls on several streams
  * may overlap when their workspaces differ.  gemm_tile forces the workgroup tile of the matrix-core GEMM:
  * 0 = chosen per shape, 1 = 256x128, 2 = 256x256 with operands staged through registers, 3 = 256x256 and
- * 4 = 256x320 with operands loaded straight into LDS (3 and 4 fall back to 1 when K % 64 != 0). */
+ * 4 = 256x320 with operands loaded straight into LDS (3 and 4 fall back to 1 when K % 64 != 0, and every forced tile
+ * is 1 where the sum runs over several ranges of K). */
 size_t mynn_dequant_matmul_workspace_bytes(int M, int N, int K, int act_dtype, int out_dtype);
 int mynn_dequant_matmul_ws(void *out, const void *act, const int8_t *wq, const void *scale,
                            int M, int N, int K, int act_dtype, int out_dtype,

@@ -92,9 +92,11 @@ __device__ inline void tile_of(int b, int nblocks, int tiles_m, int tiles_n, int
 // EPI: GEMM_PLAIN C = T(acc); GEMM_RESIDUAL C = T(R + T(acc)) with R laid out like C;
 // GEMM_SWIGLU: B's rows are gate/up interleaved in groups of 32, C is [M, N/2] and
 // C = T(swish(T(acc_gate)) * T(acc_up)) -- the roundings of separate linear, Add and SwiGLU ops.
-template <typename T, typename G, bool KTAIL, int EPI>
+// RANGES: the sum runs over `ranges` K ranges, cut where tile_gemm_kernel cuts them, each from zero and added to the sum of
+// those before it: the bits of a product that is split over workgroups there.
+template <typename T, typename G, bool KTAIL, int EPI, bool RANGES>
 __global__ __launch_bounds__(G::THREADS) void gemm_nt_mfma_kernel(T *C, const T *A, const T *B, const T *R, int M, int N,
-                                                                 int K, int Kp) {
+                                                                 int K, int Kp, int ranges) {
     constexpr int BM = G::BM, BN = G::BN, TI = G::TI, TJ = G::TJ, CA = G::CA, CB = G::CB, RPP = G::ROWS_PER_PASS;
     extern __shared__ __align__(16) uint16_t lds[];
     uint16_t *As = lds, *Bs = lds + 2 * BM * LDT;  // As[buf] = As + buf*BM*LDT, Bs[buf] = Bs + buf*BN*LDT
@@ -158,6 +160,21 @@ __global__ __launch_bounds__(G::THREADS) void gemm_nt_mfma_kernel(T *C, const T 
     };
 
     const int nk = Kp / BK;  // even: Kp is a multiple of 2*BK
+    f16x_t sum[RANGES ? TI : 1][RANGES ? TJ : 1];
+    int z = 0, border = RANGES ? (int)((long)(nk / 2) / ranges) * 2 : 0;  // first K step of range z + 1
+    auto end_of_range = [&]() {
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    sum[i][j][e] = z == 0 ? acc[i][j][e] : sum[i][j][e] + acc[i][j][e];
+                    acc[i][j][e] = 0.f;
+                }
+        ++z;
+        border = (int)((long)(nk / 2) * (z + 1) / ranges) * 2;
+    };
     Stage rA, rB;
     load_tiles(rA, 0);
     store_tiles(0, rA);
@@ -173,6 +190,15 @@ __global__ __launch_bounds__(G::THREADS) void gemm_nt_mfma_kernel(T *C, const T 
         store_tiles(0, rB);                            // tile kt+2
         load_tiles(rB, min(kt + 4, nk - 1) * BK);
         __syncthreads();
+        if constexpr (RANGES) {
+            if (kt + 2 == border) end_of_range();
+        }
+    }
+    if constexpr (RANGES) {
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) acc[i][j] = sum[i][j];
     }
 
     gemm_store<T, G, EPI>([&](int i, int j, int e) { return acc[i][j][e]; }, lds, C, R, M, N, m0, n0, wrow, wcol, lane, wave);
@@ -403,25 +429,25 @@ int dequant_weight_rows(void *dst, const int8_t *wq, const void *scale, int N, i
     });
 }
 
-template <typename T, typename G, int EPI>
+template <typename T, typename G, int EPI, bool RANGES = false>
 static int gemm_launch_tile(void *out, const void *act, const void *wt, const void *res, int M, int N, int K,
-                            hipStream_t s) {
+                            hipStream_t s, int ranges = 1) {
     const int Kp = gemm_kp(K);
     const int tiles = ((M + G::BM - 1) / G::BM) * ((N + G::BN - 1) / G::BN);
     static bool lds_set = false;  // the kernels want more LDS than the 64 KB default
     if (!lds_set) {
-        MYNN_HIP(hipFuncSetAttribute((const void *)gemm_nt_mfma_kernel<T, G, false, EPI>,
+        MYNN_HIP(hipFuncSetAttribute((const void *)gemm_nt_mfma_kernel<T, G, false, EPI, RANGES>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS));
-        MYNN_HIP(hipFuncSetAttribute((const void *)gemm_nt_mfma_kernel<T, G, true, EPI>,
+        MYNN_HIP(hipFuncSetAttribute((const void *)gemm_nt_mfma_kernel<T, G, true, EPI, RANGES>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS));
         lds_set = true;
     }
     if (K == Kp)
-        MYNN_LAUNCH((gemm_nt_mfma_kernel<T, G, false, EPI>), dim3(tiles), dim3(G::THREADS), G::LDS, s, (T *)out,
-                           (const T *)act, (const T *)wt, (const T *)res, M, N, K, Kp);
+        MYNN_LAUNCH((gemm_nt_mfma_kernel<T, G, false, EPI, RANGES>), dim3(tiles), dim3(G::THREADS), G::LDS, s, (T *)out,
+                           (const T *)act, (const T *)wt, (const T *)res, M, N, K, Kp, ranges);
     else
-        MYNN_LAUNCH((gemm_nt_mfma_kernel<T, G, true, EPI>), dim3(tiles), dim3(G::THREADS), G::LDS, s, (T *)out,
-                           (const T *)act, (const T *)wt, (const T *)res, M, N, K, Kp);
+        MYNN_LAUNCH((gemm_nt_mfma_kernel<T, G, true, EPI, RANGES>), dim3(tiles), dim3(G::THREADS), G::LDS, s, (T *)out,
+                           (const T *)act, (const T *)wt, (const T *)res, M, N, K, Kp, ranges);
     return launch_status("gemm_nt_mfma_kernel");
 }
 
@@ -497,7 +523,7 @@ static int gemm_launch(void *out, const void *act, const void *wt, const void *r
 }
 
 int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, int M, int N, int K, int dtype, int epi,
-                 hipStream_t s, int tile) {
+                 hipStream_t s, int tile, int ranges) {
     MYNN_REQUIRE(tile >= 0 && tile <= 4, MYNN_ERR_INVALID,
                  "gemm tile %d is not 0 (automatic), 1 (256x128), 2 (256x256), 3 (256x256, direct-to-LDS loads) or 4 (256x320, direct-to-LDS loads)", tile);
     MYNN_REQUIRE(out && act && wt, MYNN_ERR_INVALID, "dequant_matmul: null operand");
@@ -505,8 +531,10 @@ int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, in
     MYNN_REQUIRE(aligned16(act) && aligned16(wt), MYNN_ERR_INVALID, "dequant_matmul: act must be 16-byte aligned");
     MYNN_REQUIRE(epi != GEMM_RESIDUAL || res, MYNN_ERR_INVALID, "dequant_matmul: residual store without a residual");
     MYNN_REQUIRE(epi != GEMM_SWIGLU || N % 64 == 0, MYNN_ERR_INVALID, "dequant_matmul: SwiGLU store needs N %% 64 == 0, N=%d", N);
+    MYNN_REQUIRE(ranges >= 1 && ranges <= (K + 63) / 64 && (ranges == 1 || epi == GEMM_PLAIN), MYNN_ERR_INVALID, "dequant_matmul: %d K ranges, store %d", ranges, epi);
     return dispatch_dtype16(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
+        if (ranges > 1) return gemm_launch_tile<T, Tile256x128, GEMM_PLAIN, true>(out, act, wt, nullptr, M, N, K, s, ranges);
         if (epi == GEMM_RESIDUAL) return gemm_launch<T, GEMM_RESIDUAL>(out, act, wt, res, M, N, K, tile, s);
         if (epi == GEMM_SWIGLU) return gemm_launch<T, GEMM_SWIGLU>(out, act, wt, res, M, N, K, tile, s);
         return gemm_launch<T, GEMM_PLAIN>(out, act, wt, res, M, N, K, tile, s);
@@ -581,22 +609,30 @@ static size_t tiles_scratch(int kind, int N, int K) {
 static bool tiles_first(const TgPlan &plan, int kind, int M, int N, int K, int dtype) {
     return kind == TG_W8S || plan.us <= gemm_nt_mfma_us(M, N, K, dtype) + dequant_us(N, K);
 }
-
-int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
-                      int tile, hipStream_t s) {
-    int rc = dequant_weight_rows(ws, wq, scale, N, K, dtype, 0, 0, s);
-    if (rc) return rc;
-    return gemm_nt_mfma(out, act, ws, nullptr, M, N, K, dtype, GEMM_PLAIN, s, tile);
+// K ranges of the sums of a product of 16 and more rows: by its sizes and type alone, so that every form of the operator --
+// this one, a caller's workspace, a forced tile, a prepared weight, an operand that is not aligned for the tiles, a call that
+// is being captured -- has the same sums, bit for bit.
+static int sum_ranges(int M, int N, int K, int dtype) {
+    if (M < 16 || N <= 0 || !tile_gemm_supported(TG_W8, M, N, K)) return 1;
+    const TgPlan plan = tile_gemm_plan(TG_W8, dtype, M, N, K, tiles_scratch(TG_W8, N, K));
+    return tiles_first(plan, TG_W8, M, N, K, dtype) ? plan.ks : 1;
 }
 
-// partial sums of quantized_matmul's K ranges (0 bytes under capture when there are none yet: one range then)
-int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters, size_t *bytes) {
+int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
+                      int tile, hipStream_t s, int ranges) {
+    int rc = dequant_weight_rows(ws, wq, scale, N, K, dtype, 0, 0, s);
+    if (rc) return rc;
+    return gemm_nt_mfma(out, act, ws, nullptr, M, N, K, dtype, GEMM_PLAIN, s, tile, ranges);
+}
+
+// partial sums and arrival counters of a product's K ranges; not for a call that is being captured (tile_gemm_plan_seq)
+int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters) {
     StreamWs w;
     int rc = stream_workspace(s, need, &w);
     if (rc) return rc;
+    MYNN_REQUIRE(w.ptr && w.bytes >= need, MYNN_ERR_STATE, "the library workspace cannot grow while the stream is being captured");
     *counters = (int *)w.ptr;
     *part = w.ptr + kWsCounterBytes;
-    *bytes = w.ptr ? w.bytes : 0;
     return 0;
 }
 
@@ -637,7 +673,7 @@ extern "C" int mynn_dequant_matmul_ws(void *out, const void *act, const int8_t *
                                  (char *)workspace + kWsCounterBytes, (int *)workspace, as_stream(s));
             }
         }
-        return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, workspace, gemm_tile, as_stream(s));
+        return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, workspace, gemm_tile, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));
 }
@@ -651,11 +687,10 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
         if (tiles_first(plan, kind, M, N, K, out_dtype)) {
             void *part = nullptr;
             int *counters = nullptr;
-            size_t have = 0;
-            if (plan.ks > 1) {
-                int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters, &have);
+            if (plan.ks > 1 && stream_capturing(as_stream(s))) plan = tile_gemm_plan_seq(kind, out_dtype, M, N, K, plan.ks);
+            else if (plan.ks > 1) {
+                int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters);
                 if (rc) return rc;
-                if (have < plan.part_bytes) plan = tile_gemm_plan(kind, out_dtype, M, N, K, have);
             }
             return tile_gemm(kind, plan, out, nullptr, act, wq, nullptr, scale, nullptr, M, N, K, out_dtype, GEMM_PLAIN, part, counters, as_stream(s));
         }
@@ -667,7 +702,7 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
         if (rc) return rc;
         MYNN_REQUIRE(ws.bytes >= gemm_weight_bytes(N, K), MYNN_ERR_STATE, "dequant_matmul: the library workspace cannot grow while the stream is being captured; "
                                                                           "pass a workspace (mynn_dequant_matmul_ws) or a prepared weight");
-        return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s));
+        return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));
 }
@@ -681,5 +716,5 @@ extern "C" int mynn_dequant_weight_prepare(void *wt, const int8_t *wq, const voi
 extern "C" int mynn_dequant_matmul_prepared(void *out, const void *act, const void *wt, int M, int N, int K, int dtype,
                                             int gemm_tile, mynn_stream s) {
     MYNN_REQUIRE(M >= 16, MYNN_ERR_UNSUPPORTED, "dequant_matmul_prepared: M=%d (the prepared weight serves the matrix-core path, M >= 16)", M);
-    return gemm_nt_mfma(out, act, wt, nullptr, M, N, K, dtype, GEMM_PLAIN, as_stream(s), gemm_tile);
+    return gemm_nt_mfma(out, act, wt, nullptr, M, N, K, dtype, GEMM_PLAIN, as_stream(s), gemm_tile, sum_ranges(M, N, K, dtype));
 }

@@ -82,12 +82,13 @@ double qgemm_dma_us(int M, int N, int K);  // its time by measurement, for the c
 int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_scale, const int8_t *rhs, const void *rhs_scale,
               const void *res, int M, int N, int K, int dtype, int epi, hipStream_t s);
 // tile: 0 heuristic; 1 = 256x128, 2 = 256x256 (register staged); 3 = 256x256, 4 = 256x320 (direct to LDS)
+// ranges > 1 (GEMM_PLAIN): each K range of tile_gemm is summed up on its own and the sums are added in their order, in tiles of 256x128
 int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, int M, int N, int K, int dtype, int epi,
-                 hipStream_t s, int tile = 0);
+                 hipStream_t s, int tile = 0, int ranges = 1);
 double gemm_nt_mfma_us(int M, int N, int K, int dtype);  // its time by measurement, for the choice against tile_gemm
 // W_T = T(wq * scale) into `ws` (gemm_weight_bytes), then out = act . W_T^T
 int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
-                      int tile, hipStream_t s);
+                      int tile, hipStream_t s, int ranges = 1);
 
 // tile_gemm.hip -- products of ordinary size with operand tiles of 32 .. 128 rows, K ranges where those do not fill the
 // device.  TG_W8 / TG_W8S: 16-bit activations, int8 weights scaled before / after the products; TG_I8: QuantizedMatMul.
@@ -96,14 +97,17 @@ struct TgPlan {
     int tile = 0, ks = 1;  // which tile, how many K ranges
     double us = 0;         // the time the choice was made by
     size_t part_bytes = 0; // partial sums of the ranges
+    bool seq = false;      // the ranges one after the other in one workgroup: no scratch memory, the same sums
 };
 constexpr int kTgCounters = 4096;             // arrival counters (ints) of a launch, zero between launches
 constexpr size_t kTgScratchMax = 32u << 20;   // no plan needs more partial sums than this
 bool tile_gemm_supported(int kind, int M, int N, int K);
 // the best choice whose partial sums fit scratch_bytes (0: one K range)
 TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes);
+// the same sums as a plan of ks ranges has, without scratch memory (GEMM_PLAIN)
+TgPlan tile_gemm_plan_seq(int kind, int dtype, int M, int N, int K, int ks);
 // epi: GEMM_PLAIN, GEMM_RESIDUAL or GEMM_SWIGLU_PAIRS (gate and up rows alternate); part, counters: for plans with ranges
-int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters, size_t *bytes);  // the stream's (gemm.hip)
+int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters);  // the stream's (gemm.hip)
 int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
               const void *res, int M, int N, int K, int dtype, int epi, void *part, int *counters, hipStream_t s);
 

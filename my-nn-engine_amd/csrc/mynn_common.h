@@ -235,6 +235,14 @@ LaunchTimer &launch_timer();
         }                                                                                                          \
     } while (0)
 
+// is the stream being captured into a graph?  (what a captured launch points at has to live as long as the graph)
+inline bool stream_capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 inline int launch_status(const char *what) {
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : hip_fail(e, what);

@@ -106,11 +106,10 @@ extern "C" int mynn_quantized_matmul(void *out, int32_t *acc_out, const int8_t *
             return qgemm_dma(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, as_stream(s));
         void *part = nullptr;
         int *counters = nullptr;
-        size_t have = 0;
-        if (plan.ks > 1) {
-            int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters, &have);
+        if (plan.ks > 1 && stream_capturing(as_stream(s))) plan = tile_gemm_plan_seq(TG_I8, dtype, M, N, K, plan.ks);
+        else if (plan.ks > 1) {
+            int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters);
             if (rc) return rc;
-            if (have < plan.part_bytes) plan = tile_gemm_plan(TG_I8, dtype, M, N, K, have);
         }
         return tile_gemm(TG_I8, plan, out, acc_out, lhs, rhs, lhs_scale, rhs_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, part, counters, as_stream(s));
     }

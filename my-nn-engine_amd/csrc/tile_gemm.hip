@@ -21,6 +21,10 @@
 // When the tiles do not fill the device the K range is split over workgroups.  Each leaves its partial sums in scratch
 // memory (agent-scope stores, which go past the XCD's L2) and counts itself in; the last to arrive adds them up in the
 // order of the ranges -- the result does not depend on who was last -- and stores the output.  Nobody waits for anybody.
+// SEQ: one workgroup takes all ranges of its tile one after the other and adds them up in registers: the same bits without
+// scratch memory, for calls that are being captured (a graph may be replayed on any stream and outlive any block).
+// It costs the parallelism: bf16, 6 rows x 4096 x 14336 109 us against 25, 6 x 2048 x 2048 14.3 against 8.2, 100 x 4096 x 4096
+// 29 against 17.
 #include <algorithm>
 #include <type_traits>
 
@@ -71,7 +75,7 @@ template <typename T, bool SCALED> __device__ inline U4 weight_operand(uint32_t 
 }
 
 // TAIL: the rows are not whole K steps, the last one reads zeros past their end
-template <typename T, typename G, int EPI, bool TAIL>
+template <typename T, typename G, int EPI, bool TAIL, bool SEQ>
 __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const void *A_, const int8_t *B, int M, int N, int K, int ks, T *C,
                                                                       const T *R, const T *a_scale, const T *b_scale,
                                                                       uint64_t *part, int *counter, int32_t *acc_out) {
@@ -96,18 +100,23 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
         constexpr int XCD = 8, BAND = 8;
         const int nb = gridDim.x, x = blockIdx.x % XCD, per = nb / XCD, rem = nb % XCD;
         const int l = x * per + min(x, rem) + blockIdx.x / XCD;
-        const int band = l / (BAND * tiles_n * ks), in_band = l - band * BAND * tiles_n * ks;
+        const int side = SEQ ? 1 : ks;  // K ranges side by side
+        const int band = l / (BAND * tiles_n * side), in_band = l - band * BAND * tiles_n * side;
         const int rows_here = min(BAND, tiles_m - band * BAND);
         tm = band * BAND + in_band % rows_here;
         const int rest = in_band / rows_here;
-        kz = rest % ks;
-        tn = rest / ks;
+        kz = rest % side;
+        tn = rest / side;
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const int a_bytes = K * EA;                    // bytes of an activation row; a weight row is K bytes
     const int iters = (a_bytes + 127) / 128;
-    const int it0 = (int)((long)iters * kz / ks), it1 = (int)((long)iters * (kz + 1) / ks);
-    const int n_it = it1 - it0;
+    int it0, n_it;
+    auto range = [&](int z) {  // (gemm_nt_mfma_kernel cuts K in the same places)
+        it0 = (int)((long)iters * z / ks);
+        n_it = (int)((long)iters * (z + 1) / ks) - it0;
+    };
+    range(kz);
 
     // this lane's chunks of each operand tile: LDS position P = (CH * wave + i) * 64 + lane.  Offsets are from the tile's
     // first row, so that a step's address is a scalar base plus a 32-bit lane offset.
@@ -215,9 +224,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
     // multiplies, so that neither the barrier nor the LDS latency is in front of the MFMAs.
     constexpr int KM = G::KM, AHEAD = NS - KM;  // steps whose loads are in flight ahead of the one that is read
     static_assert(NS % KM == 0 && AHEAD >= KM, "whole groups of stages");
-#pragma unroll
-    for (int s = 0; s < AHEAD; s++) issue(s, lds + s * G::STAGE);
-    int cur = 0, fill = AHEAD, it = 0;
+    int cur, fill, it;
     auto fetch = [&](Frags &f, auto first) {
         if constexpr (decltype(first)::value) {
             constexpr int VM = (AHEAD - KM) * (CHA + CHB);  // loads that may stay in flight: those of the later stages
@@ -250,26 +257,61 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
     };
     constexpr std::true_type whole;
     constexpr std::integral_constant<bool, KM == 1> second;
-    Frags f0, f1;
-    fetch(f0, whole);
-    __builtin_amdgcn_sched_barrier(0);
-    while (it + 1 < n_it) {
-        fetch(f1, second);
-        multiply(f0);
-        end_of_step();
+    auto one_range = [&]() {
+#pragma unroll
+        for (int s = 0; s < AHEAD; s++) issue(s, lds + s * G::STAGE);
+        cur = 0;
+        fill = AHEAD;
+        it = 0;
+        Frags f0, f1;
         fetch(f0, whole);
-        multiply(f1);
-        end_of_step();
+        __builtin_amdgcn_sched_barrier(0);
+        while (it + 1 < n_it) {
+            fetch(f1, second);
+            multiply(f0);
+            end_of_step();
+            fetch(f0, whole);
+            multiply(f1);
+            end_of_step();
+        }
+        if (it < n_it) {
+            fetch(f1, second);
+            multiply(f0);
+            multiply(f1);
+        } else multiply(f0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeats of the last step too, before LDS is reused
+        __syncthreads();
+    };
+    one_range();
+    if constexpr (SEQ) {
+        acc_t sum[TI][TJ];
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) sum[i][j] = acc[i][j];
+        for (int z = 1; z < ks; z++) {
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < TJ; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
+            range(z);
+            one_range();
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < TJ; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) sum[i][j][e] += acc[i][j][e];
+        }
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) acc[i][j] = sum[i][j];
     }
-    if (it < n_it) {
-        fetch(f1, second);
-        multiply(f0);
-        multiply(f1);
-    } else multiply(f0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeats of the last step too, before LDS is reused
-    __syncthreads();
 
-    if (ks > 1) {
+    if (!SEQ && ks > 1) {
         // partial sums, two per word, [range][(i, j), pair][thread]
         const size_t tile = (size_t)tn * tiles_m + tm;
         constexpr int WORDS = TI * TJ * 8;
@@ -445,6 +487,13 @@ TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_b
     return e.plan;
 }
 
+TgPlan tile_gemm_plan_seq(int kind, int dtype, int M, int N, int K, int ks) {
+    TgPlan plan = tile_gemm_plan(kind, dtype, M, N, K, 0);
+    plan.ks = kind == TG_I8 ? 1 : ks;  // (int32 sums are the same in any order)
+    plan.seq = plan.ks > 1;
+    return plan;
+}
+
 struct TgArgs {
     void *out;
     int32_t *acc_out;
@@ -452,24 +501,28 @@ struct TgArgs {
     const int8_t *wq;
     const void *a_scale, *w_scale, *res;
     int M, N, K, ks;
+    bool seq;
     uint64_t *part;
     int *counters;
     hipStream_t s;
 };
 
-template <typename T, typename G, int EPI, bool TAIL> static int tg_go(const TgArgs &p) {
+template <typename T, typename G, int EPI, bool TAIL, bool SEQ = false> static int tg_go(const TgArgs &p) {
     static bool lds_set = false;
     if (!lds_set && G::LDS > 64 * 1024) {
-        MYNN_HIP(hipFuncSetAttribute((const void *)tile_gemm_kernel<T, G, EPI, TAIL>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
+        MYNN_HIP(hipFuncSetAttribute((const void *)tile_gemm_kernel<T, G, EPI, TAIL, SEQ>, hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
         lds_set = true;
     }
     const int tiles = ((p.M + G::BM - 1) / G::BM) * ((p.N + G::BN - 1) / G::BN);
-    MYNN_LAUNCH((tile_gemm_kernel<T, G, EPI, TAIL>), dim3(tiles * p.ks), dim3(G::THREADS), G::LDS, p.s, p.act, p.wq, p.M, p.N, p.K, p.ks, (T *)p.out,
+    MYNN_LAUNCH((tile_gemm_kernel<T, G, EPI, TAIL, SEQ>), dim3(SEQ ? tiles : tiles * p.ks), dim3(G::THREADS), G::LDS, p.s, p.act, p.wq, p.M, p.N, p.K, p.ks, (T *)p.out,
                 (const T *)p.res, (const T *)p.a_scale, (const T *)p.w_scale, p.part, p.counters, p.acc_out);
     return launch_status("tile_gemm_kernel");
 }
 template <typename T, typename G> static int tg_epi(const TgArgs &p, int epi) {
     const bool tail = (size_t)p.K * (G::KIND == TG_I8 ? 1 : 2) % 128 != 0;
+    if constexpr (G::KIND != TG_I8) {
+        if (p.seq) return tail ? tg_go<T, G, GEMM_PLAIN, true, true>(p) : tg_go<T, G, GEMM_PLAIN, false, true>(p);
+    }
     if constexpr (G::KIND == TG_W8S || sizeof(T) == 4)
         return tail ? tg_go<T, G, GEMM_PLAIN, true>(p) : tg_go<T, G, GEMM_PLAIN, false>(p);
     else {
@@ -513,8 +566,9 @@ int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const v
     MYNN_REQUIRE(epi != GEMM_RESIDUAL || res, MYNN_ERR_INVALID, "tile_gemm: residual store without a residual");
     MYNN_REQUIRE(epi != GEMM_SWIGLU_PAIRS || (N % 2 == 0 && !acc_out), MYNN_ERR_INVALID, "tile_gemm: SwiGLU store needs row pairs, N=%d", N);
     MYNN_REQUIRE(epi != GEMM_SWIGLU && (kind != TG_W8S || epi == GEMM_PLAIN), MYNN_ERR_INVALID, "tile_gemm: store %d", epi);
-    MYNN_REQUIRE(plan.ks >= 1 && (plan.ks == 1 || (part && counters && aligned16(part))), MYNN_ERR_INVALID, "tile_gemm: K ranges without scratch memory");
-    const TgArgs p{out, acc_out, act, wq, a_scale, w_scale, res, M, N, K, plan.ks, (uint64_t *)part, counters, s};
+    MYNN_REQUIRE(plan.ks >= 1 && (plan.ks == 1 || plan.seq || (part && counters && aligned16(part))), MYNN_ERR_INVALID, "tile_gemm: K ranges without scratch memory");
+    MYNN_REQUIRE(!plan.seq || (kind != TG_I8 && epi == GEMM_PLAIN), MYNN_ERR_UNSUPPORTED, "tile_gemm: ranges one after the other: kind %d, store %d", kind, epi);
+    const TgArgs p{out, acc_out, act, wq, a_scale, w_scale, res, M, N, K, plan.ks, plan.seq, (uint64_t *)part, counters, s};
     MYNN_REQUIRE(dtype != MYNN_F32 || (kind == TG_I8 && epi == GEMM_PLAIN), MYNN_ERR_UNSUPPORTED, "tile_gemm: f32 output of int8 products only");
     return dispatch_dtype(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
