@@ -14,11 +14,9 @@
 // or 256 x 256, K step 32, operands staged through registers into padded LDS tiles, any K % 8 == 0).
 // The store can add a residual (o_proj, down_proj) or apply SwiGLU to interleaved gate/up columns.
 // The int8 form of gemm_nt_dma_kernel is QuantizedMatMul for large grids (qgemm_dma).
-#include <map>
-#include <mutex>
-
 #include "gemm_store.h"
 #include "kernels.h"
+#include "stream_block.h"
 
 namespace mynn {
 
@@ -553,38 +551,10 @@ double gemm_nt_mfma_us(int M, int N, int K, int dtype) {
 // ... and of dequant_weight_rows before it (3 bytes per weight)
 static double dequant_us(int N, int K) { return 2.0 + 3.0 * N * K / 5.6e6; }
 
-// ---- library-owned workspaces of the stand-alone entry points: one per stream, so calls on different streams never
-// share a dequantised weight or partial sums; the table is guarded by a mutex.  A workspace only ever grows, and growing
-// waits for the stream's earlier work before the old block is released.  Its first bytes are tile_gemm's arrival counters,
-// zero between calls.
-struct StreamWs {
-    char *ptr = nullptr;
-    size_t bytes = 0;
-};
-static std::mutex g_ws_mu;
-static std::map<hipStream_t, StreamWs> g_ws;
+// ---- library-owned workspaces of the stand-alone entry points: dequantised weights or partial sums.  The first bytes of a
+// block are tile_gemm's arrival counters, zero between calls.
+static StreamBlocks g_ws;
 constexpr size_t kWsCounterBytes = (size_t)kTgCounters * 4;
-
-// out->bytes: what there is behind the counters; less than `need` only while the stream is being captured
-static int stream_workspace(hipStream_t s, size_t need, StreamWs *out) {
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    StreamWs &w = g_ws[s];
-    if (need + kWsCounterBytes > w.bytes) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
-            *out = StreamWs{w.ptr, w.ptr ? w.bytes - kWsCounterBytes : 0};
-            return 0;
-        }
-        MYNN_HIP(hipStreamSynchronize(s));
-        if (w.ptr) MYNN_HIP(hipFree(w.ptr));
-        w = StreamWs{};
-        MYNN_HIP(hipMalloc((void **)&w.ptr, need + kWsCounterBytes));
-        w.bytes = need + kWsCounterBytes;
-        MYNN_HIP(hipMemsetAsync(w.ptr, 0, kWsCounterBytes, s));
-    }
-    *out = StreamWs{w.ptr, w.bytes - kWsCounterBytes};
-    return 0;
-}
 
 __global__ void zero_words_kernel(uint32_t *p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -625,15 +595,16 @@ int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *
     return gemm_nt_mfma(out, act, ws, nullptr, M, N, K, dtype, GEMM_PLAIN, s, tile, ranges);
 }
 
-// partial sums and arrival counters of a product's K ranges; not for a call that is being captured (tile_gemm_plan_seq)
-int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters) {
-    StreamWs w;
-    int rc = stream_workspace(s, need, &w);
-    if (rc) return rc;
-    MYNN_REQUIRE(w.ptr && w.bytes >= need, MYNN_ERR_STATE, "the library workspace cannot grow while the stream is being captured");
-    *counters = (int *)w.ptr;
-    *part = w.ptr + kWsCounterBytes;
-    return 0;
+int tile_gemm_on_stream(int kind, TgPlan plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale,
+                        const void *w_scale, int M, int N, int K, int dtype, hipStream_t s) {
+    StreamBlocks::Lease ws;
+    if (plan.ks > 1 && stream_capturing(s)) plan = tile_gemm_plan_seq(kind, dtype, M, N, K, plan.ks);
+    else if (plan.ks > 1) {
+        int rc = g_ws.lease(s, kWsCounterBytes + plan.part_bytes, kWsCounterBytes, "matrix product", &ws);
+        if (rc) return rc;
+    }
+    return tile_gemm(kind, plan, out, acc_out, act, wq, a_scale, w_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, ws.ptr ? ws.ptr + kWsCounterBytes : nullptr,
+                     (int *)ws.ptr, s);
 }
 
 // the reference's kernel choice (cuda.rs:1518-1652): matrix cores for M >= 16 with 16-bit operands
@@ -685,23 +656,14 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
     if (scale && takes_tiles(out, act, wq, M, N, K, act_dtype, out_dtype, &kind)) {
         TgPlan plan = tile_gemm_plan(kind, out_dtype, M, N, K, tiles_scratch(kind, N, K));
         if (tiles_first(plan, kind, M, N, K, out_dtype)) {
-            void *part = nullptr;
-            int *counters = nullptr;
-            if (plan.ks > 1 && stream_capturing(as_stream(s))) plan = tile_gemm_plan_seq(kind, out_dtype, M, N, K, plan.ks);
-            else if (plan.ks > 1) {
-                int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters);
-                if (rc) return rc;
-            }
-            return tile_gemm(kind, plan, out, nullptr, act, wq, nullptr, scale, nullptr, M, N, K, out_dtype, GEMM_PLAIN, part, counters, as_stream(s));
+            return tile_gemm_on_stream(kind, plan, out, nullptr, act, wq, nullptr, scale, M, N, K, out_dtype, as_stream(s));
         }
     }
     if (takes_matrix_cores(act, wq, M, K, act_dtype, out_dtype)) {
         MYNN_REQUIRE(N > 0 && K > 0, MYNN_ERR_INVALID, "dequant_matmul: N=%d K=%d", N, K);
-        StreamWs ws;
-        int rc = stream_workspace(as_stream(s), gemm_weight_bytes(N, K), &ws);
+        StreamBlocks::Lease ws;
+        int rc = g_ws.lease(as_stream(s), kWsCounterBytes + gemm_weight_bytes(N, K), kWsCounterBytes, "dequant_matmul", &ws);
         if (rc) return rc;
-        MYNN_REQUIRE(ws.bytes >= gemm_weight_bytes(N, K), MYNN_ERR_STATE, "dequant_matmul: the library workspace cannot grow while the stream is being captured; "
-                                                                          "pass a workspace (mynn_dequant_matmul_ws) or a prepared weight");
         return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));

@@ -107,9 +107,11 @@ TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_b
 // the same sums as a plan of ks ranges has, without scratch memory (GEMM_PLAIN)
 TgPlan tile_gemm_plan_seq(int kind, int dtype, int M, int N, int K, int ks);
 // epi: GEMM_PLAIN, GEMM_RESIDUAL or GEMM_SWIGLU_PAIRS (gate and up rows alternate); part, counters: for plans with ranges
-int tile_gemm_workspace(hipStream_t s, size_t need, void **part, int **counters);  // the stream's (gemm.hip)
 int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
               const void *res, int M, int N, int K, int dtype, int epi, void *part, int *counters, hipStream_t s);
+// the product with the stream's scratch memory for its ranges (gemm.hip), with none while the stream is being captured
+int tile_gemm_on_stream(int kind, TgPlan plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale,
+                        const void *w_scale, int M, int N, int K, int dtype, hipStream_t s);
 
 // elementwise.hip
 // device-side loop state of a batch-1 decode model; a null `ids` means "no bookkeeping"

@@ -101,17 +101,10 @@ extern "C" int mynn_quantized_matmul(void *out, int32_t *acc_out, const int8_t *
     // matrix cores from three rows on (two rows of 4096 x 4096: 6.2 us as dot products, 8.1 as tiles; three: 10 and 8),
     // with the 256-row tiles of gemm.hip where enough of them make that the faster one
     if (M >= 3 && (!out || aligned16(out))) {
-        TgPlan plan = tile_gemm_plan(TG_I8, dtype, M, N, K, kTgScratchMax);
+        const TgPlan plan = tile_gemm_plan(TG_I8, dtype, M, N, K, kTgScratchMax);
         if (dtype != MYNN_F32 && qgemm_dma_us(M, N, K) < plan.us)
             return qgemm_dma(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, as_stream(s));
-        void *part = nullptr;
-        int *counters = nullptr;
-        if (plan.ks > 1 && stream_capturing(as_stream(s))) plan = tile_gemm_plan_seq(TG_I8, dtype, M, N, K, plan.ks);
-        else if (plan.ks > 1) {
-            int rc = tile_gemm_workspace(as_stream(s), plan.part_bytes, &part, &counters);
-            if (rc) return rc;
-        }
-        return tile_gemm(TG_I8, plan, out, acc_out, lhs, rhs, lhs_scale, rhs_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, part, counters, as_stream(s));
+        return tile_gemm_on_stream(TG_I8, plan, out, acc_out, lhs, rhs, lhs_scale, rhs_scale, M, N, K, dtype, as_stream(s));
     }
     return dispatch_dtype(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
