@@ -17,14 +17,19 @@
  * Process-wide state, all of it: (a) the configuration that `mynn_model_configure` leaves for the
  * next `model_init` (the reference ABI has no other way to say it; `mynn_model_create` takes the
  * configuration as an argument and touches nothing global); (b) the scratch memory of the entry
- * points that need some and are not given any: `mynn_dequant_matmul` (M >= 16) and `mynn_attention`
- * (a cache split over workgroups) keep one grown-on-demand block PER STREAM under a mutex, so calls
- * on different streams never share one; growing synchronises that stream and cannot happen while
- * the stream is being captured (the call then fails with MYNN_ERR_STATE).  The `_ws` variants take
+ * points that need some and are not given any: `mynn_dequant_matmul` (M >= 2), `mynn_quantized_matmul`
+ * (M >= 3), `mynn_attention` (a cache split over workgroups) and `mynn_attention_streaming`.  Each of
+ * these three groups keeps one grown-on-demand block PER STREAM, locked until the call's launches are
+ * made, so calls on different streams never share one and several host threads may call on one stream.
+ * Growing synchronises that stream and cannot happen while the stream is being captured: a captured call
+ * that needs a larger block than there is fails with MYNN_ERR_STATE (make it once before the capture).
+ * A block that a captured call was given stays valid for the graph's life, also when a later call makes
+ * the stream's block grow; it is shared with that stream's other calls, so replays have to be ordered
+ * with those.  Products that only split K (no weight is dequantised: see the calls) use no library
+ * memory at all while being captured; their graphs may be replayed anywhere.  The `_ws` variants take
  * the caller's block instead and touch nothing global; `mynn_attention_noalloc` uses a fixed
- * device array of the library.  `mynn_attention_streaming` keeps one grown-on-demand block per stream
- * in the same way (`mynn_attention_streaming_ws` takes the caller's).  Executors (seam 1) own
- * everything they use: nothing an executor launches touches library-global memory.
+ * device array of the library.  Executors (seam 1) own everything they use: nothing an executor
+ * launches touches library-global memory.
  *
  * Return value of every `int` function: 0 on success, a negative MYNN_ERR_* for a rejected
  * argument, or a positive hipError_t.  Nothing here calls exit().

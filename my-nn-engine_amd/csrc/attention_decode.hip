@@ -20,12 +20,12 @@
 // key bound); the matrix-core prefill kernel lives in attention_prefill.hip.
 #include <type_traits>
 
-#include <map>
 #include <mutex>
 
 #include "attention.h"
 #include "mfma.h"
 #include "attention_short.h"
+#include "stream_block.h"
 
 namespace mynn {
 
@@ -473,38 +473,18 @@ int attention_decode_launch(AttnParams p, int D, int dtype, int kv_int8, void *s
     return attention_merge_launch(p, D, dtype, s);
 }
 
-// ---- library-owned scratch, grown on demand (the streaming-KV operators below; one set for all streams)
-struct Grown {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-};
-static int ensure(Grown &g, size_t bytes, bool zero, hipStream_t s) {
-    if (bytes <= g.bytes) return 0;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
-        return fail(MYNN_ERR_STATE, "the library's scratch memory cannot grow while the stream is being captured");
-    MYNN_HIP(hipStreamSynchronize(s));
-    if (g.ptr) MYNN_HIP(hipFree(g.ptr));
-    g.ptr = nullptr;
-    g.bytes = 0;
-    MYNN_HIP(hipMalloc(&g.ptr, bytes));
-    if (zero) MYNN_HIP(hipMemset(g.ptr, 0, bytes));
-    g.bytes = bytes;
-    return 0;
-}
-// mynn_attention: the partial results of a cache split over workgroups, one block per stream
-static std::mutex g_scratch_mu;
-static std::map<hipStream_t, Grown> g_scratch;
+// mynn_attention: arrival counters (zero between calls), then the partial results of a cache split over workgroups
+static StreamBlocks g_scratch;
+constexpr size_t kArriveBytes = (size_t)kAttnArrive * 4;
 
 // mynn_attention_noalloc: the same partial results in a device array of the library (one copy per GPU, held until the
 // process ends).  The array's name is only a handle on the host: the address kernels get is asked for once per device.
 constexpr size_t kStaticScratchBytes = 8u << 20;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
-static __device__ int scratch_arrive[kAttnArrive];
 constexpr int kMaxDevices = 64;
-static void *g_static_ptr[kMaxDevices] = {}, *g_static_arrive[kMaxDevices] = {};
+static void *g_static_ptr[kMaxDevices] = {};
 static std::mutex g_static_mu;
-static int static_scratch(void **out, int **arrive) {
+static int static_scratch(void **out) {
     int dev = 0;
     MYNN_HIP(hipGetDevice(&dev));
     MYNN_REQUIRE(dev >= 0 && dev < kMaxDevices, MYNN_ERR_UNSUPPORTED, "attention_noalloc: device %d", dev);
@@ -513,11 +493,9 @@ static int static_scratch(void **out, int **arrive) {
         void *ptr = nullptr;
         MYNN_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
         MYNN_REQUIRE(ptr, MYNN_ERR_STATE, "attention_noalloc: the scratch array has no device address");
-        MYNN_HIP(hipGetSymbolAddress(&g_static_arrive[dev], HIP_SYMBOL(scratch_arrive)));
         g_static_ptr[dev] = ptr;
     }
     *out = g_static_ptr[dev];
-    *arrive = (int *)g_static_arrive[dev];
     return 0;
 }
 
@@ -551,6 +529,7 @@ static int attention_entry(void *out, const void *Q, const void *K, const void *
               &p.heads_per_wg);
     MYNN_REQUIRE(p.nsplit <= 65535, MYNN_ERR_UNSUPPORTED, "attention: cache of %d rows needs too many slices", kv_len);
     void *scr = nullptr;
+    StreamBlocks::Lease lease;
     if (p.nsplit > 1) {
         const size_t need = attn_scratch_bytes(B, num_q_heads, Sq, head_dim, p.nsplit);
         if (ws_mode == WS_CALLER) {
@@ -561,17 +540,15 @@ static int attention_entry(void *out, const void *Q, const void *K, const void *
             MYNN_REQUIRE(need <= kStaticScratchBytes, MYNN_ERR_UNSUPPORTED,
                          "attention_noalloc: this shape needs %zu bytes of partial results, the library's fixed array holds %zu", need,
                          kStaticScratchBytes);
-            int rc = static_scratch(&scr, &p.arrive);
+            int rc = static_scratch(&scr);
             if (rc) return rc;
         } else {
-            std::lock_guard<std::mutex> lk(g_scratch_mu);
-            Grown &g = g_scratch[st];
-            const size_t had = g.bytes;
-            int rc = ensure(g, need + kAttnArrive * 4, false, st);
+            int rc = g_scratch.lease(st, kArriveBytes + need, kArriveBytes, "attention", &lease);
             if (rc) return rc;
-            if (g.bytes != had) MYNN_HIP(hipMemsetAsync(g.ptr, 0, kAttnArrive * 4, st));  // the counters in front
-            p.arrive = (int *)g.ptr;
-            scr = (char *)g.ptr + kAttnArrive * 4;
+            // (a graph's launches may meet others on the counters, whatever the caller was told, and a counter that is left
+            // above zero spoils every later call; so it merges by a second launch, as the fixed array's calls do)
+            if (!stream_capturing(st)) p.arrive = (int *)lease.ptr;
+            scr = lease.ptr + kArriveBytes;
         }
     }
     return attention_decode_launch(p, head_dim, dtype, kv_int8, scr, st);
@@ -793,8 +770,7 @@ static RingCarve ring_carve(int B, int Sq, int Hq, int Hkv, int D, int dtype, in
     c.total = off;
     return c;
 }
-static std::mutex g_ring_mu;
-static std::map<hipStream_t, Grown> g_ring;  // mynn_attention_streaming: one block per stream
+static StreamBlocks g_ring;  // mynn_attention_streaming
 }  // namespace mynn
 
 extern "C" size_t mynn_attention_streaming_workspace_bytes(int B, int Sq, int cache_seq_len, int num_q_heads, int num_kv_heads,
@@ -909,15 +885,10 @@ extern "C" int mynn_attention_streaming(void *out, const void *Q, const void *K,
     // the library's block of this stream, sized once for the whole cache (it then never grows for this shape)
     const size_t need = ring_carve(B, Sq, num_q_heads, num_kv_heads, head_dim, dtype, kv_int8, rope_on, cache_seq_len).total;
     hipStream_t st = as_stream(s);
-    void *ws = nullptr;
-    {
-        std::lock_guard<std::mutex> lk(g_ring_mu);
-        Grown &g = g_ring[st];
-        int rc = ensure(g, need, false, st);
-        if (rc) return rc;
-        ws = g.ptr;
-    }
+    StreamBlocks::Lease ws;
+    int rc = g_ring.lease(st, need, 0, "attention_streaming", &ws);
+    if (rc) return rc;
     return mynn_attention_streaming_ws(out, Q, K, V, k_scale, v_scale, scale, is_causal, B, Sq, active_seq_kv, cache_seq_len, q_pos_offset,
                                        num_q_heads, num_kv_heads, head_dim, dtype, kv_int8, ring_sink, ring_window, ring_start, cos_t,
-                                       sin_t, kv_position, ws, need, s);
+                                       sin_t, kv_position, ws.ptr, need, s);
 }

@@ -29,6 +29,11 @@ def linear(g, rng, M, N, K, dt=orc.F16, aligned=True):
     return act, W, g.to_dev(orc.to_storage(rng.uniform(1e-3, 1e-2, N), dt), dt)
 
 
+def attention(g, rng, B, L, dt=orc.F16):
+    D, Hq, Hkv = 64, 32, 4
+    return [g.to_dev(orc.to_storage(rng.standard_normal(s), dt), dt) for s in ((B, Hq, 1, D), (B, Hkv, L, D), (B, Hkv, L, D))]
+
+
 def calls(g, rng):
     """(name, a small call whose graph is kept, a call that needs a larger block)"""
     m = g.mynn
@@ -39,6 +44,9 @@ def calls(g, rng):
     q = [g.to_dev(rng.integers(-127, 128, sh).astype(np.int8)) for sh in ((40, 8192), (256, 8192), (200, 8192), (4096, 8192))]
     sc = [g.to_dev(orc.to_storage(rng.uniform(1e-3, 1e-2, n), orc.F16), orc.F16) for n in (40, 256, 200, 4096)]
     yield "K ranges of int8", lambda: m.quantized_matmul(q[0], sc[0], q[1], sc[1])[0], lambda: m.quantized_matmul(q[2], sc[2], q[3], sc[3])[0]
+    a, c = attention(g, rng, 1, 2304), attention(g, rng, 8, 4096)
+    yield "key ranges", lambda: m.attention(*a, 0.125), lambda: m.attention(*c, 0.125)
+    yield "ring rows", lambda: m.attention_streaming(*a, 0.125, False, 2304, 4, 2300, 7), lambda: m.attention_streaming(*c, 0.125, False, 4004, 4, 4000, 7)
 
 
 def test_growth_between_capture_and_replay(g):
