@@ -45,8 +45,10 @@ template <int D, int QW, int KW> constexpr size_t pf_lds() {
 // KV8: an int8 cache with a scale per row.  The codes enter both products exactly; a key's scale multiplies its score, its
 // value's scale its weight.  (fp16: in units of the largest scale so far, times 2^12, so that small weights stay normal
 // numbers and none overflows; a larger scale rescales O^T as a larger maximum does, and the unit is put back at the end.)
-// The weights enter as two values of T each, rounded and rest: the row-at-a-time kernel, which also takes these calls,
-// keeps them in f32.
+// The weights enter as several values of T each, rounded and rest: the row-at-a-time kernel, which also takes these calls,
+// keeps them in f32.  Two of fp16 (22 bits: as near to the result in 64 bits as f32 is), three of bf16: with two, 0.2 % of the
+// outputs were not the nearest bf16 value where f32 weights leave 0.01 - 0.03 % (32 heads, 128 rows behind 500 keys: two values
+// 22.3 us, three 24.3 at D = 128, 13.9 and 15.4 at D = 64; one prompt of 128 rows 9.2 and 9.5).
 template <typename T, int D, bool PAGED, bool KV8, int QW, int KW>
 __global__ __launch_bounds__(QW *KW * 64, 2) void attn_prefill_kernel(AttnParams p) {
     constexpr int kPfThreads = QW * 64, kPfRows = QW * 32;  // threads of a group, query rows of the workgroup
@@ -293,20 +295,28 @@ __global__ __launch_bounds__(QW *KW * 64, 2) void attn_prefill_kernel(AttnParams
             const int e0 = 8 * (st & 1);
             const U4 pf = U4{pack2<T>(ph[e0 + 0], ph[e0 + 1]), pack2<T>(ph[e0 + 2], ph[e0 + 3]),
                              pack2<T>(ph[e0 + 4], ph[e0 + 5]), pack2<T>(ph[e0 + 6], ph[e0 + 7])};
-            U4 rest;  // KV8: what the rounding of the weights to T left out
+            constexpr int RESTS = !KV8 ? 0 : std::is_same<T, f16_t>::value ? 1 : 2;
+            U4 rest[RESTS + 1];  // KV8: what the rounding of the weights to T left out, and what its rounding left out
             if constexpr (KV8) {
-                float w[8];
-                widen8<T>(pf, w);
+                float w[8], have[8];
 #pragma unroll
-                for (int e = 0; e < 8; e++) w[e] = ph[e0 + e] - w[e];
-                rest = U4{pack2<T>(w[0], w[1]), pack2<T>(w[2], w[3]), pack2<T>(w[4], w[5]), pack2<T>(w[6], w[7])};
+                for (int e = 0; e < 8; e++) w[e] = ph[e0 + e];
+                rest[0] = pf;
+#pragma unroll
+                for (int r = 1; r <= RESTS; r++) {
+                    widen8<T>(rest[r - 1], have);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) w[e] -= have[e];
+                    rest[r] = U4{pack2<T>(w[0], w[1]), pack2<T>(w[2], w[3]), pack2<T>(w[4], w[5]), pack2<T>(w[6], w[7])};
+                }
             }
 #pragma unroll
             for (int t2 = 0; t2 < DT; t2++) {
                 const uint16_t *vr = &Vt[buf][(32 * t2 + col) * LDV + 16 * st + 4 * g];
                 const uint2 lo = *(const uint2 *)vr, hi = *(const uint2 *)(vr + 8);
                 o[t2] = Mfma<T>::run(U4{lo.x, lo.y, hi.x, hi.y}, pf, o[t2]);
-                if constexpr (KV8) o[t2] = Mfma<T>::run(U4{lo.x, lo.y, hi.x, hi.y}, rest, o[t2]);
+#pragma unroll
+                for (int r = 1; r <= RESTS; r++) o[t2] = Mfma<T>::run(U4{lo.x, lo.y, hi.x, hi.y}, rest[r], o[t2]);
             }
         }
     };
