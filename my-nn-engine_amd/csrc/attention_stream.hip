@@ -16,7 +16,7 @@
 //            an MFMA tile are dims 32c + 2r (+1),
 // then waves are combined through LDS, and key ranges by the workgroup of a (sequence, kv head) that arrives last
 // (or by a second launch, attn_merge_kernel, where the caller's scratch memory has no arrival counters).
-// P enters the second product as a sum of two storage-type values.  Replaces the reference's attention_decode (attention.cuh:495-606) for these shapes.
+// P enters the second product as a sum of storage-type values (two of fp16, three of bf16).  Replaces the reference's attention_decode (attention.cuh:495-606) for these shapes.
 #include <type_traits>
 
 #include "attention.h"
@@ -76,14 +76,19 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
     constexpr int PST = kStreamTile + 8;    // p tile row stride in elements (16-byte aligned rows)
     __shared__ __align__(16) uint16_t v_s[kStreamWaves][kStreamTile * VST];
     // the storage type keeps 8 (bf16) or 11 (fp16) bits of p, and over thousands of keys that rounding shows
-    // in small outputs: a second tile holds the remainder p - T(p) and feeds a second product
-    constexpr bool kSplitP = true;
+    // in small outputs: further tiles hold the remainder p - T(p), and what its rounding leaves out, and feed products of
+    // their own.  Two values of fp16 measure as f32 weights do against 64 bits; with two of bf16 0.15 - 0.3 % of the outputs
+    // were not the nearest value, with f32 weights or three values 0 - 0.05 % (it costs 0.3 us a launch at 8 sequences x
+    // 500 keys: the 22-layer bf16 step 816 -> 824 us)
+    constexpr int PARTS = std::is_same<T, f16_t>::value ? 2 : 3;
     // fp16 has the bits but not the range: p of a far-away key is subnormal or zero in fp16 while
     // thousands of them still add up, so p is stored times 2^12 and the factor taken out at the end
     constexpr float kPScale = std::is_same<T, f16_t>::value ? 4096.f : 1.f;
-    __shared__ __align__(16) uint16_t p_s[kStreamWaves][(kSplitP ? 2 : 1) * 16 * PST];
+    __shared__ __align__(16) uint16_t p_s[kStreamWaves][PARTS * 16 * PST];
     __shared__ float m_s[kStreamWaves][G], l_s[kStreamWaves][G];
-    __shared__ float o_s[kStreamWaves][G][D];
+    // (a wave's results take the place of its own V tile once it is through)
+    static_assert(G * D * sizeof(float) <= kStreamTile * VST * sizeof(uint16_t), "results of a wave fit its V tile");
+    auto o_s = [&](int w) { return (float(*)[D])v_s[w]; };
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int bhkv = blockIdx.x, split = blockIdx.y;
@@ -318,13 +323,13 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
                 if constexpr (KVI8) pe[e] = t + a * 16 + quad * 4 + e < k1 ? pe[e] * scale_of(sr[2 + a], e) : 0.f;
             }
             // p[head][16a + 4*quad .. +3] in the storage type
-            *(uint2 *)&pt[col * PST + a * 16 + quad * 4] =
-                uint2{pack2<T>(pe[0] * kPScale, pe[1] * kPScale), pack2<T>(pe[2] * kPScale, pe[3] * kPScale)};
-            if constexpr (kSplitP) {
-                float lo[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) lo[e] = pe[e] * kPScale - Elem<T>::rnd(pe[e] * kPScale);
-                *(uint2 *)&pt[16 * PST + col * PST + a * 16 + quad * 4] = uint2{pack2<T>(lo[0], lo[1]), pack2<T>(lo[2], lo[3])};
+            for (int e = 0; e < 4; e++) pe[e] *= kPScale;
+#pragma unroll
+            for (int part = 0; part < PARTS; part++) {
+                *(uint2 *)&pt[part * 16 * PST + col * PST + a * 16 + quad * 4] = uint2{pack2<T>(pe[0], pe[1]), pack2<T>(pe[2], pe[3])};
+#pragma unroll
+                for (int e = 0; e < 4; e++) pe[e] -= Elem<T>::rnd(pe[e]);
             }
         }
         l_run = l_run * alpha + psum;
@@ -336,9 +341,9 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
         }
         __builtin_amdgcn_wave_barrier();
         // ---- O^T += V^T . P: B operand = p[head col][keys 8*quad..+7]; A operands from V dword pairs
-        const U4 pf = *(const U4 *)&pt[col * PST + quad * 8];
-        U4 pl = U4{0u, 0u, 0u, 0u};
-        if constexpr (kSplitP) pl = *(const U4 *)&pt[16 * PST + col * PST + quad * 8];
+        U4 pf[PARTS];
+#pragma unroll
+        for (int part = 0; part < PARTS; part++) pf[part] = *(const U4 *)&pt[part * 16 * PST + col * PST + quad * 8];
 #pragma unroll
         for (int c = 0; c < KB; c++) {
             uint32_t w[8];
@@ -349,11 +354,10 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
             ev.y = __builtin_amdgcn_perm(w[3], w[2], 0x05040100u); od.y = __builtin_amdgcn_perm(w[3], w[2], 0x07060302u);
             ev.z = __builtin_amdgcn_perm(w[5], w[4], 0x05040100u); od.z = __builtin_amdgcn_perm(w[5], w[4], 0x07060302u);
             ev.w = __builtin_amdgcn_perm(w[7], w[6], 0x05040100u); od.w = __builtin_amdgcn_perm(w[7], w[6], 0x07060302u);
-            acc[c][0] = Mfma16<T>::run(ev, pf, acc[c][0]);
-            acc[c][1] = Mfma16<T>::run(od, pf, acc[c][1]);
-            if constexpr (kSplitP) {
-                acc[c][0] = Mfma16<T>::run(ev, pl, acc[c][0]);
-                acc[c][1] = Mfma16<T>::run(od, pl, acc[c][1]);
+#pragma unroll
+            for (int part = 0; part < PARTS; part++) {
+                acc[c][0] = Mfma16<T>::run(ev, pf[part], acc[c][0]);
+                acc[c][1] = Mfma16<T>::run(od, pf[part], acc[c][1]);
             }
         }
         __builtin_amdgcn_wave_barrier();
@@ -433,7 +437,7 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
 #pragma unroll
             for (int par = 0; par < 2; par++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) o_s[wave][col][c * 32 + 2 * (4 * quad + e) + par] = acc[c][par][e] * (1.0f / kPScale);
+                for (int e = 0; e < 4; e++) o_s(wave)[col][c * 32 + 2 * (4 * quad + e) + par] = acc[c][par][e] * (1.0f / kPScale);
     }
     __syncthreads();
 
@@ -449,8 +453,8 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
         for (int w = 0; w < kStreamWaves; w++) {
             const float c = m_s[w][g] == -INFINITY ? 0.f : fast_exp(m_s[w][g] - mt);
             lt = fmaf(l_s[w][g], c, lt);
-            o0 = fmaf(o_s[w][g][d], c, o0);
-            o1 = fmaf(o_s[w][g][d + 1], c, o1);
+            o0 = fmaf(o_s(w)[g][d], c, o0);
+            o1 = fmaf(o_s(w)[g][d + 1], c, o1);
         }
         const size_t row = (size_t)(b * p.Hq + head0 + g), at = (size_t)b * p.o_bs + (size_t)(head0 + g) * p.o_hs + d;
         if (n_act == 1) {

@@ -75,3 +75,35 @@ def test_prefill_over_an_int8_cache(g, dt, D):
     got = g.to_host(g.mynn.attention(g.to_dev(q, dt), g.to_dev(kq), g.to_dev(vq), D ** -0.5, True, L, q_pos_offset=L - S,
                                      k_scale=g.to_dev(ks, dt), v_scale=g.to_dev(vs, dt)))
     assert share_off(got, exact(orc.to_f32(q, dt).astype(np.float64), k, v, True), dt) <= share_allowed(dt)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("kv8", [False, True], ids=["kv16", "kv_int8"])
+@pytest.mark.parametrize("D,Hkv", [(64, 4), (128, 8)])
+def test_streaming_decode(g, dt, kv8, D, Hkv):
+    """the kernel of batched decode steps, through its paged form (which takes it at every size)"""
+    import torch
+
+    rng = np.random.default_rng(D + kv8)
+    B, Hq, L, P = 8, 32, 300, 64
+    n = (L + P - 1) // P
+    off = []
+    for _ in range(3):
+        q = orc.to_storage(rng.standard_normal((B, Hq, 1, D)), dt)
+        sc = [None, None]
+        if kv8:
+            (kq, sc[0], k), (vq, sc[1], v) = quantised(rng, (B, Hkv, n * P, D), dt), quantised(rng, (B, Hkv, n * P, D), dt)
+        else:
+            kq, vq = (orc.to_storage(rng.standard_normal((B, Hkv, n * P, D)), dt) for _ in range(2))
+            k, v = (orc.to_f32(x, dt).astype(np.float64) for x in (kq, vq))
+
+        def pool(x):  # pages of a sequence in a row
+            x = x.reshape(B, Hkv, n, P, *x.shape[3:])
+            return g.to_dev(np.ascontiguousarray(x.swapaxes(1, 2)).reshape(B * n, Hkv, P, *x.shape[4:]), dt)
+
+        table = torch.arange(B * n, dtype=torch.int32, device="cuda").view(B, n)
+        got = g.mynn.attention_paged(g.to_dev(q, dt), pool(kq), pool(vq), table, P, D ** -0.5, False, L, q_pos_offset=L - 1,
+                                     k_scale_pool=pool(sc[0]) if kv8 else None, v_scale_pool=pool(sc[1]) if kv8 else None)
+        off.append(share_off(g.to_host(got), exact(orc.to_f32(q, dt).astype(np.float64), k[:, :, :L], v[:, :, :L], False), dt))
+    assert np.mean(off) <= share_allowed(dt), off
