@@ -48,7 +48,7 @@ template <int D, int QW, int KW> constexpr size_t pf_lds() {
 // The weights enter as several values of T each, rounded and rest: the row-at-a-time kernel, which also takes these calls,
 // keeps them in f32.  Two of fp16 (22 bits: as near to the result in 64 bits as f32 is), three of bf16: with two, 0.2 % of the
 // outputs were not the nearest bf16 value where f32 weights leave 0.01 - 0.03 % (32 heads, 128 rows behind 500 keys: two values
-// 22.3 us, three 24.3 at D = 128, 13.9 and 15.4 at D = 64; one prompt of 128 rows 9.2 and 9.5).
+// 22.3 us, three 23.5 at D = 128, 13.9 and 14.3 at D = 64; one prompt of 128 rows 9.2 and 9.4).
 template <typename T, int D, bool PAGED, bool KV8, int QW, int KW>
 __global__ __launch_bounds__(QW *KW * 64, 2) void attn_prefill_kernel(AttnParams p) {
     constexpr int kPfThreads = QW * 64, kPfRows = QW * 32;  // threads of a group, query rows of the workgroup
@@ -293,30 +293,28 @@ __global__ __launch_bounds__(QW *KW * 64, 2) void attn_prefill_kernel(AttnParams
         for (int st = 0; st < 4; st++) {
             const f16x_t &ph = s[st >> 1];
             const int e0 = 8 * (st & 1);
-            const U4 pf = U4{pack2<T>(ph[e0 + 0], ph[e0 + 1]), pack2<T>(ph[e0 + 2], ph[e0 + 3]),
-                             pack2<T>(ph[e0 + 4], ph[e0 + 5]), pack2<T>(ph[e0 + 6], ph[e0 + 7])};
-            constexpr int RESTS = !KV8 ? 0 : std::is_same<T, f16_t>::value ? 1 : 2;
-            U4 rest[RESTS + 1];  // KV8: what the rounding of the weights to T left out, and what its rounding left out
+            constexpr int PARTS = KV8 ? kParts<T> : 1;
+            U4 pf[PARTS];
             if constexpr (KV8) {
-                float w[8], have[8];
+                float w[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) w[e] = ph[e0 + e];
-                rest[0] = pf;
 #pragma unroll
-                for (int r = 1; r <= RESTS; r++) {
-                    widen8<T>(rest[r - 1], have);
-#pragma unroll
-                    for (int e = 0; e < 8; e++) w[e] -= have[e];
-                    rest[r] = U4{pack2<T>(w[0], w[1]), pack2<T>(w[2], w[3]), pack2<T>(w[4], w[5]), pack2<T>(w[6], w[7])};
+                for (int part = 0; part < PARTS; part++) {
+                    pf[part].x = take_part<T>(w[0], w[1]);
+                    pf[part].y = take_part<T>(w[2], w[3]);
+                    pf[part].z = take_part<T>(w[4], w[5]);
+                    pf[part].w = take_part<T>(w[6], w[7]);
                 }
-            }
+            } else
+                pf[0] = U4{pack2<T>(ph[e0 + 0], ph[e0 + 1]), pack2<T>(ph[e0 + 2], ph[e0 + 3]),
+                           pack2<T>(ph[e0 + 4], ph[e0 + 5]), pack2<T>(ph[e0 + 6], ph[e0 + 7])};
 #pragma unroll
             for (int t2 = 0; t2 < DT; t2++) {
                 const uint16_t *vr = &Vt[buf][(32 * t2 + col) * LDV + 16 * st + 4 * g];
                 const uint2 lo = *(const uint2 *)vr, hi = *(const uint2 *)(vr + 8);
-                o[t2] = Mfma<T>::run(U4{lo.x, lo.y, hi.x, hi.y}, pf, o[t2]);
 #pragma unroll
-                for (int r = 1; r <= RESTS; r++) o[t2] = Mfma<T>::run(U4{lo.x, lo.y, hi.x, hi.y}, rest[r], o[t2]);
+                for (int part = 0; part < PARTS; part++) o[t2] = Mfma<T>::run(U4{lo.x, lo.y, hi.x, hi.y}, pf[part], o[t2]);
             }
         }
     };

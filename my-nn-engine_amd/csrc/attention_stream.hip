@@ -78,9 +78,9 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
     // the storage type keeps 8 (bf16) or 11 (fp16) bits of p, and over thousands of keys that rounding shows
     // in small outputs: further tiles hold the remainder p - T(p), and what its rounding leaves out, and feed products of
     // their own.  Two values of fp16 measure as f32 weights do against 64 bits; with two of bf16 0.15 - 0.3 % of the outputs
-    // were not the nearest value, with f32 weights or three values 0 - 0.05 % (it costs 0.3 us a launch at 8 sequences x
-    // 500 keys: the 22-layer bf16 step 816 -> 824 us)
-    constexpr int PARTS = std::is_same<T, f16_t>::value ? 2 : 3;
+    // were not the nearest value, with f32 weights or three values 0 - 0.05 % (at no cost: 32 sequences x 2048 keys, D = 128,
+    // 55.7 us with either, over an int8 cache 30.4 with two and 30.3 - 30.8 with three)
+    constexpr int PARTS = kParts<T>;
     // fp16 has the bits but not the range: p of a far-away key is subnormal or zero in fp16 while
     // thousands of them still add up, so p is stored times 2^12 and the factor taken out at the end
     constexpr float kPScale = std::is_same<T, f16_t>::value ? 4096.f : 1.f;
@@ -327,9 +327,8 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
             for (int e = 0; e < 4; e++) pe[e] *= kPScale;
 #pragma unroll
             for (int part = 0; part < PARTS; part++) {
-                *(uint2 *)&pt[part * 16 * PST + col * PST + a * 16 + quad * 4] = uint2{pack2<T>(pe[0], pe[1]), pack2<T>(pe[2], pe[3])};
-#pragma unroll
-                for (int e = 0; e < 4; e++) pe[e] -= Elem<T>::rnd(pe[e]);
+                const uint32_t w0 = take_part<T>(pe[0], pe[1]), w1 = take_part<T>(pe[2], pe[3]);
+                *(uint2 *)&pt[part * 16 * PST + col * PST + a * 16 + quad * 4] = uint2{w0, w1};
             }
         }
         l_run = l_run * alpha + psum;

@@ -41,6 +41,25 @@ template <> __device__ inline uint32_t pack2<bf16_t>(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){lo, hi}, bf2_t));
 }
 
+// A weight held in f32 as kParts<T> values of T whose sum it is: for operands that must not lose bits.  take_part packs the
+// next part of two weights (low half first) and takes it off them.  fp16: rounded, two parts hold 22 bits; bf16: the upper
+// half of the f32 number as it is, three parts are all 24 bits exactly (and the conversion is one v_perm).
+template <typename T> constexpr int kParts = std::is_same<T, f16_t>::value ? 2 : 3;
+template <typename T> __device__ inline uint32_t take_part(float &a, float &b) {
+    if constexpr (std::is_same<T, f16_t>::value) {
+        const uint32_t w = pack2<T>(a, b);
+        const h2_t h = __builtin_bit_cast(h2_t, w);
+        a -= (float)h[0];
+        b -= (float)h[1];
+        return w;
+    } else {
+        const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+        a -= __builtin_bit_cast(float, ua & 0xFFFF0000u);
+        b -= __builtin_bit_cast(float, ub & 0xFFFF0000u);
+        return __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+    }
+}
+
 // 8 int8 (two dwords) -> 8 values of T packed in a U4; exact
 template <typename T> __device__ inline U4 i8x8_to_operand(uint32_t w0, uint32_t w1) {
     if constexpr (std::is_same<T, f16_t>::value) {
