@@ -209,6 +209,10 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
     // running state of head `col`: maximum, partial sum (the 4 quads hold parts), O^T accumulators
     // acc[c][par][e] = dim 32c + 2*(4*quad + e) + par
     float m_run = -INFINITY, l_run = 0.f;
+    // UNITS: the scale of a value multiplies its key's weight, so with scales of 16 and more (values beyond 2000) the weights
+    // would pass fp16's largest number: they and the accumulators are then kept divided by a power of two, one for the wave
+    constexpr bool UNITS = KVI8 && std::is_same<T, f16_t>::value;
+    float unit = 1.f, to_unit = kPScale;  // kPScale / unit
     f4_t acc[KB][2];
 #pragma unroll
     for (int c = 0; c < KB; c++)
@@ -310,9 +314,26 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
         tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
         const float m_new = fmaxf(m_run, tmax);  // finite: the tile has at least one key in range
-        const float alpha = fast_exp(m_run - m_new);
+        float alpha = fast_exp(m_run - m_new), back = 1.f;
         m_run = m_new;
         float psum = 0.f;
+        if constexpr (UNITS) {
+            float vm = 0.f;
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) vm = fmaxf(vm, t + a * 16 + quad * 4 + e < k1 ? fabsf(scale_of(sr[2 + a], e)) : 0.f);
+            if (__builtin_amdgcn_ballot_w64(vm > 8.f * unit) != 0) {
+                vm = fmaxf(vm, __shfl_xor(vm, 16, 64));
+                vm = fmaxf(vm, __shfl_xor(vm, 32, 64));
+                // (its power of two; scales of fp16 end at 2^16)
+                const float un = fmaxf(unit, __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, fminf(vm, 65536.f)) & 0x7F800000u));
+                const float inv = __builtin_bit_cast(float, 0x7F000000u - __builtin_bit_cast(uint32_t, un));
+                back = unit * inv;
+                unit = un;
+                to_unit = kPScale * inv;
+            }
+        }
 #pragma unroll
         for (int a = 0; a < 2; a++) {
             float pe[4];
@@ -324,7 +345,7 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
             }
             // p[head][16a + 4*quad .. +3] in the storage type
 #pragma unroll
-            for (int e = 0; e < 4; e++) pe[e] *= kPScale;
+            for (int e = 0; e < 4; e++) pe[e] *= UNITS ? to_unit : kPScale;
 #pragma unroll
             for (int part = 0; part < PARTS; part++) {
                 const uint32_t w0 = take_part<T>(pe[0], pe[1]), w1 = take_part<T>(pe[2], pe[3]);
@@ -332,6 +353,7 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
             }
         }
         l_run = l_run * alpha + psum;
+        alpha *= back;
         if (alpha != 1.f) {
 #pragma unroll
             for (int c = 0; c < KB; c++)
@@ -436,7 +458,7 @@ __global__ __launch_bounds__(kStreamThreads) void attn_stream_kernel(StreamParam
 #pragma unroll
             for (int par = 0; par < 2; par++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) o_s(wave)[col][c * 32 + 2 * (4 * quad + e) + par] = acc[c][par][e] * (1.0f / kPScale);
+                for (int e = 0; e < 4; e++) o_s(wave)[col][c * 32 + 2 * (4 * quad + e) + par] = acc[c][par][e] * (UNITS ? unit * (1.0f / kPScale) : 1.0f / kPScale);
     }
     __syncthreads();
 

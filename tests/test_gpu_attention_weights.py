@@ -32,9 +32,11 @@ def share_off(got, want, dt):
     return np.mean(got != orc.to_storage(want.astype(np.float32), dt))
 
 
-def quantised(rng, shape, dt):
+def quantised(rng, shape, dt, size=1.0):
+    """codes, row scales and values; size: of the largest rows (others are up to 2^6 smaller where it is not 1)"""
     codes = np.clip(np.round(rng.standard_normal(shape) * 45), -127, 127).astype(np.int8)
-    scale = orc.to_storage(rng.uniform(0.018, 0.026, shape[:-1]), dt)
+    scale = rng.uniform(0.018, 0.026, shape[:-1]) * size * np.exp2(-rng.integers(0, 7, shape[:-1]) * (size != 1.0))
+    scale = orc.to_storage(scale, dt)
     return codes, scale, codes * orc.to_f32(scale, dt).astype(np.float64)[..., None]
 
 
@@ -79,10 +81,11 @@ def test_prefill_over_an_int8_cache(g, dt, D):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
-@pytest.mark.parametrize("kv8", [False, True], ids=["kv16", "kv_int8"])
+@pytest.mark.parametrize("kv8,size", [(False, 1.0), (True, 1.0), (True, 1.5e4), (True, 1e-3)], ids=["kv16", "kv_int8", "kv_int8_large", "kv_int8_small"])
 @pytest.mark.parametrize("D,Hkv", [(64, 4), (128, 8)])
-def test_streaming_decode(g, dt, kv8, D, Hkv):
-    """the kernel of batched decode steps, through its paged form (which takes it at every size)"""
+def test_streaming_decode(g, dt, kv8, size, D, Hkv):
+    """the kernel of batched decode steps, through its paged form (which takes it at every size); values at both ends of
+    fp16 (a value's scale multiplies its key's weight)"""
     import torch
 
     rng = np.random.default_rng(D + kv8)
@@ -93,7 +96,7 @@ def test_streaming_decode(g, dt, kv8, D, Hkv):
         q = orc.to_storage(rng.standard_normal((B, Hq, 1, D)), dt)
         sc = [None, None]
         if kv8:
-            (kq, sc[0], k), (vq, sc[1], v) = quantised(rng, (B, Hkv, n * P, D), dt), quantised(rng, (B, Hkv, n * P, D), dt)
+            (kq, sc[0], k), (vq, sc[1], v) = quantised(rng, (B, Hkv, n * P, D), dt), quantised(rng, (B, Hkv, n * P, D), dt, size)
         else:
             kq, vq = (orc.to_storage(rng.standard_normal((B, Hkv, n * P, D)), dt) for _ in range(2))
             k, v = (orc.to_f32(x, dt).astype(np.float64) for x in (kq, vq))
