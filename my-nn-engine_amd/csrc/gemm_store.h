@@ -27,7 +27,7 @@ __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const 
     const int ldc = HALF ? N >> 1 : N;
     const int c0 = HALF ? (n0 + wcol) >> 1 : n0 + wcol;
     T *patch = (T *)lds + (size_t)wave * 32 * EST;
-    const bool vec_ok = (ldc & 7) == 0;
+    const bool vec_ok = (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && (EPI != GEMM_RESIDUAL || ((uintptr_t)R & 15) == 0);  // (uniform)
 #pragma unroll
     for (int i = 0; i < TI; i++) {
         T *prow = patch + (lane & 31) * EST + (lane >> 5) * (EPI == GEMM_SWIGLU_PAIRS ? 2 : 4);

@@ -99,8 +99,9 @@ extern "C" int mynn_quantized_matmul(void *out, int32_t *acc_out, const int8_t *
     // int32 accumulators hold the exact sum as long as K * 128 * 128 < 2^31
     MYNN_REQUIRE(K <= 131071, MYNN_ERR_UNSUPPORTED, "quantized_matmul: K=%d could overflow the int32 accumulator", K);
     // matrix cores from three rows on (two rows of 4096 x 4096: 6.2 us as dot products, 8.1 as tiles; three: 10 and 8),
-    // with the 256-row tiles of gemm.hip where enough of them make that the faster one
-    if (M >= 3 && (!out || aligned16(out))) {
+    // with the 256-row tiles of gemm.hip where enough of them make that the faster one; the output may lie anywhere (their
+    // store writes element by element where it is not 16-byte aligned)
+    if (M >= 3) {
         const TgPlan plan = tile_gemm_plan(TG_I8, dtype, M, N, K, kTgScratchMax);
         if (dtype != MYNN_F32 && qgemm_dma_us(M, N, K) < plan.us)
             return qgemm_dma(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, as_stream(s));

@@ -562,7 +562,6 @@ int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const v
     MYNN_REQUIRE((out || acc_out) && act && wq && (w_scale || !out) && (kind != TG_I8 || a_scale || !out), MYNN_ERR_INVALID, "tile_gemm: null operand");
     MYNN_REQUIRE(tile_gemm_supported(kind, M, N, K), MYNN_ERR_UNSUPPORTED, "tile_gemm: M=%d N=%d K=%d", M, N, K);
     MYNN_REQUIRE(aligned16(act) && aligned16(wq), MYNN_ERR_INVALID, "tile_gemm: operands must be 16-byte aligned");
-    MYNN_REQUIRE(!out || (aligned16(out) && (!res || aligned16(res))), MYNN_ERR_INVALID, "tile_gemm: output and residual must be 16-byte aligned");
     MYNN_REQUIRE(epi != GEMM_RESIDUAL || res, MYNN_ERR_INVALID, "tile_gemm: residual store without a residual");
     MYNN_REQUIRE(epi != GEMM_SWIGLU_PAIRS || (N % 2 == 0 && !acc_out), MYNN_ERR_INVALID, "tile_gemm: SwiGLU store needs row pairs, N=%d", N);
     MYNN_REQUIRE(epi != GEMM_SWIGLU && (kind != TG_W8S || epi == GEMM_PLAIN), MYNN_ERR_INVALID, "tile_gemm: store %d", epi);
