@@ -186,7 +186,7 @@ def check(rc):
 
 # ------------------------------------------------------------------ torch plumbing
 # The host path of an operator call is most of the time of a small one (a 5632 x 2048 GEMV takes 3.9 us on the device):
-# the current stream is asked for as a raw handle (0.1 us; torch.cuda.current_stream() builds a Stream
+# the current stream is asked for as a raw handle where torch has that (0.1 us; torch.cuda.current_stream() builds a Stream
 # object, 2.7 us), outputs come from new_empty of the tensor whose device they share (1.1 us; torch.empty with a device 1.5),
 # type codes from one table.
 _torch = None
@@ -213,7 +213,10 @@ def _dt(t):
 
 def _stream():
     torch = _t()
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:  # (not part of torch's public interface)
+        return torch.cuda.current_stream().cuda_stream
 
 
 def _ptr(t):

@@ -1,5 +1,6 @@
-"""The Python side of an operator call: where its outputs live."""
+"""The Python side of an operator call: where its outputs live, and the stream it asks torch for."""
 import importlib
+import types
 
 import pytest
 
@@ -29,3 +30,8 @@ def test_outputs_live_with_the_operand_they_are_made_from(calls):
     out, acc = calls.quantized_matmul(wq, scale, torch.empty((5, 32), dtype=torch.int8), torch.empty(5, dtype=torch.bfloat16))
     assert out.device.type == acc.device.type == "meta" and (out.dtype, acc.dtype) == (torch.bfloat16, torch.int32)
 
+
+def test_stream_without_the_raw_handle(monkeypatch):
+    public = types.SimpleNamespace(_C=types.SimpleNamespace(), cuda=types.SimpleNamespace(current_stream=lambda: types.SimpleNamespace(cuda_stream=41)))
+    monkeypatch.setattr(mynn, "_t", lambda: public)
+    assert mynn._stream() == 41
