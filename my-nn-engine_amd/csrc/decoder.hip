@@ -342,8 +342,15 @@ static int linear_w8a8(Model &m, void *out, const void *act, const Lin &l, int M
         TRY(mynn_dynamic_quantize_linear(m.a8, m.a8_scale, nullptr, act, M, l.K, m.cfg.dtype, 1, m.stream));
     }
     note(m, name, (double)l.N * l.K + (double)M * l.K + l.N * eb + (double)M * l.N * eb, 2.0 * M * l.N * l.K);
-    return mynn_quantized_matmul(out, nullptr, m.a8, m.a8_scale, (const int8_t *)l.w, l.scale, M, l.N, l.K, m.cfg.dtype,
-                                 m.stream);
+    if (M >= 3 && m.cfg.dtype != MYNN_F32 && !qgemm_dma_supported(M, l.N, l.K)) {
+        // (the operator would split K with the library's scratch memory: an executor uses none but its own)
+        const TgPlan one = tile_gemm_plan(TG_I8, m.cfg.dtype, M, l.N, l.K, 0);
+        return tile_gemm(TG_I8, one, out, nullptr, m.a8, (const int8_t *)l.w, m.a8_scale, l.scale, nullptr, M, l.N, l.K, m.cfg.dtype, GEMM_PLAIN,
+                         nullptr, nullptr, m.stream);
+    }
+    if (M >= 3 && m.cfg.dtype != MYNN_F32)
+        return qgemm_dma(out, nullptr, m.a8, m.a8_scale, (const int8_t *)l.w, l.scale, nullptr, M, l.N, l.K, m.cfg.dtype, GEMM_PLAIN, m.stream);
+    return mynn_quantized_matmul(out, nullptr, m.a8, m.a8_scale, (const int8_t *)l.w, l.scale, M, l.N, l.K, m.cfg.dtype, m.stream);
 }
 
 // W8A8 on the matrix cores: (RMSNorm +) per-row quantisation of the input, then the product with the

@@ -48,3 +48,19 @@ def test_layer_equals_the_operators(g, dt, B, ffn):
     want = linear(m.rms_norm(x3, dw["final_norm"], cfg["eps"]), "lm_head")
     assert np.array_equal(np.asarray(got).reshape(B, -1), g.to_host(want))
     dec.close()
+
+
+@pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("B", [2, 3, 97])
+def test_a_forced_tile_runs_the_operators_with_the_same_bits(g, dt, B):
+    """an executor with a forced GEMM tile keeps one operator per launch (and no scratch memory for K ranges)"""
+    cfg, w = llm_weights.synthetic_int8(dict(SMALL, n_layers=1, hidden=256, ffn=5632, n_heads=4, n_kv_heads=2, head_dim=64, max_seq=4), dt, seed=B)
+    dw = dev_weights(g, w, dt)
+    ids = np.random.default_rng(B).integers(0, cfg["vocab"], B)
+    rows = []
+    for tile in (0, 1):
+        dec = g.mynn.Decoder(cfg, dw, batch=B, quantize_activations=True, gemm_tile=tile)
+        assert ("swiglu" in [k[0] for k in dec.profile(ids, [0], 0, 1)]) == (tile == 1)
+        rows.append(dec.step(ids, [0], 0, 1, want_logits=True)[1])
+        dec.close()
+    assert np.array_equal(*rows)
