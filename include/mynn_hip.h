@@ -88,9 +88,9 @@ int mynn_dequant_gemv(void *out, const void *act, const int8_t *wq, const void *
 int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq, const void *scale,
                         int M, int N, int K, int act_dtype, int out_dtype, mynn_stream s);
 
-/* The same with the caller's scratch memory: for M >= 16 (16-bit operands) the weight is dequantised into
- * `workspace` (mynn_dequant_matmul_workspace_bytes(...) bytes, 16-byte aligned, 0 = none needed) on every
- * call; nothing global is touched, so the call can be captured into a graph and calls on several streams
+/* The same with the caller's scratch memory: for M >= 16 (16-bit operands) `workspace`
+ * (mynn_dequant_matmul_workspace_bytes(...) bytes, 16-byte aligned, 0 = none needed) takes the dequantised weight of a
+ * large product or the partial sums of a small one; nothing global is touched, so the call can be captured into a graph and calls on several streams
  * may overlap when their workspaces differ.  gemm_tile forces the workgroup tile of the matrix-core GEMM:
  * 0 = chosen per shape, 1 = 256x128, 2 = 256x256 with operands staged through registers, 3 = 256x256 and
  * 4 = 256x320 with operands loaded straight into LDS (3 and 4 fall back to 1 when K % 64 != 0, and every forced tile
@@ -110,8 +110,8 @@ int mynn_dequant_weight_prepare(void *wt, const int8_t *wq, const void *scale, i
 int mynn_dequant_matmul_prepared(void *out, const void *act, const void *wt, int M, int N, int K,
                                  int dtype, int gemm_tile, mynn_stream s);
 
-/* Measurement aid, no counterpart in the reference, process-wide: 1 = the few-row (16 <= M <= 32) gate/up GEMM of a
- * batched decode step runs its loads alone (no LDS, no conversion, no MFMA, no barrier), 2 = everything but the MFMAs,
+/* Measurement aid, no counterpart in the reference, process-wide: 1 = the few-row gate/up GEMM (M <= 32, 768 row
+ * blocks of 32 and more) of a batched decode step runs its loads alone (no LDS, no conversion, no MFMA, no barrier), 2 = everything but the MFMAs,
  * 0 = the product kernel.  The ablated launches compute garbage; only their duration means anything
  * (bench.py --workload decode_batch --skinny-ablation). */
 void mynn_skinny_set_ablation(int mode);
@@ -402,7 +402,7 @@ void *mynn_model_create(const mynn_model_config *cfg, void **initializer, void *
  * share the checkpoint's device buffers by name (PersistentBuffers, src/session.rs:284-394) and derive nothing from
  * them.  Here an executor derives copies at init -- q|k|v rows concatenated and gate/up rows interleaved (decode),
  * every weight dequantised once to the 16-bit type (prefill, matrix cores), an int8 copy tiled for streaming
- * (16..64 rows), int8 gate/up interleaved in groups of 32 (quantize_activations prefill) -- and a prefill, a decode
+ * (2..64 rows), int8 gate/up interleaved in groups of 32 (quantize_activations prefill) -- and a prefill, a decode
  * and a batched executor made by mynn_model_create each derive their own.  mynn_weight_set_create makes the holder
  * (cfg: the shapes, dtype, weights_int8 and qkv_bias are what matters; initializer as mynn_model_create), and
  * mynn_model_create_shared builds an executor on it: each kind of copy is made by the first executor that needs it

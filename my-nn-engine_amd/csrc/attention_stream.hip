@@ -2,7 +2,7 @@
 // 16-bit or int8 (per-token scales) K/V, head_dim 64 or 128, up to 8 query heads per kv head.
 //
 // attention_decode.hip is built for latency (one pass, everything in flight at once, one workgroup
-// per CU); with tens of megabytes of K/V per launch the job is bandwidth instead, and this kernel
+// per CU); with megabytes of K/V per launch the job is bandwidth instead, and this kernel
 // keeps the loads streaming: a workgroup of 4 waves walks its key range in tiles of 32 keys per wave,
 // the next tile's K and V already in registers while the current one is used.  Both products run on
 // the matrix cores (v_mfma_f32_16x16x32), with the query heads as the 16 columns (zero beyond G):
@@ -39,9 +39,12 @@ template <> struct Mfma16<bf16_t> {
 };
 
 constexpr int kStreamWaves = 4, kStreamThreads = kStreamWaves * 64, kStreamTile = 32;
-// (sequences x kv heads x keys) from which this kernel is taken instead of the latency kernel of attention_decode.hip:
-// measured cross-over (head_dim 64 and 128, 1 .. 32 sequences): below it that kernel's single launch of 9-11 us wins or
-// ties, above it this one (two launches, 11 us together, one of 9 us once every CU has a pair) is 25-50 % faster
+// (sequences x kv heads x keys) from which the operator takes this kernel instead of the latency kernel of
+// attention_decode.hip.  Latency / streaming, us, 16-bit caches (profiles/attention_routes.md): from 8192 on this one is the
+// faster at every shape measured (D = 64: 16 x 128 keys 6.6 / 6.4, 2 x 1024 12.6 / 7.1, 4 x 2048 20.4 / 9.8; D = 128: 1 x 1024
+// 12.3 / 7.7, 4 x 256 9.3 / 7.8); below it goes either way (4 x 256, D = 64: 6.9 / 7.1; 2 x 256, D = 128: 7.2 / 7.7; but 1 x 1024,
+// D = 64: 10.7 / 6.8).  An executor's fused form, which saves the RoPE + append launch as well, takes this kernel for every
+// batch of two and more whatever the length.
 constexpr long kStreamMinKeys = 8192;
 
 // KVI8: int8 caches with one scale per token row (QuantizingKVCacheUpdate): K and V are widened exactly to

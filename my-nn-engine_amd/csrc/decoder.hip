@@ -174,7 +174,7 @@ struct Model {
     LinPlan pl_qkv, pl_o, pl_gu, pl_down, pl_lm;
     void *tg_part = nullptr;     // tile_gemm's partial sums and arrival counters
     int *tg_counters = nullptr;
-    bool skinny = false;      // 16..64 rows: int8 weights streamed once through the few-row matrix-core kernel
+    bool skinny = false;      // 2..64 rows: int8 weights streamed once through the few-row matrix-core kernels, from a tiled copy
     bool rowblock = false;    // ... one launch per linear (rowblock.hip), with the norm in front up to 16 rows
     float *skinny_scratch = nullptr;
     void *cos_t = nullptr, *sin_t = nullptr;
@@ -305,7 +305,7 @@ static int linear_rows(Model &m, void *out, const void *act, const Lin &l, int M
     return launch_status("dense_linear_kernel");
 }
 
-// one few-row GEMM against int8 weights (two launches: products, then sum/scale/store)
+// one few-row GEMM against int8 weights (products of K ranges, then sum/scale/store; one launch from 768 row blocks on)
 // next_norm (residual store): the weights of the RMSNorm that reads this output next; *normed = m.nrm holds it
 static int skinny_rows(Model &m, void *out, const void *act, const Lin &l, const void *packed, const void *res, int M, int epi,
                        const char *name, const void *next_norm = nullptr, bool *normed = nullptr, const SkinnyRope *rope = nullptr,

@@ -4,13 +4,16 @@
 // scales with M >= 16 take the matrix-core path whose numerics are those of
 // dequant_matmul_wmma.cuh:65-76 -- the weight is dequantised to the 16-bit type WITH the scale
 // folded in (one rounding) and the products are accumulated in f32; everything else takes the
-// scale-after-sum kernels of gemv.hip.
+// scale-after-sum kernels of gemv.hip.  Products of fewer rows than fill the device with 256-row tiles are multiplied from
+// the int8 weights as they are stored (tile_gemm.hip); this file has the large ones, the choice between the two and the
+// entry points.
 //
 // Two steps: (1) W_T[n,k] = T(wq[n,k] * scale[n]) -- a pure streaming pass (~3 bytes moved per
 // weight) into a library-owned workspace per call, or once into a resident copy that a prefill
 // executor keeps; (2) C = A . W_T^T with v_mfma_f32_32x32x16_{f16,bf16}.  Grids of at least one round
 // of 256 x 256 tiles with K % 64 == 0 run gemm_nt_dma_kernel (operand tiles loaded straight into LDS,
-// swizzled, 256 x 256 or 256 x 320 per workgroup of 8 waves); the rest runs gemm_nt_mfma_kernel (256 x 128
+// swizzled, 256 x 256 or 256 x 320 per workgroup of 8 waves); the rest -- prepared weights and operands that
+// tile_gemm does not take -- runs gemm_nt_mfma_kernel (256 x 128
 // or 256 x 256, K step 32, operands staged through registers into padded LDS tiles, any K % 8 == 0).
 // The store can add a residual (o_proj, down_proj) or apply SwiGLU to interleaved gate/up columns.
 // The int8 form of gemm_nt_dma_kernel is QuantizedMatMul for large grids (qgemm_dma).

@@ -18,7 +18,6 @@ int gemv_norm_swiglu(void *out, const void *x, const void *norm_w, float eps, co
 int dequant_gemv_dispatch(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K,
                           int act_dtype, int out_dtype, hipStream_t s);
 
-// gemm.hip -- matrix-core DequantMatMul, M >= 16, 16-bit types
 // skinny.hip -- 2 <= M <= 64 rows against int8 weights streamed once (scale after the sum); `scratch` holds
 // skinny_scratch_bytes(M, N, K) of f32 partial sums; epi is one of GEMM_* (SWIGLU: interleaved gate/up rows)
 bool skinny_gemm_supported(int M, int N, int K);

@@ -406,15 +406,16 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 }
 
 // ---- which tile, and over how many K ranges.
-// The time of a launch, in microseconds, as measured over some 300 shapes (16 <= M <= 4096, the linear layers of the
-// benchmark's models and others; every tile at 1 .. 12 ranges) and fitted per tile:
+// The time of a launch, in microseconds, fitted per tile to measured times of the linear layers of the benchmark's models
+// and others (16 <= M <= 4096, every tile at 1 .. 12 ranges):
 //
 //   t = launch + steps per range * (a * rounds + b * workgroups on the fullest CU) + e * ranges + partial sums at 4 TB/s
 //
 // a: what a step costs a CU however few workgroups it holds (latency); b: what each resident workgroup adds (LDS, MFMA and
 // dequantisation work); rounds: how often a CU takes a new set of workgroups.  Never less than the weights' bytes at 4.6
 // TB/s or the tiles' operations at the rate that long launches reach (0.93 PFLOP/s fp16, 0.88 bf16, 1.85 int8).  Choosing by it
-// is within 2 % of the best choice on average, 27 % at worst.  (Two fits where the conversion of the weights costs differ: it
+// is 2 % above the best tile and number of ranges on average over 432 shapes, 27 % at worst (profiles/tile_gemm_plans.csv has
+// them); without ranges the same shapes would take 1.5 times as long (16-bit, 4 times at worst) and 1.04 times (int8).  (Two fits where the conversion of the weights costs differ: it
 // is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
 struct TgCost {
     int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
