@@ -834,31 +834,43 @@ static int build(Model &m, void **init, void **state) {
         m.rowblock = m.skinny && c.seq_q == 1 && rowblock_supported(rows_, QD + 2 * KD, H, false) && rowblock_supported(rows_, H, QD, false) &&
                      rowblock_supported(rows_, H, F, false);
     }
-    // which linears of a matrix-core executor multiply by tiles of the int8 weights as they are: those too small for the
-    // 256-row kernels to be the faster ones (some 1500 rows for a 11264 x 2048 matrix, every int8 product below half a
-    // round of tiles); a model with none of the others never makes the resident copies.  (Up to 64 rows the few-row kernel
-    // streams a tiled copy; shapes that it does not take stay with the resident one.)
+    // which linears of a matrix-core executor multiply by tiles of the int8 weights as they are: those for which that is the
+    // faster form (up to 500 .. 1500 rows, every int8 product of a few tiles); a model with none of the others never makes the
+    // resident copies, and one that would gain less than 3 % by them does not either (2 bytes per weight and a pass at
+    // set-up).  (Up to 64 rows the few-row kernel streams a tiled copy; shapes that it does not take stay with the resident one.)
     const int tile_kind = c.quantize_activations ? TG_I8 : TG_W8;
     size_t tg_part_bytes = 0;
-    auto plan_linear = [&](LinPlan &pl, int N, int K, const void *first, const void *last) {
-        const int rows_ = c.batch * c.seq_q;
-        pl = LinPlan{};
-        if (c.gemm_tile || !tile_gemm_supported(tile_kind, rows_, N, K) || !aligned16(first) || !aligned16(last)) return;
-        pl.plan = tile_gemm_plan(tile_kind, c.dtype, rows_, N, K, kTgScratchMax);
-        pl.tile = pl.plan.us <= (tile_kind == TG_I8 ? qgemm_dma_us(rows_, N, K) : gemm_nt_mfma_us(rows_, N, K, c.dtype));
-        if (pl.tile) tg_part_bytes = std::max(tg_part_bytes, pl.plan.part_bytes);
-    };
     bool all_tiles = false;
     if (m.quant && !m.skinny && c.batch * c.seq_q >= (c.quantize_activations ? 2 : 65)) {
-        bool ok = true;
+        const int rows_ = c.batch * c.seq_q;
+        bool ok = !c.gemm_tile, every = true;
         for (const Layer &L : m.layers) ok = ok && aligned16(L.o.w) && aligned16(L.down.w);
-        const void *odd = ok ? nullptr : (const void *)1;
-        plan_linear(m.pl_qkv, QD + 2 * KD, H, nullptr, nullptr);
-        plan_linear(m.pl_o, H, QD, odd, odd);
-        plan_linear(m.pl_gu, 2 * F, H, nullptr, nullptr);
-        plan_linear(m.pl_down, H, F, odd, odd);
-        plan_linear(m.pl_lm, V, H, m.lm_head.w, m.lm_head.w);
-        all_tiles = m.pl_qkv.tile && m.pl_o.tile && m.pl_gu.tile && m.pl_down.tile && m.pl_lm.tile;
+        double us_tiles = 0, us_best = 0;
+        auto plan_linear = [&](LinPlan &pl, int N, int K, bool can, int count, bool swiglu) {
+            pl = LinPlan{};
+            if (!can || !tile_gemm_supported(tile_kind, rows_, N, K)) {
+                every = false;
+                return;
+            }
+            pl.plan = tile_gemm_plan(tile_kind, c.dtype, rows_, N, K, kTgScratchMax);
+            const double other = tile_kind == TG_I8 ? qgemm_dma_us(rows_, N, K, swiglu) : gemm_nt_mfma_us(rows_, N, K, c.dtype, swiglu);
+            pl.tile = pl.plan.us <= other;
+            us_tiles += count * pl.plan.us;
+            us_best += count * std::min(pl.plan.us, other);
+        };
+        plan_linear(m.pl_qkv, QD + 2 * KD, H, !c.gemm_tile, c.n_layers, false);
+        plan_linear(m.pl_o, H, QD, ok, c.n_layers, false);
+        plan_linear(m.pl_gu, 2 * F, H, !c.gemm_tile, c.n_layers, true);
+        plan_linear(m.pl_down, H, F, ok, c.n_layers, false);
+        plan_linear(m.pl_lm, V, H, !c.gemm_tile && aligned16(m.lm_head.w), 1, false);
+        // (without whole groups of 32 gate rows there is no resident form of the layer)
+        const bool no_copies = tile_kind == TG_W8 && every && (us_tiles <= 1.03 * us_best || F % 32 != 0);
+        all_tiles = true;
+        for (LinPlan *pl : {&m.pl_qkv, &m.pl_o, &m.pl_gu, &m.pl_down, &m.pl_lm}) {
+            pl->tile = pl->tile || no_copies;
+            all_tiles = all_tiles && pl->tile;
+            if (pl->tile) tg_part_bytes = std::max(tg_part_bytes, pl->plan.part_bytes);
+        }
     }
     if (m.skinny) {
         // one more int8 copy of every linear weight, tiled for sequential streaming (1 byte per weight)

@@ -472,11 +472,25 @@ static int gemm_launch_dma(void *out, const void *act, const void *wt, const voi
 bool qgemm_dma_supported(int M, int N, int K) {
     return K % 128 == 0 && (long)((M + 255) / 256) * ((N + 255) / 256) >= 128;
 }
-// its time, microseconds: rounds over the 256 CUs, a last one that is half empty a little faster than a full one
-double qgemm_dma_us(int M, int N, int K) {
+// The time of a launch of 256-row tiles, microseconds, from rounds over the 256 CUs: a full round takes `fixed` (its store
+// and the ramp of its loads) plus `per_k` for every 1000 values of K, an empty one `empty` of that (fewer tiles leave each
+// more power and bandwidth), one of 320 columns `wide` times that.  wide_ok: 320 columns where they save rounds, as the
+// launchers take them.
+struct DmaCost {
+    double launch, fixed, per_k, empty, wide;
+};
+static double dma_us(const DmaCost &c, int M, int N, int K, bool wide_ok) {
+    const long t256 = (long)((M + 255) / 256) * ((N + 255) / 256), t320 = (long)((M + 255) / 256) * ((N + 319) / 320);
+    const bool wide = wide_ok && (t320 + 255) / 256 * 320 < (t256 + 255) / 256 * 256;
+    const long tiles = wide ? t320 : t256, last = tiles % 256;
+    const double rounds = tiles / 256 + (last ? c.empty + (1 - c.empty) * last / 256 : 0);
+    return c.launch + rounds * (c.fixed + c.per_k * K * 1e-3) * (wide ? c.wide : 1);
+}
+// (within 3 % of 180 measured products on average, 300 <= M <= 8192: 3000 x 5632 x 2048 46.8 us as one round of 320 columns,
+// where two rounds of 256 would take 67 and tile_gemm takes 60)
+double qgemm_dma_us(int M, int N, int K, bool swiglu) {
     if (!qgemm_dma_supported(M, N, K)) return 1e30;
-    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256), rounds = (tiles + 255) / 256;
-    return 4.0 + K * 1e-3 * (tiles < 256 ? 9.5 + 6.0 * tiles / 256 : 15.5 * rounds);
+    return dma_us(DmaCost{2.2, 9.6, 13.5, 0.61, 1.28}, M, N, K, !swiglu);
 }
 int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_scale, const int8_t *rhs, const void *rhs_scale,
               const void *res, int M, int N, int K, int dtype, int epi, hipStream_t s) {
@@ -498,18 +512,21 @@ int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_sc
     });
 }
 
+static bool gemm_fills(int M, int N) { return (long)((M + 255) / 256) * ((N + 127) / 128) > 256; }
 // tile: 0 = heuristic, 1 = 256x128, 2 = 256x256 via registers, 3 = 256x256 / 4 = 256x320 direct to LDS
 template <typename T, int EPI>
 static int gemm_launch(void *out, const void *act, const void *wt, const void *res, int M, int N, int K, int tile, hipStream_t s) {
     const int g_gemm_tile_override = tile;
-    // the large tile needs fewer LDS reads per MFMA (measured 10-25% faster) but runs one workgroup per CU:
-    // it is chosen once it fills the 256 CUs at least once (a partly filled second round still wins: the
-    // CUs left running clock higher)
-    const long big_tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
-    bool big = big_tiles >= 256;
-    if (g_gemm_tile_override) big = g_gemm_tile_override == 2;
     // the direct-to-LDS kernel is the faster 256 x 256 one (measured +5..20%); it needs whole 64-wide K steps
     const bool dma_ok = K % 64 == 0 && g_gemm_tile_override != 2;
+    // the large tile needs fewer LDS reads per MFMA (measured 10-25% faster) but runs one workgroup per CU:
+    // it is chosen once it fills the 256 CUs at least once (a partly filled second round still wins: the
+    // CUs left running clock higher), or, loaded straight to LDS, once the tiles of half its width are more than one per CU
+    // (gemm_fills; fp16: 5000 x 2560 x 2048 60 us against 72, 1500 x 5632 x 2048 52 against 65; below 2048 x 4096 x 4096 99
+    // against 85)
+    const long big_tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
+    bool big = big_tiles >= 256 || (dma_ok && gemm_fills(M, N));
+    if (g_gemm_tile_override) big = g_gemm_tile_override == 2;
     if (g_gemm_tile_override == 3 || g_gemm_tile_override == 4) big = dma_ok;
     if constexpr (EPI != GEMM_SWIGLU) {
         // 320 columns per tile when that saves rounds over the CUs (rounds x tile width = time)
@@ -542,14 +559,11 @@ int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, in
     });
 }
 
-// The time of gemm_nt_mfma, microseconds: grids of at least one round of 256 x 256 tiles run at 1.0 - 1.1 PFLOP/s (fp16;
-// bf16 5 % above) of whole tiles, those that take 320 columns at a time (gemm_launch) at 1.13; smaller ones take as long as
-// one tile does on its CU, which tile_gemm beats at every size measured.
-double gemm_nt_mfma_us(int M, int N, int K, int dtype) {
-    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256), wide = (long)((M + 255) / 256) * ((N + 319) / 320);
-    if (tiles < 256) return 1e30;
-    if (K % 64 == 0 && (wide + 255) / 256 * 320 < (tiles + 255) / 256 * 256) return 6.0 + 2.0 * 256 * 320 * K * (double)wide / 1.13e9;
-    return 6.0 + 2.0 * 256 * 256 * K * (double)tiles / (dtype == MYNN_BF16 ? 1.10e9 : 1.03e9);
+// The time of gemm_nt_mfma, microseconds (within 3 % of 100 measured products on average); grids that do not fill the
+// device with its 256-column tiles take as long as one tile does on its CU, which tile_gemm beats at every size measured.
+double gemm_nt_mfma_us(int M, int N, int K, int dtype, bool swiglu) {
+    if (K % 64 ? (long)((M + 255) / 256) * ((N + 255) / 256) < 256 : !gemm_fills(M, N)) return 1e30;
+    return dma_us(dtype == MYNN_BF16 ? DmaCost{2.8, 5.8, 27.5, 0.45, 1.19} : DmaCost{1.0, 6.9, 28.9, 0.47, 1.19}, M, N, K, !swiglu && K % 64 == 0);
 }
 // ... and of dequant_weight_rows before it (3 bytes per weight)
 static double dequant_us(int N, int K) { return 2.0 + 3.0 * N * K / 5.6e6; }

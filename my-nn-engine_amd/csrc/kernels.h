@@ -77,14 +77,14 @@ int interleave_row_groups(void *dst, const void *src, size_t rows, size_t row_by
 // QuantizedMatMul (int8 x int8 -> exact int32 -> two scales) with the large direct-to-LDS tiles of the
 // matrix-core GEMM; res (optional) is added to the rounded result and rounded again
 bool qgemm_dma_supported(int M, int N, int K);
-double qgemm_dma_us(int M, int N, int K);  // its time by measurement, for the choice against tile_gemm
+double qgemm_dma_us(int M, int N, int K, bool swiglu = false);  // its time by measurement, for the choice against tile_gemm
 int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_scale, const int8_t *rhs, const void *rhs_scale,
               const void *res, int M, int N, int K, int dtype, int epi, hipStream_t s);
 // tile: 0 heuristic; 1 = 256x128, 2 = 256x256 (register staged); 3 = 256x256, 4 = 256x320 (direct to LDS)
 // ranges > 1 (GEMM_PLAIN): each K range of tile_gemm is summed up on its own and the sums are added in their order, in tiles of 256x128
 int gemm_nt_mfma(void *out, const void *act, const void *wt, const void *res, int M, int N, int K, int dtype, int epi,
                  hipStream_t s, int tile = 0, int ranges = 1);
-double gemm_nt_mfma_us(int M, int N, int K, int dtype);  // its time by measurement, for the choice against tile_gemm
+double gemm_nt_mfma_us(int M, int N, int K, int dtype, bool swiglu = false);  // its time by measurement, for the choice against tile_gemm
 // W_T = T(wq * scale) into `ws` (gemm_weight_bytes), then out = act . W_T^T
 int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
                       int tile, hipStream_t s, int ranges = 1);
