@@ -274,10 +274,10 @@ static int gemm_rows(Model &m, const LinPlan &pl, void *out, const void *act, co
                      const char *name) {
     const int N = l.N, K = l.K;
     const double eb = 2.0, n_out = epi == GEMM_SWIGLU ? N / 2 : N;
-    if (pl.tile) {
+    if (pl.tile) {  // (SwiGLU as the layer would have it otherwise: the resident copies of whole groups of 32 rows the hardware's, else mynn_swiglu)
         note(m, name, (double)N * K + N * eb + ((double)M * K + (double)M * n_out * (epi == GEMM_RESIDUAL ? 2 : 1)) * eb, 2.0 * M * N * K);
         return tile_gemm(TG_W8, pl.plan, out, nullptr, act, (const int8_t *)l.w, nullptr, l.scale, res, M, N, K, m.cfg.dtype,
-                         epi == GEMM_SWIGLU ? GEMM_SWIGLU_PAIRS : epi, m.tg_part, m.tg_counters, m.stream);
+                         epi != GEMM_SWIGLU ? epi : N % 64 == 0 ? GEMM_SWIGLU_PAIRS : GEMM_SWIGLU_PAIRS_EXP, m.tg_part, m.tg_counters, m.stream);
     }
     note(m, name, ((double)N * K + (double)M * K + (double)M * n_out * (epi == GEMM_RESIDUAL ? 2 : 1)) * eb, 2.0 * M * N * K);
     return gemm_nt_mfma(out, act, wt, res, M, N, K, m.cfg.dtype, epi, m.stream, m.cfg.gemm_tile);
@@ -370,7 +370,7 @@ static int qlinear_fused(Model &m, const LinPlan &pl, void *out, const void *act
     note(m, name, (double)N * K + (double)M * K + N * eb + (double)M * n_out * eb * (res ? 2 : 1), 2.0 * M * N * K);
     if (pl.tile)
         return tile_gemm(TG_I8, pl.plan, out, nullptr, m.a8, (const int8_t *)l.w, m.a8_scale, l.scale, res, M, N, K, m.cfg.dtype,
-                         epi == GEMM_SWIGLU ? GEMM_SWIGLU_PAIRS : epi, m.tg_part, m.tg_counters, m.stream);
+                         epi == GEMM_SWIGLU ? GEMM_SWIGLU_PAIRS_EXP : epi, m.tg_part, m.tg_counters, m.stream);
     // (w32, scale32: the rows of gate and up in groups of 32, as the large tiles' SwiGLU store wants them)
     return qgemm_dma(out, nullptr, m.a8, m.a8_scale, (const int8_t *)(w32 ? w32 : l.w), scale32 ? scale32 : l.scale, res, M, N, K, m.cfg.dtype, epi,
                      m.stream);

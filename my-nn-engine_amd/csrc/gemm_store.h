@@ -13,7 +13,7 @@ namespace mynn {
 // operand buffers are free by now) and writes it out, and reads the residual, 16 bytes per lane, rows
 // contiguous.
 // GEMM_SWIGLU: gate and up columns alternate in groups of 32 (two column tiles of a wave); GEMM_SWIGLU_PAIRS: they
-// alternate one by one (column 2i gate_i, 2i+1 up_i: two neighbours in a lane).
+// and _EXP alternate one by one (column 2i gate_i, 2i+1 up_i: two neighbours in a lane).
 // at(i, j, e): element e of the accumulator of MFMA tile (i, j), as f32 ready to be rounded.
 template <typename T, typename G, int EPI, typename AccAt>
 __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const T *R, int M, int N, int m0,
@@ -21,7 +21,8 @@ __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const 
     constexpr int TI = G::TI, TJ = G::TJ;
     constexpr int EST = G::EST;
     static_assert(EPI != GEMM_SWIGLU || TJ % 2 == 0, "the SwiGLU store pairs neighbouring column tiles");
-    constexpr bool HALF = EPI == GEMM_SWIGLU || EPI == GEMM_SWIGLU_PAIRS;  // two accumulator columns per output column
+    constexpr bool PAIRS = EPI == GEMM_SWIGLU_PAIRS || EPI == GEMM_SWIGLU_PAIRS_EXP;
+    constexpr bool HALF = EPI == GEMM_SWIGLU || PAIRS;  // two accumulator columns per output column
     constexpr int OC = HALF ? TJ * 16 : TJ * 32;  // output columns of the wave tile
     constexpr int CPR = OC / 8;                   // 16-byte chunks per strip row
     const int ldc = HALF ? N >> 1 : N;
@@ -30,13 +31,13 @@ __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const 
     const bool vec_ok = (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && (EPI != GEMM_RESIDUAL || ((uintptr_t)R & 15) == 0);  // (uniform)
 #pragma unroll
     for (int i = 0; i < TI; i++) {
-        T *prow = patch + (lane & 31) * EST + (lane >> 5) * (EPI == GEMM_SWIGLU_PAIRS ? 2 : 4);
-        // GEMM_SWIGLU: hardware 2^x and reciprocal (about 1 ulp of f32 each, far below the 16-bit rounding that
-        // follows); the exact expf and division cost ~35 instructions per element there.  GEMM_SWIGLU_PAIRS: those of
-        // mynn_swiglu, whose place this store takes (500 x 28672 x 4096 int8, the pass of 8 layers 1948 us with either)
+        T *prow = patch + (lane & 31) * EST + (lane >> 5) * (PAIRS ? 2 : 4);
+        // hardware 2^x and reciprocal (about 1 ulp of f32 each, far below the 16-bit rounding that follows); the exact
+        // expf and division cost ~35 instructions per element here (a layer of 300 x 5632 outputs 1.7 us).  _EXP has them:
+        // for executors whose SwiGLU would otherwise be mynn_swiglu's
         auto swiglu = [](float gate, float up) {
             const float g = Elem<T>::rnd(gate), u = Elem<T>::rnd(up);
-            if constexpr (EPI == GEMM_SWIGLU_PAIRS) return (g * (1.0f / (1.0f + expf(-g)))) * u;
+            if constexpr (EPI == GEMM_SWIGLU_PAIRS_EXP) return (g * (1.0f / (1.0f + expf(-g)))) * u;
             else return (g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f))) * u;
         };
 #pragma unroll
@@ -49,7 +50,7 @@ __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const 
                     for (int x = 0; x < 4; x++) o[x] = swiglu(at(i, j, 4 * q + x), at(i, j + 1, 4 * q + x));
                     *(uint2 *)(prow + j * 16 + 8 * q) = uint2{pack2<T>(o[0], o[1]), pack2<T>(o[2], o[3])};
                 }
-            } else if constexpr (EPI == GEMM_SWIGLU_PAIRS) {
+            } else if constexpr (PAIRS) {
 #pragma unroll
                 for (int j = 0; j < TJ; j++)
                     *(uint32_t *)(prow + j * 16 + 4 * q) = pack2<T>(swiglu(at(i, j, 4 * q), at(i, j, 4 * q + 1)), swiglu(at(i, j, 4 * q + 2), at(i, j, 4 * q + 3)));

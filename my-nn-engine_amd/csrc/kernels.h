@@ -64,7 +64,7 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
 // matrix-core GEMM pieces.  A dequantised weight is [N, Kp] of the 16-bit type, Kp = K rounded up to 64,
 // zero padded (gemm_weight_bytes); dequant_weight_rows writes one (group/which: see gemm.hip), and
 // gemm_nt_mfma multiplies by it: out = store(act . wt^T) with the store one of GEMM_*.
-enum { GEMM_PLAIN = 0, GEMM_RESIDUAL = 1, GEMM_SWIGLU = 2, GEMM_SWIGLU_PAIRS = 3 };
+enum { GEMM_PLAIN = 0, GEMM_RESIDUAL = 1, GEMM_SWIGLU = 2, GEMM_SWIGLU_PAIRS = 3, GEMM_SWIGLU_PAIRS_EXP = 4 };
 size_t gemm_weight_bytes(int N, int K);
 int dequant_weight_rows(void *dst, const int8_t *wq, const void *scale, int N, int K, int dtype, int group, int which,
                         hipStream_t s);
@@ -105,7 +105,8 @@ bool tile_gemm_supported(int kind, int M, int N, int K);
 TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes);
 // the same sums as a plan of ks ranges has, without scratch memory (GEMM_PLAIN)
 TgPlan tile_gemm_plan_seq(int kind, int dtype, int M, int N, int K, int ks);
-// epi: GEMM_PLAIN, GEMM_RESIDUAL or GEMM_SWIGLU_PAIRS (gate and up rows alternate); part, counters: for plans with ranges
+// epi: GEMM_PLAIN, GEMM_RESIDUAL or one of GEMM_SWIGLU_PAIRS (gate and up rows alternate; _EXP: expf and a division, TG_I8 has that
+// form only); part, counters: for plans with ranges
 int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
               const void *res, int M, int N, int K, int dtype, int epi, void *part, int *counters, hipStream_t s);
 // the product with the stream's scratch memory for its ranges (gemm.hip), with none while the stream is being captured

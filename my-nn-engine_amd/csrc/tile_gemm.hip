@@ -531,7 +531,10 @@ template <typename T, typename G> static int tg_epi(const TgArgs &p, int epi) {
         return tail ? tg_go<T, G, GEMM_PLAIN, true>(p) : tg_go<T, G, GEMM_PLAIN, false>(p);
     else {
         if (epi == GEMM_RESIDUAL) return tail ? tg_go<T, G, GEMM_RESIDUAL, true>(p) : tg_go<T, G, GEMM_RESIDUAL, false>(p);
-        if (epi == GEMM_SWIGLU_PAIRS) return tail ? tg_go<T, G, GEMM_SWIGLU_PAIRS, true>(p) : tg_go<T, G, GEMM_SWIGLU_PAIRS, false>(p);
+        if (epi == GEMM_SWIGLU_PAIRS_EXP) return tail ? tg_go<T, G, GEMM_SWIGLU_PAIRS_EXP, true>(p) : tg_go<T, G, GEMM_SWIGLU_PAIRS_EXP, false>(p);
+        if constexpr (G::KIND == TG_W8) {
+            if (epi == GEMM_SWIGLU_PAIRS) return tail ? tg_go<T, G, GEMM_SWIGLU_PAIRS, true>(p) : tg_go<T, G, GEMM_SWIGLU_PAIRS, false>(p);
+        }
         return tail ? tg_go<T, G, GEMM_PLAIN, true>(p) : tg_go<T, G, GEMM_PLAIN, false>(p);
     }
 }
@@ -567,8 +570,8 @@ int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const v
     MYNN_REQUIRE(tile_gemm_supported(kind, M, N, K), MYNN_ERR_UNSUPPORTED, "tile_gemm: M=%d N=%d K=%d", M, N, K);
     MYNN_REQUIRE(aligned16(act) && aligned16(wq), MYNN_ERR_INVALID, "tile_gemm: operands must be 16-byte aligned");
     MYNN_REQUIRE(epi != GEMM_RESIDUAL || res, MYNN_ERR_INVALID, "tile_gemm: residual store without a residual");
-    MYNN_REQUIRE(epi != GEMM_SWIGLU_PAIRS || (N % 2 == 0 && !acc_out), MYNN_ERR_INVALID, "tile_gemm: SwiGLU store needs row pairs, N=%d", N);
-    MYNN_REQUIRE(epi != GEMM_SWIGLU && (kind != TG_W8S || epi == GEMM_PLAIN), MYNN_ERR_INVALID, "tile_gemm: store %d", epi);
+    MYNN_REQUIRE((epi != GEMM_SWIGLU_PAIRS && epi != GEMM_SWIGLU_PAIRS_EXP) || (N % 2 == 0 && !acc_out), MYNN_ERR_INVALID, "tile_gemm: SwiGLU store needs row pairs, N=%d", N);
+    MYNN_REQUIRE(epi != GEMM_SWIGLU && (kind != TG_W8S || epi == GEMM_PLAIN) && (kind != TG_I8 || epi != GEMM_SWIGLU_PAIRS), MYNN_ERR_INVALID, "tile_gemm: store %d", epi);
     MYNN_REQUIRE(plan.ks >= 1 && (plan.ks == 1 || plan.seq || (part && counters && aligned16(part))), MYNN_ERR_INVALID, "tile_gemm: K ranges without scratch memory");
     MYNN_REQUIRE(!plan.seq || (kind != TG_I8 && epi == GEMM_PLAIN), MYNN_ERR_UNSUPPORTED, "tile_gemm: ranges one after the other: kind %d, store %d", kind, epi);
     const TgArgs p{out, acc_out, act, wq, a_scale, w_scale, res, M, N, K, plan.ks, plan.seq, (uint64_t *)part, counters, s};
