@@ -407,7 +407,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 
 // ---- which tile, and over how many K ranges.
 // The time of a launch, in microseconds, fitted per tile to measured times of the linear layers of the benchmark's models
-// and others (16 <= M <= 4096, every tile at 1 .. 12 ranges):
+// and others (every tile at 1 .. 12 ranges):
 //
 //   t = launch + steps per range * (a * rounds + b * workgroups on the fullest CU) + g * further workgroups + e * ranges
 //       + partial sums at 4 TB/s
@@ -415,37 +415,55 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 // a: what a step costs a CU however few workgroups it holds (latency); b: what each resident workgroup adds (LDS, MFMA and
 // dequantisation work); rounds: how often a CU takes a new set of workgroups; g: what every workgroup on the fullest CU but
 // the first adds outside its steps (ramp and store).  Never less than the weights' bytes at 4.6 TB/s or the tiles'
-// operations at the rate the tile keeps up in long launches (padding included: 0.45 .. 0.9 PFLOP/s, int8 0.8 .. 1.8: larger tiles convert and
-// load less per product).  Choosing by it, and by the models of gemm.hip against the 256-row kernels, is 1 - 2 % above the
-// best measured choice on average (628 shapes, 3 <= M <= 8192; 25 % at worst, profiles/tile_gemm_plans.csv has
-// them); without ranges the shapes of up to 1000 rows would take 1.5 times as long (16-bit, 4 times at worst) and 1.04 times
-// (int8).  (Two fits where the conversion of the weights costs differ: it
-// is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
+// operations at the rate the tile keeps up in long launches (padding included).  From 256 rows on the constants are those
+// that, over 260 shapes per type, choose best (not those that predict best: some tiles have a `g` that only says that they
+// are never taken for more than one workgroup per CU); launches of fewer rows, one or two workgroups per CU and bound by
+// latency, keep a fit of their own.  Choosing by it, and by the models of gemm.hip against the 256-row kernels, is 1 % above
+// the best measured choice on average (1050 shapes, 2 <= M <= 8192; 33 of them by more than 10 %, 24 % at worst,
+// profiles/tile_gemm_plans.csv has them); without ranges 16-bit products of fewer than 256 rows would take 1.6 times as long
+// (4.4 at worst) and int8 ones 1.07 times.  (Two columns where the conversion of the weights costs differ: it is 14 vector
+// operations per 8 fp16 weights, 20 per 8 bf16 weights.)
 struct TgCost {
     int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
     float launch[2], a[2], b[2], e[2], g[2], rate[2];  // [0] fp16, [1] bf16; rate: 10^9 operations per microsecond
 };
 // (the order of the tiles in tg_launch)
+constexpr TgCost kTgW8Few[] = {
+    {32, 64, 3, {2.85f, 3.26f}, {0.308f, 0.311f}, {0.070f, 0.076f}, {0.53f, 0.47f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
+    {32, 128, 3, {2.95f, 3.26f}, {0.241f, 0.254f}, {0.150f, 0.145f}, {0.67f, 0.66f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
+    {64, 64, 2, {3.24f, 3.67f}, {0.237f, 0.236f}, {0.131f, 0.141f}, {0.62f, 0.60f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
+    {64, 128, 2, {2.87f, 3.61f}, {0.296f, 0.313f}, {0.165f, 0.147f}, {1.07f, 1.06f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
+    {128, 128, 1, {4.17f, 5.17f}, {0.281f, 0.312f}, {0.234f, 0.267f}, {0.95f, 0.90f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
+    {128, 128, 2, {4.51f, 5.83f}, {0.231f, 0.319f}, {0.323f, 0.316f}, {1.65f, 1.65f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
+};
 constexpr TgCost kTgW8[] = {
-    {32, 64, 3, {2.85f, 3.26f}, {0.308f, 0.311f}, {0.070f, 0.076f}, {0.53f, 0.47f}, {0.0f, 0.0f}, {0.45f, 0.45f}},
-    {32, 128, 3, {2.95f, 3.26f}, {0.241f, 0.254f}, {0.150f, 0.145f}, {0.67f, 0.66f}, {0.0f, 0.0f}, {0.55f, 0.5f}},
-    {64, 64, 2, {3.24f, 3.67f}, {0.237f, 0.236f}, {0.131f, 0.141f}, {0.62f, 0.60f}, {0.0f, 0.0f}, {0.5f, 0.5f}},
-    {64, 128, 2, {2.87f, 3.61f}, {0.296f, 0.313f}, {0.165f, 0.147f}, {1.07f, 1.06f}, {0.0f, 0.0f}, {0.7f, 0.7f}},
-    {128, 128, 1, {4.17f, 5.17f}, {0.281f, 0.312f}, {0.234f, 0.267f}, {0.95f, 0.90f}, {4.5f, 5.0f}, {0.75f, 0.7f}},
-    {128, 128, 2, {4.51f, 5.83f}, {0.231f, 0.319f}, {0.323f, 0.316f}, {1.65f, 1.65f}, {0.0f, 3.5f}, {0.9f, 0.8f}},
+    {32, 64, 3, {2.84f, 3.17f}, {0.308f, 0.300f}, {0.062f, 0.066f}, {0.41f, 0.42f}, {0.0f, 0.0f}, {0.77f, 0.37f}},
+    {32, 128, 3, {2.07f, 2.89f}, {0.322f, 0.254f}, {0.105f, 0.148f}, {0.62f, 0.62f}, {0.0f, 0.0f}, {0.63f, 0.94f}},
+    {64, 64, 2, {2.96f, 3.84f}, {0.254f, 0.239f}, {0.110f, 0.122f}, {0.79f, 0.72f}, {0.5f, 0.0f}, {0.94f, 1.41f}},
+    {64, 128, 2, {2.81f, 3.22f}, {0.342f, 0.327f}, {0.153f, 0.169f}, {0.69f, 0.76f}, {0.0f, 0.0f}, {0.71f, 0.72f}},
+    {128, 128, 1, {3.70f, 5.54f}, {0.309f, 0.317f}, {0.240f, 0.282f}, {0.29f, 2.88f}, {32.0f, 35.0f}, {0.88f, 0.64f}},
+    {128, 128, 2, {4.53f, 5.49f}, {0.234f, 0.426f}, {0.306f, 0.324f}, {3.14f, 1.06f}, {2.5f, 0.5f}, {0.88f, 0.80f}},
 };
 constexpr TgCost kTgW8S[] = {
     {32, 32, 3, {2.42f, 2.26f}, {0.300f, 0.350f}, {0.049f, 0.024f}, {0.65f, 0.71f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
     {32, 64, 3, {2.26f, 2.02f}, {0.266f, 0.320f}, {0.101f, 0.067f}, {0.68f, 0.73f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
     {32, 128, 3, {1.92f, 1.71f}, {0.229f, 0.245f}, {0.177f, 0.166f}, {1.00f, 1.05f}, {0.0f, 0.0f}, {0.93f, 0.88f}},
 };
+constexpr TgCost kTgI8Few[] = {
+    {32, 64, 2, {3.61f, 3.61f}, {0.001f, 0.001f}, {0.179f, 0.179f}, {0.63f, 0.63f}, {0.0f, 0.0f}, {1.85f, 1.85f}},
+    {64, 64, 1, {3.28f, 3.28f}, {0.146f, 0.146f}, {0.096f, 0.096f}, {0.93f, 0.93f}, {0.0f, 0.0f}, {1.85f, 1.85f}},
+    {64, 128, 1, {3.54f, 3.54f}, {0.190f, 0.190f}, {0.141f, 0.141f}, {0.80f, 0.80f}, {0.0f, 0.0f}, {1.85f, 1.85f}},
+    {64, 128, 2, {3.47f, 3.47f}, {0.101f, 0.101f}, {0.271f, 0.271f}, {1.12f, 1.12f}, {0.0f, 0.0f}, {1.85f, 1.85f}},
+    {128, 128, 1, {4.44f, 4.44f}, {0.244f, 0.244f}, {0.197f, 0.197f}, {0.92f, 0.92f}, {0.0f, 0.0f}, {1.85f, 1.85f}},
+    {128, 256, 1, {6.13f, 6.13f}, {0.377f, 0.377f}, {0.334f, 0.334f}, {1.76f, 1.76f}, {0.0f, 0.0f}, {1.85f, 1.85f}},
+};
 constexpr TgCost kTgI8[] = {
-    {32, 64, 2, {3.61f, 3.61f}, {0.001f, 0.001f}, {0.179f, 0.179f}, {0.63f, 0.63f}, {0.0f, 0.0f}, {0.8f, 0.8f}},
-    {64, 64, 1, {3.28f, 3.28f}, {0.146f, 0.146f}, {0.096f, 0.096f}, {0.93f, 0.93f}, {1.0f, 1.0f}, {1.2f, 1.2f}},
-    {64, 128, 1, {3.54f, 3.54f}, {0.190f, 0.190f}, {0.141f, 0.141f}, {0.80f, 0.80f}, {2.0f, 2.0f}, {1.5f, 1.5f}},
-    {64, 128, 2, {3.47f, 3.47f}, {0.101f, 0.101f}, {0.271f, 0.271f}, {1.12f, 1.12f}, {1.0f, 1.0f}, {1.5f, 1.5f}},
-    {128, 128, 1, {4.44f, 4.44f}, {0.244f, 0.244f}, {0.197f, 0.197f}, {0.92f, 0.92f}, {5.0f, 5.0f}, {1.6f, 1.6f}},
-    {128, 256, 1, {6.13f, 6.13f}, {0.377f, 0.377f}, {0.334f, 0.334f}, {1.76f, 1.76f}, {10.0f, 10.0f}, {1.8f, 1.8f}},
+    {32, 64, 2, {3.40f, 3.40f}, {0.002f, 0.002f}, {0.177f, 0.177f}, {0.55f, 0.55f}, {9.0f, 9.0f}, {0.65f, 0.65f}},
+    {64, 64, 1, {2.98f, 2.98f}, {0.146f, 0.146f}, {0.094f, 0.094f}, {0.47f, 0.47f}, {53.0f, 53.0f}, {1.02f, 1.02f}},
+    {64, 128, 1, {3.70f, 3.70f}, {0.141f, 0.141f}, {0.130f, 0.130f}, {1.63f, 1.63f}, {19.0f, 19.0f}, {1.52f, 1.52f}},
+    {64, 128, 2, {3.55f, 3.55f}, {0.049f, 0.049f}, {0.262f, 0.262f}, {1.37f, 1.37f}, {2.0f, 2.0f}, {1.14f, 1.14f}},
+    {128, 128, 1, {4.20f, 4.20f}, {0.270f, 0.270f}, {0.218f, 0.218f}, {1.38f, 1.38f}, {5.5f, 5.5f}, {1.83f, 1.83f}},
+    {128, 256, 1, {6.54f, 6.54f}, {0.509f, 0.509f}, {0.321f, 0.321f}, {0.44f, 0.44f}, {9.0f, 9.0f}, {2.03f, 2.03f}},
 };
 
 bool tile_gemm_supported(int kind, int M, int N, int K) {
@@ -453,7 +471,8 @@ bool tile_gemm_supported(int kind, int M, int N, int K) {
 }
 
 static TgPlan tg_choose(int kind, int dtype, int M, int N, int K, size_t scratch_bytes) {
-    const TgCost *tab = kind == TG_W8 ? kTgW8 : kind == TG_W8S ? kTgW8S : kTgI8;
+    const bool few = M < 256;
+    const TgCost *tab = kind == TG_W8S ? kTgW8S : kind == TG_W8 ? (few ? kTgW8Few : kTgW8) : few ? kTgI8Few : kTgI8;
     const int n_tiles = kind == TG_W8S ? 3 : 6, d = dtype == MYNN_BF16 ? 1 : 0;
     const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
     const double weights_us = (double)N * K / 4.6e6;
