@@ -168,7 +168,10 @@ struct Model {
     std::vector<Layer> layers;
     void *wt_lm_head = nullptr, *pk_lm_head = nullptr;
     WeightSet *wset = nullptr;  // the derived weight copies (shared with the session's other executors)
-    bool w8a8_fused = false;  // W8A8 with the large int8 tiles: norm+quantise, residual and SwiGLU ride on the launches
+    bool w8a8_fused = false;  // W8A8 on the matrix cores: norm+quantise, residual and SwiGLU ride on the launches
+    // every W8A8 linear fills the 256-row tiles: their SwiGLU is the hardware's form (expf and a division in the others, as
+    // the operators': 70 -> 74 us for 500 x 28672 x 4096)
+    bool all_large = false;
     bool qgemv1 = false;      // W8A8 at batch 1: norm, quantiser, int8 GEMV and residual / SwiGLU of a linear in one launch
     bool resident16 = false;  // the matrix-core path with fused stores: tiles of the int8 weights or the wt_* copies, by plan
     LinPlan pl_qkv, pl_o, pl_gu, pl_down, pl_lm;
@@ -372,8 +375,8 @@ static int qlinear_fused(Model &m, const LinPlan &pl, void *out, const void *act
         return tile_gemm(TG_I8, pl.plan, out, nullptr, m.a8, (const int8_t *)l.w, m.a8_scale, l.scale, res, M, N, K, m.cfg.dtype,
                          epi == GEMM_SWIGLU ? GEMM_SWIGLU_PAIRS_EXP : epi, m.tg_part, m.tg_counters, m.stream);
     // (w32, scale32: the rows of gate and up in groups of 32, as the large tiles' SwiGLU store wants them)
-    return qgemm_dma(out, nullptr, m.a8, m.a8_scale, (const int8_t *)(w32 ? w32 : l.w), scale32 ? scale32 : l.scale, res, M, N, K, m.cfg.dtype, epi,
-                     m.stream);
+    return qgemm_dma(out, nullptr, m.a8, m.a8_scale, (const int8_t *)(w32 ? w32 : l.w), scale32 ? scale32 : l.scale, res, M, N, K, m.cfg.dtype,
+                     epi == GEMM_SWIGLU && !m.all_large ? GEMM_SWIGLU_EXP : epi, m.stream);
 }
 
 // The attention block of the streaming-KV graph, op for op (decoder.rs:281-347, 472-487): RoPE(q); k and v un-rotated
@@ -949,6 +952,8 @@ static int build(Model &m, void **init, void **state) {
     // large tiles take the gate/up product, its rows (and scales) are interleaved in groups of 32 once
     if (m.quant && c.quantize_activations && c.batch * c.seq_q >= 2 && c.dtype != MYNN_F32) {
         const int rows_ = c.batch * c.seq_q;
+        auto large = [&](int N, int K) { return qgemm_dma_supported(rows_, N, K); };
+        m.all_large = large(QD + 2 * KD, H) && large(H, QD) && large(2 * F, H) && large(H, F) && large(V, H);
         auto either = [&](const LinPlan &pl, int N, int K) { return pl.tile || qgemm_dma_supported(rows_, N, K); };
         if ((m.pl_gu.tile || F % 32 == 0) && either(m.pl_qkv, QD + 2 * KD, H) && either(m.pl_o, H, QD) && either(m.pl_gu, 2 * F, H) &&
             either(m.pl_down, H, F) && either(m.pl_lm, V, H)) {

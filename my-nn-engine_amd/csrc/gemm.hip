@@ -496,11 +496,13 @@ int qgemm_dma(void *out, int32_t *acc_out, const int8_t *lhs, const void *lhs_sc
               const void *res, int M, int N, int K, int dtype, int epi, hipStream_t s) {
     MYNN_REQUIRE(qgemm_dma_supported(M, N, K), MYNN_ERR_UNSUPPORTED, "quantized_matmul (large tiles): M=%d N=%d K=%d", M, N, K);
     MYNN_REQUIRE(epi != GEMM_RESIDUAL || res, MYNN_ERR_INVALID, "quantized_matmul: residual store without a residual");
-    MYNN_REQUIRE(epi != GEMM_SWIGLU || (N % 64 == 0 && !acc_out), MYNN_ERR_INVALID, "quantized_matmul: SwiGLU store needs N %% 64 == 0, N=%d", N);
+    MYNN_REQUIRE((epi != GEMM_SWIGLU && epi != GEMM_SWIGLU_EXP) || (N % 64 == 0 && !acc_out), MYNN_ERR_INVALID, "quantized_matmul: SwiGLU store needs N %% 64 == 0, N=%d", N);
     return dispatch_dtype16(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
         const long t256 = (long)((M + 255) / 256) * ((N + 255) / 256), t320 = (long)((M + 255) / 256) * ((N + 319) / 320);
         const bool wide = (t320 + 255) / 256 * 320 < (t256 + 255) / 256 * 256;
+        if (epi == GEMM_SWIGLU_EXP)
+            return gemm_launch_dma<T, TileDma, GEMM_SWIGLU_EXP, true>(out, lhs, rhs, nullptr, M, N, K, s, lhs_scale, rhs_scale, nullptr);
         if (epi == GEMM_SWIGLU)
             return gemm_launch_dma<T, TileDma, GEMM_SWIGLU, true>(out, lhs, rhs, nullptr, M, N, K, s, lhs_scale, rhs_scale, nullptr);
         if (epi == GEMM_RESIDUAL) {

@@ -13,16 +13,17 @@ namespace mynn {
 // operand buffers are free by now) and writes it out, and reads the residual, 16 bytes per lane, rows
 // contiguous.
 // GEMM_SWIGLU: gate and up columns alternate in groups of 32 (two column tiles of a wave); GEMM_SWIGLU_PAIRS: they
-// and _EXP alternate one by one (column 2i gate_i, 2i+1 up_i: two neighbours in a lane).
+// alternate one by one (column 2i gate_i, 2i+1 up_i: two neighbours in a lane); _EXP: the same with expf and a division.
 // at(i, j, e): element e of the accumulator of MFMA tile (i, j), as f32 ready to be rounded.
 template <typename T, typename G, int EPI, typename AccAt>
 __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const T *R, int M, int N, int m0,
                                            int n0, int wrow, int wcol, int lane, int wave) {
     constexpr int TI = G::TI, TJ = G::TJ;
     constexpr int EST = G::EST;
-    static_assert(EPI != GEMM_SWIGLU || TJ % 2 == 0, "the SwiGLU store pairs neighbouring column tiles");
+    constexpr bool GROUPS = EPI == GEMM_SWIGLU || EPI == GEMM_SWIGLU_EXP;
+    static_assert(!GROUPS || TJ % 2 == 0, "the SwiGLU store pairs neighbouring column tiles");
     constexpr bool PAIRS = EPI == GEMM_SWIGLU_PAIRS || EPI == GEMM_SWIGLU_PAIRS_EXP;
-    constexpr bool HALF = EPI == GEMM_SWIGLU || PAIRS;  // two accumulator columns per output column
+    constexpr bool HALF = GROUPS || PAIRS;  // two accumulator columns per output column
     constexpr int OC = HALF ? TJ * 16 : TJ * 32;  // output columns of the wave tile
     constexpr int CPR = OC / 8;                   // 16-byte chunks per strip row
     const int ldc = HALF ? N >> 1 : N;
@@ -37,12 +38,12 @@ __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const 
         // for executors whose SwiGLU would otherwise be mynn_swiglu's
         auto swiglu = [](float gate, float up) {
             const float g = Elem<T>::rnd(gate), u = Elem<T>::rnd(up);
-            if constexpr (EPI == GEMM_SWIGLU_PAIRS_EXP) return (g * (1.0f / (1.0f + expf(-g)))) * u;
+            if constexpr (EPI == GEMM_SWIGLU_PAIRS_EXP || EPI == GEMM_SWIGLU_EXP) return (g * (1.0f / (1.0f + expf(-g)))) * u;
             else return (g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f))) * u;
         };
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            if constexpr (EPI == GEMM_SWIGLU) {
+            if constexpr (GROUPS) {
 #pragma unroll
                 for (int j = 0; j < TJ; j += 2) {
                     float o[4];

@@ -1,5 +1,6 @@
-"""SwiGLU in the store of a W8A8 executor's gate/up product (tile_gemm.hip) against the operators one by one: int32 sums
-are exact, so one-token sequences, whose attention returns their value row, have to agree in every bit of every row."""
+"""SwiGLU in the store of a W8A8 executor's gate/up product (tile_gemm.hip; 500 x 11264: gate/up, and no other linear, in
+the 256-row tiles of gemm.hip) against the operators one by one: int32 sums are exact, so one-token sequences, whose
+attention returns their value row, have to agree in every bit of every row."""
 import numpy as np
 import pytest
 
@@ -18,8 +19,8 @@ def g():
 
 
 @pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
-@pytest.mark.parametrize("B,ffn", [(2, 320), (97, 5632), (300, 5632)])
-def test_layer_equals_the_operators(g, dt, B, ffn):
+@pytest.mark.parametrize("B,ffn,gates", [(2, 320, "both"), (97, 5632, "both"), (300, 5632, "both"), (300, 5632, "negative"), (500, 11264, "negative")])
+def test_layer_equals_the_operators(g, dt, B, ffn, gates):
     import torch
 
     m = g.mynn
@@ -27,6 +28,11 @@ def test_layer_equals_the_operators(g, dt, B, ffn):
     dw = dev_weights(g, w, dt)
     # gates of every size up to some ten: wide enough for both ends of the sigmoid
     dw["layers.0.gate"] = (dw["layers.0.gate"][0], dw["layers.0.gate"][1] * 4)
+    if gates == "negative":
+        # (all around -5: there the largest of a row, which sets the codes of the others, comes from the sigmoid's tail)
+        dw["layers.0.gate"] = (-dw["layers.0.gate"][0].abs().clamp(max=127), dw["layers.0.gate"][1] * 0.375)
+        dw["embed"] = (dw["embed"][0].abs().clamp(max=127), dw["embed"][1])
+        dw["layers.0.up"] = (dw["layers.0.up"][0], dw["layers.0.up"][1] * 64)
     dec = m.Decoder(cfg, dw, batch=B, quantize_activations=True)
     ids = np.random.default_rng(B).integers(0, cfg["vocab"], B)
     names = [k[0] for k in dec.profile(ids, [0], 0, 1)]
