@@ -543,11 +543,12 @@ static int attention_entry(void *out, const void *Q, const void *K, const void *
             int rc = static_scratch(&scr);
             if (rc) return rc;
         } else {
-            int rc = g_scratch.lease(st, kArriveBytes + need, kArriveBytes, "attention", &lease);
+            const bool capturing = stream_capturing(st);
+            int rc = g_scratch.lease(st, capturing, kArriveBytes + need, kArriveBytes, "attention", &lease);
             if (rc) return rc;
             // (a graph's launches may meet others on the counters, whatever the caller was told, and a counter that is left
             // above zero spoils every later call; so it merges by a second launch, as the fixed array's calls do)
-            if (!stream_capturing(st)) p.arrive = (int *)lease.ptr;
+            if (!capturing) p.arrive = (int *)lease.ptr;
             scr = lease.ptr + kArriveBytes;
         }
     }
@@ -886,7 +887,7 @@ extern "C" int mynn_attention_streaming(void *out, const void *Q, const void *K,
     const size_t need = ring_carve(B, Sq, num_q_heads, num_kv_heads, head_dim, dtype, kv_int8, rope_on, cache_seq_len).total;
     hipStream_t st = as_stream(s);
     StreamBlocks::Lease ws;
-    int rc = g_ring.lease(st, need, 0, "attention_streaming", &ws);
+    int rc = g_ring.lease(st, stream_capturing(st), need, 0, "attention_streaming", &ws);
     if (rc) return rc;
     return mynn_attention_streaming_ws(out, Q, K, V, k_scale, v_scale, scale, is_causal, B, Sq, active_seq_kv, cache_seq_len, q_pos_offset,
                                        num_q_heads, num_kv_heads, head_dim, dtype, kv_int8, ring_sink, ring_window, ring_start, cos_t,

@@ -619,7 +619,7 @@ int tile_gemm_on_stream(int kind, TgPlan plan, void *out, int32_t *acc_out, cons
     StreamBlocks::Lease ws;
     if (plan.ks > 1 && stream_capturing(s)) plan = tile_gemm_plan_seq(kind, dtype, M, N, K, plan.ks);
     else if (plan.ks > 1) {
-        int rc = g_ws.lease(s, kWsCounterBytes + plan.part_bytes, kWsCounterBytes, "matrix product", &ws);
+        int rc = g_ws.lease(s, false, kWsCounterBytes + plan.part_bytes, kWsCounterBytes, "matrix product", &ws);
         if (rc) return rc;
     }
     return tile_gemm(kind, plan, out, acc_out, act, wq, a_scale, w_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, ws.ptr ? ws.ptr + kWsCounterBytes : nullptr,
@@ -681,7 +681,7 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
     if (takes_matrix_cores(act, wq, M, K, act_dtype, out_dtype)) {
         MYNN_REQUIRE(N > 0 && K > 0, MYNN_ERR_INVALID, "dequant_matmul: N=%d K=%d", N, K);
         StreamBlocks::Lease ws;
-        int rc = g_ws.lease(as_stream(s), kWsCounterBytes + gemm_weight_bytes(N, K), kWsCounterBytes, "dequant_matmul", &ws);
+        int rc = g_ws.lease(as_stream(s), stream_capturing(as_stream(s)), kWsCounterBytes + gemm_weight_bytes(N, K), kWsCounterBytes, "dequant_matmul", &ws);
         if (rc) return rc;
         return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }
