@@ -416,7 +416,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 // dequantisation work); rounds: how often a CU takes a new set of workgroups; g: what every workgroup on the fullest CU but
 // the first adds outside its steps (ramp and store).  Never less than the weights' bytes at 4.6 TB/s or the tiles'
 // operations at the rate the tile keeps up in long launches (padding included).  From 256 rows on the constants are those
-// that, over 260 shapes per type, choose best (not those that predict best: some tiles have a `g` that only says that they
+// that, over some 250 shapes per type, choose best (not those that predict best: some tiles have a `g` that only says that they
 // are never taken for more than one workgroup per CU); launches of fewer rows, one or two workgroups per CU and bound by
 // latency, keep a fit of their own.  Choosing by it, and by the models of gemm.hip against the 256-row kernels, is 1 % above
 // the best measured choice on average (1050 shapes, 2 <= M <= 8192; 33 of them by more than 10 %, 24 % at worst,
