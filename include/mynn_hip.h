@@ -26,7 +26,8 @@
  * A block that a captured call was given stays valid for the graph's life, also when a later call makes
  * the stream's block grow; it is shared with that stream's other calls, so replays have to be ordered
  * with those.  Products that only split K (no weight is dequantised: see the calls) use no library
- * memory at all while being captured; their graphs may be replayed anywhere.  The `_ws` variants take
+ * memory at all while being captured, and one that would dequantise its weight, for which the block is
+ * too small, takes the int8 weights instead; their graphs may be replayed anywhere.  The `_ws` variants take
  * the caller's block instead and touch nothing global; `mynn_attention_noalloc` uses a fixed
  * device array of the library.  Executors (seam 1) own everything they use: nothing an executor
  * launches touches library-global memory.

@@ -672,7 +672,8 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
                                    int K, int act_dtype, int out_dtype, mynn_stream s) {
     MYNN_REQUIRE(M >= 1, MYNN_ERR_INVALID, "dequant_matmul: M=%d", M);
     int kind = 0;
-    if (scale && takes_tiles(out, act, wq, M, N, K, act_dtype, out_dtype, &kind)) {
+    const bool tiles = scale && takes_tiles(out, act, wq, M, N, K, act_dtype, out_dtype, &kind);
+    if (tiles) {
         TgPlan plan = tile_gemm_plan(kind, out_dtype, M, N, K, tiles_scratch(kind, N, K));
         if (tiles_first(plan, kind, M, N, K, out_dtype)) {
             return tile_gemm_on_stream(kind, plan, out, nullptr, act, wq, nullptr, scale, M, N, K, out_dtype, as_stream(s));
@@ -682,6 +683,10 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
         MYNN_REQUIRE(N > 0 && K > 0, MYNN_ERR_INVALID, "dequant_matmul: N=%d K=%d", N, K);
         StreamBlocks::Lease ws;
         int rc = g_ws.lease(as_stream(s), stream_capturing(as_stream(s)), kWsCounterBytes + gemm_weight_bytes(N, K), kWsCounterBytes, "dequant_matmul", &ws);
+        // (captured, and the stream's block does not hold the dequantised weight: the same sums from the int8 weights)
+        if (rc == MYNN_ERR_STATE && tiles)
+            return tile_gemm(kind, tile_gemm_plan(kind, out_dtype, M, N, K, 0), out, nullptr, act, wq, nullptr, scale, nullptr, M, N, K, out_dtype,
+                             GEMM_PLAIN, nullptr, nullptr, as_stream(s));
         if (rc) return rc;
         return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }

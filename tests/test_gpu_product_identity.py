@@ -30,10 +30,11 @@ def captured(torch, call):
     return out
 
 
-# one and two row tiles of 16 .. 300 rows x few and many columns; K of two steps, of half a step more, of 4 .. 8 ranges
+# one and two row tiles of 16 .. 300 rows x few and many columns; K of two steps, of half a step more, of 4 .. 8 ranges; the
+# last two: 256-row tiles that do not fill the device once, whole and ragged (captured on a new stream: the int8 tiles)
 @pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
 @pytest.mark.parametrize("M,N,K", [(16, 2048, 2048), (64, 2048, 2048), (33, 65, 4112), (100, 256, 8192), (128, 4096, 4096), (300, 4096, 14336),
-                                   (300, 1000, 4096), (17, 31, 128), (40, 72, 2200)])
+                                   (300, 1000, 4096), (17, 31, 128), (40, 72, 2200), (1500, 5632, 2048), (1300, 7177, 1088)])
 @pytest.mark.parametrize("size", [1.0, 1e-5])  # (1e-5: fp16 weights that are subnormal once scaled)
 def test_same_bits_from_every_form(g, dt, M, N, K, size):
     import torch
