@@ -25,12 +25,30 @@ template <> struct Mfma<bf16_t> {
     }
 };
 
+// ds_read_b64_tr_b16: of each 16 lanes, lane i names the 8 bytes at row i / 4, columns 4 * (i % 4) .. +3 of a 4 x 16 block of 16-bit
+// values (anywhere in LDS, 8-byte aligned), and receives the block's column i, rows 0 .. 3
+typedef short s4_t __attribute__((ext_vector_type(4)));
+__device__ inline uint2 lds_read_tr16(const char *p) {
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4_t *)p));
+}
+
+// 16 bytes per lane from base + off to LDS byte lds + 16 * lane (base and lds wave-uniform).  As an instruction of its own and not
+// through the builtin: behind the builtin the compiler puts a wait for EVERY load in flight before the next ds_read_*_tr, the
+// tile after the one that is read among them.  The caller waits (vmcnt, then a barrier) before it reads what was loaded.
+__device__ inline uint32_t lds_offset(const char *p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p; }
+__device__ inline void load_to_lds(const char *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+
 // two f32 -> one dword of two storage-type values (low half first), round to nearest even: one packed
 // convert instruction.  The inputs are values ALREADY rounded to f32 (the empty asm keeps the compiler from
 // fusing the producing multiply into a mixed-precision op that would round the exact product once).
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+template <typename T> __device__ inline uint32_t cvt2(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){lo, hi}, std::conditional_t<std::is_same<T, f16_t>::value, h2_t, bf2_t>));
+}
 template <typename T> __device__ inline uint32_t pack2(float lo, float hi);
 template <> __device__ inline uint32_t pack2<f16_t>(float lo, float hi) {
     asm volatile("" : "+v"(lo), "+v"(hi));
