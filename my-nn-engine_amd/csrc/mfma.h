@@ -32,12 +32,42 @@ __device__ inline uint2 lds_read_tr16(const char *p) {
     return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4_t *)p));
 }
 
-// 16 bytes per lane from base + off to LDS byte lds + 16 * lane (base and lds wave-uniform).  As an instruction of its own and not
-// through the builtin: behind the builtin the compiler puts a wait for EVERY load in flight before the next ds_read_*_tr, the
-// tile after the one that is read among them.  The caller waits (vmcnt, then a barrier) before it reads what was loaded.
-__device__ inline uint32_t lds_offset(const char *p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p; }
+// 16 bytes per lane to LDS byte lds + 16 * lane (wave-uniform), from base + off (base wave-uniform) or from p.  As instructions of
+// their own and not through the builtin: behind the builtin the compiler puts a wait for EVERY load in flight before the next
+// ds_read that it cannot tell apart from what is being written, the stages further ahead among them.  The caller waits (vmcnt,
+// then a barrier) before it reads what was loaded.
+__device__ inline uint32_t lds_offset(const void *p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p; }
+__device__ inline const char *scalar_pointer(const char *p) {  // (nothing where it is in scalar registers already)
+    const uint64_t u = (uint64_t)(uintptr_t)p;
+    return (const char *)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(u >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)u));
+}
 __device__ inline void load_to_lds(const char *base, uint32_t off, uint32_t lds) {
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    base = scalar_pointer(base);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
+}
+__device__ inline void load_to_lds(const char *p, uint32_t lds) {
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+}
+
+// N <= 4 of them to consecutive kilobytes of LDS from one setting of m0: load i adds 1024 * i to both of its addresses, so off[i] is
+// 1024 * i short of the distance from base.
+template <int N> __device__ inline void load_group_to_lds(const char *base, const uint32_t *off, uint32_t lds) {
+    static_assert(N >= 1 && N <= 4, "the offset has 12 bits");
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    base = scalar_pointer(base);
+#define MYNN_LOAD(i, o) "\n\tglobal_load_lds_dwordx4 %" #i ", %1 offset:" #o
+    if constexpr (N == 1) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) ::"s"(lds), "s"(base), "v"(off[0]) : "memory", "m0");
+    else if constexpr (N == 2) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) MYNN_LOAD(3, 1024) ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]) : "memory", "m0");
+    else if constexpr (N == 3)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) MYNN_LOAD(3, 1024) MYNN_LOAD(4, 2048) ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2])
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) MYNN_LOAD(3, 1024) MYNN_LOAD(4, 2048) MYNN_LOAD(5, 3072) ::"s"(lds), "s"(base), "v"(off[0]),
+                     "v"(off[1]), "v"(off[2]), "v"(off[3])
+                     : "memory", "m0");
+#undef MYNN_LOAD
 }
 
 // two f32 -> one dword of two storage-type values (low half first), round to nearest even: one packed

@@ -153,8 +153,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             for (int c = wave; c < M * CPR; c += WAVES) {
                 const int m = c / CPR, k = p * PK + (c % CPR) * 512 + lane * 8;
                 if (k - lane * 8 >= K) continue;
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(act + (size_t)m * K + min(k, K - 8)),
-                                                 (__attribute__((address_space(3))) void *)(dst + (size_t)m * AS + (c % CPR) * 1024), 16, 0, 0);
+                load_to_lds((const char *)(act + (size_t)m * K + min(k, K - 8)), lds_offset(dst + (size_t)m * AS + (c % CPR) * 1024));
             }
         };
         issue_panel(0);
