@@ -89,7 +89,7 @@ double gemm_nt_mfma_us(int M, int N, int K, int dtype, bool swiglu = false);  //
 int dequant_gemm_mfma(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, void *ws,
                       int tile, hipStream_t s, int ranges = 1);
 
-// tile_gemm.hip -- products of ordinary size with operand tiles of 32 .. 128 rows, K ranges where those do not fill the
+// tile_gemm.hip -- products of ordinary size with operand tiles of 32 .. 160 rows, K ranges where those do not fill the
 // device.  TG_W8 / TG_W8S: 16-bit activations, int8 weights scaled before / after the products; TG_I8: QuantizedMatMul.
 enum { TG_W8 = 0, TG_W8S = 1, TG_I8 = 2 };
 struct TgPlan {
