@@ -185,8 +185,9 @@ def check(rc):
 
 
 # ------------------------------------------------------------------ torch plumbing
-# The host path of an operator call is most of the time of a small one (a 5632 x 2048 GEMV takes 3.9 us on the device):
-# the current stream is asked for as a raw handle where torch has that (0.1 us; torch.cuda.current_stream() builds a Stream
+# The host path of an operator call is most of the time of a small one (a 5632 x 2048 GEMV takes 3.9 us on the device).  The four
+# operators a program calls most go through a module of their own (csrc/host_ops.cpp), which takes plain tensors and answers None
+# to everything else; the rest, and what it does not take, through ctypes: the current stream is asked for as a raw handle where torch has that (0.1 us; torch.cuda.current_stream() builds a Stream
 # object, 2.7 us), outputs come from new_empty of the tensor whose device they share (1.1 us; torch.empty with a device 1.5),
 # type codes from one table.
 _torch = None
@@ -226,6 +227,29 @@ def _ptr(t):
     return t.data_ptr()
 
 
+_ops = None
+
+
+def _host_ops():
+    """lib/_host_ops.so, with the addresses of the library's entry points."""
+    global _ops
+    if _ops is None:
+        import importlib.machinery
+        import importlib.util
+
+        l = lib()
+        path = os.path.join(_HERE, "lib", "_host_ops.so")
+        if not os.path.exists(path):
+            raise MynnError("host module not built: %s is missing (run __graft_entry__.build())" % path)
+        loader = importlib.machinery.ExtensionFileLoader("_host_ops", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_host_ops", path, loader=loader))
+        loader.exec_module(module)
+        module.bind(MynnError, *(C.cast(getattr(l, n), _vp).value for n in (
+            "mynn_last_error", "mynn_dequant_matmul", "mynn_quantized_matmul", "mynn_dynamic_quantize_linear", "mynn_attention")))
+        _ops = module
+    return _ops
+
+
 def device_info():
     cu, wave, lds = _i(), _i(), _i()
     arch = C.create_string_buffer(64)
@@ -251,6 +275,10 @@ def dequant_gemv(act, wq, scale):
 
 
 def dequant_matmul(act, wq, scale):
+    if wq.is_cuda:
+        out = (_ops or _host_ops()).dequant_matmul(act, wq, scale)
+        if out is not None:
+            return out
     N, K = wq.shape
     M = act.numel() // K
     out = wq.new_empty(act.shape[:-1] + (N,), dtype=scale.dtype)
@@ -294,6 +322,10 @@ def dequant_matmul_prepared(act, wt, N, gemm_tile=0):
 
 
 def quantized_matmul(lhs, lhs_scale, rhs, rhs_scale, want_acc=True):
+    if not want_acc and lhs.is_cuda:
+        out = (_ops or _host_ops()).quantized_matmul(lhs, lhs_scale, rhs, rhs_scale)
+        if out is not None:
+            return out, None
     M, K = lhs.shape
     N = rhs.shape[0]
     out = lhs.new_empty((M, N), dtype=rhs_scale.dtype)
@@ -304,6 +336,10 @@ def quantized_matmul(lhs, lhs_scale, rhs, rhs_scale, want_acc=True):
 
 
 def dynamic_quantize_linear(x, symmetric=True):
+    if symmetric and x.is_cuda:
+        out = (_ops or _host_ops()).dynamic_quantize_linear(x)
+        if out is not None:
+            return out
     rows = x.shape[0]
     inner = x.numel() // rows
     y = x.new_empty(x.shape, dtype=_t().int8 if symmetric else _t().uint8)
@@ -316,6 +352,10 @@ def dynamic_quantize_linear(x, symmetric=True):
 
 def attention(q, k, v, scale, is_causal=False, active=None, d_active=None, q_pos_offset=None, k_scale=None,
               v_scale=None):
+    if d_active is None and q.is_cuda:
+        out = (_ops or _host_ops()).attention(q, k, v, scale, is_causal, active, q_pos_offset, k_scale, v_scale)
+        if out is not None:
+            return out
     B, Hq, Sq, D = q.shape
     Hkv, cache_len = k.shape[1], k.shape[2]
     if active is None:
