@@ -63,7 +63,7 @@ size_t attn_scratch_bytes(int B, int Hq, int Sq, int D, int nsplit);
 int attention_decode_launch(AttnParams p, int D, int dtype, int kv_int8, void *scratch, hipStream_t s);
 int attention_prefill_launch(const AttnParams &p, int D, int dtype, int kv_int8, hipStream_t s);
 bool attention_prefill_supported(const AttnParams &p, int D, int dtype, int kv_int8);
-// streaming decode kernel (attention_stream.hip): taken when eligible; attn_plan then returns its plan
+// streaming decode kernel (attention_stream.h, .hip): taken when eligible; attn_plan then returns its plan
 bool attn_stream_eligible(int B, int Sq, int Hq, int Hkv, int D, int dtype, int kv_int8, int kv_len, int cache_len);
 void attn_stream_plan(int B, int Hkv, int kv_len, int *slice, int *nsplit);
 int attn_stream_max_ranges(int B, int Hkv, int kv_len_max);  // most key ranges any length <= kv_len_max is planned with
