@@ -68,7 +68,11 @@ template <typename T, int D, int W> struct StreamLds {
     static constexpr int V = kStreamTile * (D + 4) * 2, P = kParts<T> * 16 * (kStreamTile + 8) * 2, ML = 8 * 4;
     static constexpr int P0 = W * V, M0 = P0 + W * P, L0 = M0 + W * ML, ROW0 = L0 + W * ML, SCALE0 = ROW0 + 2 * D * 2, BYTES = SCALE0 + 16;
 };
-template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W>
+// ONCE: value rows, whole lines per instruction, are read with the hint that they won't be wanted again (stream_once below).  Key
+// rows are read 64 bytes at a time, a line by two instructions: the hint there gave 2.5 % of a decode step of 32 sequences x 2048
+// keys where this one gives 3.2, both together 3.0.
+__device__ __forceinline__ U4 load_once(const U4 *p) { return __builtin_nontemporal_load(p); }
+template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, bool ONCE>
 __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
     using Lds = StreamLds<T, D, W>;
     constexpr int kStreamWaves = W, kStreamThreads = W * 64;
@@ -252,7 +256,9 @@ __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
 #pragma unroll
         for (int q = 0; q < NP; q++) {
             const int vrow = min(t0 + q * KPP + vk, k1 - 1);
-            vr[q] = *(const Chunk *)(Vp + at(vrow) * D + vd);
+            const Chunk *src = (const Chunk *)(Vp + at(vrow) * D + vd);
+            if constexpr (ONCE) vr[q] = load_once(src);
+            else vr[q] = *src;
         }
     };
 
@@ -566,6 +572,16 @@ __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
 
 // Waves of a workgroup, four or eight, from its key range (attn_stream_plan, which makes ranges of 256 rows where eight are wanted)
 inline bool stream_eight_waves(int slice, int nsplit) { return slice == 256 && (nsplit == 1 || nsplit >= 8); }
+
+// Whether 16-bit value rows are read as not wanted again (four waves only: eight have little to read).  In an executor's step (the
+// length in device memory) the other layers' caches and weights pass before the same rows are read again; an operator's caches
+// may still be in the Infinity Cache, 256 MB, from the call before unless they are larger than it.  Us per launch without /
+// with, D = 128, 8 kv heads: operator, 17 sequences x 1056 keys (74 MB) 14.7 / 16.2, 24 x 2000 29.9 / 31.0, 32 x 2000 (262 MB) 41.5 /
+// 42.0, 32 x 3000 (393 MB) 68.8 / 57.9, 64 x 3000 133.5 / 122.7; step of an 8-layer executor, 16 x 1000 804 / 790, 32 x 1000 930 / 916,
+// 64 x 3000 2020 / 1915; launch of 32 x 2048 in a 32-layer step, paged, 47.6 / 43.9.  (int8 caches, 32 x 3000: no difference.)
+inline bool stream_once(const StreamParams &p, int B, size_t row_bytes) {
+    return p.d_active || 2 * (size_t)B * p.Hkv * min(p.active, p.cache_len) * row_bytes > (320u << 20);
+}
 
 // by type, a translation unit each
 template <typename T> int attn_stream_go(const StreamParams &p, int B, int D, int kv_int8, bool fuse, hipStream_t s);
