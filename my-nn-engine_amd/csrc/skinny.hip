@@ -300,6 +300,24 @@ int skinny_pack_weight(void *dst, const int8_t *wq, int N, int K, hipStream_t s)
 
 // sum of the K ranges, scale, store (with the residual or SwiGLU when asked); SWIGLU: rows of the weight
 // were gate/up interleaved (row 2i gate_i, 2i+1 up_i) and out is [M, N/2]
+// A sum over K ranges, in their order: N4 consecutive columns of the partial sums [range][M][N] at `src`, `pitch` = M * N apart.
+// The loads of up to MAXS ranges are issued together (ranges past the last repeat it and do not count): behind a test per
+// range the compiler waited for the first load before it asked for the others.
+template <int MAXS, typename V> struct PartSum {
+    V v[MAXS];
+    __device__ __forceinline__ void request(const float *src, size_t pitch, int ksplit) {
+#pragma unroll
+        for (int s = 0; s < MAXS; s++) v[s] = *(const V *)(src + (size_t)min(s, ksplit - 1) * pitch);
+    }
+    __device__ __forceinline__ void add(float *t, int ksplit) const {
+        constexpr int W = sizeof(V) / sizeof(float);
+#pragma unroll
+        for (int s = 0; s < MAXS; s++)
+#pragma unroll
+            for (int i = 0; i < W; i++) t[i] += s < ksplit ? ((const float *)&v[s])[i] : 0.f;
+    }
+};
+
 template <typename T, int EPI>
 __global__ __launch_bounds__(256) void skinny_reduce_kernel(T *out, const float *part, const T *scale, const T *res, int M,
                                                           int N, int ksplit) {
@@ -307,19 +325,28 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(T *out, const float 
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)M * n_out) return;
     const int m = (int)(idx / n_out), c = (int)(idx % n_out);
-    auto total = [&](int n) {
-        float t = 0.f;
-        for (int s = 0; s < ksplit; s++) t += part[((size_t)s * M + m) * N + n];
-        return t;
+    const size_t pitch = (size_t)M * N;
+    auto total = [&](auto t2, int n, float *t) {
+        using V = decltype(t2);
+        PartSum<8, V> p;
+        for (int s0 = 0; s0 < ksplit; s0 += 8) {
+            p.request(part + s0 * pitch + (size_t)m * N + n, pitch, ksplit - s0);
+            p.add(t, ksplit - s0);
+        }
     };
     if (EPI == GEMM_SWIGLU) {
-        const float g = Elem<T>::rnd(total(2 * c) * Elem<T>::ld(scale, 2 * c));
-        const float u = Elem<T>::rnd(total(2 * c + 1) * Elem<T>::ld(scale, 2 * c + 1));
+        float t[2] = {0.f, 0.f};
+        total(float2{}, 2 * c, t);  // (N is even)
+        const float g = Elem<T>::rnd(t[0] * Elem<T>::ld(scale, 2 * c));
+        const float u = Elem<T>::rnd(t[1] * Elem<T>::ld(scale, 2 * c + 1));
         const float sig = 1.0f / (1.0f + expf(-g));
         Elem<T>::st(out, idx, (g * sig) * u);
     } else {
-        float y = total(c) * Elem<T>::ld(scale, c);
-        if (EPI == GEMM_RESIDUAL) y = Elem<T>::rnd(y) + Elem<T>::ld(res, idx);
+        const float sc = Elem<T>::ld(scale, c), rs = EPI == GEMM_RESIDUAL ? Elem<T>::ld(res, idx) : 0.f;
+        float t = 0.f;
+        total(0.f, c, &t);
+        float y = t * sc;
+        if (EPI == GEMM_RESIDUAL) y = Elem<T>::rnd(y) + rs;
         Elem<T>::st(out, idx, y);
     }
 }
@@ -329,32 +356,19 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(T *out, const float 
 // thread, every load issued before the first sum; x_out = T(T(sum * scale) + res), nrm_out = T((x * inv) * w)
 // with inv = 1 / sqrt(mean(x^2) + eps) over the stored (rounded) x, as the separate operators compute them.
 constexpr int kReduceNormThreads = 1024, kReduceNormMaxSplit = 12;  // (2048 x 5632: 11 ranges)
-template <typename T>
+template <typename T, int MAXS>
 __global__ __launch_bounds__(kReduceNormThreads) void skinny_reduce_norm_kernel(T *x_out, T *nrm_out, const float *part, const T *scale,
                                                                               const T *res, const T *norm_w, int M, int N, int ksplit,
                                                                               float eps) {
     __shared__ float red[kReduceNormThreads / 64];
     const int m = blockIdx.x, c0 = threadIdx.x * 4;
     const bool live = c0 < N;
-    float4 pv[kReduceNormMaxSplit];
-    uint2 sc2 = uint2{0u, 0u}, rs2 = sc2, nw2 = sc2;
-#pragma unroll
-    for (int s = 0; s < kReduceNormMaxSplit; s++) {
-        pv[s] = float4{0.f, 0.f, 0.f, 0.f};
-        if (live && s < ksplit) pv[s] = *(const float4 *)(part + ((size_t)s * M + m) * N + c0);
-    }
-    if (live) {
-        sc2 = *(const uint2 *)(scale + c0);
-        rs2 = *(const uint2 *)(res + (size_t)m * N + c0);
-        nw2 = *(const uint2 *)(norm_w + c0);
-    }
+    const int cl = live ? c0 : 0;
+    PartSum<MAXS, float4> p;
+    p.request(part + (size_t)m * N + cl, (size_t)M * N, ksplit);
+    const uint2 sc2 = *(const uint2 *)(scale + cl), rs2 = *(const uint2 *)(res + (size_t)m * N + cl), nw2 = *(const uint2 *)(norm_w + cl);
     float t[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < kReduceNormMaxSplit; s++) {  // the order of skinny_reduce_kernel: K ranges ascending
-        if (s < ksplit) {
-            t[0] += pv[s].x; t[1] += pv[s].y; t[2] += pv[s].z; t[3] += pv[s].w;
-        }
-    }
+    p.add(t, ksplit);  // the order of skinny_reduce_kernel: K ranges ascending
     float sc[8], rs[8], nw[8], x[4];
     widen8<T>(U4{sc2.x, sc2.y, 0u, 0u}, sc);
     widen8<T>(U4{rs2.x, rs2.y, 0u, 0u}, rs);
@@ -363,7 +377,7 @@ __global__ __launch_bounds__(kReduceNormThreads) void skinny_reduce_norm_kernel(
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         x[i] = Elem<T>::rnd(Elem<T>::rnd(t[i] * sc[i]) + rs[i]);
-        ss += x[i] * x[i];
+        ss += live ? x[i] * x[i] : 0.f;
     }
     if (live) *(uint2 *)(x_out + (size_t)m * N + c0) = uint2{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
     ss = wave_sum(ss);
@@ -386,7 +400,7 @@ __global__ __launch_bounds__(kReduceNormThreads) void skinny_reduce_norm_kernel(
 // to T, v as stored; s = amax / 127 stored as T, q = trunc(x * 127 / amax +- 0.5) clamped to [-128, 127]); every head
 // then takes D/8 threads (4 low + 4 high elements each), an aligned lane group, and the row maximum is a DPP reduction.
 constexpr int kReduceRopeThreads = 128;  // two waves: a row's units spread over ~7 workgroups, ~220 workgroups per launch
-template <typename T, bool KV8>
+template <typename T, bool KV8, int MAXS>
 __global__ __launch_bounds__(kReduceRopeThreads) void skinny_reduce_rope_kernel(const float *part, const T *scale, int M, int N, int ksplit,
                                                                               T *q_out, void *k_cache_v, void *v_cache_v, T *k_scale,
                                                                               T *v_scale, const T *cos_t, const T *sin_t,
@@ -397,27 +411,23 @@ __global__ __launch_bounds__(kReduceRopeThreads) void skinny_reduce_rope_kernel(
     const int rot_units = (Hq + Hkv) * upr, units = rot_units + Hkv * upv;
     const int past = *d_past;
     const size_t tab = (size_t)position[sq] * D;
-    auto total4 = [&](int col, float *t) {
-        float4 pv[kReduceNormMaxSplit];
-#pragma unroll
-        for (int s = 0; s < kReduceNormMaxSplit; s++) {
-            pv[s] = float4{0.f, 0.f, 0.f, 0.f};
-            if (s < ksplit) pv[s] = *(const float4 *)(part + ((size_t)s * M + m) * N + col);
-        }
-        const uint2 sc2 = *(const uint2 *)(scale + col);
+    struct Four {  // four columns of the projection, as requested
+        PartSum<MAXS, float4> p;
+        uint2 sc;
+    };
+    auto request = [&](int col, Four &f) {
+        f.p.request(part + (size_t)m * N + col, (size_t)M * N, ksplit);
+        f.sc = *(const uint2 *)(scale + col);
+    };
+    auto total4 = [&](const Four &f, float *t) {
         float sc[8];
-        widen8<T>(U4{sc2.x, sc2.y, 0u, 0u}, sc);
+        widen8<T>(U4{f.sc.x, f.sc.y, 0u, 0u}, sc);
         t[0] = t[1] = t[2] = t[3] = 0.f;
-#pragma unroll
-        for (int s = 0; s < kReduceNormMaxSplit; s++)
-            if (s < ksplit) {
-                t[0] += pv[s].x; t[1] += pv[s].y; t[2] += pv[s].z; t[3] += pv[s].w;
-            }
+        f.p.add(t, ksplit);
 #pragma unroll
         for (int i = 0; i < 4; i++) t[i] = Elem<T>::rnd(t[i] * sc[i]);
     };
-    auto ld4 = [&](const T *p, float *f) {
-        const uint2 v = *(const uint2 *)p;
+    auto widen4 = [](const uint2 &v, float *f) {
         float w[8];
         widen8<T>(U4{v.x, v.y, 0u, 0u}, w);
 #pragma unroll
@@ -450,13 +460,18 @@ __global__ __launch_bounds__(kReduceRopeThreads) void skinny_reduce_rope_kernel(
             if constexpr (KV8) {
                 const int hv = (u - rot_units) / upr, j = ((u - rot_units) % upr) * 4;
                 float lo[4], hi[4];
-                total4((Hq + Hkv + hv) * D + j, lo);
-                total4((Hq + Hkv + hv) * D + j + half, hi);
+                Four l4, h4;
+                request((Hq + Hkv + hv) * D + j, l4);
+                request((Hq + Hkv + hv) * D + j + half, h4);
+                total4(l4, lo);
+                total4(h4, hi);
                 quantise_store(lo, hi, (int8_t *)v_cache_v, v_scale, kv_cache_row(pg, b, hv, past + sq, Hkv, max_seq), j);
             } else {
                 const int hv = (u - rot_units) / upv, j = ((u - rot_units) % upv) * 4;
                 float t[4];
-                total4((Hq + Hkv + hv) * D + j, t);
+                Four f;
+                request((Hq + Hkv + hv) * D + j, f);
+                total4(f, t);
                 T *dst = (T *)v_cache_v + kv_cache_row(pg, b, hv, past + sq, Hkv, max_seq) * D + j;
                 *(uint2 *)dst = uint2{pack2<T>(t[0], t[1]), pack2<T>(t[2], t[3])};
             }
@@ -464,12 +479,17 @@ __global__ __launch_bounds__(kReduceRopeThreads) void skinny_reduce_rope_kernel(
         }
         const int head = u / upr, j = (u % upr) * 4;
         float xl[4], xh[4], cl[4], ch[4], sl[4], sh[4];
-        total4(head * D + j, xl);
-        total4(head * D + j + half, xh);
-        ld4(cos_t + tab + j, cl);
-        ld4(cos_t + tab + j + half, ch);
-        ld4(sin_t + tab + j, sl);
-        ld4(sin_t + tab + j + half, sh);
+        Four l4, h4;
+        request(head * D + j, l4);
+        request(head * D + j + half, h4);
+        const uint2 cs[4] = {*(const uint2 *)(cos_t + tab + j), *(const uint2 *)(cos_t + tab + j + half), *(const uint2 *)(sin_t + tab + j),
+                             *(const uint2 *)(sin_t + tab + j + half)};
+        total4(l4, xl);
+        total4(h4, xh);
+        widen4(cs[0], cl);
+        widen4(cs[1], ch);
+        widen4(cs[2], sl);
+        widen4(cs[3], sh);
         float ol[4], oh[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -562,11 +582,18 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
         if (ks_used == 1 && epi == GEMM_PLAIN) return gemm(std::integral_constant<int, GEMM_PLAIN>{});
         int rc = gemm(std::integral_constant<int, -1>{});
         if (rc) return rc;
+        auto by_split = [&](auto f) {  // (loads past the last range repeat it: as few of those as a choice of three leaves)
+            if (ks_used <= 4) f(std::integral_constant<int, 4>{});
+            else if (ks_used <= 8) f(std::integral_constant<int, 8>{});
+            else f(std::integral_constant<int, kReduceNormMaxSplit>{});
+        };
         if (epi == GEMM_RESIDUAL && norm_w && nrm_out && normed && N % 4 == 0 && N <= 4 * kReduceNormThreads &&
             ks_used <= kReduceNormMaxSplit && aligned16(out) && aligned16(res) && aligned16(nrm_out) && ((uintptr_t)norm_w & 7) == 0 &&
             ((uintptr_t)scale & 7) == 0) {
-            MYNN_LAUNCH(skinny_reduce_norm_kernel<T>, dim3(M), dim3(kReduceNormThreads), 0, s, (T *)out, (T *)nrm_out, scratch,
-                        (const T *)scale, (const T *)res, (const T *)norm_w, M, N, ks_used, eps);
+            by_split([&](auto most) {
+                MYNN_LAUNCH((skinny_reduce_norm_kernel<T, decltype(most)::value>), dim3(M), dim3(kReduceNormThreads), 0, s, (T *)out, (T *)nrm_out, scratch,
+                            (const T *)scale, (const T *)res, (const T *)norm_w, M, N, ks_used, eps);
+            });
             *normed = true;
             return launch_status("skinny_reduce_norm_kernel");
         }
@@ -576,16 +603,19 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
             ((uintptr_t)rope->sin_t & 7) == 0 && (!rope->k_scale || ((rope->D == 64 || rope->D == 128) && rope->v_scale))) {
             const int rope_units = (rope->Hq + rope->Hkv) * (rope->D / 8) + rope->Hkv * (rope->k_scale ? rope->D / 8 : rope->D / 4);
             const dim3 rope_grid(M, (rope_units + kReduceRopeThreads - 1) / kReduceRopeThreads);
-            if (rope->k_scale)
-                MYNN_LAUNCH((skinny_reduce_rope_kernel<T, true>), rope_grid, dim3(kReduceRopeThreads), 0, s, scratch, (const T *)scale, M, N,
-                            ks_used, (T *)rope->q_out, rope->k_cache, rope->v_cache, (T *)rope->k_scale, (T *)rope->v_scale,
-                            (const T *)rope->cos_t, (const T *)rope->sin_t, rope->position, rope->d_past, rope->S, rope->Hq, rope->Hkv,
-                            rope->D, rope->max_seq, rope->paging);
-            else
-                MYNN_LAUNCH((skinny_reduce_rope_kernel<T, false>), rope_grid, dim3(kReduceRopeThreads), 0, s, scratch, (const T *)scale, M, N,
-                            ks_used, (T *)rope->q_out, rope->k_cache, rope->v_cache, (T *)nullptr, (T *)nullptr, (const T *)rope->cos_t,
-                            (const T *)rope->sin_t, rope->position, rope->d_past, rope->S, rope->Hq, rope->Hkv, rope->D, rope->max_seq,
-                            rope->paging);
+            by_split([&](auto most) {
+                constexpr int MAXS = decltype(most)::value;
+                if (rope->k_scale)
+                    MYNN_LAUNCH((skinny_reduce_rope_kernel<T, true, MAXS>), rope_grid, dim3(kReduceRopeThreads), 0, s, scratch, (const T *)scale, M, N,
+                                ks_used, (T *)rope->q_out, rope->k_cache, rope->v_cache, (T *)rope->k_scale, (T *)rope->v_scale,
+                                (const T *)rope->cos_t, (const T *)rope->sin_t, rope->position, rope->d_past, rope->S, rope->Hq, rope->Hkv,
+                                rope->D, rope->max_seq, rope->paging);
+                else
+                    MYNN_LAUNCH((skinny_reduce_rope_kernel<T, false, MAXS>), rope_grid, dim3(kReduceRopeThreads), 0, s, scratch, (const T *)scale, M, N,
+                                ks_used, (T *)rope->q_out, rope->k_cache, rope->v_cache, (T *)nullptr, (T *)nullptr, (const T *)rope->cos_t,
+                                (const T *)rope->sin_t, rope->position, rope->d_past, rope->S, rope->Hq, rope->Hkv, rope->D, rope->max_seq,
+                                rope->paging);
+            });
             *roped = true;
             return launch_status("skinny_reduce_rope_kernel");
         }
