@@ -50,34 +50,39 @@ __global__ __launch_bounds__(kEwThreads) void rms_norm_kernel(T *out, const T *x
 }
 
 // Rows of 16-bit values whose length is a multiple of 8 and at most 8 * 4 * kEwThreads: 128-bit
-// loads, the row read once and kept in registers between the two passes.
-template <typename T>
+// loads, the row read once and kept in registers between the two passes.  The launch is one round trip to memory and a
+// reduction: all loads, the weights' too, are requested without a test around them (pieces past the row repeat its last one and
+// count as zero) -- behind a test each, the compiler waited for every load before it asked for the next, and for the weights
+// once more behind the reduction (32 rows of 4096: 3.3 -> 2.9 us).
+// NCH pieces a thread: no more than the row has (8192 rows of 2048: 13.1 us before, 11.8; with four for every length 15.7)
+template <typename T, int NCH>
 __global__ __launch_bounds__(kEwThreads) void rms_norm_vec_kernel(T *out, const T *x, const T *w, int dim, float eps) {
     __shared__ float red[4];
     const size_t base = (size_t)blockIdx.x * dim;
     const int chunks = dim >> 3;
-    U4 v[4];
+    U4 v[NCH], nw[NCH];
+#pragma unroll
+    for (int q = 0; q < NCH; q++) v[q] = *(const U4 *)(x + base + (size_t)min((int)threadIdx.x + q * kEwThreads, chunks - 1) * 8);
+#pragma unroll
+    for (int q = 0; q < NCH; q++) nw[q] = *(const U4 *)(w + (size_t)min((int)threadIdx.x + q * kEwThreads, chunks - 1) * 8);
     float ss = 0.f;
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const int c = threadIdx.x + q * kEwThreads;
-        if (c < chunks) {
-            v[q] = *(const U4 *)(x + base + (size_t)c * 8);
-            float f[8];
-            widen8<T>(v[q], f);
+    for (int q = 0; q < NCH; q++) {
+        if ((int)threadIdx.x + q * kEwThreads >= chunks) v[q] = U4{0u, 0u, 0u, 0u};
+        float f[8];
+        widen8<T>(v[q], f);
 #pragma unroll
-            for (int i = 0; i < 8; i++) ss += f[i] * f[i];
-        }
+        for (int i = 0; i < 8; i++) ss += f[i] * f[i];
     }
     const float tot = block_sum(ss, red);
     const float inv = 1.0f / sqrtf(tot / (float)dim + eps);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
+    for (int q = 0; q < NCH; q++) {
         const int c = threadIdx.x + q * kEwThreads;
         if (c < chunks) {
             float f[8], g[8];
             widen8<T>(v[q], f);
-            widen8<T>(*(const U4 *)(w + (size_t)c * 8), g);
+            widen8<T>(nw[q], g);
             U4 o;
             o.x = pack2<T>((f[0] * inv) * g[0], (f[1] * inv) * g[1]);
             o.y = pack2<T>((f[2] * inv) * g[2], (f[3] * inv) * g[3]);
@@ -268,7 +273,8 @@ __global__ __launch_bounds__(kEwThreads) void dynquant_kernel(void *y_, T *y_sca
 // Symmetric per-row quantisation of 16-bit rows of at most 8 * 64 * W * NCH values (a multiple of 8): the row read once
 // with 128-bit loads and kept in registers; same arithmetic as dynquant_kernel<T, true>.  W = 1: one wave per row,
 // reductions inside the wave.  W = 4: a workgroup per row, for few rows (a wave per row left most CUs without one: 97 rows
-// of 4096 took 6.4 us) and for rows that one wave cannot hold (500 of 14336 on the looping kernel: 28 us).
+// of 4096 took 6.4 us) and for rows that one wave cannot hold (500 of 14336 on the looping kernel: 28 us).  All pieces of a
+// row are requested without a test around them, as in rms_norm_vec_kernel (500 rows of 14336: 8.7 -> 6.8 us, of 4096 with the norm 5.7 -> 5.6).
 // NORM: the row is first RMS-normalised exactly as rms_norm_vec_kernel does (rounded to the storage type)
 // and only the quantised form is written -- the normalised activations of a W8A8 layer have no other reader.
 template <typename T, bool NORM, int NCH, int W>
@@ -284,22 +290,18 @@ __global__ __launch_bounds__(kEwThreads) void dynquant_rows_vec_kernel(int8_t *y
     float ss = 0.f;
 #pragma unroll
     for (int q = 0; q < NCH; q++) {
-        const int c = lane + q * 64 * W;
-        v[q] = U4{0u, 0u, 0u, 0u};
-        if (c < chunks) {
-            v[q] = *(const U4 *)(x + base + (size_t)c * 8);
-            if (NORM && W > 1) nw[q] = *(const U4 *)(w + (size_t)c * 8);
-        }
+        const int c = min(lane + q * 64 * W, chunks - 1);
+        v[q] = *(const U4 *)(x + base + (size_t)c * 8);
+        if (NORM && W > 1) nw[q] = *(const U4 *)(w + (size_t)c * 8);
     }
 #pragma unroll
     for (int q = 0; q < NCH; q++) {
-        if (lane + q * 64 * W < chunks) {
-            if (NORM) {
-                float f[8];
-                widen8<T>(v[q], f);
+        if (lane + q * 64 * W >= chunks) v[q] = U4{0u, 0u, 0u, 0u};
+        if (NORM) {
+            float f[8];
+            widen8<T>(v[q], f);
 #pragma unroll
-                for (int i = 0; i < 8; i++) ss += f[i] * f[i];
-            }
+            for (int i = 0; i < 8; i++) ss += f[i] * f[i];
         }
     }
     if (NORM) {
@@ -594,8 +596,14 @@ extern "C" int mynn_rms_norm(void *out, const void *x, const void *w, int rows, 
         using T = std::remove_pointer_t<decltype(t)>;
         if constexpr (sizeof(T) == 2) {
             if (dim % 8 == 0 && dim <= 8 * 4 * kEwThreads && aligned16(out) && aligned16(x) && aligned16(w)) {
-                MYNN_LAUNCH(rms_norm_vec_kernel<T>, dim3(rows), dim3(kEwThreads), 0, as_stream(s), (T *)out,
-                                   (const T *)x, (const T *)w, dim, eps);
+                auto go = [&](auto nch) {
+                    MYNN_LAUNCH((rms_norm_vec_kernel<T, decltype(nch)::value>), dim3(rows), dim3(kEwThreads), 0, as_stream(s), (T *)out,
+                                (const T *)x, (const T *)w, dim, eps);
+                };
+                const int nch = (dim / 8 + kEwThreads - 1) / kEwThreads;
+                if (nch == 1) go(std::integral_constant<int, 1>{});
+                else if (nch == 2) go(std::integral_constant<int, 2>{});
+                else go(std::integral_constant<int, 4>{});
                 return launch_status("rms_norm_vec_kernel");
             }
         }
