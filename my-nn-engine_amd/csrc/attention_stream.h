@@ -63,16 +63,20 @@ struct StreamParams {
     float scale;
     int Hq, Hkv, cache_len, active, nsplit, slice, page_shift, pages_per_seq;
 };
+enum StreamForm { kOneTile, kTiles, kTilesOnce };
 // LDS of a workgroup of W waves, in bytes: V tiles, p tiles, (m, l) of the waves, the new row and its scales
 template <typename T, int D, int W> struct StreamLds {
     static constexpr int V = kStreamTile * (D + 4) * 2, P = kParts<T> * 16 * (kStreamTile + 8) * 2, ML = 8 * 4;
     static constexpr int P0 = W * V, M0 = P0 + W * P, L0 = M0 + W * ML, ROW0 = L0 + W * ML, SCALE0 = ROW0 + 2 * D * 2, BYTES = SCALE0 + 16;
 };
-// ONCE: value rows, whole lines per instruction, are read with the hint that they won't be wanted again (stream_once below).  Key
+// FORM: kOneTile where the key range has a tile per wave, kTiles where a wave walks several, the next one's loads in flight (with both
+// in one kernel, chosen by the range, the walk is 1 - 2 % slower: 17 sequences x 1056 keys, D = 128, 14.7 us against 14.4; the walk
+// over a single tile 5 %: 4 x 1000, D = 64, 7.2 against 6.9).
+// kTilesOnce: value rows, whole lines per instruction, are read with the hint that they won't be wanted again (stream_once below).  Key
 // rows are read 64 bytes at a time, a line by two instructions: the hint there gave 2.5 % of a decode step of 32 sequences x 2048
 // keys where this one gives 3.2, both together 3.0.
 __device__ __forceinline__ U4 load_once(const U4 *p) { return __builtin_nontemporal_load(p); }
-template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, bool ONCE>
+template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, int FORM>
 __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
     using Lds = StreamLds<T, D, W>;
     constexpr int kStreamWaves = W, kStreamThreads = W * 64;
@@ -257,7 +261,7 @@ __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
         for (int q = 0; q < NP; q++) {
             const int vrow = min(t0 + q * KPP + vk, k1 - 1);
             const Chunk *src = (const Chunk *)(Vp + at(vrow) * D + vd);
-            if constexpr (ONCE) vr[q] = load_once(src);
+            if constexpr (FORM == kTilesOnce) vr[q] = load_once(src);
             else vr[q] = *src;
         }
     };
@@ -409,7 +413,7 @@ __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
     // workgroup (heads out of step as well): 60 us; a contiguous cache is indifferent to all three (50 us).  The
     // order of the tiles changes nothing but the rounding of the online softmax, and it is a fixed function of the
     // grid.
-    const int nt = (k1 - k0 - wave * kStreamTile + tstep - 1) / tstep;
+    const int nt = (k1 - k0 - wave * kStreamTile + tstep - 1) / tstep;  // (kOneTile: one, or none or fewer)
     NewRow fresh;
     if constexpr (FUSE) {
         if (new_mine) request(fresh);
@@ -446,7 +450,7 @@ __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
             if (new_mine) append(fresh);
             __builtin_amdgcn_wave_barrier();
         }
-        if (nt == 1) process(tile_at(0), kA, vA, sA);  // (no tile to have in flight meanwhile)
+        if constexpr (FORM == kOneTile) process(tile_at(0), kA, vA, sA);
         else while (true) {
             load_tile(tile_at(n + 1), kB, vB, sB);
             process(tile_at(n), kA, vA, sA);

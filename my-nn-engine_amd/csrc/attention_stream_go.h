@@ -4,25 +4,27 @@
 
 namespace mynn {
 
-template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, bool ONCE> static int stream_go(const StreamParams &p, int B, hipStream_t s) {
+template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, int FORM> static int stream_go(const StreamParams &p, int B, hipStream_t s) {
     constexpr int lds = StreamLds<T, D, W>::BYTES;
     static bool lds_set = false;
     if (!lds_set && lds > 64 * 1024) {
-        MYNN_HIP(hipFuncSetAttribute((const void *)attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        MYNN_HIP(hipFuncSetAttribute((const void *)attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         lds_set = true;
     }
-    MYNN_LAUNCH((attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, ONCE>), dim3(B * p.Hkv, p.nsplit), dim3(W * 64), lds, s, p);
+    MYNN_LAUNCH((attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, FORM>), dim3(B * p.Hkv, p.nsplit), dim3(W * 64), lds, s, p);
     return launch_status("attn_stream_kernel");
 }
 template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE> static int stream_w(const StreamParams &p, int B, hipStream_t s) {
-    if (stream_eight_waves(p.slice, p.nsplit)) return stream_go<T, D, G, KVI8, PAGED, FUSE, 8, false>(p, B, s);
+    // (eight waves: ranges of 256 keys)
+    if (stream_eight_waves(p.slice, p.nsplit)) return stream_go<T, D, G, KVI8, PAGED, FUSE, 8, kOneTile>(p, B, s);
+    if (p.slice == 4 * kStreamTile) return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, kOneTile>(p, B, s);
     if constexpr (KVI8) {
-        return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, false>(p, B, s);
+        return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, kTiles>(p, B, s);
     } else if constexpr (FUSE) {  // (executors only)
-        return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, true>(p, B, s);
+        return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, kTilesOnce>(p, B, s);
     } else {
-        if (stream_once(p, B, D * sizeof(T))) return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, true>(p, B, s);
-        return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, false>(p, B, s);
+        if (stream_once(p, B, D * sizeof(T))) return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, kTilesOnce>(p, B, s);
+        return stream_go<T, D, G, KVI8, PAGED, FUSE, 4, kTiles>(p, B, s);
     }
 }
 template <typename T, int D, bool KVI8, bool PAGED, bool FUSE>

@@ -24,6 +24,7 @@ def g():
     (2, 16, 4, 2048), (8, 8, 1, 2041),                     # four waves, sixteen ranges
     (4, 8, 4, 2048), (16, 2, 1, 1993), (1, 32, 4, 4090),   # eight waves, eight and more ranges
     (1, 8, 4, 8192), (1, 4, 1, 16300),                     # more than sixteen
+    (17, 16, 8, 1056), (64, 8, 8, 1300),                   # a wave walks several tiles; caches beyond 320 MB (D = 128)
 ])
 def test_ranges(g, dt, kv8, D, B, Hq, Hkv, active):
     import torch
