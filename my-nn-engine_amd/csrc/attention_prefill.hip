@@ -240,7 +240,8 @@ __global__ __launch_bounds__(QW *KW * 64, 2) void attn_prefill_kernel(AttnParams
     // one barrier per tile: behind it the tile is whole and the other stage free
     int t0 = 0, stage = 0;
     auto next = [&]() {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+        // vmcnt(0) lgkmcnt(0): this wave's share of the tile is in LDS, and its reads of the stage that is filled next are through
+        __builtin_amdgcn_s_waitcnt(0x0070);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
