@@ -23,10 +23,10 @@ class MynnError(RuntimeError):
 
 
 def build(jobs=8):
-    """Compiles every HIP source for gfx950 (hipcc cross-compiles without a GPU)."""
+    """Compiles every HIP source for gfx950 (hipcc cross-compiles without a GPU), and the module of host_ops.cpp."""
     import subprocess
 
-    subprocess.check_call(["make", "-C", CSRC, "-j%d" % jobs, "--no-print-directory"])
+    subprocess.check_call(["make", "-C", CSRC, "-j%d" % jobs, "--no-print-directory", "all", "host_ops"])
     return LIB_PATH
 
 
