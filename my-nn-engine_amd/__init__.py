@@ -230,23 +230,42 @@ def _ptr(t):
 _ops = None
 
 
+class _NoHostOps:
+    """In the place of the module where it cannot be had: takes nothing, so that every call goes the long way."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_host_ops():
+    import importlib.machinery
+    import importlib.util
+
+    l = lib()
+    path = os.path.join(_HERE, "lib", "_host_ops.so")
+    loader = importlib.machinery.ExtensionFileLoader("_host_ops", path)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_host_ops", path, loader=loader))
+    loader.exec_module(module)
+    if module.torch_version != _t().__version__.split("+")[0]:
+        raise ImportError("%s was built against torch %s, this is %s" % (path, module.torch_version, _torch.__version__))
+    module.bind(MynnError, *(C.cast(getattr(l, n), _vp).value for n in (
+        "mynn_last_error", "mynn_dequant_matmul", "mynn_quantized_matmul", "mynn_dynamic_quantize_linear", "mynn_attention")))
+    return module
+
+
 def _host_ops():
-    """lib/_host_ops.so, with the addresses of the library's entry points."""
+    """lib/_host_ops.so, with the addresses of the library's entry points.  The kernels are the same without it, so where it is missing or
+    does not load (another torch), that is said once."""
     global _ops
     if _ops is None:
-        import importlib.machinery
-        import importlib.util
+        try:
+            _ops = _load_host_ops()
+        except ImportError as e:
+            import warnings
 
-        l = lib()
-        path = os.path.join(_HERE, "lib", "_host_ops.so")
-        if not os.path.exists(path):
-            raise MynnError("host module not built: %s is missing (run __graft_entry__.build())" % path)
-        loader = importlib.machinery.ExtensionFileLoader("_host_ops", path)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_host_ops", path, loader=loader))
-        loader.exec_module(module)
-        module.bind(MynnError, *(C.cast(getattr(l, n), _vp).value for n in (
-            "mynn_last_error", "mynn_dequant_matmul", "mynn_quantized_matmul", "mynn_dynamic_quantize_linear", "mynn_attention")))
-        _ops = module
+            warnings.warn("my-nn-engine_amd: operator calls go through ctypes, a few microseconds longer each (make -C %s host_ops): %s" % (CSRC, e),
+                          RuntimeWarning, stacklevel=3)
+            _ops = _NoHostOps()
     return _ops
 
 

@@ -9,6 +9,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "../../include/mynn_hip.h"
 
@@ -190,4 +191,9 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host_ops", nullptr, -1, g_metho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_ops(void) { return PyModule_Create(&g_module); }
+PyMODINIT_FUNC PyInit__host_ops(void) {
+    PyObject *m = PyModule_Create(&g_module);
+    // (torch's classes are used as its headers lay them out: a module built against another one is not to be called)
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}

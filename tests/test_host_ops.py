@@ -34,6 +34,50 @@ def test_what_is_not_a_plain_gpu_tensor_is_left_alone():
         ops.bind(mynn.MynnError, 0, 0, 0, 0, 0)
 
 
+def make_nothing(path, monkeypatch):
+    pass
+
+
+def make_garbage(path, monkeypatch):
+    (path / "lib").mkdir()
+    (path / "lib" / "_host_ops.so").write_bytes(b"not a module")
+
+
+def make_one_for_another_torch(path, monkeypatch):
+    (path / "lib").mkdir()
+    import os
+    import shutil
+
+    shutil.copy(os.path.join(mynn._HERE, "lib", "_host_ops.so"), path / "lib" / "_host_ops.so")
+    monkeypatch.setattr(torch, "__version__", "2.3.1+other")
+
+
+@pytest.mark.parametrize("make", [make_nothing, make_garbage, make_one_for_another_torch])
+def test_without_the_module_the_long_way_stays_open(make, tmp_path, monkeypatch):
+    import warnings
+
+    make(tmp_path, monkeypatch)
+    mynn.lib()
+    monkeypatch.setattr(mynn, "_HERE", str(tmp_path))
+    monkeypatch.setattr(mynn, "_ops", None)
+    with pytest.warns(RuntimeWarning, match="ctypes"):
+        ops = mynn._host_ops()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert mynn._host_ops() is ops  # said once
+    assert ops.dequant_matmul(1, 2, 3) is None and ops.attention() is None
+
+
+@pytest.mark.gpu
+def test_operators_work_without_the_module(tmp_path, monkeypatch):
+    w, s = torch.ones((8, 64), dtype=torch.int8, device="cuda"), torch.ones(8, device="cuda")
+    x = torch.ones((2, 64), device="cuda")
+    monkeypatch.setattr(mynn, "_HERE", str(tmp_path))
+    monkeypatch.setattr(mynn, "_ops", None)
+    with pytest.warns(RuntimeWarning, match="ctypes"):
+        assert torch.equal(mynn.dequant_matmul(x, w, s), torch.full((2, 8), 64.0, device="cuda"))
+
+
 @pytest.fixture
 def both(monkeypatch):
     """f -> (its result through the module, its result without)"""
