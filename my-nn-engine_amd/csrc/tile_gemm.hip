@@ -58,14 +58,20 @@ constexpr TgCost kTgI8[] = {
     {128, 256, 1, {6.54f, 6.54f}, {0.509f, 0.509f}, {0.321f, 0.321f}, {0.44f, 0.44f}, {9.0f, 9.0f}, {2.03f, 2.03f}},
 };
 
+static const TgCost *tg_table(int kind, int M, int *n) {
+    *n = kind == TG_W8S ? 3 : kind == TG_W8 ? 7 : 6;
+    return kind == TG_W8S ? kTgW8S : kind == TG_W8 ? kTgW8 : M < 256 ? kTgI8Few : kTgI8;
+}
+
 bool tile_gemm_supported(int kind, int M, int N, int K) {
     return M >= 1 && N >= 1 && K >= 16 && K % (kind == TG_I8 ? 32 : 16) == 0 && (long)K * 256 * 2 < (1l << 31);
 }
 
 // seq: for a plan whose ranges one workgroup takes, which has two sets of sums in its registers
 static TgPlan tg_choose(int kind, int dtype, int M, int N, int K, size_t scratch_bytes, bool seq) {
-    const TgCost *tab = kind == TG_W8S ? kTgW8S : kind == TG_W8 ? kTgW8 : M < 256 ? kTgI8Few : kTgI8;
-    const int n_tiles = kind == TG_W8S ? 3 : kind == TG_W8 ? 7 : 6, d = dtype == MYNN_BF16 ? 1 : 0;
+    int n_tiles;
+    const TgCost *tab = tg_table(kind, M, &n_tiles);
+    const int d = dtype == MYNN_BF16 ? 1 : 0;
     const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
     const double weights_us = (double)N * K / 4.6e6;
     TgPlan best;
@@ -109,8 +115,9 @@ TgPlan tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_b
 }
 
 TgPlan tile_gemm_plan_seq(int kind, int dtype, int M, int N, int K, int ks) {
-    TgPlan plan = tg_remembered(kind, dtype, M, N, K, 0, true);
-    plan.ks = kind == TG_I8 ? 1 : ks;  // (int32 sums are the same in any order)
+    const bool i8 = kind == TG_I8;  // (int32 sums are the same in any order: one range)
+    TgPlan plan = tg_remembered(kind, dtype, M, N, K, 0, !i8);
+    plan.ks = i8 ? 1 : ks;
     plan.seq = plan.ks > 1;
     return plan;
 }
@@ -136,3 +143,36 @@ int tile_gemm(int kind, const TgPlan &plan, void *out, int32_t *acc_out, const v
 }
 
 }  // namespace mynn
+
+// For the tests, and for measuring what the constants above are fitted to; not part of the library's interface.
+// plan[6] = tile, its rows and columns, K ranges, whether one workgroup takes them one after the other, bytes of partial sums.
+// seq_ks > 0: the plan without scratch memory for the sums of seq_ks ranges
+extern "C" int mynn_tile_gemm_plan(int kind, int dtype, int M, int N, int K, size_t scratch_bytes, int seq_ks, long *plan, double *us) {
+    using namespace mynn;
+    MYNN_REQUIRE(plan && kind >= TG_W8 && kind <= TG_I8 && tile_gemm_supported(kind, M, N, K), MYNN_ERR_UNSUPPORTED, "tile_gemm_plan: kind %d, M=%d N=%d K=%d", kind, M, N, K);
+    const TgPlan p = seq_ks > 0 ? tile_gemm_plan_seq(kind, dtype, M, N, K, seq_ks) : tile_gemm_plan(kind, dtype, M, N, K, scratch_bytes);
+    int n;
+    const TgCost &c = tg_table(kind, M, &n)[p.tile];
+    const long v[6] = {p.tile, c.bm, c.bn, p.ks, p.seq, (long)p.part_bytes};
+    for (int i = 0; i < 6; i++) plan[i] = v[i];
+    if (us) *us = p.us;
+    return MYNN_OK;
+}
+// a product by the tile and the ranges given; part, counters (zero): for ranges that workgroups take side by side
+extern "C" int mynn_tile_gemm(int kind, int tile, int ks, int seq, void *out, int32_t *acc_out, const void *act, const int8_t *wq, const void *a_scale, const void *w_scale,
+                              const void *res, int M, int N, int K, int dtype, int epi, void *part, size_t part_bytes, int *counters, mynn_stream s) {
+    using namespace mynn;
+    MYNN_REQUIRE(kind >= TG_W8 && kind <= TG_I8 && tile_gemm_supported(kind, M, N, K), MYNN_ERR_UNSUPPORTED, "tile_gemm: kind %d, M=%d N=%d K=%d", kind, M, N, K);
+    int n;
+    const TgCost *tab = tg_table(kind, M, &n);
+    MYNN_REQUIRE(tile >= 0 && tile < n, MYNN_ERR_INVALID, "tile_gemm: tile %d of %d", tile, n);
+    const long tiles = (long)((M + tab[tile].bm - 1) / tab[tile].bm) * ((N + tab[tile].bn - 1) / tab[tile].bn);
+    const int iters = (K * (kind == TG_I8 ? 1 : 2) + 127) / 128;
+    MYNN_REQUIRE(ks >= 1 && ks <= iters && (ks == 1 || seq || (tiles <= kTgCounters && part_bytes >= (size_t)tiles * ks * tab[tile].bm * tab[tile].bn * 4)),
+                 MYNN_ERR_INVALID, "tile_gemm: %d K ranges of %ld tiles", ks, tiles);
+    TgPlan p;
+    p.tile = tile;
+    p.ks = ks;
+    p.seq = seq != 0 && ks > 1;
+    return tile_gemm(kind, p, out, acc_out, act, wq, a_scale, w_scale, res, M, N, K, dtype, epi, part, counters, as_stream(s));
+}
