@@ -141,18 +141,22 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
     const uint32_t lds0 = lds_offset(lds);
     const char *anext, *bnext;  // the bases of the next step to be requested
     int wanted;                 // its number within the range
+    int whole_steps;            // steps below this one lie within the rows
     uint32_t fill;              // the stage it goes to, in bytes
     auto first_request = [&]() {
+        whole_steps = it0 + n_it == iters ? n_it - 1 : 1 << 30;
         anext = A + (size_t)m0 * a_bytes + (size_t)it0 * 128 - 4096;
         bnext = (const char *)B + (size_t)n0 * K + (size_t)it0 * BROW - 4096;
         wanted = 0;
         fill = 0;
     };
     // A step's loads in two halves, the activations' and the weights'; past the range the last step once more, never read: it
-    // keeps the counts
-    auto request_a = [&]() {
+    // keeps the counts.  at_end: the step may reach past the rows' end.  A lane then picks its address by itself, a dozen instructions a
+    // load, so only the steps from whole_steps on are asked for in that way, by a loop of their own (us a call, all steps in that way / those
+    // alone: int8, 64 x 4330 x 4000 11.6 / 10.3, 33 x 6496 x 6592 15.6 / 12.8; int8 weights, 300 x 5476 x 7456, fp16 59 / 49, bf16 67 / 49).
+    auto request_a = [&](auto at_end) {
         const uint32_t to = lds0 + fill + CHA * wave * 1024;
-        if constexpr (TAIL) {
+        if constexpr (decltype(at_end)::value) {
 #pragma unroll
             for (int i = 0; i < CHA; i++) {
                 const int P = (CHA * wave + i) * 64 + lane;
@@ -163,9 +167,9 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
             if constexpr (CHA > 4) load_group_to_lds<CHA - 4>(anext, aoff + 4, to + 4096);
         }
     };
-    auto request_b = [&]() {
+    auto request_b = [&](auto at_end) {
         const uint32_t to = lds0 + fill + BM * 128 + CHB * wave * 1024;
-        if constexpr (TAIL) {
+        if constexpr (decltype(at_end)::value) {
 #pragma unroll
             for (int i = 0; i < CHB; i++) {
                 const int P = (CHB * wave + i) * 64 + lane, c = BROW == 128 ? (P & 7) ^ ((P >> 4) & 7) : (P & 3) ^ ((P >> 4) & 3);
@@ -180,6 +184,17 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
         bnext += more ? BROW : 0;
         wanted += more ? 1 : 0;
         fill = fill + G::STAGE == NS * G::STAGE ? 0 : fill + G::STAGE;
+    };
+    constexpr std::integral_constant<bool, TAIL> end_too;  // steps of any kind
+    constexpr std::false_type whole_only;
+    auto request = [&]() {
+        if (TAIL && wanted >= whole_steps) {
+            request_a(end_too);
+            request_b(end_too);
+        } else {
+            request_a(whole_only);
+            request_b(whole_only);
+        }
     };
 
     using acc_t = std::conditional_t<I8, i16x_t, f16x_t>;
@@ -256,7 +271,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
         ++it;
     };
     // the step in `now` is multiplied, the one in stage cur read into `next`
-    auto step = [&](const Frags &now, Frags &next, auto first) {
+    auto step = [&](const Frags &now, Frags &next, auto first, auto at_end) {
         if constexpr (decltype(first)::value) meet();
         const char *st = lds + cur;
         auto quarter = [&](auto part) {
@@ -264,8 +279,8 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
             if constexpr (s < 2) {
                 read(st, next, 2 * s);
                 read(st, next, 2 * s + 1);
-            } else if constexpr (s == 2) request_a();
-            else request_b();
+            } else if constexpr (s == 2) request_a(at_end);
+            else request_b(at_end);
             multiply(fb[s & 1], now.a[s]);
 #pragma unroll
             for (int j = 0; j < TJ; j++) fb[(s + 1) & 1][j] = convert(s < 3 ? now.w[(s + 1) & 3][j] : next.w[0][j], j);
@@ -298,28 +313,30 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
     auto one_range_step = [&]() {
         first_request();
 #pragma unroll
-        for (int s = 0; s < AHEAD; s++) {
-            request_a();
-            request_b();
-        }
+        for (int s = 0; s < AHEAD; s++) request();
         cur = 0;
         it = 0;
         Frags f0, f1;
         meet();
 #pragma unroll
         for (int s = 0; s < 4; s++) read(lds, f0, s);
-        request_a();
-        request_b();
+        request();
         advance();
 #pragma unroll
         for (int j = 0; j < TJ; j++) fb[0][j] = convert(f0.w[0][j], j);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (TAIL) {
+            while (it + 1 < n_it && wanted + 1 < whole_steps) {
+                step(f0, f1, second, whole_only);
+                step(f1, f0, whole, whole_only);
+            }
+        }
         while (it + 1 < n_it) {
-            step(f0, f1, second);
-            step(f1, f0, whole);
+            step(f0, f1, second, end_too);
+            step(f1, f0, whole, end_too);
         }
         if (it < n_it) {
-            step(f0, f1, second);
+            step(f0, f1, second, end_too);
             last(f1);
         } else last(f0);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeats of the last step too, before LDS is reused
@@ -343,12 +360,12 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
             for (int j = 0; j < TJ; j++) w[S & 1][j] = *(const w_t *)(st + bbase[S] + j * (32 * BROW));
         };
         const char *st = lds, *nx = lds;  // the stages of this step and of the next
-        auto quarter = [&](auto s, auto request) {
+        auto quarter = [&](auto s, auto half, auto at_end) {
             constexpr int S = decltype(s)::value;
             read_a(S < 3 ? st : nx, std::integral_constant<int, S + 1>{});
             read_w(S < 2 ? st : nx, std::integral_constant<int, S + 2>{});
-            if constexpr (decltype(request)::value == 1) request_a();
-            if constexpr (decltype(request)::value == 2) request_b();
+            if constexpr (decltype(half)::value == 1) request_a(at_end);
+            if constexpr (decltype(half)::value == 2) request_b(at_end);
             multiply(fb[S & 1], a[S & 1]);
 #pragma unroll
             for (int j = 0; j < TJ; j++) fb[(S + 1) & 1][j] = convert(w[(S + 1) & 1][j], j);
@@ -374,10 +391,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
         };
         first_request();
 #pragma unroll
-        for (int s = 0; s < NS - 1; s++) {
-            request_a();
-            request_b();
-        }
+        for (int s = 0; s < NS - 1; s++) request();
         cur = 0;
         it = 0;
         meet_wide(std::integral_constant<int, (NS - 2) * (CHA + CHB)>{});
@@ -387,21 +401,26 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
 #pragma unroll
         for (int j = 0; j < TJ; j++) fb[0][j] = convert(w[0][j], j);
         __builtin_amdgcn_sched_barrier(0);
-        quarter(q0, q0);
-        quarter(q1, q0);
-        for (; it + 1 < n_it; ++it) {
+        quarter(q0, q0, whole_only);
+        quarter(q1, q0, whole_only);
+        auto round = [&](auto at_end) {
             meet_wide(std::integral_constant<int, KEEP>{});
             cur = cur + G::STAGE == NS * G::STAGE ? 0 : cur + G::STAGE;
             nx = lds + cur;
-            quarter(q2, q1);
-            quarter(q3, q2);
+            quarter(q2, q1, at_end);
+            quarter(q3, q2, at_end);
             st = nx;
-            quarter(q0, q0);
-            quarter(q1, q0);
+            quarter(q0, q0, at_end);
+            quarter(q1, q0, at_end);
+            ++it;
+        };
+        if constexpr (TAIL) {
+            while (it + 1 < n_it && wanted < whole_steps) round(whole_only);
         }
+        while (it + 1 < n_it) round(end_too);
         nx = st;  // (reads past the last step stay within it and are not used)
-        quarter(q2, q0);
-        quarter(q3, q0);
+        quarter(q2, q0, whole_only);
+        quarter(q3, q0, whole_only);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     };
