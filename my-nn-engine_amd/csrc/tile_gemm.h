@@ -22,6 +22,8 @@
 // setting of m0 and one scalar base per operand, fragment addresses that need one addition per MFMA step.  fp16, us a call before /
 // now: 300 x 28672 x 4096 115 / 75, 700 x 11264 x 2048 47.5 / 38.5, 500 x 4096 x 14336 81 / 72, 1000 x 28672 x 4096 264 / 236; bf16
 // 500 x 28672 x 4096 156 / 118, 700 x 4096 x 14336 133 / 99.
+// PIN: not in 64 x 64 with one fragment of each operand a wave, where the order the compiler finds is the better one, together with KM = 2
+// (fp16, 300 x 2048 x 2048: pinned 12.8 us a call, KM = 2 12.7, not pinned 12.8, both 11.8; bf16 13.8 / 13.3 / 13.8 / 13.1).
 // KM: the waves meet at a barrier every KM steps; 2 helps where a step is short against the meeting (the eight waves of the int8
 // 64 x 128 tile, 500 x 4096 x 14336: 55.5 -> 50.6 us together with six stages against three).
 //
@@ -44,8 +46,9 @@ namespace mynn {
 typedef int i4x_t __attribute__((ext_vector_type(4)));
 typedef int i16x_t __attribute__((ext_vector_type(16)));
 
-template <int KIND_, int BM_, int BN_, int WM_, int WN_, int NS_, int WPE_, int KM_>
+template <int KIND_, int BM_, int BN_, int WM_, int WN_, int NS_, int WPE_, int KM_, bool PIN_ = true>
 struct TgTile {
+    static constexpr bool PIN = PIN_;
     static constexpr int KIND = KIND_, BM = BM_, BN = BN_, WM = WM_, WN = WN_, NS = NS_, WPE = WPE_, KM = KM_;
     static constexpr int THREADS = WM * WN * 64;
     static constexpr int TI = BM / WM / 32, TJ = BN / WN / 32;
@@ -284,6 +287,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
             multiply(fb[s & 1], now.a[s]);
 #pragma unroll
             for (int j = 0; j < TJ; j++) fb[(s + 1) & 1][j] = convert(s < 3 ? now.w[(s + 1) & 3][j] : next.w[0][j], j);
+            if constexpr (!G::PIN) return;
             constexpr int NM = TI * TJ, RPM = s < 2 ? (2 * (TI + TJ) + NM - 1) / NM : 0, VPM = I8 ? 1 : (std::is_same<T, f16_t>::value ? 16 : 22) / TI;
 #pragma unroll
             for (int n = 0; n < NM; n++) {
@@ -297,6 +301,7 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
         quarter(std::integral_constant<int, 1>{});
         quarter(std::integral_constant<int, 2>{});
         quarter(std::integral_constant<int, 3>{});
+        if constexpr (!G::PIN) __builtin_amdgcn_sched_barrier(0);
         advance();
     };
     auto last = [&](const Frags &now) {

@@ -6,8 +6,7 @@
 namespace mynn {
 
 // ---- which tile, and over how many K ranges.
-// The time of a launch, in microseconds, fitted per tile to measured times of the linear layers of the benchmark's models
-// and others (every tile at 1 .. 16 ranges):
+// The time of a launch, in microseconds, fitted per tile to measured times (every tile at 1 .. 16 ranges):
 //
 //   t = launch + steps per range * (a * rounds + b * workgroups on the fullest CU) + g * further workgroups + e * ranges
 //       + partial sums at 4 TB/s
@@ -17,24 +16,29 @@ namespace mynn {
 // the first adds outside its steps (ramp and store).  Never less than the weights' bytes at 4.6 TB/s or the tiles'
 // operations at the rate the tile keeps up in long launches (padding included).  The constants are those that choose best, not
 // those that predict best (some tiles have a `g` that only says that they are never taken for more than one workgroup per CU).
-// 16-bit activations: choosing by them is 0.5 % above the best of all tiles and ranges on average, over some 280 shapes of
-// 16 .. 8192 rows for each type, 11 % at worst; against the 256-row kernel by its model (gemm.hip) 0.2 %, 5 % at worst; fewer
-// than 16 rows 1 % over 98 shapes, 9 % at worst (profiles/tile_gemm_plans.csv has the shapes).  int8: 1 % above the best measured
-// choice on average, two tables, below and from 256 rows on.  (Two columns where the conversion of the weights costs differ: it
-// is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
+// How well (profiles/tile_gemm_plans.csv: matrices of the benchmark's models and as many others, tests/test_tile_plans.py): from 16 rows
+// on 0.5 % above the best of all tiles and ranges on average over 574 shapes of each type, 14 % at worst; against the 256-row kernel by
+// its model (gemm.hip) within 0.4 % on average, 10 % at worst.  Fewer than 16 rows 2.1 and 2.8 %.  int8 2.3 %, one in 25 more than 15 %:
+// two tables, below and from 256 rows on, fitted to the models' matrices with an earlier form of the loop.  (Two columns where the
+// conversion of the weights costs differ: it is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
+// Of the tiles of fewer than 96 rows, 64 x 128 is the best at 1 in 10 shapes, by up to 13 % (fp16, 97 x 5476 x 7456 33.6 us without it, 29.6
+// with; 255 x 4096 x 4096 22.9 / 19.7; 33 x 14336 x 4096 22.9 / 19.3), 64 x 64 where 32 x 128 and 64 x 128 leave CUs without a workgroup and
+// there is too little K for ranges (300 x 2048 x 2048 12.7 / 11.8).
 struct TgCost {
     int bm, bn, per_cu;  // rows and columns of the tile, workgroups a CU holds
     float launch[2], a[2], b[2], e[2], g[2], rate[2];  // [0] fp16, [1] bf16; rate: 10^9 operations per microsecond
 };
 // (the order of the tiles in tg_launch_w8 and tg_launch_i8)
 constexpr TgCost kTgW8[] = {
-    {32, 64, 3, {3.069f, 3.006f}, {0.215f, 0.274f}, {0.059f, 0.055f}, {0.460f, 0.420f}, {0.0f, 0.0f}, {1.000f, 1.000f}},
-    {32, 128, 3, {2.660f, 2.645f}, {0.150f, 0.245f}, {0.142f, 0.122f}, {0.651f, 0.565f}, {0.0f, 0.0f}, {1.000f, 1.000f}},
-    {96, 128, 2, {3.423f, 3.160f}, {0.068f, 0.070f}, {0.299f, 0.310f}, {1.306f, 1.114f}, {2.393f, 2.507f}, {0.924f, 0.944f}},
-    {128, 128, 1, {3.203f, 2.991f}, {0.349f, 0.310f}, {0.080f, 0.125f}, {1.766f, 1.610f}, {9.206f, 7.137f}, {0.907f, 0.913f}},
-    {160, 128, 1, {3.530f, 3.123f}, {0.346f, 0.470f}, {0.243f, 0.140f}, {1.549f, 1.499f}, {7.907f, 6.479f}, {1.022f, 1.009f}},
-    {128, 256, 1, {4.305f, 4.159f}, {0.540f, 0.537f}, {0.223f, 0.200f}, {1.949f, 3.274f}, {11.418f, 13.552f}, {1.089f, 1.105f}},
-    {160, 256, 1, {5.169f, 3.896f}, {0.591f, 0.780f}, {0.325f, 0.157f}, {2.159f, 2.208f}, {13.363f, 11.788f}, {1.117f, 1.130f}},
+    {32, 64, 3, {4.933f, 3.914f}, {0.155f, 0.274f}, {0.081f, 0.077f}, {0.215f, 0.357f}, {0.000f, 0.000f}, {0.400f, 0.961f}},
+    {32, 128, 3, {4.207f, 3.949f}, {0.164f, 0.311f}, {0.128f, 0.089f}, {0.478f, 0.434f}, {0.524f, 0.865f}, {0.437f, 0.400f}},
+    {64, 64, 2, {4.188f, 4.469f}, {0.140f, 0.201f}, {0.152f, 0.135f}, {0.478f, 0.497f}, {0.000f, 0.023f}, {0.458f, 0.404f}},
+    {64, 128, 2, {4.556f, 4.333f}, {0.185f, 0.194f}, {0.144f, 0.205f}, {1.030f, 1.051f}, {3.900f, 2.375f}, {0.815f, 0.763f}},
+    {96, 128, 2, {4.886f, 4.760f}, {0.033f, 0.241f}, {0.293f, 0.153f}, {1.153f, 1.183f}, {3.844f, 4.341f}, {0.861f, 0.797f}},
+    {128, 128, 1, {5.311f, 5.482f}, {0.370f, 0.406f}, {0.095f, 0.096f}, {1.007f, 0.933f}, {9.915f, 8.754f}, {0.972f, 0.968f}},
+    {160, 128, 1, {5.472f, 6.941f}, {0.398f, 0.427f}, {0.091f, 0.064f}, {2.595f, 1.467f}, {13.523f, 12.953f}, {0.973f, 0.998f}},
+    {128, 256, 1, {6.476f, 7.126f}, {0.488f, 0.242f}, {0.208f, 0.487f}, {2.786f, 3.010f}, {7.963f, 7.300f}, {1.079f, 1.084f}},
+    {160, 256, 1, {8.920f, 9.232f}, {0.821f, 0.221f}, {0.122f, 0.768f}, {1.187f, 0.019f}, {5.301f, 4.490f}, {1.131f, 1.150f}},
 };
 constexpr TgCost kTgW8S[] = {
     {32, 32, 3, {3.394f, 3.360f}, {0.190f, 0.203f}, {0.014f, 0.016f}, {0.504f, 0.503f}, {0.0f, 0.0f}, {0.90f, 0.90f}},
@@ -59,7 +63,7 @@ constexpr TgCost kTgI8[] = {
 };
 
 static const TgCost *tg_table(int kind, int M, int *n) {
-    *n = kind == TG_W8S ? 3 : kind == TG_W8 ? 7 : 6;
+    *n = kind == TG_W8S ? 3 : kind == TG_W8 ? 9 : 6;
     return kind == TG_W8S ? kTgW8S : kind == TG_W8 ? kTgW8 : M < 256 ? kTgI8Few : kTgI8;
 }
 

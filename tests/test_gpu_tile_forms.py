@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 W8, W8S, I8 = 0, 1, 2  # (kernels.h)
 PLAIN, RESIDUAL, PAIRS, PAIRS_EXP = 0, 1, 3, 4
-TILES = {W8: [(32, 64), (32, 128), (96, 128), (128, 128), (160, 128), (128, 256), (160, 256)], W8S: [(32, 32), (32, 64), (32, 128)],
+TILES = {W8: [(32, 64), (32, 128), (64, 64), (64, 128), (96, 128), (128, 128), (160, 128), (128, 256), (160, 256)], W8S: [(32, 32), (32, 64), (32, 128)],
          I8: [(32, 64), (64, 64), (64, 128), (64, 128), (128, 128), (128, 256)]}
 STEP = {W8: 64, W8S: 64, I8: 128}  # values of K in a step
 GRAIN = {W8: 16, W8S: 16, I8: 32}  # K is a multiple of it
@@ -52,7 +52,7 @@ def sizes(kind, tile):
 
 
 @pytest.mark.parametrize("T", ["float16", "bfloat16"])
-@pytest.mark.parametrize("kind,tile", [(W8, t) for t in range(7)] + [(W8S, t) for t in range(3)])
+@pytest.mark.parametrize("kind,tile", [(W8, t) for t in range(9)] + [(W8S, t) for t in range(3)])
 def test_tiles_of_int8_weights(g, T, kind, tile):
     import torch
 

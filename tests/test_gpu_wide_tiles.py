@@ -1,6 +1,6 @@
-"""int8-weight products of 97 and more rows: the tiles of 96 .. 160 rows (tile_gemm.h, the loop that reads less than a K step ahead)
-at rows and columns that do not fill them, fewer K steps than they have stages, rows that are not whole steps, with and without
-K ranges; captured, where a smaller tile takes the ranges one after the other, the same bits."""
+"""int8-weight products of 97 and more rows by the tiles and ranges that their sizes choose: rows and columns that do not fill a tile, few K
+steps, rows that are not whole steps; captured, where a smaller tile may take the ranges one after the other, the same bits.  (Every tile by
+name: test_gpu_tile_forms.py.)"""
 import pytest
 
 import oracle as orc
@@ -17,12 +17,9 @@ def g():
 
 @pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
 @pytest.mark.parametrize("M,N,K", [
-    (97, 11264, 2048), (129, 11250, 1040), (168, 6469, 5792),     # 96 x 128, the last in two ranges
-    (200, 5000, 8208), (1000, 4096, 4096), (127, 28672, 4096),    # 128 x 128, the first in three ranges
-    (300, 11264, 2048), (319, 11001, 1040), (300, 4096, 14336),   # 160 x 128, the last in ranges
-    (481, 11250, 528), (500, 11264, 2048), (321, 15000, 272),     # 128 x 256
-    (640, 15000, 144), (639, 15001, 80), (700, 11264, 2048),      # 160 x 256
-    (640, 15000, 16), (257, 9001, 272), (160, 4090, 14352),
+    (97, 11264, 2048), (129, 11250, 1040), (168, 6469, 5792), (200, 5000, 8208), (1000, 4096, 4096), (127, 28672, 4096), (300, 11264, 2048),
+    (319, 11001, 1040), (300, 4096, 14336), (481, 11250, 528), (500, 11264, 2048), (321, 15000, 272), (640, 15000, 144), (639, 15001, 80),
+    (700, 11264, 2048), (640, 15000, 16), (257, 9001, 272), (160, 4090, 14352),
 ])
 def test_wide_tiles(g, dt, M, N, K):
     import torch
