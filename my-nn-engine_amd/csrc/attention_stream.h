@@ -574,8 +574,10 @@ __global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
     else merge(std::integral_constant<int, 8>{}, std::false_type{});
 }
 
-// Waves of a workgroup, four or eight, from its key range (attn_stream_plan, which makes ranges of 256 rows where eight are wanted)
-inline bool stream_eight_waves(int slice, int nsplit) { return slice == 256 && (nsplit == 1 || nsplit >= 8); }
+// Waves of a workgroup, four or eight, from its key range: attn_stream_plan makes ranges of 256 rows where eight are wanted, one or five
+// and more of them.  Where the pairs of (sequence, kv head) ask for 256 rows anyway, eight waves with a tile each are as fast as four
+// with two or faster (us, four / eight: D = 64, 32 pairs x 1500 keys, int8 cache 8.3 / 7.9; D = 128, 36 x 1500 11.7 / 10.9, 40 x 1100 11.1 / 10.4).
+inline bool stream_eight_waves(int slice, int nsplit) { return slice == 256 && (nsplit == 1 || nsplit >= 5); }
 
 // Whether 16-bit value rows are read as not wanted again (four waves only: eight have little to read).  In an executor's step (the
 // length in device memory) the other layers' caches and weights pass before the same rows are read again; an operator's caches

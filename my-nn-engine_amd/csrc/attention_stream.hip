@@ -79,12 +79,17 @@ void attn_stream_plan(int B, int Hkv, int kv_len, int *slice, int *nsplit) {
     if (n < 1) n = 1;
     int rows = ((kv_len + n - 1) / n + step - 1) / step * step;
     // Eight waves to a workgroup and ranges of twice the length where that leaves nothing to merge, or where four would make so
-    // many ranges that their arrivals and the merge are most of the launch (us of an operator call, four / eight waves: D = 64, 16 x
-    // 250 keys 6.0 / 4.6, 32 x 200 5.9 / 4.5, 4 x 2048 8.8 / 7.6, 1 x 4096 9.6 / 7.5; D = 128, 8 x 250 7.1 / 6.2, 2 x 2048 10.5 / 9.3;
-    // but four ranges against two, 8 x 500, 6.1 / 6.8, eight against four, 4 x 1000, 6.7 / 7.0, and sixteen on half of the
-    // CUs, D = 128, 1 x 2000, 7.8 / 8.2)
+    // many ranges that their arrivals and the merge, beyond eight of them two waits for memory instead of one, are most of the launch:
+    // more than 16, or more than 8 that fill most of the CUs.  Us of an operator call, four / eight waves, fp16, 32 query heads:
+    //   nothing left to merge    D = 64: 16 x 250 keys 6.0 / 4.6, 32 x 200 5.9 / 4.5; D = 128: 8 x 250 7.1 / 6.2; but 8 x 500 6.1 / 6.8
+    //   16 pairs of (sequence, kv head), by keys          1000        1100        1200        1400        1700        1900        2048
+    //     D = 64, 4 kv heads                         7.0 / 7.4   7.7 / 7.4   8.1 / 7.4   8.4 / 7.5   8.6 / 7.6   8.8 / 7.8   9.1 / 7.9
+    //     D = 128, 8 kv heads                        8.0 / 8.7   8.3 / 9.0   8.7 / 8.9   9.2 / 9.1   9.8 / 9.4  10.3 / 9.6  10.7 / 9.6
+    //   8 pairs:  D = 64, 4 kv heads                             7.0 / 7.1   7.0 / 7.2   7.3 / 6.9   7.3 / 7.2   7.6 / 7.1   7.6 / 7.5
+    //     D = 128, 8 kv heads                                    7.8 / 8.3   7.8 / 8.4   7.9 / 8.4   8.1 / 8.7   8.2 / 8.7   8.5 / 8.7
+    //   more than 16 ranges      8 pairs x 3000: D = 64 9.5 / 8.2, D = 128 10.7 / 9.6; 4 pairs x 4000: 9.8 / 7.8, 14.6 / 10.6
     const int ranges = (kv_len + rows - 1) / rows;
-    if (rows == step && ranges > 1 && (ranges == 2 || ranges > 16 || (ranges == 16 && pairs * ranges >= stream_slots()))) rows = 2 * step;
+    if (rows == step && (ranges == 2 || ranges > 16 || (ranges > 8 && pairs * ranges * 8 >= stream_slots() * 5))) rows = 2 * step;
     *slice = rows;
     *nsplit = (kv_len + rows - 1) / rows;
 }

@@ -23,6 +23,7 @@ def g():
     (16, 32, 4, 257), (8, 4, 4, 500), (4, 32, 4, 1000),    # four waves, a few ranges
     (2, 16, 4, 2048), (8, 8, 1, 2041),                     # four waves, sixteen ranges
     (4, 8, 4, 2048), (16, 2, 1, 1993), (1, 32, 4, 4090),   # eight waves, eight and more ranges
+    (4, 32, 4, 1153), (3, 8, 4, 1790), (9, 8, 4, 1500),    # ... and five to seven
     (1, 8, 4, 8192), (1, 4, 1, 16300),                     # more than sixteen
     (17, 16, 8, 1056), (64, 8, 8, 1300),                   # a wave walks several tiles; caches beyond 320 MB (D = 128)
 ])
