@@ -641,19 +641,25 @@ template <typename T, int D> static int pf_go_kv8(const AttnParams &p, hipStream
 //   1 x  300             7.6          6.9          7.1      1 x  128              7.4          6.9          7.0          9.3
 //   1 x  777            14.4         11.2         12.2      1 x  500             15.2         12.1         13.3         15.3
 //   1 x 1200            20.0         15.8         17.8      1 x  777             20.5         18.8         18.2         19.3
-//   1 x 2048            32.9         33.2         32.1      1 x 1200             30.3         34.2         25.8         25.7
+//   1 x 1300            21.3         17.0         18.5      1 x 1200             30.1         34.8         26.3         25.9
+//   1 x 1600            25.5         23.5         23.3      1 x 1300             32.0         38.2         27.9         28.6
+//   1 x 1900            30.4         30.0         28.9      1 x 1600             38.9         47.0         37.4         36.4
+//   1 x 2048            32.8         32.7         32.1      1 x 1900             47.9         61.5         50.4         44.7
 //   2 x  936            17.9         20.1         17.9      1 x 2048             52.1         67.6         53.8         48.7
 //   8 x 1024            56.8         84.4         69.3      2 x  936             27.6         41.8         33.6         32.9
-// (4 x 1 and 32 / 2 x 2 share a CU with a second workgroup.)  Up to 64 rows there is one tile and nothing to split.
+// (4 x 1 and 32 / 2 x 2 share a CU with a second workgroup.)  Beyond 320 workgroups it is the heads that count, as a launch lasts as long
+// as the last rows of one: up to 32 of them (over all sequences) the groups of keys pay, 48 heads x 1100 rows take 4 x 1 (D = 64 20.1 us
+// against 21.0, D = 128 30.1 against 32.1), 40 are a tie.  Up to 64 rows there is one tile and nothing to split.
 template <typename T, int D, bool PAGED> static int pf_pick(const AttnParams &p, hipStream_t s) {
     const long wgs = (long)p.B * p.Hq * ((p.Sq + 127) / 128);
+    const bool few_heads = wgs <= 512 && (long)p.B * p.Hq <= 32;
     if (p.Sq > 64) {
         if constexpr (D == 64) {
-            if (wgs <= 320) return pf_go<T, D, PAGED, 64, 2, 2>(p, s);
+            if (wgs <= 320 || few_heads) return pf_go<T, D, PAGED, 64, 2, 2>(p, s);
         } else {
             if (wgs <= 128) return pf_go<T, D, PAGED, 64, 2, 2>(p, s);
             if (p.Sq > 128 && wgs <= 320) return pf_go<T, D, PAGED, 32, 2, 2>(p, s);
-            if (p.Sq >= 2000 && wgs <= 512) return pf_go<T, D, PAGED, 64, 4, 2>(p, s);
+            if (few_heads) return pf_go<T, D, PAGED, 64, 4, 2>(p, s);
         }
     }
     return pf_go<T, D, PAGED, 64, 4, 1>(p, s);

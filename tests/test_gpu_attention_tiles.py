@@ -46,6 +46,8 @@ def reference(q, k, v, scale, causal, active):
     (5, 32, 8, 128, 161, 30, True),   # 2 x 2, 32 keys: 320 blocks
     (5, 32, 8, 128, 129, 0, False),
     (1, 32, 8, 128, 2001, 30, True),  # 4 x 2: many rows of few heads
+    (1, 32, 8, 128, 1281, 3, True),
+    (1, 32, 8, 64, 1345, 0, True),    # ... and 2 x 2 at D = 64
 ])
 @pytest.mark.parametrize("paged", [False, True])
 def test_tiles(g, dt, B, Hq, Hkv, D, S, past, causal, paged):
