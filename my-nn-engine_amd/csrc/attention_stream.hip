@@ -5,11 +5,11 @@
 namespace mynn {
 
 // (sequences x kv heads x keys) from which the operator takes this kernel instead of the latency kernel of
-// attention_decode.hip.  Latency / streaming, us, 16-bit caches (profiles/attention_routes.md): from 8192 on this one is the
-// faster at every shape measured (D = 64: 16 x 128 keys 6.6 / 6.4, 2 x 1024 12.6 / 7.1, 4 x 2048 20.4 / 9.8; D = 128: 1 x 1024
-// 12.3 / 7.7, 4 x 256 9.3 / 7.8); below it goes either way (4 x 256, D = 64: 6.9 / 7.1; 2 x 256, D = 128: 7.2 / 7.7; but 1 x 1024,
-// D = 64: 10.7 / 6.8).  An executor's fused form, which saves the RoPE + append launch as well, takes this kernel for every
-// batch of two and more whatever the length.
+// attention_decode.hip.  Latency / streaming, us a call, 16-bit caches (profiles/attention_routes.md): from 8192 on this one is the
+// faster at every shape measured (D = 64: 16 x 128 keys 7.2 / 5.2, 2 x 1024 13.0 / 6.7, 4 x 2048 20.5 / 8.3; D = 128: 1 x 1024 12.7 / 7.5,
+// 4 x 256 9.2 / 6.1).  The line was drawn when 4096 went either way; with eight waves and one wait in the merge it does no longer
+// (D = 64, 4 x 256 7.0 / 5.3; D = 128, 2 x 256 7.3 / 6.2, 1 x 512 10.5 / 7.3), and it could come down.  An executor's fused form, which
+// saves the RoPE + append launch as well, takes this kernel for every batch of two and more whatever the length.
 constexpr long kStreamMinKeys = 8192;
 
 // ---- merge of key ranges: out[row, d] = sum_s o_s * exp(m_s - m) / sum_s l_s * exp(m_s - m).

@@ -856,11 +856,12 @@ static int build(Model &m, void **init, void **state) {
                 return;
             }
             pl.plan = tile_gemm_plan(tile_kind, c.dtype, rows_, N, K, kTgScratchMax);
-            // (in the middle of a pass long products run at the power limit, where tiles of int8 weights, which convert what they
-            // multiply, keep up less of the rate that they have on their own: 8 x 1024 rows of the 4096-wide layers 21.8 ms a pass
-            // with them throughout, 20.8 without, though each is predicted within 3 %; 2048 rows of 2048-wide ones, 30 - 110 us
-            // each, gain 9 % by them as predicted)
-            if (tile_kind == TG_W8 && pl.plan.us > 150) pl.plan.us *= 1.06;
+            // (Inside a pass tiles of int8 weights, which convert what they multiply, keep up less of the rate they have on their own than
+            // the kernels of the resident copy do, the more the longer they run.  Over 30 passes -- TinyLlama 1400 .. 8192 rows, 8B layers
+            // 700 .. 4096, both types -- the choice is above the best of all seven rules tried by, on average and at most: as predicted
+            // 1.1 and 4.2 %, 6 % on products beyond 150 us 0.7 and 4.2, 10 % beyond 150 us 0.7 and 4.1, 15 % 1.0 and 6.5, 10 % beyond 80 us
+            // 0.6 and 2.3: bf16 6 x 1000 TinyLlama rows 14.8 ms as predicted, 14.3 with it, fp16 4 x 1024 8B rows 11.2 and 10.8.)
+            if (tile_kind == TG_W8 && pl.plan.us > 80) pl.plan.us *= 1.1;
             const double other = tile_kind == TG_I8 ? qgemm_dma_us(rows_, N, K, swiglu) : gemm_nt_mfma_us(rows_, N, K, c.dtype, swiglu);
             pl.tile = pl.plan.us <= other;
             us_tiles += count * pl.plan.us;
