@@ -41,6 +41,9 @@ __device__ inline const char *scalar_pointer(const char *p) {  // (nothing where
     const uint64_t u = (uint64_t)(uintptr_t)p;
     return (const char *)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(u >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)u));
 }
+// (m0 is a register that the compiler keeps for itself and sets in front of whatever uses it: named as overwritten, which it warns of)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ inline void load_to_lds(const char *base, uint32_t off, uint32_t lds) {
     lds = __builtin_amdgcn_readfirstlane(lds);
     base = scalar_pointer(base);
@@ -69,6 +72,7 @@ template <int N> __device__ inline void load_group_to_lds(const char *base, cons
                      : "memory", "m0");
 #undef MYNN_LOAD
 }
+#pragma clang diagnostic pop
 
 // two f32 -> one dword of two storage-type values (low half first), round to nearest even: one packed
 // convert instruction.  The inputs are values ALREADY rounded to f32 (the empty asm keeps the compiler from
