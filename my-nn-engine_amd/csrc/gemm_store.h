@@ -71,7 +71,7 @@ __device__ __forceinline__ void gemm_store(AccAt at, uint16_t *lds, T *C, const 
             if (row >= M || col >= ldc) continue;
             U4 v = *(const U4 *)&patch[r * EST + cc];
             const size_t at = (size_t)row * ldc + col;
-            if (vec_ok && col + 8 <= ldc) {
+            if (vec_ok) {  // (col, like ldc, is a multiple of 8: all eight lie within the row)
                 if (EPI == GEMM_RESIDUAL) {
                     float fv[8], fr8[8];
                     widen8<T>(v, fv);

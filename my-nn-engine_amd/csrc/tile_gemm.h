@@ -417,12 +417,11 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
             st = nx;
             quarter(q0, q0, at_end);
             quarter(q1, q0, at_end);
-            ++it;
         };
         if constexpr (TAIL) {
-            while (it + 1 < n_it && wanted < whole_steps) round(whole_only);
+            for (; it + 1 < n_it && wanted < whole_steps; ++it) round(whole_only);
         }
-        while (it + 1 < n_it) round(end_too);
+        for (; it + 1 < n_it; ++it) round(end_too);
         nx = st;  // (reads past the last step stay within it and are not used)
         quarter(q2, q0, whole_only);
         quarter(q3, q0, whole_only);

@@ -17,10 +17,11 @@ namespace mynn {
 // operations at the rate the tile keeps up in long launches (padding included).  The constants are those that choose best, not
 // those that predict best (some tiles have a `g` that only says that they are never taken for more than one workgroup per CU).
 // How well (profiles/tile_gemm_plans.csv: matrices of the benchmark's models and as many others, tests/test_tile_plans.py): from 16 rows
-// on 0.5 % above the best of all tiles and ranges on average over 574 shapes of each type, 14 % at worst; against the 256-row kernel by
-// its model (gemm.hip) within 0.4 % on average, 10 % at worst.  Fewer than 16 rows 2.1 and 2.8 %.  int8 2.3 %, one in 25 more than 15 %:
-// two tables, below and from 256 rows on, fitted to the models' matrices with an earlier form of the loop.  (Two columns where the
-// conversion of the weights costs differ: it is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
+// on 0.6 % above the best of all tiles and ranges on average over 660 shapes of each type, 6 % at the 97th percentile, one in 660 more
+// than 15 % (16 and 24 rows of 15871 x 8096, bf16, where two plans meet the line of the weights' bytes, by 20 %).  Fewer than 16 rows 2.1
+// and 2.8 %: launches alone; each further range of a call also costs its host path, so there the older constants stay.  int8 2.3 %, one
+// in 25 more than 15 %: two tables, below and from 256 rows on, fitted to the models' matrices with an earlier form of the loop.  (Two
+// columns where the conversion of the weights costs differ: it is 14 vector operations per 8 fp16 weights, 20 per 8 bf16 weights.)
 // Of the tiles of fewer than 96 rows, 64 x 128 is the best at 1 in 10 shapes, by up to 13 % (fp16, 97 x 5476 x 7456 33.6 us without it, 29.6
 // with; 255 x 4096 x 4096 22.9 / 19.7; 33 x 14336 x 4096 22.9 / 19.3), 64 x 64 where 32 x 128 and 64 x 128 leave CUs without a workgroup and
 // there is too little K for ranges (300 x 2048 x 2048 12.7 / 11.8).
@@ -30,15 +31,15 @@ struct TgCost {
 };
 // (the order of the tiles in tg_launch_w8 and tg_launch_i8)
 constexpr TgCost kTgW8[] = {
-    {32, 64, 3, {4.933f, 3.914f}, {0.155f, 0.274f}, {0.081f, 0.077f}, {0.215f, 0.357f}, {0.000f, 0.000f}, {0.400f, 0.961f}},
-    {32, 128, 3, {4.207f, 3.949f}, {0.164f, 0.311f}, {0.128f, 0.089f}, {0.478f, 0.434f}, {0.524f, 0.865f}, {0.437f, 0.400f}},
-    {64, 64, 2, {4.188f, 4.469f}, {0.140f, 0.201f}, {0.152f, 0.135f}, {0.478f, 0.497f}, {0.000f, 0.023f}, {0.458f, 0.404f}},
-    {64, 128, 2, {4.556f, 4.333f}, {0.185f, 0.194f}, {0.144f, 0.205f}, {1.030f, 1.051f}, {3.900f, 2.375f}, {0.815f, 0.763f}},
-    {96, 128, 2, {4.886f, 4.760f}, {0.033f, 0.241f}, {0.293f, 0.153f}, {1.153f, 1.183f}, {3.844f, 4.341f}, {0.861f, 0.797f}},
-    {128, 128, 1, {5.311f, 5.482f}, {0.370f, 0.406f}, {0.095f, 0.096f}, {1.007f, 0.933f}, {9.915f, 8.754f}, {0.972f, 0.968f}},
-    {160, 128, 1, {5.472f, 6.941f}, {0.398f, 0.427f}, {0.091f, 0.064f}, {2.595f, 1.467f}, {13.523f, 12.953f}, {0.973f, 0.998f}},
-    {128, 256, 1, {6.476f, 7.126f}, {0.488f, 0.242f}, {0.208f, 0.487f}, {2.786f, 3.010f}, {7.963f, 7.300f}, {1.079f, 1.084f}},
-    {160, 256, 1, {8.920f, 9.232f}, {0.821f, 0.221f}, {0.122f, 0.768f}, {1.187f, 0.019f}, {5.301f, 4.490f}, {1.131f, 1.150f}},
+    {32, 64, 3, {4.933f, 3.913f}, {0.155f, 0.274f}, {0.081f, 0.078f}, {0.215f, 0.357f}, {0.000f, 0.000f}, {0.400f, 0.673f}},
+    {32, 128, 3, {4.207f, 3.940f}, {0.164f, 0.311f}, {0.128f, 0.088f}, {0.478f, 0.439f}, {0.524f, 1.596f}, {0.437f, 0.400f}},
+    {64, 64, 2, {4.188f, 4.423f}, {0.140f, 0.200f}, {0.152f, 0.141f}, {0.478f, 0.479f}, {0.000f, 0.000f}, {0.458f, 0.412f}},
+    {64, 128, 2, {4.556f, 4.389f}, {0.185f, 0.195f}, {0.144f, 0.208f}, {1.030f, 1.032f}, {3.900f, 2.289f}, {0.815f, 1.237f}},
+    {96, 128, 2, {4.886f, 5.084f}, {0.033f, 0.239f}, {0.293f, 0.161f}, {1.153f, 1.268f}, {3.844f, 3.201f}, {0.861f, 0.805f}},
+    {128, 128, 1, {5.311f, 5.250f}, {0.370f, 0.391f}, {0.095f, 0.108f}, {1.007f, 1.068f}, {9.915f, 8.787f}, {0.972f, 0.953f}},
+    {160, 128, 1, {5.472f, 6.763f}, {0.398f, 0.468f}, {0.091f, 0.047f}, {2.595f, 1.541f}, {13.523f, 12.223f}, {0.973f, 0.979f}},
+    {128, 256, 1, {6.476f, 5.986f}, {0.488f, 0.307f}, {0.208f, 0.444f}, {2.786f, 3.029f}, {7.963f, 6.760f}, {1.079f, 1.075f}},
+    {160, 256, 1, {8.920f, 9.339f}, {0.821f, 0.251f}, {0.122f, 0.733f}, {1.187f, 0.037f}, {5.301f, 4.901f}, {1.131f, 1.162f}},
 };
 constexpr TgCost kTgW8S[] = {
     {32, 32, 3, {3.394f, 3.360f}, {0.190f, 0.203f}, {0.014f, 0.016f}, {0.504f, 0.503f}, {0.0f, 0.0f}, {0.90f, 0.90f}},
