@@ -55,21 +55,30 @@ __device__ inline void load_to_lds(const char *p, uint32_t lds) {
 }
 
 // N <= 4 of them to consecutive kilobytes of LDS from one setting of m0: load i adds 1024 * i to both of its addresses, so off[i] is
-// 1024 * i short of the distance from base.
-template <int N> __device__ inline void load_group_to_lds(const char *base, const uint32_t *off, uint32_t lds) {
+// 1024 * i short of the distance from base.  NT: with the non-temporal hint, for what is read once.
+template <int N, bool NT = false> __device__ inline void load_group_to_lds(const char *base, const uint32_t *off, uint32_t lds) {
     static_assert(N >= 1 && N <= 4, "the offset has 12 bits");
     lds = __builtin_amdgcn_readfirstlane(lds);
     base = scalar_pointer(base);
-#define MYNN_LOAD(i, o) "\n\tglobal_load_lds_dwordx4 %" #i ", %1 offset:" #o
-    if constexpr (N == 1) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) ::"s"(lds), "s"(base), "v"(off[0]) : "memory", "m0");
-    else if constexpr (N == 2) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) MYNN_LOAD(3, 1024) ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]) : "memory", "m0");
-    else if constexpr (N == 3)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) MYNN_LOAD(3, 1024) MYNN_LOAD(4, 2048) ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2])
+#define MYNN_LOAD(i, o, nt) "\n\tglobal_load_lds_dwordx4 %" #i ", %1 offset:" #o nt
+#define MYNN_GROUP(nt)                                                                                                                                          \
+    if constexpr (N == 1) asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0, nt) ::"s"(lds), "s"(base), "v"(off[0]) : "memory", "m0");                  \
+    else if constexpr (N == 2)                                                                                                                                  \
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0, nt) MYNN_LOAD(3, 1024, nt) ::"s"(lds), "s"(base), "v"(off[0]), "v"(off[1]) : "memory", "m0"); \
+    else if constexpr (N == 3)                                                                                                                                  \
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0, nt) MYNN_LOAD(3, 1024, nt) MYNN_LOAD(4, 2048, nt) ::"s"(lds), "s"(base), "v"(off[0]),       \
+                     "v"(off[1]), "v"(off[2])                                                                                                                   \
+                     : "memory", "m0");                                                                                                                         \
+    else                                                                                                                                                        \
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0, nt) MYNN_LOAD(3, 1024, nt) MYNN_LOAD(4, 2048, nt) MYNN_LOAD(5, 3072, nt) ::"s"(lds),        \
+                     "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3])                                                                              \
                      : "memory", "m0");
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" MYNN_LOAD(2, 0) MYNN_LOAD(3, 1024) MYNN_LOAD(4, 2048) MYNN_LOAD(5, 3072) ::"s"(lds), "s"(base), "v"(off[0]),
-                     "v"(off[1]), "v"(off[2]), "v"(off[3])
-                     : "memory", "m0");
+    if constexpr (NT) {
+        MYNN_GROUP(" nt")
+    } else {
+        MYNN_GROUP("")
+    }
+#undef MYNN_GROUP
 #undef MYNN_LOAD
 }
 #pragma clang diagnostic pop

@@ -2,15 +2,26 @@
 //
 // At this size a linear is a few microseconds, of which skinny.hip's form -- K ranges over workgroups, partial sums through
 // memory, a second launch that adds them up -- spends more on the second launch than on the weights.  Here one workgroup
-// owns 16 .. 64 weight rows (RB row blocks of RH) over the WHOLE K range: its waves split K among themselves, every wave has
-// its share of the weights in flight before the first product, and the partial sums meet in LDS, so the workgroup stores
-// finished output: scale, residual or SwiGLU, and in front the RMSNorm of the activation rows while they are staged (NORM).
+// owns 16 .. 96 weight rows (NB blocks of 16) over the WHOLE K range, its waves share K, and the partial sums meet in LDS, so the
+// workgroup stores finished output: scale, residual or SwiGLU, and in front the RMSNorm of the activation rows (NORM, up to 16 rows).
 //
 //   out[m,n] = T(scale[n] * sum_k act[m,k] * wq[n,k])   (scale after the f32 sum, as skinny.hip)
 //
-// The weights are skinny.hip's tiled copy: a wave's step of 32 rows x 128 k is 4 KB, read by four sequential loads, and
-// turned exactly into the A operand of v_mfma_f32_32x32x16 (or half of it into that of 16x16x32); the activation rows are the
-// B operand's columns, read from LDS.
+// A wave's share of K is its own alone, weights and activations: both go global -> LDS by the load unit into rings that no other
+// wave touches, so up to the final sum nothing is waited for but the wave's own loads, by count.  A step is 64 k: a kilobyte of
+// weights per row block (skinny.hip's tiled copy: 16 rows x 4 pieces of 16 bytes) and a kilobyte of activations per 8 rows (whole 128-byte
+// lines; through registers, as the matrix cores want them, a load would touch half lines of 16 rows, and half the rate came of it).
+// The waves of a workgroup take steps in turn, so that they sweep the copy together.
+//
+// What bounds it: few rows, the weights (4096 x 14336, 8 rows: 12.2 us of which a flat read is 9); many, what a CU gets of the
+// activations, which every workgroup reads in full: some 80 KB a microsecond from the XCD's L2 (that keeps large K with many rows out
+// of this kernel: rowblock_supported).  Against panels of activations for all waves, two in turn behind a barrier each, with the
+// weights in registers, fp16, us: 8 rows, 2048 x 2048 4.3 -> 3.7, 2048 x 5632 6.2 -> 5.6, 4096 x 4096 7.0 -> 5.2, 6144 x 4096 8.7 -> 6.5,
+// 4096 x 14336 14.7 -> 12.2, 11264 x 2048 7.4 -> 6.1; 32 rows, 2048 x 2048 5.4 -> 4.0, 11264 x 2048 9.7 -> 8.4.
+//
+// NORM: a wave squares what it loaded, the waves add up the rows' sums over one barrier, and each normalises its share in place; all of
+// it is in LDS and all weights are in flight in registers meanwhile.  8 rows, 2560 x 2048 5.8 -> 5.0 us, 11264 x 2048 8.2 -> 7.5, 6144 x
+// 4096 10.2 -> 9.7 (with whole rows a wave each, normalised by every workgroup before its first product).
 #include <type_traits>
 
 #include "kernels.h"
@@ -18,258 +29,304 @@
 
 namespace mynn {
 
-// The waves of a workgroup: row blocks times shares of a slab of WK * 128 k (a step per wave) times groups of activation rows.  DEPTH slabs of
-// weights are in flight per wave.  Activations, plain form: panels of SPP slabs, [M] rows, copied global -> LDS by the load
-// unit, the next panel while one is multiplied; NORM > 0: whole rows at once, NORM 16-byte pieces per lane.
-constexpr int kRbMaxRows = 64, kRbDepth = 4;
-// RB row blocks of RH weight rows per workgroup, WK waves that share a slab's K, CG groups of waves with MC tiles of RH
-// activation rows each
-template <int RB_, int RH_, int WK_, int CG_, int MC_, int SPP_> struct RbShape {
-    static constexpr int RB = RB_, RH = RH_, WK = WK_, CG = CG_, MC = MC_, SPP = SPP_, WAVES = RB * WK * CG, ROWS = CG * MC * RH;
-    static constexpr int PANEL = WK * 128 * SPP, ROW_BYTES = (PANEL + 511) / 512 * 1024 + 16;
-    static constexpr int RED = RH + 4;  // floats per row of partial sums
-    static size_t lds(int M, int K, bool norm) {
-        const size_t act = norm ? (size_t)M * (K * 2 + 16) : (size_t)(K > PANEL ? 2 : 1) * M * ROW_BYTES, red = (size_t)WK * RB * M * RED * sizeof(float);
-        return act > red ? act : red;
+constexpr int kRbMaxRows = 64;
+// NB row blocks of 16 per workgroup, A8 groups of 8 activation rows, ND stages of weights, NA stages of activations, WAVES waves
+// (NORM: NA >= the steps of a wave; its weights are in registers, ND = 0)
+template <int NB_, int A8_, int ND_, int NA_, int WAVES_> struct RbShape {
+    static constexpr int NB = NB_, A8 = A8_, ND = ND_, NA = NA_, WAVES = WAVES_, MT = (A8 + 1) / 2;
+    static constexpr int WAVE_BYTES = (ND * NB + NA * A8) * 1024;
+    static constexpr int RED = 16 + 4;  // floats per row of partial sums
+    static constexpr int SQUARES = ND ? 0 : WAVES * A8 * 8 * 4;
+    static size_t lds(int M) {
+        const size_t st = (size_t)WAVES * WAVE_BYTES + SQUARES, red = (size_t)WAVES * NB * M * RED * sizeof(float);
+        return st > red ? st : red;
     }
 };
 
 typedef float f4x_t __attribute__((ext_vector_type(4)));
-template <typename T> __device__ inline f16x_t rb_mfma(const U4 &a, const U4 &b, f16x_t c) { return Mfma<T>::run(a, b, c); }
+// D[16 x 16] += A[16 x 32] . B[32 x 16]: lane l holds row (column) l % 16, k = 8 * (l / 16) .. +7, of D column l % 16, rows 4 * (l / 16) .. +3
 template <typename T> __device__ inline f4x_t rb_mfma(const U4 &a, const U4 &b, f4x_t c) {
     if constexpr (std::is_same<T, f16_t>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, a), __builtin_bit_cast(h8_t, b), c, 0, 0, 0);
     else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8_t, a), __builtin_bit_cast(b8_t, b), c, 0, 0, 0);
 }
 
-template <typename T, typename S, int EPI, int NORM>
-__global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, const T *scale, const T *res, const T *norm_w, T *out,
-                                                                      int M, int N, int K, float eps) {
-    constexpr int RB = S::RB, RH = S::RH, WK = S::WK, MC = S::MC, SPP = S::SPP, WAVES = S::WAVES, DEPTH = kRbDepth, RS = S::RED;
+template <typename T, typename S, int EPI, bool NORM>
+__global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, int M, int N, int K, const T *scale, const T *res,
+                                                                      const T *norm_w, T *out, float eps) {
+    constexpr int NB = S::NB, A8 = S::A8, ND = S::ND, NA = S::NA, MT = S::MT, WAVES = S::WAVES, RS = S::RED;
     extern __shared__ __align__(16) char lds[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane % RH, h = lane / RH, cg = wave / (RB * WK), rb = wave / WK % RB, kw = wave % WK;
-    const int row_blocks = (N + 31) / 32, iters = K / 128, slabs = (iters + WK - 1) / WK;
-    const size_t pitch = (size_t)row_blocks * 256;  // 16-byte pieces of one step over all row blocks
-    // The copy's 16-byte piece of k 64 * a + 16 * j, row i of a block is number 64 * j + 32 * a + i of its step.  A lane of
-    // the 32-row form reads pieces (h, 0 .. 3), of the 16-row form (h % 2, h / 2) and (h % 2, 2 + h / 2).
-    const int block = min((int)blockIdx.x * RB + rb, row_blocks * (32 / RH) - 1);
-    constexpr int LPW = RH / 8;  // loads of a step
-    const U4 *wsrc = pk + (size_t)(block / (32 / RH)) * 256 + (RH == 32 ? lane : (h >> 1) * 64 + (h & 1) * 32 + (block & 1) * 16 + r);
-    U4 w[DEPTH][LPW];
-    auto load_w = [&](int sl, U4 *dst) {
-        const U4 *p = wsrc + (size_t)min(sl * WK + kw, iters - 1) * pitch;
+    const int tid = threadIdx.x, lane = tid & 63, kw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, h = lane >> 4;
+    const int row_blocks = (N + 31) / 32, b0 = (int)blockIdx.x * NB;
+    const int halves = K / 64, n = __builtin_amdgcn_readfirstlane((halves - kw + WAVES - 1) / WAVES);  // steps in all, of this wave
+    char *ring_w = lds + kw * S::WAVE_BYTES, *ring_a = ring_w + ND * NB * 1024;
+    // Addresses of this lane's 16 bytes, as load_group_to_lds takes them, from 4096 bytes in front of a step.  Activations: row 8 * i +
+    // lane / 8, and of its 8 chunks the one that makes the fragment reads below meet different banks.  Weights: row r of the block, piece h
+    // of the step's half of 128 k (the copy's piece of k 64 * a + 16 * j, row i of 32, is number 64 * j + 32 * a + i).
+    uint32_t aoff[A8], woff[NB];
 #pragma unroll
-        for (int j = 0; j < LPW; j++) dst[j] = __builtin_nontemporal_load(p + j * (RH == 32 ? 64 : 128));
+    for (int i = 0; i < A8; i++) {
+        const int row = 8 * i + (lane >> 3);
+        aoff[i] = (uint32_t)(min(row, M - 1) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4) + 4096 - 1024 * (i % 4));
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int block = min(b0 + b, row_blocks * 2 - 1);
+        woff[b] = (uint32_t)((block >> 1) * 4096 + (64 * h + (block & 1) * 16 + r) * 16 + 4096 - 1024 * (b % 4));
+    }
+    // the i-th step of this wave (within the matrix whatever i: a wave without steps of its own asks for the last one's where NORM counts on it)
+    auto half_of = [&](int i) { return min(i * WAVES + kw, halves - 1); };
+    auto step_w = [&](int i) {
+        const int hs = half_of(i);
+        return (const char *)pk + (size_t)(hs >> 1) * row_blocks * 4096 + (hs & 1) * 512 - 4096;
+    };
+    auto request_w = [&](int i, int slot) {
+        const uint32_t to = lds_offset(ring_w) + slot * NB * 1024;
+        load_group_to_lds<(NB < 4 ? NB : 4), true>(step_w(i), woff, to);
+        if constexpr (NB > 4) load_group_to_lds<NB - 4, true>(step_w(i), woff + 4, to + 4096);
+    };
+    auto request_a = [&](int i, int slot) {
+        const char *src = (const char *)act + (size_t)half_of(i) * 128 - 4096;
+        const uint32_t to = lds_offset(ring_a) + slot * A8 * 1024;
+        load_group_to_lds<(A8 < 4 ? A8 : 4)>(src, aoff, to);
+        if constexpr (A8 > 4) load_group_to_lds<A8 - 4>(src, aoff + 4, to + 4096);
+    };
+    auto wait = [&](auto left) {  // until no more than `left` loads are in flight, and all LDS reads are through
+        constexpr int V = decltype(left)::value;
+        static_assert(V < 64, "a counter of six bits");
+        __builtin_amdgcn_s_waitcnt((V & 15) | (V >> 4) << 14 | 0x70);
+        asm volatile("" ::: "memory");
     };
     // what the store of this thread's first output needs (mostly its only one), fetched in front of everything else
-    constexpr int PR = EPI == GEMM_SWIGLU ? RH / 2 : RH;  // outputs per row block and activation row
+    constexpr int PR = EPI == GEMM_SWIGLU ? 8 : 16;  // outputs per row block and activation row
     T sc0, sc1, rs0;
     {
-        const int o = min(tid, RB * M * PR - 1), c = o % PR, m = (o / PR) % M, n = min((((int)blockIdx.x * RB + o / (PR * M)) * RH) + (EPI == GEMM_SWIGLU ? 2 * c : c), N - 1);
-        sc0 = scale[n];
-        if constexpr (EPI == GEMM_SWIGLU) sc1 = scale[min(n + 1, N - 1)];
-        if constexpr (EPI == GEMM_RESIDUAL) rs0 = res[(size_t)m * N + n];
+        const int o = min(tid, NB * M * PR - 1), c = o % PR, m = (o / PR) % M, c0 = min((b0 + o / (PR * M)) * 16 + (EPI == GEMM_SWIGLU ? 2 * c : c), N - 1);
+        sc0 = scale[c0];
+        if constexpr (EPI == GEMM_SWIGLU) sc1 = scale[min(c0 + 1, N - 1)];
+        if constexpr (EPI == GEMM_RESIDUAL) rs0 = res[(size_t)m * N + c0];
     }
-    std::conditional_t<RH == 32, f16x_t, f4x_t> acc[MC];
-    int arow0[MC];  // this lane's activation row of each tile (rows past M repeat the last one and are not stored)
+    f4x_t acc[NB][MT];
 #pragma unroll
-    for (int mc = 0; mc < MC; mc++) {
+    for (int b = 0; b < NB; b++)
 #pragma unroll
-        for (int e = 0; e < RH * RH / 64; e++) acc[mc][e] = 0.f;
-        arow0[mc] = min((cg * MC + mc) * RH + r, M - 1);
-    }
-    auto multiply = [&](const U4 *q, const char *a0, int pitch) {  // a0: the activations at the step's first k
-        U4 b[MC][2 * LPW];
+        for (int t = 0; t < MT; t++) acc[b][t] = f4x_t{0.f, 0.f, 0.f, 0.f};
+    const int fr = A8 == 1 ? r & 7 : r;  // (rows past the loaded ones: columns that are not stored)
+    const int frag = fr * 128, f0 = frag + (((2 * h) ^ (fr & 7)) << 4), f1 = frag + (((2 * h + 1) ^ (fr & 7)) << 4);
+    U4 w[NB], a[MT][2];
+    auto read_a = [&](int slot) {
+        const char *st = ring_a + slot * A8 * 1024;
 #pragma unroll
-        for (int mc = 0; mc < MC; mc++)
+        for (int t = 0; t < MT; t++) {
+            a[t][0] = *(const U4 *)(st + f0 + t * 2048);
+            a[t][1] = *(const U4 *)(st + f1 + t * 2048);
+        }
+    };
+    auto multiply = [&]() {
 #pragma unroll
-            for (int i = 0; i < 2 * LPW; i++)
-                b[mc][i] = *(const U4 *)(a0 + (size_t)arow0[mc] * pitch + (RH == 32 ? 128 * h + 16 * i : 128 * (h & 1) + 32 * (h >> 1) + 64 * (i >> 1) + 16 * (i & 1)));
+        for (int b = 0; b < NB; b++) {
+            const U4 lo = i8x8_to_operand<T>(w[b].x, w[b].y), hi = i8x8_to_operand<T>(w[b].z, w[b].w);
 #pragma unroll
-        for (int i = 0; i < LPW; i++) {
-            U4 c = q[i];
-            pin(c);  // (converted here, not when they were loaded)
-            const U4 lo = i8x8_to_operand<T>(c.x, c.y), hi = i8x8_to_operand<T>(c.z, c.w);
-#pragma unroll
-            for (int mc = 0; mc < MC; mc++) {
-                acc[mc] = rb_mfma<T>(lo, b[mc][2 * i], acc[mc]);
-                acc[mc] = rb_mfma<T>(hi, b[mc][2 * i + 1], acc[mc]);
+            for (int t = 0; t < MT; t++) {
+                acc[b][t] = rb_mfma<T>(lo, a[t][0], acc[b][t]);
+                acc[b][t] = rb_mfma<T>(hi, a[t][1], acc[b][t]);
             }
         }
     };
-    if constexpr (NORM > 0) {
-        // whole rows, a wave each: requested before the weights, as loads return in order
-        const int AS = K * 2 + 16, pieces = K >> 3;
-        for (int m = wave; m < M || m == wave; m += WAVES) {
-            U4 v[NORM], nw[NORM];
-            const int ml = min(m, M - 1);
+    asm volatile("" ::: "memory");  // (the counts below rely on the order of the requests)
+    if constexpr (NORM) {
+        // (steps past the wave's share are the matrix's last one and not used: they keep the counts)
+        U4 nw[NA], wr[NA][NB];
 #pragma unroll
-            for (int q = 0; q < NORM; q++) {
-                const int c = min(lane + q * 64, pieces - 1);
-                v[q] = *(const U4 *)(act + (size_t)ml * K + c * 8);
-                nw[q] = *(const U4 *)(norm_w + c * 8);
+        for (int i = 0; i < NA; i++) nw[i] = *(const U4 *)(norm_w + half_of(i) * 64 + (((lane & 7) ^ (lane >> 3)) << 3));
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < NA; i++) request_a(i, i);
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) wr[i][b] = __builtin_nontemporal_load((const U4 *)(step_w(i) + woff[b] + 1024 * (b % 4)));
+        wait(std::integral_constant<int, (NA * NB < 63 ? NA * NB : 63)>{});
+        float ss[A8];
+#pragma unroll
+        for (int g = 0; g < A8; g++) ss[g] = 0.f;
+        auto mine = [&](int i, int g) { return (U4 *)(ring_a + (i * A8 + g) * 1024 + lane * 16); };  // what this lane loaded
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int g = 0; g < A8; g++) {
+                float f[8], t = 0.f;
+                widen8<T>(*mine(i, g), f);
+#pragma unroll
+                for (int x = 0; x < 8; x++) t += f[x] * f[x];
+                ss[g] += i < n ? t : 0.f;
             }
-            if (m == wave) {
+        float *squares = (float *)(lds + WAVES * S::WAVE_BYTES);  // [wave][row]
 #pragma unroll
-                for (int d = 0; d < DEPTH; d++) load_w(d, w[d]);
-            }
-            if (m >= M) break;
-            float ss = 0.f;
-#pragma unroll
-            for (int q = 0; q < NORM; q++) {
-                float f[8];
-                widen8<T>(v[q], f);
-                if (lane + q * 64 < pieces) {
-#pragma unroll
-                    for (int i = 0; i < 8; i++) ss += f[i] * f[i];
-                }
-            }
-            const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)K + eps);
-#pragma unroll
-            for (int q = 0; q < NORM; q++) {
-                const int c = lane + q * 64;
-                float f[8], g[8];
-                widen8<T>(v[q], f);
-                widen8<T>(nw[q], g);
-                if (c < pieces)
-                    *(U4 *)(lds + (size_t)m * AS + c * 16) = U4{pack2<T>((f[0] * inv) * g[0], (f[1] * inv) * g[1]), pack2<T>((f[2] * inv) * g[2], (f[3] * inv) * g[3]),
-                                                               pack2<T>((f[4] * inv) * g[4], (f[5] * inv) * g[5]), pack2<T>((f[6] * inv) * g[6], (f[7] * inv) * g[7])};
-            }
+        for (int g = 0; g < A8; g++) {
+            ss[g] = group_sum<8>(ss[g]);
+            if ((lane & 7) == 0) squares[kw * 8 * A8 + 8 * g + (lane >> 3)] = ss[g];
         }
         __syncthreads();
-        for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
 #pragma unroll
-            for (int d = 0; d < DEPTH; d++) {
-                const int sl = s0 + d;
-                if (sl * WK + kw < iters) multiply(w[d], lds + (size_t)(sl * WK + kw) * 256, AS);
-                if (s0 + DEPTH < slabs) load_w(sl + DEPTH, w[d]);
-            }
-        }
-    } else {
-        constexpr int PK = S::PANEL, AS = S::ROW_BYTES, CPR = (PK + 511) / 512;  // 1 KB copies per row
-        const int panels = (slabs + SPP - 1) / SPP;
-        auto issue_panel = [&](int p) {
-            char *dst = lds + (size_t)(p & 1) * M * AS;
-            for (int c = wave; c < M * CPR; c += WAVES) {
-                const int m = c / CPR, k = p * PK + (c % CPR) * 512 + lane * 8;
-                if (k - lane * 8 >= K) continue;
-                load_to_lds((const char *)(act + (size_t)m * K + min(k, K - 8)), lds_offset(dst + (size_t)m * AS + (c % CPR) * 1024));
-            }
-        };
-        issue_panel(0);
-        asm volatile("" ::: "memory");  // (the counts below rely on the order of the requests)
-#pragma unroll
-        for (int d = 0; d < DEPTH; d++) load_w(d, w[d]);
-        constexpr int AGE = (SPP < DEPTH ? SPP : DEPTH) * LPW;  // weight loads younger than the panel that is waited for, at least
-        for (int s0 = 0; s0 < slabs; s0 += DEPTH) {
-#pragma unroll
-            for (int d = 0; d < DEPTH; d++) {
-                const int sl = s0 + d;
-                if (sl < slabs) {
-                    if (sl % SPP == 0) {
-                        // this panel is here, everyone is done with the one before it: its buffer takes the next
-                        __builtin_amdgcn_s_waitcnt((AGE & 15) | (AGE >> 4) << 14 | 0x70);
-                        asm volatile("" ::: "memory");
-                        __builtin_amdgcn_s_barrier();
-                        asm volatile("" ::: "memory");
-                        if (sl / SPP + 1 < panels) issue_panel(sl / SPP + 1);
-                        asm volatile("" ::: "memory");
-                    }
-                    if (sl * WK + kw < iters) multiply(w[d], lds + (size_t)((sl / SPP) & 1) * M * AS + (size_t)((sl % SPP) * WK + kw) * 256, AS);
-                }
-                load_w(sl + DEPTH, w[d]);  // (past the end: the last step once more, unused; it keeps the counts)
-            }
-        }
-    }
-    __syncthreads();  // the activations are done with: their memory takes the partial sums
-
-    // D[n][m]: lane holds column m = lane % RH and rows n = 4 * (lane / RH) + e % 4, + 8 * (e / 4) in the 32-row form
-    float *red = (float *)lds;
-#pragma unroll
-    for (int mc = 0; mc < MC; mc++) {
-        const int m = (cg * MC + mc) * RH + r;
-        if (m >= M) continue;
-        float *dst = red + ((size_t)(kw * RB + rb) * M + m) * RS + 4 * h;
-#pragma unroll
-        for (int e4 = 0; e4 < RH * RH / 256; e4++) *(float4 *)(dst + e4 * 8) = float4{acc[mc][e4 * 4], acc[mc][e4 * 4 + 1], acc[mc][e4 * 4 + 2], acc[mc][e4 * 4 + 3]};
-    }
-    __syncthreads();
-    for (int o = tid; o < RB * M * PR; o += WAVES * 64) {
-        const int c = o % PR, m = (o / PR) % M, b = o / (PR * M);
-        const int n0 = ((int)blockIdx.x * RB + b) * RH;
-        const bool first = o == tid;
-        auto total = [&](int n) {
+        for (int g = 0; g < A8; g++) {
             float t = 0.f;
 #pragma unroll
-            for (int k = 0; k < WK; k++) t += red[((size_t)(k * RB + b) * M + m) * RS + n];
+            for (int k = 0; k < WAVES; k++) t += squares[k * 8 * A8 + 8 * g + (lane >> 3)];
+            const float inv = 1.0f / sqrtf(t / (float)K + eps);
+#pragma unroll
+            for (int i = 0; i < NA; i++) {
+                float f[8], q[8];
+                widen8<T>(*mine(i, g), f);
+                widen8<T>(nw[i], q);
+                *mine(i, g) = U4{pack2<T>((f[0] * inv) * q[0], (f[1] * inv) * q[1]), pack2<T>((f[2] * inv) * q[2], (f[3] * inv) * q[3]),
+                                 pack2<T>((f[4] * inv) * q[4], (f[5] * inv) * q[5]), pack2<T>((f[6] * inv) * q[6], (f[7] * inv) * q[7])};
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NA; i++) {
+            if (i >= n) break;
+            read_a(i);
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                w[b] = wr[i][b];
+                pin(w[b]);  // (converted here, not when they were loaded)
+            }
+            multiply();
+        }
+    } else {
+        constexpr int C = A8 + NB;  // loads of a step
+        static_assert(NORM || NA == ND, "one count for both rings");
+        auto request = [&](int i, int slot) {
+            request_w(i, slot);
+            request_a(i, slot);
+        };
+        int i = 0, slot = 0;
+        auto take = [&]() {
+#pragma unroll
+            for (int b = 0; b < NB; b++) w[b] = *(const U4 *)(ring_w + (slot * NB + b) * 1024 + lane * 16);
+            read_a(slot);
+        };
+#pragma unroll
+        for (int d = 0; d < ND - 1; d++)
+            if (d < n) request(d, d);
+        for (; i + ND - 1 < n; i++) {
+            wait(std::integral_constant<int, (ND - 2) * C>{});
+            take();
+            request(i + ND - 1, slot == 0 ? ND - 1 : slot - 1);  // (the stage that the step before was read from)
+            multiply();
+            slot = slot + 1 == ND ? 0 : slot + 1;
+        }
+        // the last ND - 1 steps, with nothing left to ask for
+        auto rest = [&](auto left) {
+            constexpr int L = decltype(left)::value;
+            if constexpr (L < ND) {
+                if (n - i != L) return;
+                wait(std::integral_constant<int, (L - 1) * C>{});
+                take();
+                multiply();
+                slot = slot + 1 == ND ? 0 : slot + 1;
+                i++;
+            }
+        };
+        static_assert(NORM || (ND >= 2 && ND <= 8), "");
+        rest(std::integral_constant<int, 7>{});
+        rest(std::integral_constant<int, 6>{});
+        rest(std::integral_constant<int, 5>{});
+        rest(std::integral_constant<int, 4>{});
+        rest(std::integral_constant<int, 3>{});
+        rest(std::integral_constant<int, 2>{});
+        rest(std::integral_constant<int, 1>{});
+    }
+    __syncthreads();  // the rings are done with: their memory takes the partial sums
+    float *red = (float *)lds;
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            const int m = t * 16 + r;
+            if (m < M) *(float4 *)(red + ((size_t)(kw * NB + b) * M + m) * RS + 4 * h) = float4{acc[b][t][0], acc[b][t][1], acc[b][t][2], acc[b][t][3]};
+        }
+    __syncthreads();
+    for (int o = tid; o < NB * M * PR; o += WAVES * 64) {
+        const int c = o % PR, m = (o / PR) % M, b = o / (PR * M);
+        const int c0 = (b0 + b) * 16;
+        const bool first = o == tid;
+        auto total = [&](int col) {
+            float t = 0.f;
+#pragma unroll
+            for (int k = 0; k < WAVES; k++) t += red[((size_t)(k * NB + b) * M + m) * RS + col];
             return t;
         };
         if constexpr (EPI == GEMM_SWIGLU) {  // rows 2i / 2i+1 of the weight are gate_i / up_i
-            const int n = n0 + 2 * c;
-            if (n + 1 < N) {
-                const T sg = first ? sc0 : scale[n], su = first ? sc1 : scale[n + 1];
+            const int col = c0 + 2 * c;
+            if (col + 1 < N) {
+                const T sg = first ? sc0 : scale[col], su = first ? sc1 : scale[col + 1];
                 const float g = Elem<T>::rnd(total(2 * c) * Elem<T>::ld(&sg, 0)), u = Elem<T>::rnd(total(2 * c + 1) * Elem<T>::ld(&su, 0));
                 const float sig = 1.0f / (1.0f + expf(-g));
-                Elem<T>::st(out, (size_t)m * (N >> 1) + (n >> 1), (g * sig) * u);
+                Elem<T>::st(out, (size_t)m * (N >> 1) + (col >> 1), (g * sig) * u);
             }
         } else {
-            const int n = n0 + c;
-            if (n < N) {
-                const T sn = first ? sc0 : scale[n];
+            const int col = c0 + c;
+            if (col < N) {
+                const T sn = first ? sc0 : scale[col];
                 float y = total(c) * Elem<T>::ld(&sn, 0);
                 if constexpr (EPI == GEMM_RESIDUAL) {
-                    const T rn = first ? rs0 : res[(size_t)m * N + n];
+                    const T rn = first ? rs0 : res[(size_t)m * N + col];
                     y = Elem<T>::rnd(y) + Elem<T>::ld(&rn, 0);
                 }
-                Elem<T>::st(out, (size_t)m * N + n, y);
+                Elem<T>::st(out, (size_t)m * N + col, y);
             }
         }
     }
 }
 
-// ---- which form: as many workgroups as there are CUs and no more, each with whole row blocks.
-// HALF   up to 256 blocks of 16 rows
-// ONE    one block of 32 rows per workgroup while that is at most one per CU (more than 32 activation rows: two of 16)
-// THREE  three blocks of 16 rows, twelve waves, up to 256 such workgroups (16 activation rows; with a norm over more than 2048
-//        values its rows do not fit the registers of twelve waves)
-// TWO    two blocks of 32 rows; from 768 row blocks on skinny.hip's one-launch form streams the weights just as fast
-//        (28672 x 4096, 8 rows: 23 us) and this kernel is not taken
-// 8 rows, us, 32-row forms / HALF or THREE: 2560 x 2048 with norm 7.2 / 6.1, 2048 x 2048 6.3 / 4.9, 2048 x 5632 9.4 / 7.2, 4096 x
-// 14336 18.6 / 14.5, 11264 x 2048 with norm 9.5 / 7.9, 10000 x 4096 12.6 / 11.2; but 6144 x 4096 9.1 / 9.7, 10000 x 4096 with norm
-// 14.1 / 15.9.  24 rows, ONE or TWO / HALF with two tiles of activation rows: 2048 x 2048 6.9 / 5.7, 2048 x 5632 11.0 / 9.0.  48 rows,
-// here / two launches of skinny.hip: 2560 x 2048 7.4 / 12, 2048 x 2048 7.0 / 12, 11264 x 2048 11.5 / 18, 2048 x 5632 13.1 / 12.6.
-// A CU gets some 50 GB/s of weights and 180 GB/s of activations, which every workgroup reads in full: that is what keeps
-// large K with many rows out of this kernel (rowblock_supported).
-// The norm rides along up to 16 rows (8 rows x 2560 x 2048: 7.2 us with it in the ONE form against 6.0 + a launch of 2.5;
-// every workgroup normalises all rows for itself, at 32 rows that costs 3.7 us).
-template <typename F> static auto rb_shape(int M, int N, int K, bool norm, F &&f) {
-    if (N <= 256 * 16) {
-        if (M > 32) return f(RbShape<1, 16, 4, 2, 2, 1>{});
-        if (M > 16) return f(RbShape<1, 16, 8, 1, 2, 1>{});
-        if (norm || K > 8192) return f(RbShape<1, 16, 8, 1, 1, 1>{});  // (4096 x 14336: 14.5 us against 15.4 with two slabs per panel)
-        return f(RbShape<1, 16, 8, 1, 1, 2>{});
-    }
-    if (N <= 256 * 32) return M > 32 ? f(RbShape<2, 16, 4, 1, 4, 1>{}) : f(RbShape<1, 32, 8, 1, 1, 1>{});
-    if (M <= 16 && N <= 256 * 48 && (!norm || K <= 2048)) return f(RbShape<3, 16, 4, 1, 1, 2>{});
-    return M > 32 ? f(RbShape<2, 32, 4, 1, 2, 1>{}) : f(RbShape<2, 32, 4, 1, 1, 2>{});
+// ---- which form: as many row blocks per workgroup as leave one workgroup per CU (its rings take most of the LDS), stages as the
+// 160 KB allow.
+template <bool NORM, typename F> static auto rb_shape(int M, int N, int K, F &&f) {
+    auto rows = [&](auto b) {
+        constexpr int NB = decltype(b)::value;
+        if constexpr (NORM) {
+            if (K <= 2048) return M <= 8 ? f(RbShape<NB, 1, 0, 4, 8>{}) : f(RbShape<NB, 2, 0, 4, 8>{});
+            if constexpr (NB <= 3) return M <= 8 ? f(RbShape<NB, 1, 0, 8, 8>{}) : f(RbShape<NB, 2, 0, 8, 8>{});
+            return f(RbShape<NB, 2, 0, 4, 8>{});  // (refused by rowblock_supported)
+        } else {
+            constexpr int D1 = 20 / (NB + 1) < 8 ? 20 / (NB + 1) : 8, D2 = 20 / (NB + 2), D4 = 20 / (NB + 4);
+            if (M <= 8) return f(RbShape<NB, 1, D1, D1, 8>{});
+            if (M <= 16) return f(RbShape<NB, 2, D2, D2, 8>{});
+            if (M <= 32) return f(RbShape<NB, 4, D4, D4, 8>{});
+            if constexpr (NB <= 2) return f(RbShape<NB, 8, 2, 2, 8>{});
+            else return f(RbShape<NB, 8, 40 / (NB + 8), 40 / (NB + 8), 4>{});  // (a stage of eight waves would be the only one)
+        }
+    };
+    if (N <= 256 * 16) return rows(std::integral_constant<int, 1>{});
+    if (N <= 256 * 32) return rows(std::integral_constant<int, 2>{});
+    if (N <= 256 * 48) return rows(std::integral_constant<int, 3>{});
+    if (N <= 256 * 64) return rows(std::integral_constant<int, 4>{});
+    return rows(std::integral_constant<int, 6>{});
 }
+// From 768 row blocks of 32 on skinny.hip's one-launch form streams the weights just as fast (28672 x 4096, 8 rows: 23 us).
+// More than 16 rows: the activations' bytes keep large K out unless there are many weight rows to use them for.
+// The norm rides along up to 16 rows (it costs 1.0 us for 8 rows x 2048, 2.2 for 16, 2.9 for 8 x 4096, against a launch of 2.5 - 5); over
+// 2048 values with more than 12288 weight rows it would cost 6 (the weights that wait in registers meanwhile).
 bool rowblock_supported(int M, int N, int K, bool norm) {
-    return M >= 1 && M <= kRbMaxRows && (M <= 16 || (long)N * K <= (12l << 20) || (N + 31) / 32 > 256) && K % 128 == 0 && N >= 1 && (N + 31) / 32 < 768 && (!norm || (M <= 16 && K <= 4096)) &&
-           rb_shape(M, N, K, norm, [&](auto s) { return decltype(s)::lds(M, K, norm); }) <= 160 * 1024;
+    return M >= 1 && M <= kRbMaxRows && (M <= 16 || (long)N * K <= (12l << 20) || (N + 31) / 32 > 256) && K % 128 == 0 && N >= 1 && (N + 31) / 32 < 768 &&
+           (long)M * K * 2 < (1l << 31) && (!norm || (M <= 16 && K <= (N <= 256 * 48 ? 4096 : 2048)));
 }
 
-template <typename T, typename S, int EPI, int NORM>
+template <typename T, typename S, int EPI, bool NORM>
 static int rb_go(const void *act, const void *pk, const void *scale, const void *res, const void *norm_w, void *out, int M, int N, int K, float eps,
                  hipStream_t s) {
     static size_t lds_set = 64 * 1024;
-    const size_t lds = S::lds(M, K, NORM > 0);
+    const size_t lds = S::lds(M);
+    static_assert(S::WAVES * S::WAVE_BYTES + S::SQUARES <= 160 * 1024 && S::WAVES * S::NB * S::A8 * 8 * S::RED * 4 <= 160 * 1024, "");
     if (lds > lds_set) {
         MYNN_HIP(hipFuncSetAttribute((const void *)rowblock_gemm_kernel<T, S, EPI, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         lds_set = 160 * 1024;
     }
-    constexpr int rows = S::RB * S::RH;
-    MYNN_LAUNCH((rowblock_gemm_kernel<T, S, EPI, NORM>), dim3((N + rows - 1) / rows), dim3(S::WAVES * 64), lds, s, (const T *)act,
-                (const U4 *)pk, (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, M, N, K, eps);
+    constexpr int rows = S::NB * 16;
+    MYNN_LAUNCH((rowblock_gemm_kernel<T, S, EPI, NORM>), dim3((N + rows - 1) / rows), dim3(S::WAVES * 64), lds, s, (const T *)act, (const U4 *)pk, M, N, K,
+                (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, eps);
     return launch_status("rowblock_gemm_kernel");
 }
 
@@ -280,21 +337,16 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
     MYNN_REQUIRE(aligned16(act) && aligned16(packed) && (!norm_w || aligned16(norm_w)), MYNN_ERR_INVALID, "rowblock_gemm: operands must be 16-byte aligned");
     return dispatch_dtype16(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
-        return rb_shape(M, N, K, norm_w != nullptr, [&](auto shape) {
-            using S = decltype(shape);
-            auto go = [&](auto e) {
-                constexpr int EPI = decltype(e)::value;
-                if constexpr (S::ROWS <= 32 && !(S::ROWS == 32 && S::RH == 16)) {  // (the shapes of up to 16 rows)
-                    if (norm_w && K <= 2048) return rb_go<T, S, EPI, 4>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
-                    if constexpr (S::RB != 3)
-                        if (norm_w) return rb_go<T, S, EPI, 8>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
-                }
-                return rb_go<T, S, EPI, 0>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
-            };
-            if (epi == GEMM_RESIDUAL) return go(std::integral_constant<int, GEMM_RESIDUAL>{});
-            if (epi == GEMM_SWIGLU) return go(std::integral_constant<int, GEMM_SWIGLU>{});
-            return go(std::integral_constant<int, GEMM_PLAIN>{});
-        });
+        auto go = [&](auto norm) {
+            constexpr bool NORM = decltype(norm)::value;
+            return rb_shape<NORM>(M, N, K, [&](auto shape) {
+                using S = decltype(shape);
+                if (epi == GEMM_RESIDUAL) return rb_go<T, S, GEMM_RESIDUAL, NORM>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
+                if (epi == GEMM_SWIGLU) return rb_go<T, S, GEMM_SWIGLU, NORM>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
+                return rb_go<T, S, GEMM_PLAIN, NORM>(act, packed, scale, res, norm_w, out, M, N, K, eps, s);
+            });
+        };
+        return norm_w ? go(std::true_type{}) : go(std::false_type{});
     });
 }
 

@@ -1,0 +1,40 @@
+"""The one-launch linears of decode batches (rowblock.hip) where a wave's steps of 64 k run out: fewer steps than the eight waves, one
+more than they share evenly, fewer and more than the stages of the rings, one to six row blocks per workgroup with a ragged last one,
+one to eight groups of activation rows, with the norm inside and without; against the oracle."""
+import numpy as np
+import pytest
+
+import llm_weights
+import oracle as orc
+from conftest import max_err_rel_to_max
+from test_gpu_decoder import SMALL, dev_weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def g():
+    import gpu_util
+
+    return gpu_util
+
+
+# (K of a linear is hidden or ffn: 128 -> 2 steps, 640 -> 10, 4224 -> 66; the gate/up matrix has 2 ffn rows, the lm_head vocab rows)
+@pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("B", [2, 8, 9, 16, 24, 47])
+@pytest.mark.parametrize("hidden,ffn,vocab", [(128, 128, 300), (640, 4224, 4111), (128, 6272, 12305), (128, 8576, 16401)])
+def test_steps_of_a_wave(g, dt, B, hidden, ffn, vocab):
+    cfg, w = llm_weights.synthetic_int8(dict(SMALL, n_layers=1, hidden=hidden, ffn=ffn, vocab=vocab, n_heads=hidden // 64, n_kv_heads=hidden // 128, head_dim=64), dt, seed=B)
+    dec = g.mynn.Decoder(cfg, dev_weights(g, w, dt), batch=B)
+    rng = np.random.default_rng(B)
+    refs = {b: orc.Model(cfg, w) for b in (0, B - 1)}
+    for step in range(2):
+        toks = rng.integers(0, vocab, B)
+        _, got = dec.step(toks, [step], step, step + 1, want_logits=True)
+        got = got.reshape(B, -1)
+        for b, ref in refs.items():
+            want = ref.forward([toks[b]], [step], step, step + 1, False)
+            # 13 stored values lie between a token and its logits, each up to half a unit of its type off: 13 * 2^-9 of bf16 (one of
+            # 128 hidden values showed 1.2e-2), far less of fp16, which keeps test_gpu_rowblock.py's bound
+            assert max_err_rel_to_max(g.f32(got[b], dt), g.f32(want[0], dt)) <= (1e-2 if dt == orc.F16 else 13 * 2.0**-9), (step, b)
+    dec.close()
