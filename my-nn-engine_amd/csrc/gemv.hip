@@ -168,9 +168,13 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv_kernel(GemvParams p
 // (group g, g + total_waves, ...).  For a group every lane issues all R x NC 16-byte weight loads
 // before the first multiply, dequantises in registers (int8 -> f32 convert + FMA) and the partial
 // sums meet in a wave64 butterfly; the scale is applied after the sum.  NC = ceil(K / 1024).
+// D < NC: only D chunks of each row are in flight, the next is asked for when one is used up: with all of a long row at once the
+// device delivers less (fp16, us, all / D as in gemv1_dispatch: 4096 x 14336 13.4 / 11.9, 8192 x 14000 24.8 / 21.5, 2048 x 9600 7.3 /
+// 6.0, 8192 x 8192 13.5 / 12.7, 4096 x 6000 6.2 / 5.8; bf16 12.6 / 10.8, 21.0 / 19.4, 6.8 / 5.2, 13.1 / 12.7, 6.4 / 5.6; rows of up to
+// 4096 are short enough: 28672 x 4096 19.8 us whatever D).
 // What the first loads need (pointers, sizes) are leading scalar arguments: they arrive preloaded in SGPRs with
 // the wave (-amdgpu-kernarg-preload-count) instead of through a scalar load from the kernarg segment.
-template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false>
+template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false, int D = NC>
 __global__ __launch_bounds__(kGemvThreads) void dequant_gemv1_kernel(const int8_t *wq, const void *act, const void *scale_p, const void *norm_w,
                                                                        const void *residual, int N, int K, int groups,
                                                                        int total_waves, GemvParams p) {
@@ -255,19 +259,18 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv1_kernel(const int8_
     // one row group's operands: R x NC weight chunks per lane, plus, in lane r < R, what the store of row r
     // needs (scale, the next row's scale for SwiGLU, the residual) -- fetched with the weights, not after the sum
     struct Group {
-        U4 w[R][NC];
+        U4 w[R][D];
         T sc, sc1, res;  // as loaded: widening them here would make the wave wait for every load above
     };
     const T *scale = (const T *)scale_p;
+    // (unconditional: the wait for the activation can then be counted exactly; chunks past K are not used)
+    auto load_chunk = [&](int gg, Group &G, int r, int j) {
+        const int row = gg * R + r < N ? gg * R + r : N - 1;
+        G.w[r][j % D] = __builtin_nontemporal_load((const U4 *)(wq + (size_t)row * K) + min(lane + j * kWave, nchunks - 1));
+    };
     auto load_group = [&](int gg, Group &G) {
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int row = gg * R + r < N ? gg * R + r : N - 1;
-            const U4 *wrow = (const U4 *)(wq + (size_t)row * K);
-#pragma unroll
-            for (int j = 0; j < NC; j++)  // (unconditional: the wait for the activation can then be counted exactly;
-                G.w[r][j] = __builtin_nontemporal_load(&wrow[min(lane + j * kWave, nchunks - 1)]);  // chunks past K are not used)
-        }
+        for (int i = 0; i < R * D; i++) load_chunk(gg, G, D == NC ? i / D : i % R, D == NC ? i % D : i / R);
         const int row = min(gg * R + min(lane, R - 1), N - 1);
         G.sc = scale[row];
         if constexpr (EPI == EPI_SWIGLU) G.sc1 = scale[min(row + 1, N - 1)];
@@ -333,7 +336,11 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv1_kernel(const int8_
     T *out = (T *)p.out;
     auto compute = [&](int gg, Group &G) {
         float acc[R];
-        gemv_rows_dot<T, R, NC>(act_lds, K, lane, G.w, acc);
+        if constexpr (D == NC) gemv_rows_dot<T, R, NC>(act_lds, K, lane, G.w, acc);
+        else gemv_rows_dot<T, R, NC, D>(act_lds, K, lane, G.w, acc, [&](int j) {
+#pragma unroll
+            for (int r = 0; r < R; r++) load_chunk(gg, G, r, j);
+        });
 #pragma unroll
         for (int r = 0; r < R; r++) acc[r] = wave_sum(acc[r]);
         const int row0 = gg * R;
@@ -379,7 +386,7 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv1_kernel(const int8_
         }
     }
 }
-template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false>
+template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false, int D = NC>
 static int launch_gemv1(const GemvParams &p, hipStream_t s) {
     const int groups = (p.N + R - 1) / R;
     const int max_waves = 256 * 16;  // four resident waves per SIMD (measured best of 8/12/16/20/24/32 per CU)
@@ -387,7 +394,7 @@ static int launch_gemv1(const GemvParams &p, hipStream_t s) {
     int waves = (groups + passes - 1) / passes;
     const int blocks = (waves + kGemvWaves - 1) / kGemvWaves;
     waves = blocks * kGemvWaves;
-    MYNN_LAUNCH((dequant_gemv1_kernel<T, R, NC, EPI, NORM, ARGMAX>), dim3(blocks + (ARGMAX ? 1 : 0)), dim3(kGemvThreads),
+    MYNN_LAUNCH((dequant_gemv1_kernel<T, R, NC, EPI, NORM, ARGMAX, D>), dim3(blocks + (ARGMAX ? 1 : 0)), dim3(kGemvThreads),
                 (size_t)p.K * sizeof(float), s, p.wq, p.act, p.scale, p.norm_w, p.residual, p.N, p.K, groups, waves, p);
     return launch_status("dequant_gemv1_kernel");
 }
@@ -499,9 +506,9 @@ static int gemv1_dispatch(const GemvParams &p, hipStream_t s) {
     if (nc <= 1) { MYNN_GEMV1(1); }
     if (nc <= 2) { MYNN_GEMV1(2); }
     if (nc <= 4) { MYNN_GEMV1(4); }
-    if (nc <= 6) { MYNN_GEMV1(6); }
-    if (nc <= 8) { MYNN_GEMV1(8); }
-    if (nc <= 14) { MYNN_GEMV1(14); }
+    if (nc <= 6) return launch_gemv1<T, 2, 6, EPI, NORM, false, 3>(p, s);
+    if (nc <= 8) return launch_gemv1<T, 2, 8, EPI, NORM, false, 4>(p, s);
+    if (nc <= 14) return launch_gemv1<T, 2, 14, EPI, NORM, false, 5>(p, s);
 #undef MYNN_GEMV1
     // longer rows: the looping kernel
     if (wide) return launch_gemv<T, T, 4, 1, EPI, NORM>(p, s);

@@ -62,9 +62,13 @@ __device__ inline float gemv_dot16_biased(const U4 &w, const U4 &a0, const U4 &a
     return acc;
 }
 
-// acc[r] = this lane's share of row r: chunks lane, lane + 64, .. of the R rows in w[r][j]
-template <typename T, int R, int NC>
-__device__ __forceinline__ void gemv_rows_dot(const float *lds, int K, int lane, U4 (*w)[NC], float *acc) {
+// acc[r] = this lane's share of row r: chunks lane, lane + 64, .. of the R rows in w[r][j % D]; more(j) asks for chunk j of the rows when
+// the one whose place it takes has been used
+struct GemvNoMore {
+    __device__ void operator()(int) const {}
+};
+template <typename T, int R, int NC, int D = NC, typename More = GemvNoMore>
+__device__ __forceinline__ void gemv_rows_dot(const float *lds, int K, int lane, U4 (*w)[D], float *acc, More more = More()) {
     const int nchunks = K >> 4;
 #pragma unroll
     for (int r = 0; r < R; r++) acc[r] = 0.f;
@@ -81,10 +85,11 @@ __device__ __forceinline__ void gemv_rows_dot(const float *lds, int K, int lane,
                 bias += s.x + s.y;
 #pragma unroll
                 for (int r = 0; r < R; r++) {
-                    pin(w[r][j]);
-                    acc[r] = gemv_dot16_biased(w[r][j], a0, a1, acc[r]);
+                    pin(w[r][j % D]);
+                    acc[r] = gemv_dot16_biased(w[r][j % D], a0, a1, acc[r]);
                 }
             }
+            if (j + D < NC) more(j + D);
         }
 #pragma unroll
         for (int r = 0; r < R; r++) acc[r] -= bias;
@@ -103,12 +108,13 @@ __device__ __forceinline__ void gemv_rows_dot(const float *lds, int K, int lane,
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     float wf[16];
-                    pin(w[r][j]);
-                    widen16_i8(w[r][j], wf);
+                    pin(w[r][j % D]);
+                    widen16_i8(w[r][j % D], wf);
 #pragma unroll
                     for (int i = 0; i < 16; i++) acc[r] = fmaf(a[i], wf[i], acc[r]);
                 }
             }
+            if (j + D < NC) more(j + D);
         }
     }
 }
