@@ -60,6 +60,9 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
 bool rowblock_supported(int M, int N, int K, bool norm);
 int rowblock_gemm(void *out, const void *act, const void *packed, const void *scale, const void *res, const void *norm_w, float eps, int M, int N,
                   int K, int dtype, int epi, hipStream_t s);
+// ... from row-major weights, 2 .. 15 rows (16-bit types)
+bool rowblock_rows_supported(const void *out, const void *act, const void *wq, const void *scale, int M, int N, int K);
+int rowblock_rows_gemm(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, hipStream_t s);
 
 // matrix-core GEMM pieces.  A dequantised weight is [N, Kp] of the 16-bit type, Kp = K rounded up to 64,
 // zero padded (gemm_weight_bytes); dequant_weight_rows writes one (group/which: see gemm.hip), and

@@ -11,7 +11,8 @@
 // wave touches, so up to the final sum nothing is waited for but the wave's own loads, by count.  A step is 64 k: a kilobyte of
 // weights per row block (skinny.hip's tiled copy: 16 rows x 4 pieces of 16 bytes) and a kilobyte of activations per 8 rows (whole 128-byte
 // lines; through registers, as the matrix cores want them, a load would touch half lines of 16 rows, and half the rate came of it).
-// The waves of a workgroup take steps in turn, so that they sweep the copy together.
+// The waves of a workgroup take steps in turn, so that they sweep the copy together.  PACKED false: weights as they are stored, row by row
+// (operator calls), two steps at a time.
 //
 // What bounds it: few rows, the weights (4096 x 14336, 8 rows: 12.2 us of which a flat read is 9); many, what a CU gets of the
 // activations, which every workgroup reads in full: some 80 KB a microsecond from the XCD's L2 (that keeps large K with many rows out
@@ -32,9 +33,11 @@ namespace mynn {
 constexpr int kRbMaxRows = 64;
 // NB row blocks of 16 per workgroup, A8 groups of 8 activation rows, ND stages of weights, NA stages of activations, WAVES waves
 // (NORM: NA >= the steps of a wave; its weights are in registers, ND = 0)
-template <int NB_, int A8_, int ND_, int NA_, int WAVES_> struct RbShape {
+template <int NB_, int A8_, int ND_, int NA_, int WAVES_, bool PACKED_ = true> struct RbShape {
+    static constexpr bool PACKED = PACKED_;
+    static constexpr int H = PACKED ? 1 : 2;  // steps of 64 k that are asked for together
     static constexpr int NB = NB_, A8 = A8_, ND = ND_, NA = NA_, WAVES = WAVES_, MT = (A8 + 1) / 2;
-    static constexpr int WAVE_BYTES = (ND * NB + NA * A8) * 1024;
+    static constexpr int WAVE_BYTES = (ND * NB + NA * A8) * H * 1024;
     static constexpr int RED = 16 + 4;  // floats per row of partial sums
     static constexpr int SQUARES = ND ? 0 : WAVES * A8 * 8 * 4;
     static size_t lds(int M) {
@@ -53,22 +56,29 @@ template <typename T> __device__ inline f4x_t rb_mfma(const U4 &a, const U4 &b, 
 template <typename T, typename S, int EPI, bool NORM>
 __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, int M, int N, int K, const T *scale, const T *res,
                                                                       const T *norm_w, T *out, float eps) {
-    constexpr int NB = S::NB, A8 = S::A8, ND = S::ND, NA = S::NA, MT = S::MT, WAVES = S::WAVES, RS = S::RED;
+    constexpr int NB = S::NB, A8 = S::A8, ND = S::ND, NA = S::NA, MT = S::MT, WAVES = S::WAVES, RS = S::RED, H = S::H;
+    constexpr bool PACKED = S::PACKED;
+    static_assert(PACKED || !NORM, "");
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, kw = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, h = lane >> 4;
     const int row_blocks = (N + 31) / 32, b0 = (int)blockIdx.x * NB;
-    const int halves = K / 64, n = __builtin_amdgcn_readfirstlane((halves - kw + WAVES - 1) / WAVES);  // steps in all, of this wave
-    char *ring_w = lds + kw * S::WAVE_BYTES, *ring_a = ring_w + ND * NB * 1024;
+    const int halves = K / (64 * H), n = __builtin_amdgcn_readfirstlane((halves - kw + WAVES - 1) / WAVES);  // steps in all, of this wave
+    char *ring_w = lds + kw * S::WAVE_BYTES, *ring_a = ring_w + ND * NB * H * 1024;
     // Addresses of this lane's 16 bytes, as load_group_to_lds takes them, from 4096 bytes in front of a step.  Activations: row 8 * i +
     // lane / 8, and of its 8 chunks the one that makes the fragment reads below meet different banks.  Weights: row r of the block, piece h
     // of the step's half of 128 k (the copy's piece of k 64 * a + 16 * j, row i of 32, is number 64 * j + 32 * a + i).
-    uint32_t aoff[A8], woff[NB];
+    uint32_t aoff[A8], woff[NB * H];
 #pragma unroll
     for (int i = 0; i < A8; i++) {
         const int row = 8 * i + (lane >> 3);
         aoff[i] = (uint32_t)(min(row, M - 1) * K * 2 + (((lane & 7) ^ (lane >> 3)) << 4) + 4096 - 1024 * (i % 4));
     }
+    if constexpr (!PACKED) {
+#pragma unroll
+        for (int j = 0; j < NB * H; j++)
+            woff[j] = (uint32_t)(min(8 * j + (lane >> 3), N - 1 - b0 * 16) * K + (((lane & 7) ^ (lane >> 3)) << 4) + 4096 - 1024 * (j % 4));
+    } else
 #pragma unroll
     for (int b = 0; b < NB; b++) {
         const int block = min(b0 + b, row_blocks * 2 - 1);
@@ -78,18 +88,25 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
     auto half_of = [&](int i) { return min(i * WAVES + kw, halves - 1); };
     auto step_w = [&](int i) {
         const int hs = half_of(i);
-        return (const char *)pk + (size_t)(hs >> 1) * row_blocks * 4096 + (hs & 1) * 512 - 4096;
+        if constexpr (!PACKED) return (const char *)pk + (size_t)b0 * 16 * K + (size_t)hs * 128 - 4096;
+        else return (const char *)pk + (size_t)(hs >> 1) * row_blocks * 4096 + (hs & 1) * 512 - 4096;
     };
     auto request_w = [&](int i, int slot) {
-        const uint32_t to = lds_offset(ring_w) + slot * NB * 1024;
-        load_group_to_lds<(NB < 4 ? NB : 4), true>(step_w(i), woff, to);
-        if constexpr (NB > 4) load_group_to_lds<NB - 4, true>(step_w(i), woff + 4, to + 4096);
+        constexpr int L = NB * H;
+        const uint32_t to = lds_offset(ring_w) + slot * L * 1024;
+        const char *src = step_w(i);
+        load_group_to_lds<(L < 4 ? L : 4), true>(src, woff, to);
+        if constexpr (L > 4) load_group_to_lds<(L < 8 ? L - 4 : 4), true>(src, woff + 4, to + 4096);
+        if constexpr (L > 8) load_group_to_lds<L - 8, true>(src, woff + 8, to + 8192);
     };
     auto request_a = [&](int i, int slot) {
-        const char *src = (const char *)act + (size_t)half_of(i) * 128 - 4096;
-        const uint32_t to = lds_offset(ring_a) + slot * A8 * 1024;
-        load_group_to_lds<(A8 < 4 ? A8 : 4)>(src, aoff, to);
-        if constexpr (A8 > 4) load_group_to_lds<A8 - 4>(src, aoff + 4, to + 4096);
+#pragma unroll
+        for (int x = 0; x < H; x++) {
+            const char *src = (const char *)act + (size_t)(half_of(i) * H + x) * 128 - 4096;
+            const uint32_t to = lds_offset(ring_a) + (slot * H + x) * A8 * 1024;
+            load_group_to_lds<(A8 < 4 ? A8 : 4)>(src, aoff, to);
+            if constexpr (A8 > 4) load_group_to_lds<A8 - 4>(src, aoff + 4, to + 4096);
+        }
     };
     auto wait = [&](auto left) {  // until no more than `left` loads are in flight, and all LDS reads are through
         constexpr int V = decltype(left)::value;
@@ -195,26 +212,32 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             multiply();
         }
     } else {
-        constexpr int C = A8 + NB;  // loads of a step
+        constexpr int C = (A8 + NB) * H;  // loads of a step
         static_assert(NORM || NA == ND, "one count for both rings");
         auto request = [&](int i, int slot) {
             request_w(i, slot);
             request_a(i, slot);
         };
         int i = 0, slot = 0;
-        auto take = [&]() {
+        const int wrow = r * 128;  // !PACKED: row r's chunks of 16 bytes, placed as those of the activations
+        auto use = [&](int x) {
 #pragma unroll
-            for (int b = 0; b < NB; b++) w[b] = *(const U4 *)(ring_w + (slot * NB + b) * 1024 + lane * 16);
-            read_a(slot);
+            for (int b = 0; b < NB; b++)
+                w[b] = *(const U4 *)(ring_w + (slot * NB + b) * H * 1024 + (PACKED ? lane * 16 : wrow + (((4 * x + h) ^ (r & 7)) << 4)));
+            read_a(slot * H + x);
         };
 #pragma unroll
         for (int d = 0; d < ND - 1; d++)
             if (d < n) request(d, d);
         for (; i + ND - 1 < n; i++) {
             wait(std::integral_constant<int, (ND - 2) * C>{});
-            take();
+            use(0);
             request(i + ND - 1, slot == 0 ? ND - 1 : slot - 1);  // (the stage that the step before was read from)
             multiply();
+            if constexpr (H > 1) {
+                use(1);
+                multiply();
+            }
             slot = slot + 1 == ND ? 0 : slot + 1;
         }
         // the last ND - 1 steps, with nothing left to ask for
@@ -223,8 +246,12 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             if constexpr (L < ND) {
                 if (n - i != L) return;
                 wait(std::integral_constant<int, (L - 1) * C>{});
-                take();
+                use(0);
                 multiply();
+                if constexpr (H > 1) {
+                    use(1);
+                    multiply();
+                }
                 slot = slot + 1 == ND ? 0 : slot + 1;
                 i++;
             }
@@ -347,6 +374,36 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
             });
         };
         return norm_w ? go(std::true_type{}) : go(std::false_type{});
+    });
+}
+
+// ---- row-major weights, up to 16 rows: stages of 128 k, so that a load touches whole lines of 8 weight rows.  One workgroup per CU up to
+// 12288 weight rows, as above; beyond, workgroups of four waves, two per CU, whose ramps and stores overlap (6 rows, bf16, us, eight waves /
+// four: 14336 x 4096 12.6 with 64 rows each / 12.8 with 32, 15 rows 18.2 with 48 / 14.1 with 32; 28672 x 4096 25.7 with 32 / 22.9 with 64).
+template <typename F> static int rb_rows_shape(int M, int N, F &&f) {
+    auto form = [&](auto b, auto waves) {
+        constexpr int NB = decltype(b)::value, W = decltype(waves)::value, D1 = 20 / (2 * NB + 2), D2 = 20 / (2 * NB + 4);
+        if constexpr (D2 < 2) return f(RbShape<NB, 1, D1, D1, W, false>{});
+        else return M <= 8 ? f(RbShape<NB, 1, D1, D1, W, false>{}) : f(RbShape<NB, 2, D2, D2, W, false>{});
+    };
+    using std::integral_constant;
+    if (N <= 256 * 16) return form(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    if (N <= 256 * 32) return form(integral_constant<int, 2>{}, integral_constant<int, 8>{});
+    if (N <= 256 * 48) return form(integral_constant<int, 3>{}, integral_constant<int, 8>{});
+    if (N <= 512 * 32 || M > 8) return form(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    return form(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+}
+// (one row streams faster through the GEMV, and more than 15 are summed with the scale inside)
+bool rowblock_rows_supported(const void *out, const void *act, const void *wq, const void *scale, int M, int N, int K) {
+    return out && act && wq && scale && M >= 2 && M <= 15 && N >= 1 && K >= 128 && K % 128 == 0 && (long)K * 128 < (1l << 31) && aligned16(act) && aligned16(wq);
+}
+int rowblock_rows_gemm(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, hipStream_t s) {
+    MYNN_REQUIRE(rowblock_rows_supported(out, act, wq, scale, M, N, K), MYNN_ERR_UNSUPPORTED, "rowblock_rows_gemm: M=%d N=%d K=%d", M, N, K);
+    return dispatch_dtype16(dtype, [&](auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        return rb_rows_shape(M, N, [&](auto shape) {
+            return rb_go<T, decltype(shape), GEMM_PLAIN, false>(act, wq, scale, nullptr, nullptr, out, M, N, K, 0.f, s);
+        });
     });
 }
 
