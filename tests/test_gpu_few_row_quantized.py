@@ -1,0 +1,34 @@
+"""QuantizedMatMul of 2 .. 32 rows (qrows.hip): one to four groups of 8 rows, fewer weight rows than a block and ragged blocks of every
+workgroup form, K of fewer steps than waves and of one more than they share evenly; integer sums and outputs, bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def g():
+    import gpu_util
+
+    return gpu_util
+
+
+@pytest.mark.parametrize("dt", [orc.F32, orc.F16, orc.BF16])
+@pytest.mark.parametrize("M", [2, 8, 9, 17, 32])
+@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336)])
+def test_few_rows_int8(g, dt, M, N, K):
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    a, w = rng.integers(-128, 128, (M, K)).astype(np.int8), rng.integers(-128, 128, (N, K)).astype(np.int8)
+    sa, sw = orc.to_storage(rng.uniform(1e-3, 1e-2, M), dt), orc.to_storage(rng.uniform(1e-3, 1e-2, N), dt)
+    da, dw, dsa, dsw = g.to_dev(a), g.to_dev(w), g.to_dev(sa, dt), g.to_dev(sw, dt)
+    out, acc = g.mynn.quantized_matmul(da, dsa, dw, dsw)
+    want = (a.astype(np.float64) @ w.astype(np.float64).T).astype(np.int64)  # (below 2^53: exact)
+    assert np.array_equal(acc.cpu().numpy().astype(np.int64), want)
+    y = (want.astype(np.float32) * g.f32(sa, dt).reshape(M, 1)) * g.f32(sw, dt).reshape(1, N)
+    assert np.array_equal(g.to_host(out).reshape(M, N), orc.to_storage(y, dt).reshape(M, N))
+    alone, none = g.mynn.quantized_matmul(da, dsa, dw, dsw, want_acc=False)
+    assert none is None and torch.equal(alone, out)
