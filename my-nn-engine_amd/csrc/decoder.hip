@@ -320,10 +320,17 @@ static int skinny_rows(Model &m, void *out, const void *act, const Lin &l, const
                                m.cfg.dtype, epi, m.skinny_scratch, m.stream, next_norm, m.cfg.eps, m.nrm, normed, rope, roped);
 }
 
+static int rowblock_product(Model &m, void *out, const void *x, const void *norm_w, const Lin &l, const void *packed, const void *res, int M, int epi,
+                            const char *name) {
+    const double eb = dtype_size(m.cfg.dtype), n_out = epi == GEMM_SWIGLU ? l.N / 2 : l.N;
+    note(m, name, (double)l.N * l.K + l.N * eb + (double)M * l.K * eb + (double)M * n_out * eb * (epi == GEMM_RESIDUAL ? 2 : 1), 2.0 * M * l.N * l.K);
+    return rowblock_gemm(out, x, packed, l.scale, res, norm_w, m.cfg.eps, M, l.N, l.K, m.cfg.dtype, epi, m.stream);
+}
+
 // a linear of a rowblock executor on x, or on its RMSNorm: one launch where the kernel has the form, else norm + product
 static int rowblock_rows(Model &m, void *out, const void *x, const void *norm_w, const Lin &l, const void *packed, const void *res, int M, int epi,
                          const char *name) {
-    const double eb = dtype_size(m.cfg.dtype), n_out = epi == GEMM_SWIGLU ? l.N / 2 : l.N;
+    const double eb = dtype_size(m.cfg.dtype);
     const bool norm_in = norm_w && rowblock_supported(M, l.N, l.K, true);
     if (norm_w && !norm_in) {
         note(m, "rms_norm", 2.0 * M * l.K * eb + l.K * eb);
@@ -331,8 +338,7 @@ static int rowblock_rows(Model &m, void *out, const void *x, const void *norm_w,
         x = m.nrm;
     }
     if (!rowblock_supported(M, l.N, l.K, norm_in)) return skinny_rows(m, out, x, l, packed, res, M, epi, name);
-    note(m, name, (double)l.N * l.K + l.N * eb + (double)M * l.K * eb + (double)M * n_out * eb * (epi == GEMM_RESIDUAL ? 2 : 1), 2.0 * M * l.N * l.K);
-    return rowblock_gemm(out, x, packed, l.scale, res, norm_in ? norm_w : nullptr, m.cfg.eps, M, l.N, l.K, m.cfg.dtype, epi, m.stream);
+    return rowblock_product(m, out, x, norm_in ? norm_w : nullptr, l, packed, res, M, epi, name);
 }
 
 // Options::quantize_activations: DynamicQuantizeLinear (per row, symmetric) then QuantizedMatMul.
@@ -502,7 +508,12 @@ static int enqueue_step(Model &m) {
                 // RoPE and both cache appends (an int8 cache: with its quantiser) ride on the launch that sums the projection's K ranges
                 const SkinnyRope rp{m.q, L.k_cache, L.v_cache, m.cos_t, m.sin_t, m.d_pos, m.d_past, S, Hq, Hkv, D, c.max_seq, m.paging,
                                     kv8 ? L.k_scale : nullptr, kv8 ? L.v_scale : nullptr};
-                TRY(skinny_rows(m, m.qkv, m.nrm, L.qkv, L.pk_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv", nullptr, nullptr,
+                // ... or on the attention, behind a product in one launch: 2 us more there, one launch fewer (us a step, 8 layers of 4096,
+                // 17 / 32 / 48 / 64 sequences, 200 tokens 717 -> 696, 760 -> 741, 988 -> 969, 1054 -> 1037; 2048 tokens 938 -> 914, 1065 -> 1049,
+                // 1486 -> 1450, 1599 -> 1572; int8 caches -1.2 ... -1.8 %; rows of 8192 the other way: 16.4 us with the sums / 17.3)
+                if (m.attn_stream_fuse && L.pk_qkv && H <= 4096 && rowblock_fits(rows, L.qkv.N, H, false))
+                    TRY(rowblock_product(m, m.qkv, m.nrm, nullptr, L.qkv, L.pk_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv"));
+                else TRY(skinny_rows(m, m.qkv, m.nrm, L.qkv, L.pk_qkv, nullptr, rows, GEMM_PLAIN, "linear_qkv", nullptr, nullptr,
                                 (kv8 && D != 64 && D != 128) || streaming || L.qkv_b || c.unfused_decode ? nullptr : &rp, &roped));
             }
             else if (w8a8) TRY(linear_w8a8(m, m.qkv, m.nrm, L.qkv, rows, true, "qlinear_qkv"));

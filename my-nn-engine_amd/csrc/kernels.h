@@ -57,7 +57,8 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
 
 // rowblock.hip -- the same product in one launch, where that is the faster form (packed: skinny_pack_weight's copy); norm_w: of the
 // RMS-normalised rows.  epi: GEMM_PLAIN, GEMM_RESIDUAL, GEMM_SWIGLU (interleaved gate/up rows)
-bool rowblock_supported(int M, int N, int K, bool norm);
+bool rowblock_fits(int M, int N, int K, bool norm);       // the kernel has a form for it
+bool rowblock_supported(int M, int N, int K, bool norm);  // ... which is the one to take
 int rowblock_gemm(void *out, const void *act, const void *packed, const void *scale, const void *res, const void *norm_w, float eps, int M, int N,
                   int K, int dtype, int epi, hipStream_t s);
 // ... from row-major weights, 2 .. 15 rows (16-bit types)

@@ -336,9 +336,11 @@ template <bool NORM, typename F> static auto rb_shape(int M, int N, int K, F &&f
 // More than 16 rows: the activations' bytes keep large K out unless there are many weight rows to use them for.
 // The norm rides along up to 16 rows (it costs 1.0 us for 8 rows x 2048, 2.2 for 16, 2.9 for 8 x 4096, against a launch of 2.5 - 5); over
 // 2048 values with more than 12288 weight rows it would cost 6 (the weights that wait in registers meanwhile).
+bool rowblock_fits(int M, int N, int K, bool norm) {
+    return M >= 1 && M <= kRbMaxRows && K % 128 == 0 && N >= 1 && (N + 31) / 32 < 768 && (long)M * K * 2 < (1l << 31) && (!norm || (M <= 16 && K <= (N <= 256 * 48 ? 4096 : 2048)));
+}
 bool rowblock_supported(int M, int N, int K, bool norm) {
-    return M >= 1 && M <= kRbMaxRows && (M <= 16 || (long)N * K <= (12l << 20) || (N + 31) / 32 > 256) && K % 128 == 0 && N >= 1 && (N + 31) / 32 < 768 &&
-           (long)M * K * 2 < (1l << 31) && (!norm || (M <= 16 && K <= (N <= 256 * 48 ? 4096 : 2048)));
+    return rowblock_fits(M, N, K, norm) && (M <= 16 || (long)N * K <= (12l << 20) || (N + 31) / 32 > 256);
 }
 
 template <typename T, typename S, int EPI, bool NORM>
@@ -360,7 +362,7 @@ static int rb_go(const void *act, const void *pk, const void *scale, const void 
 int rowblock_gemm(void *out, const void *act, const void *packed, const void *scale, const void *res, const void *norm_w, float eps, int M, int N,
                   int K, int dtype, int epi, hipStream_t s) {
     MYNN_REQUIRE(out && act && packed && scale && (epi != GEMM_RESIDUAL || res), MYNN_ERR_INVALID, "rowblock_gemm: null operand");
-    MYNN_REQUIRE(rowblock_supported(M, N, K, norm_w != nullptr) && (epi != GEMM_SWIGLU || N % 2 == 0), MYNN_ERR_UNSUPPORTED, "rowblock_gemm: M=%d N=%d K=%d", M, N, K);
+    MYNN_REQUIRE(rowblock_fits(M, N, K, norm_w != nullptr) && (epi != GEMM_SWIGLU || N % 2 == 0), MYNN_ERR_UNSUPPORTED, "rowblock_gemm: M=%d N=%d K=%d", M, N, K);
     MYNN_REQUIRE(aligned16(act) && aligned16(packed) && (!norm_w || aligned16(norm_w)), MYNN_ERR_INVALID, "rowblock_gemm: operands must be 16-byte aligned");
     return dispatch_dtype16(dtype, [&](auto *t) {
         using T = std::remove_pointer_t<decltype(t)>;
