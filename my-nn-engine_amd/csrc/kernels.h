@@ -64,7 +64,7 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
 // ... from row-major weights, 2 .. 15 rows (16-bit types)
 bool rowblock_rows_supported(const void *out, const void *act, const void *wq, const void *scale, int M, int N, int K);
 int rowblock_rows_gemm(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, hipStream_t s);
-// qrows.hip -- QuantizedMatMul of 2 .. 32 rows in one launch without scratch memory
+// qrows.hip -- QuantizedMatMul of 2 .. 32 rows (narrow matrices 128) in one launch without scratch memory
 bool qrows_supported(int M, int N, int K);
 int qrows_gemm(void *out, int32_t *acc_out, const int8_t *lhs, const void *a_scale, const int8_t *rhs, const void *b_scale, int M, int N, int K, int dtype, hipStream_t s);
 

@@ -4,7 +4,7 @@
 // Replaces quantized_gemv_int8.cuh:13-51 (one 32-lane warp per row, __dp4a) and
 // quantized_matmul_int8.cuh:112-269 (mma.m16n8k32.s8, 3-stage cp.async); CPU twin
 // src/codegen/cpu/kernels/qgemv_i8i8.rs:38-80.
-//   2 .. 32 rows, K % 128 == 0: v_mfma_i32_16x16x64_i8, a stream per wave (qrows.hip)
+//   2 .. 32 rows (narrow matrices 128), K % 128 == 0: v_mfma_i32_16x16x64_i8, a stream per wave (qrows.hip)
 //   M < 3  : wave64 rows, 16 int8 per lane per load, v_dot4_i32_i8, integer butterfly (this file)
 //   else   : v_mfma_i32_32x32x32_i8 with tiles of 32 .. 128 rows (tile_gemm.hip) or 256 (gemm.hip)
 // Integer accumulation is associative, so both are bit-exact whatever the order.

@@ -1,8 +1,8 @@
-// QuantizedMatMul of 2 .. 64 rows, one launch without scratch memory: the streams of rowblock.hip with int8 on both sides.
+// QuantizedMatMul of 2 .. 128 rows, one launch without scratch memory: the streams of rowblock.hip with int8 on both sides.
 //
 //   out[m,n] = T((acc * a_scale[m]) * b_scale[n]), acc = sum_k lhs[m,k] * rhs[n,k] in exact int32 (the order does not matter)
 //
-// A workgroup owns 16 .. 64 rows of rhs over all of K; its waves take steps of 128 k in turn.  A step is 128 bytes of every row, whole lines:
+// A workgroup owns 16 .. 64 rows of rhs and up to 32 of lhs (grid y) over all of K; its waves take steps of 128 k in turn.  A step is 128 bytes of every row, whole lines:
 // both operands go global -> LDS by the load unit into rings that no other wave touches and are waited for by count; nobody meets
 // anybody before the sums of the waves, in LDS at the end.  v_mfma_i32_16x16x64_i8: lane l holds row l % 16, k = 16 * (l / 16) .. +15.
 //
@@ -35,7 +35,9 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, kw = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, h = lane >> 4;
-    const int b0 = (int)blockIdx.x * NB, n0 = b0 * 16;
+    const int b0 = (int)blockIdx.x * NB, n0 = b0 * 16, m0 = (int)blockIdx.y * A8 * 8;
+    lhs += (size_t)m0 * K;
+    M = min(M - m0, A8 * 8);
     const int steps = K / 128, n = __builtin_amdgcn_readfirstlane((steps - kw + WAVES - 1) / WAVES);  // in all, of this wave
     char *ring = lds + kw * ND * S::STAGE;
     // Row 8 * i + lane / 8 of an operand, and of its 8 chunks of 16 bytes the one that makes the fragment reads meet different banks;
@@ -52,8 +54,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
         const uint32_t to = lds_offset(ring) + slot * S::STAGE;
         load_group_to_lds<(NB < 2 ? 2 : 4), true>(w, woff, to);
         if constexpr (NB > 2) load_group_to_lds<2 * NB - 4, true>(w, woff + 4, to + 4096);
-        load_group_to_lds<(A8 < 4 ? A8 : 4)>(a, aoff, to + 2 * NB * 1024);
-        if constexpr (A8 > 4) load_group_to_lds<A8 - 4>(a, aoff + 4, to + 2 * NB * 1024 + 4096);
+        load_group_to_lds<A8>(a, aoff, to + 2 * NB * 1024);
     };
     auto wait = [&](auto left) {  // until no more than `left` loads are in flight, and all LDS reads are through
         constexpr int V = decltype(left)::value;
@@ -133,9 +134,9 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
         int t = 0;
 #pragma unroll
         for (int k = 0; k < WAVES; k++) t += red[((size_t)(k * NB + b) * M + m) * RS + c];
-        const size_t at = (size_t)m * N + col;
+        const size_t at = (size_t)(m0 + m) * N + col;
         if (acc_out) acc_out[at] = t;
-        if (out) Elem<T>::st(out, at, ((float)t * Elem<T>::ld(a_scale, m)) * Elem<T>::ld(b_scale, col));
+        if (out) Elem<T>::st(out, at, ((float)t * Elem<T>::ld(a_scale, m0 + m)) * Elem<T>::ld(b_scale, col));
     }
 }
 
@@ -148,13 +149,14 @@ template <typename F> static int qr_shape(int M, int N, F &&f) {
         return f(QrShape<NB, A8, D < 8 ? D : 8, decltype(waves)::value>{});
     };
     using std::integral_constant;
+    const long cols = (long)N * ((M + 31) / 32);  // (as many workgroups as one group of rows of a matrix so wide)
     auto by_columns = [&](auto groups) {
         constexpr integral_constant<int, 8> eight;
         constexpr integral_constant<int, 4> four;
-        if (N <= 256 * 16) return form(integral_constant<int, 1>{}, eight, groups);
-        if (N <= 256 * 32) return form(integral_constant<int, 2>{}, eight, groups);
-        if (N <= 256 * 48) return form(integral_constant<int, 3>{}, eight, groups);
-        if constexpr (decltype(groups)::value <= 2) return N <= 256 * 64 ? form(four, eight, groups) : form(four, four, groups);
+        if (cols <= 256 * 16) return form(integral_constant<int, 1>{}, eight, groups);
+        if (cols <= 256 * 32) return form(integral_constant<int, 2>{}, eight, groups);
+        if (cols <= 256 * 48) return form(integral_constant<int, 3>{}, eight, groups);
+        if constexpr (decltype(groups)::value <= 2) return cols <= 256 * 64 ? form(four, eight, groups) : form(four, four, groups);
         else return form(integral_constant<int, 2>{}, four, groups);
     };
     if (M <= 8) return by_columns(integral_constant<int, 1>{});
@@ -164,19 +166,23 @@ template <typename F> static int qr_shape(int M, int N, F &&f) {
 template <typename T, typename S>
 static int qr_go(const int8_t *lhs, const int8_t *rhs, const void *a_scale, const void *b_scale, void *out, int32_t *acc_out, int M, int N, int K, hipStream_t s) {
     static size_t lds_set = 64 * 1024;
-    const size_t lds = S::lds(M);
+    const size_t lds = S::lds(M < S::A8 * 8 ? M : S::A8 * 8);
     if (lds > lds_set) {
         MYNN_HIP(hipFuncSetAttribute((const void *)qrows_gemm_kernel<T, S>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         lds_set = 160 * 1024;
     }
-    MYNN_LAUNCH((qrows_gemm_kernel<T, S>), dim3((N + S::NB * 16 - 1) / (S::NB * 16)), dim3(S::WAVES * 64), lds, s, lhs, rhs, M, N, K, (const T *)a_scale,
+    MYNN_LAUNCH((qrows_gemm_kernel<T, S>), dim3((N + S::NB * 16 - 1) / (S::NB * 16), (M + S::A8 * 8 - 1) / (S::A8 * 8)), dim3(S::WAVES * 64), lds, s, lhs, rhs, M, N, K, (const T *)a_scale,
                 (const T *)b_scale, (T *)out, acc_out);
     return launch_status("qrows_gemm_kernel");
 }
 
-// 2 .. 32 rows whose K is whole steps.  More rows: the lhs bytes of every workgroup (64 rows, us, tiles / so: 2048 x 2048 5.6 / 5.6, 4096 x 4096
-// 8.9 / 8.9, 4096 x 14336 18.3 / 22.5).  Two rows of a very wide matrix: the dot products of qmatmul.hip (28672 x 4096 21.5 / 22.6).
-bool qrows_supported(int M, int N, int K) { return M >= 2 && M <= 32 && N >= 1 && K >= 128 && K % 128 == 0 && (M > 2 || N <= 256 * 64); }
+// 2 .. 32 rows whose K is whole steps; two rows of a very wide matrix stay with the dot products of qmatmul.hip (28672 x 4096 21.5 us / 22.6
+// so).  Groups of 32 rows where a narrow matrix leaves CUs for them (us, tiles / so: 40 rows, 2048 x 2048 5.8 / 4.3, 2048 x 5632 8.5 / 7.0; 64 rows 5.8 /
+// 4.4, 9.2 / 7.2, 4096 x 4096 8.7 / 8.4; 97 rows, 2048 x 5632 9.2 / 8.9; but 64 rows, 4096 x 14336 18.3 / 20.0, 97 rows, 4096 x 4096 9.2 / 10.7).
+bool qrows_supported(int M, int N, int K) {
+    if (M < 2 || M > 128 || N < 1 || K < 128 || K % 128 != 0) return false;
+    return M == 2 ? N <= 256 * 64 : M <= 32 || ((long)N * ((M + 31) / 32) <= 256 * 32 && K <= 6144);
+}
 int qrows_gemm(void *out, int32_t *acc_out, const int8_t *lhs, const void *a_scale, const int8_t *rhs, const void *b_scale, int M, int N, int K, int dtype,
                hipStream_t s) {
     MYNN_REQUIRE((out || acc_out) && lhs && rhs && (!out || (a_scale && b_scale)), MYNN_ERR_INVALID, "qrows_gemm: null operand");

@@ -1,4 +1,4 @@
-"""QuantizedMatMul of 2 .. 32 rows (qrows.hip): one to four groups of 8 rows, fewer weight rows than a block and ragged blocks of every
+"""QuantizedMatMul of 2 .. 128 rows (qrows.hip): one to four groups of 8 rows and several of 32, fewer weight rows than a block and ragged blocks of every
 workgroup form, K of fewer steps than waves and of one more than they share evenly; integer sums and outputs, bit for bit."""
 import numpy as np
 import pytest
@@ -16,8 +16,8 @@ def g():
 
 
 @pytest.mark.parametrize("dt", [orc.F32, orc.F16, orc.BF16])
-@pytest.mark.parametrize("M", [2, 8, 9, 17, 32])
-@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336)])
+@pytest.mark.parametrize("M", [2, 8, 9, 17, 32, 33, 65, 128])
+@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336), (2050, 1152)])
 def test_few_rows_int8(g, dt, M, N, K):
     import torch
 
