@@ -61,6 +61,10 @@ bool rowblock_fits(int M, int N, int K, bool norm);       // the kernel has a fo
 bool rowblock_supported(int M, int N, int K, bool norm);  // ... which is the one to take
 int rowblock_gemm(void *out, const void *act, const void *packed, const void *scale, const void *res, const void *norm_w, float eps, int M, int N,
                   int K, int dtype, int epi, hipStream_t s);
+// ... the f32 sums [kRbRanges][M][N] of K ranges, 17 .. 64 rows
+constexpr int kRbRanges = 2;
+bool rowblock_parts_supported(int M, int N, int K);
+int rowblock_parts(float *part, const void *act, const void *packed, int M, int N, int K, int dtype, hipStream_t s);
 // ... from row-major weights, 2 .. 15 rows (16-bit types)
 bool rowblock_rows_supported(const void *out, const void *act, const void *wq, const void *scale, int M, int N, int K);
 int rowblock_rows_gemm(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, hipStream_t s);

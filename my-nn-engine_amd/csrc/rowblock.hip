@@ -53,6 +53,8 @@ template <typename T> __device__ inline f4x_t rb_mfma(const U4 &a, const U4 &b, 
     else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8_t, a), __builtin_bit_cast(b8_t, b), c, 0, 0, 0);
 }
 
+// EPI: the store, GEMM_*, or kRbParts: out is f32 sums [K range][M][N] that another launch adds up and finishes
+constexpr int kRbParts = -1;
 template <typename T, typename S, int EPI, bool NORM>
 __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *act, const U4 *pk, int M, int N, int K, const T *scale, const T *res,
                                                                       const T *norm_w, T *out, float eps) {
@@ -63,7 +65,10 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
     const int tid = threadIdx.x, lane = tid & 63, kw = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, h = lane >> 4;
     const int row_blocks = (N + 31) / 32, b0 = (int)blockIdx.x * NB;
-    const int halves = K / (64 * H), n = __builtin_amdgcn_readfirstlane((halves - kw + WAVES - 1) / WAVES);  // steps in all, of this wave
+    // steps up to the end of this workgroup's K range (PARTS: one of gridDim.y), the range's first, and how many are this wave's
+    constexpr bool PARTS = EPI == kRbParts;
+    const int total = K / (64 * H), halves = PARTS ? total * ((int)blockIdx.y + 1) / (int)gridDim.y : total, first_half = PARTS ? total * (int)blockIdx.y / (int)gridDim.y : 0;
+    const int n = __builtin_amdgcn_readfirstlane(max(halves - first_half - kw + WAVES - 1, 0) / WAVES);
     char *ring_w = lds + kw * S::WAVE_BYTES, *ring_a = ring_w + ND * NB * H * 1024;
     // Addresses of this lane's 16 bytes, as load_group_to_lds takes them, from 4096 bytes in front of a step.  Activations: row 8 * i +
     // lane / 8, and of its 8 chunks the one that makes the fragment reads below meet different banks.  Weights: row r of the block, piece h
@@ -85,7 +90,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
         woff[b] = (uint32_t)((block >> 1) * 4096 + (64 * h + (block & 1) * 16 + r) * 16 + 4096 - 1024 * (b % 4));
     }
     // the i-th step of this wave (within the matrix whatever i: a wave without steps of its own asks for the last one's where NORM counts on it)
-    auto half_of = [&](int i) { return min(i * WAVES + kw, halves - 1); };
+    auto half_of = [&](int i) { return min(first_half + i * WAVES + kw, halves - 1); };
     auto step_w = [&](int i) {
         const int hs = half_of(i);
         if constexpr (!PACKED) return (const char *)pk + (size_t)b0 * 16 * K + (size_t)hs * 128 - 4096;
@@ -117,7 +122,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
     // what the store of this thread's first output needs (mostly its only one), fetched in front of everything else
     constexpr int PR = EPI == GEMM_SWIGLU ? 8 : 16;  // outputs per row block and activation row
     T sc0, sc1, rs0;
-    {
+    if constexpr (!PARTS) {
         const int o = min(tid, NB * M * PR - 1), c = o % PR, m = (o / PR) % M, c0 = min((b0 + o / (PR * M)) * 16 + (EPI == GEMM_SWIGLU ? 2 * c : c), N - 1);
         sc0 = scale[c0];
         if constexpr (EPI == GEMM_SWIGLU) sc1 = scale[min(c0 + 1, N - 1)];
@@ -275,11 +280,25 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             if (m < M) *(float4 *)(red + ((size_t)(kw * NB + b) * M + m) * RS + 4 * h) = float4{acc[b][t][0], acc[b][t][1], acc[b][t][2], acc[b][t][3]};
         }
     __syncthreads();
+    if constexpr (PARTS) {  // (N % 16 == 0)
+        float *part = (float *)out + (size_t)blockIdx.y * M * N;
+        for (int o = tid; o < NB * M * 4; o += WAVES * 64) {
+            const int c = o % 4 * 4, b = (o / 4) % NB, m = o / (4 * NB), col = (b0 + b) * 16 + c;
+            float4 t = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < WAVES; k++) {
+                const float4 v = *(const float4 *)(red + ((size_t)(k * NB + b) * M + m) * RS + c);
+                t.x += v.x, t.y += v.y, t.z += v.z, t.w += v.w;
+            }
+            if (col < N) *(float4 *)(part + (size_t)m * N + col) = t;
+        }
+        return;
+    }
     for (int o = tid; o < NB * M * PR; o += WAVES * 64) {
         const int c = o % PR, m = (o / PR) % M, b = o / (PR * M);
         const int c0 = (b0 + b) * 16;
         const bool first = o == tid;
-        auto total = [&](int col) {
+        auto sum = [&](int col) {
             float t = 0.f;
 #pragma unroll
             for (int k = 0; k < WAVES; k++) t += red[((size_t)(k * NB + b) * M + m) * RS + col];
@@ -289,7 +308,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             const int col = c0 + 2 * c;
             if (col + 1 < N) {
                 const T sg = first ? sc0 : scale[col], su = first ? sc1 : scale[col + 1];
-                const float g = Elem<T>::rnd(total(2 * c) * Elem<T>::ld(&sg, 0)), u = Elem<T>::rnd(total(2 * c + 1) * Elem<T>::ld(&su, 0));
+                const float g = Elem<T>::rnd(sum(2 * c) * Elem<T>::ld(&sg, 0)), u = Elem<T>::rnd(sum(2 * c + 1) * Elem<T>::ld(&su, 0));
                 const float sig = 1.0f / (1.0f + expf(-g));
                 Elem<T>::st(out, (size_t)m * (N >> 1) + (col >> 1), (g * sig) * u);
             }
@@ -297,7 +316,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             const int col = c0 + c;
             if (col < N) {
                 const T sn = first ? sc0 : scale[col];
-                float y = total(c) * Elem<T>::ld(&sn, 0);
+                float y = sum(c) * Elem<T>::ld(&sn, 0);
                 if constexpr (EPI == GEMM_RESIDUAL) {
                     const T rn = first ? rs0 : res[(size_t)m * N + col];
                     y = Elem<T>::rnd(y) + Elem<T>::ld(&rn, 0);
@@ -345,7 +364,7 @@ bool rowblock_supported(int M, int N, int K, bool norm) {
 
 template <typename T, typename S, int EPI, bool NORM>
 static int rb_go(const void *act, const void *pk, const void *scale, const void *res, const void *norm_w, void *out, int M, int N, int K, float eps,
-                 hipStream_t s) {
+                 hipStream_t s, int ranges = 1) {
     static size_t lds_set = 64 * 1024;
     const size_t lds = S::lds(M);
     static_assert(S::WAVES * S::WAVE_BYTES + S::SQUARES <= 160 * 1024 && S::WAVES * S::NB * S::A8 * 8 * S::RED * 4 <= 160 * 1024, "");
@@ -354,7 +373,7 @@ static int rb_go(const void *act, const void *pk, const void *scale, const void 
         lds_set = 160 * 1024;
     }
     constexpr int rows = S::NB * 16;
-    MYNN_LAUNCH((rowblock_gemm_kernel<T, S, EPI, NORM>), dim3((N + rows - 1) / rows), dim3(S::WAVES * 64), lds, s, (const T *)act, (const U4 *)pk, M, N, K,
+    MYNN_LAUNCH((rowblock_gemm_kernel<T, S, EPI, NORM>), dim3((N + rows - 1) / rows, ranges), dim3(S::WAVES * 64), lds, s, (const T *)act, (const U4 *)pk, M, N, K,
                 (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, eps);
     return launch_status("rowblock_gemm_kernel");
 }
@@ -376,6 +395,26 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
             });
         };
         return norm_w ? go(std::true_type{}) : go(std::false_type{});
+    });
+}
+
+// ---- sums of two K ranges for a launch that adds them up (and makes the norm of the row): half of K for twice the weight rows halves what
+// a workgroup reads of the activations.  Against skinny.hip's product of some 1000 waves' ranges, us a pass: TinyLlama, 17 rows 890 / 850, 32
+// rows 943 / 905, 64 rows 1153 / 1102; 8B widths, 8 layers, 64 rows 904 / 886, steps of 48 sequences 991 / 971, of 64 1045 / 1036; but of 32
+// 759 / 770 (4096 x 14336: the bytes of a workgroup again), so up to 32 rows for narrow matrices alone.
+bool rowblock_parts_supported(int M, int N, int K) {
+    return M >= 17 && M <= kRbMaxRows && N <= (M <= 32 ? 256 * 8 : 256 * 16) && N % 16 == 0 && K % 128 == 0 && K >= 4 * 128 && (long)M * K * 2 < (1l << 31);
+}
+int rowblock_parts(float *part, const void *act, const void *packed, int M, int N, int K, int dtype, hipStream_t s) {
+    MYNN_REQUIRE(part && act && packed && rowblock_parts_supported(M, N, K), MYNN_ERR_UNSUPPORTED, "rowblock_parts: M=%d N=%d K=%d", M, N, K);
+    MYNN_REQUIRE(aligned16(act) && aligned16(packed) && aligned16(part), MYNN_ERR_INVALID, "rowblock_parts: operands must be 16-byte aligned");
+    return dispatch_dtype16(dtype, [&](auto *t) {
+        using T = std::remove_pointer_t<decltype(t)>;
+        return rb_shape<false>(M, 2 * N, K, [&](auto shape) {  // (two ranges: as many workgroups as twice the rows)
+            using S = decltype(shape);
+            if constexpr (S::NB <= 2 && S::A8 >= 4) return rb_go<T, S, kRbParts, false>(act, packed, nullptr, nullptr, nullptr, part, M, N, K, 0.f, s, kRbRanges);
+            return (int)MYNN_ERR_UNSUPPORTED;
+        });
     });
 }
 

@@ -357,9 +357,8 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(T *out, const float 
 // with inv = 1 / sqrt(mean(x^2) + eps) over the stored (rounded) x, as the separate operators compute them.
 constexpr int kReduceNormThreads = 1024, kReduceNormMaxSplit = 12;  // (2048 x 5632: 11 ranges)
 template <typename T, int MAXS>
-__global__ __launch_bounds__(kReduceNormThreads) void skinny_reduce_norm_kernel(T *x_out, T *nrm_out, const float *part, const T *scale,
-                                                                              const T *res, const T *norm_w, int M, int N, int ksplit,
-                                                                              float eps) {
+__global__ __launch_bounds__(kReduceNormThreads) void skinny_reduce_norm_kernel(const float *part, int M, int N, int ksplit, const T *scale,
+                                                                              const T *res, const T *norm_w, T *x_out, T *nrm_out, float eps) {
     __shared__ float red[kReduceNormThreads / 64];
     const int m = blockIdx.x, c0 = threadIdx.x * 4;
     const bool live = c0 < N;
@@ -580,19 +579,23 @@ int dequant_gemm_skinny(void *out, const void *act, const int8_t *wq, bool packe
         }
         if (ks_used == 1 && epi == GEMM_SWIGLU) return gemm(std::integral_constant<int, GEMM_SWIGLU>{});
         if (ks_used == 1 && epi == GEMM_PLAIN) return gemm(std::integral_constant<int, GEMM_PLAIN>{});
-        int rc = gemm(std::integral_constant<int, -1>{});
+        const bool residual_norm = epi == GEMM_RESIDUAL && norm_w && nrm_out && normed && N % 4 == 0 && N <= 4 * kReduceNormThreads &&
+                                   ks_used <= kReduceNormMaxSplit && aligned16(out) && aligned16(res) && aligned16(nrm_out) && ((uintptr_t)norm_w & 7) == 0 &&
+                                   ((uintptr_t)scale & 7) == 0;
+        const bool two = residual_norm && packed && ks_used >= kRbRanges && rowblock_parts_supported(M, N, K);
+        int rc = two ? rowblock_parts(scratch, act, wq, M, N, K, dtype, s) : gemm(std::integral_constant<int, -1>{});
         if (rc) return rc;
+        const int ranges = two ? kRbRanges : ks_used;
         auto by_split = [&](auto f) {  // (loads past the last range repeat it: as few of those as a choice of three leaves)
-            if (ks_used <= 4) f(std::integral_constant<int, 4>{});
+            if (ranges <= 2) f(std::integral_constant<int, 2>{});
+            else if (ks_used <= 4) f(std::integral_constant<int, 4>{});
             else if (ks_used <= 8) f(std::integral_constant<int, 8>{});
             else f(std::integral_constant<int, kReduceNormMaxSplit>{});
         };
-        if (epi == GEMM_RESIDUAL && norm_w && nrm_out && normed && N % 4 == 0 && N <= 4 * kReduceNormThreads &&
-            ks_used <= kReduceNormMaxSplit && aligned16(out) && aligned16(res) && aligned16(nrm_out) && ((uintptr_t)norm_w & 7) == 0 &&
-            ((uintptr_t)scale & 7) == 0) {
+        if (residual_norm) {
             by_split([&](auto most) {
-                MYNN_LAUNCH((skinny_reduce_norm_kernel<T, decltype(most)::value>), dim3(M), dim3(kReduceNormThreads), 0, s, (T *)out, (T *)nrm_out, scratch,
-                            (const T *)scale, (const T *)res, (const T *)norm_w, M, N, ks_used, eps);
+                MYNN_LAUNCH((skinny_reduce_norm_kernel<T, decltype(most)::value>), dim3(M), dim3(kReduceNormThreads), 0, s, scratch, M, N, ranges,
+                            (const T *)scale, (const T *)res, (const T *)norm_w, (T *)out, (T *)nrm_out, eps);
             });
             *normed = true;
             return launch_status("skinny_reduce_norm_kernel");

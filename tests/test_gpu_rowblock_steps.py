@@ -38,3 +38,22 @@ def test_steps_of_a_wave(g, dt, B, hidden, ffn, vocab):
             # 128 hidden values showed 1.2e-2), far less of fp16, which keeps test_gpu_rowblock.py's bound
             assert max_err_rel_to_max(g.f32(got[b], dt), g.f32(want[0], dt)) <= (1e-2 if dt == orc.F16 else 13 * 2.0**-9), (step, b)
     dec.close()
+
+
+# chunks of a prompt: o and down as two K ranges (hidden 1152 and ffn 640: 18 and 10 steps, a range ends inside a 128-k step of the copy)
+@pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("rows", [17, 32, 33, 64])
+@pytest.mark.parametrize("hidden,ffn", [(1152, 640), (2176, 1152)])
+def test_two_ranges(g, dt, rows, hidden, ffn):
+    cfg, w = llm_weights.synthetic_int8(dict(SMALL, n_layers=1, hidden=hidden, ffn=ffn, n_heads=hidden // 64, n_kv_heads=hidden // 128, head_dim=64, max_seq=128), dt, seed=rows)
+    dec, ref = g.mynn.Decoder(cfg, dev_weights(g, w, dt), seq_q=rows), orc.Model(cfg, w)
+    rng = np.random.default_rng(rows)
+    for past in (0, rows):
+        if past + rows > 128:
+            break
+        ids, pos = rng.integers(0, cfg["vocab"], rows), np.arange(past, past + rows)
+        want = ref.forward(ids, pos, past, past + rows, True)
+        _, got = dec.step(ids, pos, past, past + rows, want_logits=True)
+        # (as above)
+        assert max_err_rel_to_max(g.f32(got, dt), g.f32(want, dt)) <= (1e-2 if dt == orc.F16 else 13 * 2.0**-9), past
+    dec.close()
