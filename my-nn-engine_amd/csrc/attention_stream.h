@@ -52,16 +52,23 @@ constexpr int kStreamTile = 32;
 // them from when it comes to their tile: the RoPE + append launch in front of it disappears and nobody waits for a store.
 // (Written first and read back like any other row, behind a barrier: 8 us more at 32 sequences x 2048 keys.)
 // What the kernel needs of AttnParams (a launch pays for its argument bytes: 0.9 us of host time for 300 against 60).
-struct StreamParams {
+struct StreamRest {
     void *out;
-    const void *q, *k, *v, *k_scale, *v_scale, *cos_t, *sin_t;
-    const int64_t *d_pos;
-    const int32_t *d_active, *d_past, *page_table;
+    const void *k_scale, *v_scale, *cos_t, *sin_t;
+    const int32_t *page_table;
     float *part_o, *part_ml;
     int *arrive;
     long q_bs, q_hs, o_bs, o_hs;
     float scale;
-    int Hq, Hkv, cache_len, active, nsplit, slice, page_shift, pages_per_seq;
+    int Hq, cache_len, active, nsplit, page_shift, pages_per_seq;
+};
+// ... and what its first loads need: leading scalar arguments, which arrive preloaded with the wave, where members of a struct take a load first (4 sequences x 2048
+// keys, D = 64: 7.66 -> 7.48 us)
+struct StreamParams : StreamRest {
+    const void *q, *k, *v;
+    const int32_t *d_active, *d_past;
+    const int64_t *d_pos;
+    int Hkv, slice;
 };
 enum StreamForm { kOneTile, kTiles, kTilesOnce };
 // LDS of a workgroup of W waves, in bytes: V tiles, p tiles, (m, l) of the waves, the new row and its scales
@@ -77,7 +84,9 @@ template <typename T, int D, int W> struct StreamLds {
 // keys where this one gives 3.2, both together 3.0.
 __device__ __forceinline__ U4 load_once(const U4 *p) { return __builtin_nontemporal_load(p); }
 template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, int FORM>
-__global__ __launch_bounds__(W * 64) void attn_stream_kernel(StreamParams p) {
+__global__ __launch_bounds__(W * 64) void attn_stream_kernel(const void *q, const void *k, const void *v, const int32_t *d_active, const int32_t *d_past,
+                                                               const int64_t *d_pos, int Hkv, int slice, StreamRest rest) {
+    const StreamParams p{rest, q, k, v, d_active, d_past, d_pos, Hkv, slice};
     using Lds = StreamLds<T, D, W>;
     constexpr int kStreamWaves = W, kStreamThreads = W * 64;
     extern __shared__ __align__(16) char sm[];

@@ -156,10 +156,10 @@ int attention_stream_launch(const AttnParams &p, int D, int dtype, int kv_int8, 
     }
     const bool fuse = p.qkv != nullptr;
     MYNN_REQUIRE(!fuse || (p.nsplit == 1 || p.arrive), MYNN_ERR_INVALID, "streaming attention: the fused form merges its own key ranges");
-    const StreamParams sp{p.out, fuse ? p.qkv : p.q, p.k, p.v, p.k_scale, p.v_scale, p.cos_t, p.sin_t, p.d_pos, p.d_active, p.d_past, p.page_table, p.part_o,
-                          p.part_ml, p.nsplit > 1 && p.B * p.Hkv <= kAttnArrive ? p.arrive : nullptr, fuse ? (long)(p.Hq + 2 * p.Hkv) * D : p.q_bs,
-                          fuse ? (long)D : p.q_hs, p.o_bs, p.o_hs, p.scale, p.Hq, p.Hkv, p.cache_len, p.active, p.nsplit, p.slice, p.page_shift,
-                          p.pages_per_seq};
+    const StreamParams sp{{p.out, p.k_scale, p.v_scale, p.cos_t, p.sin_t, p.page_table, p.part_o, p.part_ml,
+                           p.nsplit > 1 && p.B * p.Hkv <= kAttnArrive ? p.arrive : nullptr, fuse ? (long)(p.Hq + 2 * p.Hkv) * D : p.q_bs,
+                           fuse ? (long)D : p.q_hs, p.o_bs, p.o_hs, p.scale, p.Hq, p.cache_len, p.active, p.nsplit, p.page_shift, p.pages_per_seq},
+                          fuse ? p.qkv : p.q, p.k, p.v, p.d_active, p.d_past, p.d_pos, p.Hkv, p.slice};
     const int rc = dtype == MYNN_F16 ? attn_stream_go<f16_t>(sp, p.B, D, kv_int8, fuse, s) : attn_stream_go<bf16_t>(sp, p.B, D, kv_int8, fuse, s);
     if (sp.arrive) return rc;
     if (rc || p.nsplit == 1) return rc;

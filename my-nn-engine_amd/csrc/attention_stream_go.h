@@ -11,7 +11,7 @@ template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE, int W, int
         MYNN_HIP(hipFuncSetAttribute((const void *)attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, FORM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         lds_set = true;
     }
-    MYNN_LAUNCH((attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, FORM>), dim3(B * p.Hkv, p.nsplit), dim3(W * 64), lds, s, p);
+    MYNN_LAUNCH((attn_stream_kernel<T, D, G, KVI8, PAGED, FUSE, W, FORM>), dim3(B * p.Hkv, p.nsplit), dim3(W * 64), lds, s, p.q, p.k, p.v, p.d_active, p.d_past, p.d_pos, p.Hkv, p.slice, (const StreamRest &)p);
     return launch_status("attn_stream_kernel");
 }
 template <typename T, int D, int G, bool KVI8, bool PAGED, bool FUSE> static int stream_w(const StreamParams &p, int B, hipStream_t s) {
