@@ -1106,6 +1106,14 @@ static int build(Model &m, void **init, void **state) {
             m.qkv_attn = true;
         }
     }
+    // ... or, over a cache too long for that, the lm_head launch alone finds the token and moves the loop state on (us, 128256 rows of 4096: 82 +
+    // two launches of 9.4 -> 85)
+    if (m.quant && rows == 1 && !c.quantize_activations && !c.unfused_decode && !c.streaming_kv && !m.qkv_attn && m.attn_stream_fuse &&
+        gemv_norm_argmax_supported(m.x, m.final_norm, (const int8_t *)m.lm_head.w, V, H)) {
+        MYNN_HIP(hipMemset(m.lm_cand, 0xFF, (size_t)kGemvArgmaxWords * 8));
+        MYNN_HIP(hipDeviceSynchronize());
+        m.lm_argmax = true;
+    }
 
     // ---- batch-1 decode with quantize_activations: one launch per linear (norm, quantiser, int8 GEMV, residual / SwiGLU)
     if (m.quant && rows == 1 && c.quantize_activations && !c.streaming_kv && !c.unfused_decode && c.dtype != MYNN_F32) {
@@ -1223,16 +1231,24 @@ static int upload_inputs(Model &m, const int64_t *ids, const int64_t *pos, int64
     return 0;
 }
 
+// launches of this executor's step wait for each other's results inside
+static bool handover_used(const Model &m) { return m.qkv_attn || m.lm_argmax; }
+// the hand-over vectors (of the layers: where they are in use) and the candidates empty, the error word cleared
+static int handover_empty(Model &m, bool layers) {
+    const mynn_model_config &c = m.cfg;
+    if (layers) MYNN_HIP(hipMemset(m.qkv, 0xFF, (size_t)((char *)m.attn + (size_t)c.n_heads * c.head_dim * dtype_size(c.dtype) - (char *)m.qkv)));
+    MYNN_HIP(hipMemset(m.lm_cand, 0xFF, (size_t)kGemvArgmaxWords * 8));
+    MYNN_HIP(hipMemset(m.d_past + 3, 0, 4));
+    return 0;
+}
+
 // A wait inside a fused launch ran out (the error word is set; read back after the stream has drained): the step's
 // results -- logits, token, loop state, the KV row it appended -- are undefined.  The executor empties the hand-over
 // vectors, gives up sharing launches for good (every op becomes a launch of its own: same arithmetic, bit-identical
 // results, no workgroup ever waits for another) and captures its step again; the caller then repeats the step from
 // its host-side inputs, which overwrites the KV row.
 static int handover_recover(Model &m) {
-    const mynn_model_config &c = m.cfg;
-    MYNN_HIP(hipMemset(m.qkv, 0xFF, (size_t)((char *)m.attn + (size_t)c.n_heads * c.head_dim * dtype_size(c.dtype) - (char *)m.qkv)));
-    MYNN_HIP(hipMemset(m.lm_cand, 0xFF, (size_t)kGemvArgmaxWords * 8));
-    MYNN_HIP(hipMemset(m.d_past + 3, 0, 4));
+    TRY(handover_empty(m, m.qkv_attn));
     if (!m.fell_back && m.handover_failures == 0) {
         m.shared_qkv_attn = m.qkv_attn;
         m.shared_lm_argmax = m.lm_argmax;
@@ -1258,10 +1274,7 @@ static int handover_clean_steps(Model &m, long steps) {
     if (!m.fell_back || m.rearm_after <= 0) return 0;
     m.clean_steps += steps;
     if (m.clean_steps < m.rearm_after) return 0;
-    const mynn_model_config &c = m.cfg;
-    MYNN_HIP(hipMemset(m.qkv, 0xFF, (size_t)((char *)m.attn + (size_t)c.n_heads * c.head_dim * dtype_size(c.dtype) - (char *)m.qkv)));
-    MYNN_HIP(hipMemset(m.lm_cand, 0xFF, (size_t)kGemvArgmaxWords * 8));
-    MYNN_HIP(hipMemset(m.d_past + 3, 0, 4));
+    TRY(handover_empty(m, m.shared_qkv_attn));
     m.qkv_attn = m.shared_qkv_attn;
     m.lm_argmax = m.shared_lm_argmax;
     m.fell_back = false;
@@ -1417,13 +1430,13 @@ static int step_once(Model &m, const int64_t *input_ids, const int64_t *position
     const mynn_model_config &c = m.cfg;
     char *h_next = m.h_stage + m.stage_bytes - m.next_stage;
     // (fused projection + attention: the error word travels in the same copy, d_past[3] .. d_next[0])
-    if (m.qkv_attn) MYNN_HIP(hipMemcpyAsync(h_next, m.d_past + 3, 24, hipMemcpyDeviceToHost, m.stream));
+    if (handover_used(m)) MYNN_HIP(hipMemcpyAsync(h_next, m.d_past + 3, 24, hipMemcpyDeviceToHost, m.stream));
     else if (next_token) MYNN_HIP(hipMemcpyAsync(h_next, m.d_next, (size_t)c.batch * 4, hipMemcpyDeviceToHost, m.stream));
     if (logits_host)
         MYNN_HIP(hipMemcpyAsync(logits_host, m.logits, (size_t)c.batch * c.seq_q * c.vocab * dtype_size(c.dtype),
                                 hipMemcpyDeviceToHost, m.stream));
     MYNN_HIP(hipStreamSynchronize(m.stream));
-    if (m.qkv_attn) {
+    if (handover_used(m)) {
         if (*(const int32_t *)h_next) {
             *handover_failed = true;
             return 0;
@@ -1553,9 +1566,9 @@ extern "C" int mynn_model_decode_loop(void *state, int32_t token, int64_t past_l
         for (; done < n_steps; done++) TRY(run_once(m));
         MYNN_HIP(hipMemcpyAsync(m.h_stage, m.d_tokens, (size_t)n_steps * 4, hipMemcpyDeviceToHost, m.stream));
         char *h_err = m.h_stage + m.stage_bytes - m.next_stage;
-        if (m.qkv_attn) MYNN_HIP(hipMemcpyAsync(h_err, m.d_past + 3, 4, hipMemcpyDeviceToHost, m.stream));
+        if (handover_used(m)) MYNN_HIP(hipMemcpyAsync(h_err, m.d_past + 3, 4, hipMemcpyDeviceToHost, m.stream));
         MYNN_HIP(hipStreamSynchronize(m.stream));
-        if (m.qkv_attn && *(const int32_t *)h_err) {
+        if (handover_used(m) && *(const int32_t *)h_err) {
             // some step's hand-over gave up: every later token is undefined.  Rebuild with one op per launch and run the
             // whole loop again from the same inputs (the KV rows are overwritten).
             TRY(handover_recover(m));
