@@ -171,13 +171,19 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv_kernel(GemvParams p
 // D < NC: only D chunks of each row are in flight, the next is asked for when one is used up: with all of a long row at once the
 // device delivers less (fp16, us, all / D as in gemv1_dispatch: 4096 x 14336 13.4 / 10.5, 8192 x 14000 24.8 / 19.2, 2048 x 9600 7.3 /
 // 5.3, 8192 x 8192 13.5 / 12.7, 4096 x 6000 6.2 / 5.8; bf16 12.6 / 10.8, 21.0 / 19.4, 6.8 / 5.2, 13.1 / 12.7, 6.4 / 5.6; rows of up to
-// 4096 are short enough: 28672 x 4096 19.8 us whatever D).  Forms that fit them are held to the registers of four waves a
-// SIMD: left alone the compiler took 154 for 14 chunks of fp16 (4096 x 14336 11.5 us, 5120 x 13824 16.0 against 13.5), and scheduled the
-// short rows no better (batch-1 generation 0.3 %); held to eight waves a step of 8B widths takes a fifth longer, to three 2 % of the TinyLlama shape.
+// 4096 are short enough: 28672 x 4096 19.8 us whatever D).
 // What the first loads need (pointers, sizes) are leading scalar arguments: they arrive preloaded in SGPRs with
 // the wave (-amdgpu-kernarg-preload-count) instead of through a scalar load from the kernarg segment.
+//
+// Waves a SIMD whose registers a form is held to (1: left alone).  Left alone the compiler took 154 registers for 14 chunks of fp16
+// (4096 x 14336 11.5 us, 5120 x 13824 16.0 against 13.5), and scheduled the short rows no better (batch-1 generation 0.3 %); held to eight
+// waves a step of 8B widths takes a fifth longer, to three 2 % of the TinyLlama shape.  With a norm over more than 8192 values a thread's
+// activation and norm pieces (56 registers) join its weights (40): that fits three waves (133 .. 136 registers) but not four, where 21
+// to 27 of them went through scratch memory (batch-1 steps of two layers, vocabulary 32000, hidden 9216 / 12288 / 14336, us, four waves
+// with the values kept in f32 as well / so: fp16 294, 436, 516 / 250, 360, 433; bf16 311, 456, 536 / 256, 368, 439).
+template <int R, int NC, int D, bool NORM> constexpr int gemv1_waves() { return R * D > 10 ? 1 : NORM && NC > 8 ? 3 : 4; }
 template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false, int D = NC>
-__global__ __launch_bounds__(kGemvThreads, (R * D <= 10 ? 4 : 1)) void dequant_gemv1_kernel(const int8_t *wq, const void *act, const void *scale_p, const void *norm_w,
+__global__ __launch_bounds__(kGemvThreads, (gemv1_waves<R, NC, D, NORM>())) void dequant_gemv1_kernel(const int8_t *wq, const void *act, const void *scale_p, const void *norm_w,
                                                                        const void *residual, int N, int K, int groups,
                                                                        int total_waves, GemvParams p) {
     extern __shared__ float act_lds[];  // [K]
@@ -324,6 +330,10 @@ __global__ __launch_bounds__(kGemvThreads, (R * D <= 10 ? 4 : 1)) void dequant_g
             const int pc = tid + q * kGemvThreads;
             if (pc < npieces) {
                 if constexpr (NORM) {
+                    if constexpr (PMAX > 4) {  // (widened again: a long row's values held in f32 over the barrier would be 56 registers more)
+                        pin(apv[q]);
+                        widen8<T>(apv[q], f[q]);
+                    }
                     float nw[8];
                     widen8<T>(nwv[q], nw);
 #pragma unroll
