@@ -181,9 +181,15 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv_kernel(GemvParams p
 // activation and norm pieces (56 registers) join its weights (40): that fits three waves (133 .. 136 registers) but not four, where 21
 // to 27 of them went through scratch memory (batch-1 steps of two layers, vocabulary 32000, hidden 9216 / 12288 / 14336, us, four waves
 // with the values kept in f32 as well / so: fp16 294, 436, 516 / 250, 360, 433; bf16 311, 456, 536 / 256, 368, 439).
-template <int R, int NC, int D, bool NORM> constexpr int gemv1_waves() { return R * D > 10 ? 1 : NORM && NC > 8 ? 3 : 4; }
+// bf16 rows of 4097 to 6144 values are left alone: scheduled for four waves, the staging of the activation waited for the first weights too
+// (us, all chunks at once / a ring, held / a ring, left alone: 512 x 4608 3.26 / 3.52 / 3.09, 2048 x 5120 4.06 / 4.32 / 3.64, 2048 x 5632 4.33 / 4.54 /
+// 3.88, 4096 x 6144 6.49 / 5.80 / 5.55, 11264 x 6144 13.5 / 12.0 / 11.9).
+template <typename T, int R, int NC, int D, bool NORM> constexpr int gemv1_waves() {
+    if (R * D > 10 || (!std::is_same<T, f16_t>::value && NC == 6)) return 1;
+    return NORM && NC > 8 ? 3 : 4;
+}
 template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false, int D = NC>
-__global__ __launch_bounds__(kGemvThreads, (gemv1_waves<R, NC, D, NORM>())) void dequant_gemv1_kernel(const int8_t *wq, const void *act, const void *scale_p, const void *norm_w,
+__global__ __launch_bounds__(kGemvThreads, (gemv1_waves<T, R, NC, D, NORM>())) void dequant_gemv1_kernel(const int8_t *wq, const void *act, const void *scale_p, const void *norm_w,
                                                                        const void *residual, int N, int K, int groups,
                                                                        int total_waves, GemvParams p) {
     extern __shared__ float act_lds[];  // [K]
