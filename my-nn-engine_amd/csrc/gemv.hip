@@ -183,9 +183,10 @@ __global__ __launch_bounds__(kGemvThreads) void dequant_gemv_kernel(GemvParams p
 // with the values kept in f32 as well / so: fp16 294, 436, 516 / 250, 360, 433; bf16 311, 456, 536 / 256, 368, 439).
 // bf16 rows of 4097 to 6144 values are left alone: scheduled for four waves, the staging of the activation waited for the first weights too
 // (us, all chunks at once / a ring, held / a ring, left alone: 512 x 4608 3.26 / 3.52 / 3.09, 2048 x 5120 4.06 / 4.32 / 3.64, 2048 x 5632 4.33 / 4.54 /
-// 3.88, 4096 x 6144 6.49 / 5.80 / 5.55, 11264 x 6144 13.5 / 12.0 / 11.9).
+// 3.88, 4096 x 6144 6.49 / 5.80 / 5.55, 11264 x 6144 13.5 / 12.0 / 11.9).  So are rows of 1025 to 2048 without a norm (fp16, held / left alone: 32000 x
+// 1280 8.73 / 7.97, 32000 x 1536 9.48 / 9.09, 4096 x 2048 3.25 / 3.15, 32000 x 2048 11.17 / 11.24; bf16 32000 x 1536 9.84 / 9.22).
 template <typename T, int R, int NC, int D, bool NORM> constexpr int gemv1_waves() {
-    if (R * D > 10 || (!std::is_same<T, f16_t>::value && NC == 6)) return 1;
+    if (R * D > 10 || (!std::is_same<T, f16_t>::value && NC == 6) || (!NORM && NC == 2)) return 1;
     return NORM && NC > 8 ? 3 : 4;
 }
 template <typename T, int R, int NC, int EPI, bool NORM, bool ARGMAX = false, int D = NC>
