@@ -598,12 +598,14 @@ int gemv_norm_argmax(void *out, const void *x, const void *norm_w, float eps, co
     MYNN_REQUIRE(cand && next && err && gemv_norm_argmax_supported(x, norm_w, wq, N, K), MYNN_ERR_UNSUPPORTED,
                  "gemv_norm_argmax: N=%d K=%d", N, K);
     const int nc = (K + 1023) / 1024;
-    if (nc <= 1) return launch_gemv1<T, 2, 1, EPI_PLAIN, true, true>(p, s);
-    if (nc <= 2) return launch_gemv1<T, 4, 2, EPI_PLAIN, true, true>(p, s);  // (short rows: four per wave, as gemv1_dispatch)
+    // (rows per wave and chunks in flight as gemv1_dispatch has them.  us a step of two layers over a long cache, vocabulary 128256, two rows per
+    // wave / four: fp16, hidden 512 62.6 / 55.0, 1024 70.9 / 62.8; all chunks of a row at once / in a ring, bf16, hidden 5120 229 / 227, 6144 332 / 329)
+    if (nc <= 1) return launch_gemv1<T, 4, 1, EPI_PLAIN, true, true>(p, s);
+    if (nc <= 2) return launch_gemv1<T, 4, 2, EPI_PLAIN, true, true>(p, s);
     if (nc <= 4) return launch_gemv1<T, 2, 4, EPI_PLAIN, true, true>(p, s);
-    if (nc <= 6) return launch_gemv1<T, 2, 6, EPI_PLAIN, true, true>(p, s);
-    if (nc <= 8) return launch_gemv1<T, 2, 8, EPI_PLAIN, true, true>(p, s);
-    return launch_gemv1<T, 2, 14, EPI_PLAIN, true, true>(p, s);
+    if (nc <= 6) return launch_gemv1<T, 2, 6, EPI_PLAIN, true, true, 3>(p, s);
+    if (nc <= 8) return launch_gemv1<T, 2, 8, EPI_PLAIN, true, true, 4>(p, s);
+    return launch_gemv1<T, 2, 14, EPI_PLAIN, true, true, 5>(p, s);
 }
 template int gemv_norm_argmax<bf16_t>(void *, const void *, const void *, float, const int8_t *, const void *, int, int, uint64_t *,
                                       int32_t *, AdvanceState, int *, int, hipStream_t);
