@@ -630,7 +630,8 @@ int tile_gemm_on_stream(int kind, TgPlan plan, void *out, int32_t *acc_out, cons
 // over K ranges or by the GEMV / so: bf16, 2 rows, 2048 x 2048 5.8 / 4.0, 4096 x 14336 18.3 / 10.9; 6 rows, 5632 x 2048 9.3 / 4.7, 6144 x 4096
 // 12.1 / 7.0, 4096 x 14336 19.1 / 11.7, 28672 x 4096 29.2 / 22.9; 15 rows, 2048 x 5632 10.6 / 7.0, 4096 x 14336 20.6 / 15.3; fp16 the same.
 static bool takes_few_rows(const void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int act_dtype, int out_dtype) {
-    return act_dtype != MYNN_F32 && act_dtype == out_dtype && dtype_ok(act_dtype) && rowblock_rows_supported(out, act, wq, scale, M, N, K);
+    return act_dtype != MYNN_F32 && act_dtype == out_dtype && dtype_ok(act_dtype) && rowblock_rows_supported(out, act, wq, scale, M, N, K) &&
+           rowblock_rows_first(M, N, K);
 }
 
 // the reference's kernel choice (cuda.rs:1518-1652): matrix cores for M >= 16 with 16-bit operands

@@ -65,11 +65,13 @@ int rowblock_gemm(void *out, const void *act, const void *packed, const void *sc
 constexpr int kRbRanges = 2;
 bool rowblock_parts_supported(int M, int N, int K);
 int rowblock_parts(float *part, const void *act, const void *packed, int M, int N, int K, int dtype, hipStream_t s);
-// ... from row-major weights, 2 .. 15 rows (16-bit types)
+// ... from row-major weights, 2 .. 15 rows (16-bit types); first: it is the form to take
 bool rowblock_rows_supported(const void *out, const void *act, const void *wq, const void *scale, int M, int N, int K);
+bool rowblock_rows_first(int M, int N, int K);
 int rowblock_rows_gemm(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, hipStream_t s);
 // qrows.hip -- QuantizedMatMul of 2 .. 32 rows (narrow matrices 128) in one launch without scratch memory
 bool qrows_supported(int M, int N, int K);
+bool qrows_first(int M, int N, int K);  // ... which is the form to take
 int qrows_gemm(void *out, int32_t *acc_out, const int8_t *lhs, const void *a_scale, const int8_t *rhs, const void *b_scale, int M, int N, int K, int dtype, hipStream_t s);
 
 // matrix-core GEMM pieces.  A dequantised weight is [N, Kp] of the 16-bit type, Kp = K rounded up to 64,

@@ -4,7 +4,7 @@
 // Replaces quantized_gemv_int8.cuh:13-51 (one 32-lane warp per row, __dp4a) and
 // quantized_matmul_int8.cuh:112-269 (mma.m16n8k32.s8, 3-stage cp.async); CPU twin
 // src/codegen/cpu/kernels/qgemv_i8i8.rs:38-80.
-//   2 .. 32 rows (narrow matrices 128), K % 128 == 0: v_mfma_i32_16x16x64_i8, a stream per wave (qrows.hip)
+//   2 .. 32 rows (narrow matrices 128), K % 128 == 0, by qrows_first: v_mfma_i32_16x16x64_i8, a stream per wave (qrows.hip)
 //   M < 3  : wave64 rows, 16 int8 per lane per load, v_dot4_i32_i8, integer butterfly (this file)
 //   else   : v_mfma_i32_32x32x32_i8 with tiles of 32 .. 128 rows (tile_gemm.hip) or 256 (gemm.hip)
 // Integer accumulation is associative, so both are bit-exact whatever the order.
@@ -99,9 +99,8 @@ extern "C" int mynn_quantized_matmul(void *out, int32_t *acc_out, const int8_t *
     MYNN_REQUIRE(aligned16(lhs) && aligned16(rhs), MYNN_ERR_INVALID, "quantized_matmul: operands must be 16-byte aligned");
     // int32 accumulators hold the exact sum as long as K * 128 * 128 < 2^31
     MYNN_REQUIRE(K <= 131071, MYNN_ERR_UNSUPPORTED, "quantized_matmul: K=%d could overflow the int32 accumulator", K);
-    // rows by the streams of qrows.hip where K is whole steps of them (two rows, us, as dot products / so: 2048 x 5632 6.2 / 4.8, 4096 x 4096
-    // 5.9 / 5.3, 11264 x 2048 6.9 / 5.9)
-    if (qrows_supported(M, N, K)) return qrows_gemm(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, M, N, K, dtype, as_stream(s));
+    // rows by the streams of qrows.hip where K is whole steps of them and they are the faster form
+    if (qrows_first(M, N, K)) return qrows_gemm(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, M, N, K, dtype, as_stream(s));
     // else matrix cores from three rows on (two rows of 4096 x 4096: 6.2 us as dot products, 8.1 as tiles; three: 10 and 8),
     // with the 256-row tiles of gemm.hip where enough of them make that the faster one; the output may lie anywhere (their
     // store writes element by element where it is not 16-byte aligned)
