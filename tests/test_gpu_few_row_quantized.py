@@ -1,5 +1,6 @@
 """QuantizedMatMul of 2 .. 128 rows (qrows.hip): one to four groups of 8 rows and several of 32, fewer weight rows than a block and ragged blocks of every
-workgroup form, K of fewer steps than waves and of one more than they share evenly; integer sums and outputs, bit for bit."""
+workgroup form, K of fewer steps than waves, of one more than they share evenly and of twice the stages of the rings and more for each wave;
+integer sums and outputs, bit for bit."""
 import numpy as np
 import pytest
 
@@ -15,10 +16,7 @@ def g():
     return gpu_util
 
 
-@pytest.mark.parametrize("dt", [orc.F32, orc.F16, orc.BF16])
-@pytest.mark.parametrize("M", [2, 8, 9, 17, 32, 33, 65, 128])
-@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336), (2050, 1152)])
-def test_few_rows_int8(g, dt, M, N, K):
+def check(g, dt, M, N, K):
     import torch
 
     rng = np.random.default_rng(M + N + K)
@@ -32,3 +30,20 @@ def test_few_rows_int8(g, dt, M, N, K):
     assert np.array_equal(g.to_host(out).reshape(M, N), orc.to_storage(y, dt).reshape(M, N))
     alone, none = g.mynn.quantized_matmul(da, dsa, dw, dsw, want_acc=False)
     assert none is None and torch.equal(alone, out)
+
+
+@pytest.mark.parametrize("dt", [orc.F32, orc.F16, orc.BF16])
+@pytest.mark.parametrize("M", [2, 8, 9, 17, 32, 33, 65, 128])
+@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336), (2050, 1152)])
+def test_few_rows_int8(g, dt, M, N, K):
+    check(g, dt, M, N, K)
+
+
+# (row blocks, groups of 8 lhs rows, waves: 20 / (2 blocks + groups) stages of 128 k, 8 at most)
+@pytest.mark.parametrize("M,N,K,blocks,groups,waves", [
+    (8, 700, 12288, 1, 1, 8), (16, 700, 10240, 1, 2, 8), (32, 700, 6272, 1, 4, 8), (65, 300, 6144, 1, 4, 8), (8, 5700, 8320, 2, 1, 8), (9, 5700, 8320, 2, 2, 8),
+    (31, 5700, 8320, 2, 4, 8), (64, 2560, 4096, 2, 4, 8), (3, 8200, 4224, 3, 1, 8), (15, 8200, 4224, 3, 2, 8), (32, 8200, 4224, 3, 4, 8), (8, 12290, 4224, 4, 1, 8),
+    (16, 12290, 4224, 4, 2, 8), (5, 16400, 2176, 4, 1, 4), (12, 16400, 2176, 4, 2, 4), (24, 12290, 2176, 2, 4, 4), (32, 16400, 3200, 2, 4, 4)])
+def test_rings_in_turn(g, M, N, K, blocks, groups, waves):
+    assert K // 128 // waves >= 2 * min(8, 20 // (2 * blocks + groups)) and g.mynn.lib().mynn_few_rows_first(1, M, N, K)
+    check(g, orc.F16, M, N, K)

@@ -1,6 +1,6 @@
 """The one-launch linears of decode batches (rowblock.hip) where a wave's steps of 64 k run out: fewer steps than the eight waves, one
-more than they share evenly, fewer and more than the stages of the rings, one to six row blocks per workgroup with a ragged last one,
-one to eight groups of activation rows, with the norm inside and without; against the oracle."""
+more than they share evenly, fewer than the stages of the rings and (two to six row blocks) twice as many and more, one to six row blocks
+per workgroup with a ragged last one, one to eight groups of activation rows, with the norm inside and without; against the oracle."""
 import numpy as np
 import pytest
 
@@ -37,6 +37,24 @@ def test_steps_of_a_wave(g, dt, B, hidden, ffn, vocab):
             # 13 stored values lie between a token and its logits, each up to half a unit of its type off: 13 * 2^-9 of bf16 (one of
             # 128 hidden values showed 1.2e-2), far less of fp16, which keeps test_gpu_rowblock.py's bound
             assert max_err_rel_to_max(g.f32(got[b], dt), g.f32(want[0], dt)) <= (1e-2 if dt == orc.F16 else 13 * 2.0**-9), (step, b)
+    dec.close()
+
+
+# Every wave of the wide forms goes round its rings: lm_head (four row blocks), gate/up (six), q|k|v (three) 66 steps of 64 k, eight to a wave and more, down (two) 130;
+# a ring has 20 / (row blocks + groups of 8 rows) stages, 47 rows of the wide ones 40 / that with four waves.  (o and down of 17 and more rows are K ranges elsewhere.)
+@pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("B", [8, 16, 24, 47])
+def test_rings_in_turn(g, dt, B):
+    hidden, ffn, vocab = 4224, 8320, 12305
+    cfg, w = llm_weights.synthetic_int8(dict(SMALL, n_layers=1, hidden=hidden, ffn=ffn, vocab=vocab, n_heads=hidden // 64, n_kv_heads=hidden // 128, head_dim=64), dt, seed=B)
+    dec = g.mynn.Decoder(cfg, dev_weights(g, w, dt), batch=B)
+    toks = np.random.default_rng(B).integers(0, vocab, B)
+    _, got = dec.step(toks, [0], 0, 1, want_logits=True)
+    got = got.reshape(B, -1)
+    for b in (0, B - 1):
+        want = orc.Model(cfg, w).forward([toks[b]], [0], 0, 1, False)
+        # (as above)
+        assert max_err_rel_to_max(g.f32(got[b], dt), g.f32(want[0], dt)) <= (1e-2 if dt == orc.F16 else 13 * 2.0**-9), b
     dec.close()
 
 
