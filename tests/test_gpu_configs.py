@@ -154,8 +154,8 @@ LLAMA3_WIDTHS = dict(n_layers=2, hidden=4096, n_heads=32, n_kv_heads=8, head_dim
 def test_config4_llama3_8b_widths_batch32_decode_vs_per_sequence_oracles(g, bench):
     """configs[4] at its real widths (hidden 4096, 32 / 8 heads of 128, ffn 14336, vocab 128256; two layers instead
     of 32 -- the layers are identical in shape): 32 sequences decoded together for 24 steps, three of them followed
-    step by step by their own batch-1 oracle.  The few-row int8 GEMM, the RoPE + append in its reducing launch and
-    the decode attention at D = 128 run at the shapes the benchmark times."""
+    step by step by their own batch-1 oracle.  The few-row int8 GEMM, q|k|v in one launch and the decode attention at
+    D = 128 with RoPE and the appends inside run at the shapes the benchmark times."""
     import torch
 
     dt = orc.F16
