@@ -33,9 +33,9 @@ PROFILE_JSON = {"decode": "decode_tinyllama_int8_bs1.json", "prefill": "prefill_
                 "attention": "attention_decode_b16_l4096.json", "gemv": "gemv_rotating_weight_sets.json"}
 # launch role (the executor's name for a launch) -> pattern of the mangled kernel name
 ROLE_PATTERNS = {
-    "gemv_norm_gateup_swiglu": r"dequant_gemv1_kernelI\w+?Li\d+ELi\d+ELi2ELb1ELb0EE",
-    "gemv_down_residual": r"dequant_gemv1_kernelI\w+?Li\d+ELi\d+ELi1ELb0ELb0EE",
-    "gemv_norm_lm_head_argmax": r"dequant_gemv1_kernelI\w+?Li\d+ELi\d+ELi0ELb1ELb1EE",
+    "gemv_norm_gateup_swiglu": r"dequant_gemv1_kernelI\w+?Li\d+ELi\d+ELi2ELb1ELb0ELi\d+EE",
+    "gemv_down_residual": r"dequant_gemv1_kernelI\w+?Li\d+ELi\d+ELi1ELb0ELb0ELi\d+EE",
+    "gemv_norm_lm_head_argmax": r"dequant_gemv1_kernelI\w+?Li\d+ELi\d+ELi0ELb1ELb1ELi\d+EE",
     "qkv_attention_o": r"qkv_attention_kernelI\w+?Li\d+ELi\d+ELb0ELb0ELb0EE",   # <T, D, NC, EMBED = false, KV8 = false, PAGED = false>
     "embed_qkv_attention_o": r"qkv_attention_kernelI\w+?Li\d+ELi\d+ELb1ELb0ELb0EE",
     "linear_gateup_swiglu": r"(gemm_nt_dma_kernelI\w+?Li2ELb0EE|skinny_gemm_kernelI\w+?Li\d+ELb\dELi2ELi0EE)",  # (skinny: <T, MT, PACKED, FEPI = SwiGLU, ABL = 0>)
@@ -43,10 +43,10 @@ ROLE_PATTERNS = {
     "attention": r"(attn_stream_kernel|attn_prefill_kernel)",
     # --workload gemv: the stand-alone GEMV launches and the read probe of the same geometry
     "gemv_configs0_f32": r"dequant_gemv_kernelIffLi\d+ELi1ELi0ELb0EE",
-    "gemv_gate_up": r"dequant_gemv1_kernelI\w+?Li4ELi2ELi0ELb0ELb0EE",
-    "gemv_down": r"dequant_gemv1_kernelI\w+?Li2ELi6ELi0ELb0ELb0EE",
-    "read_probe_gate_up": r"gemv_read_probe_kernelILi4ELi2EE",
-    "read_probe_down": r"gemv_read_probe_kernelILi2ELi6EE",
+    "gemv_gate_up": r"dequant_gemv1_kernelI\w+?Li4ELi2ELi0ELb0ELb0ELi2EE",
+    "gemv_down": r"dequant_gemv1_kernelI\w+?Li2ELi6ELi0ELb0ELb0ELi3EE",
+    "read_probe_gate_up": r"gemv_read_probe_kernelILi4ELi2ELi2EE",
+    "read_probe_down": r"gemv_read_probe_kernelILi2ELi6ELi3EE",
 }
 MFMA_PEAK_TFLOPS = 2500.0  # MI355X published dense bf16/fp16 matrix rate
 INT8_PEAK_TOPS = 5000.0    # MI355X published dense int8 matrix rate

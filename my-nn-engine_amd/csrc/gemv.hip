@@ -535,32 +535,43 @@ static int gemv1_dispatch(const GemvParams &p, hipStream_t s) {
 }
 
 // ---- measurement aid: the weight stream of dequant_gemv1_kernel and nothing else.  Same grid, same row groups per
-// wave, the same R x NC non-temporal 16-byte loads per lane and group, no activation, no arithmetic beyond an xor
-// that keeps the loads alive, no store.  Launched like the GEMV (dependent launches on one stream, a different
-// matrix each time) it gives the time a launch of this geometry needs just to pull its bytes in: the floor the
+// wave, the same non-temporal 16-byte loads per lane and group, R x NC with R x D of them in flight (long rows: D < NC, as gemv1_dispatch), no
+// activation, no arithmetic beyond an xor that keeps the loads alive, no store.  Launched like the GEMV (dependent launches on one
+// stream, a different matrix each time) it gives the time a launch of this geometry needs just to pull its bytes in: the floor the
 // GEMV's duration is judged against.
-template <int R, int NC>
+template <int R, int NC, int D>
 __global__ __launch_bounds__(kGemvThreads) void gemv_read_probe_kernel(const int8_t *wq, uint32_t *sink, int N, int K, int groups,
                                                                          int total_waves) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nchunks = K >> 4;
     uint32_t acc = 0;
     for (int g = blockIdx.x * kGemvWaves + wave; g < groups; g += total_waves) {
-        U4 w[R][NC];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
+        U4 w[R][D];
+        auto load = [&](int r, int j) {
             const int row = g * R + r < N ? g * R + r : N - 1;
-            const U4 *wrow = (const U4 *)(wq + (size_t)row * K);
+            w[r][j % D] = __builtin_nontemporal_load((const U4 *)(wq + (size_t)row * K) + min(lane + j * kWave, nchunks - 1));
+        };
 #pragma unroll
-            for (int j = 0; j < NC; j++) w[r][j] = __builtin_nontemporal_load(&wrow[min(lane + j * kWave, nchunks - 1)]);
+        for (int i = 0; i < R * D; i++) load(D == NC ? i / D : i % R, D == NC ? i % D : i / R);
+#pragma unroll
+        for (int j = 0; j < NC; j++) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                U4 &c = w[r][j % D];
+                if constexpr (D < NC) pin(c);
+                acc ^= c.x ^ c.y ^ c.z ^ c.w;
+            }
+            if constexpr (D < NC) {
+                asm volatile("" : "+v"(acc)::"memory");  // (the next chunk is asked for when one is used up)
+                if (j + D < NC) {
+#pragma unroll
+                    for (int r = 0; r < R; r++) load(r, j + D);
+                }
+            }
         }
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int j = 0; j < NC; j++) acc ^= w[r][j].x ^ w[r][j].y ^ w[r][j].z ^ w[r][j].w;
     }
     if (acc == 0x9E3779B9u && sink) sink[0] = acc;  // (never true for the patterns the benchmark fills in; keeps the loads)
 }
-template <int R, int NC>
+template <int R, int NC, int D = NC>
 static int launch_read_probe(const int8_t *wq, uint32_t *sink, int N, int K, bool empty, hipStream_t s) {
     const int groups = (N + R - 1) / R;
     const int max_waves = 256 * 16;
@@ -568,7 +579,7 @@ static int launch_read_probe(const int8_t *wq, uint32_t *sink, int N, int K, boo
     int waves = (groups + passes - 1) / passes;
     const int blocks = (waves + kGemvWaves - 1) / kGemvWaves;
     waves = blocks * kGemvWaves;
-    MYNN_LAUNCH((gemv_read_probe_kernel<R, NC>), dim3(blocks), dim3(kGemvThreads), 0, s, wq, sink, N, K, empty ? 0 : groups, waves);
+    MYNN_LAUNCH((gemv_read_probe_kernel<R, NC, D>), dim3(blocks), dim3(kGemvThreads), 0, s, wq, sink, N, K, empty ? 0 : groups, waves);
     return launch_status("gemv_read_probe_kernel");
 }
 
@@ -665,7 +676,7 @@ extern "C" int mynn_gemv_read_probe(const int8_t *wq, void *sink, int N, int K, 
     if (nc <= 1) return launch_read_probe<4, 1>(wq, (uint32_t *)sink, N, K, empty != 0, st);
     if (nc <= 2) return launch_read_probe<4, 2>(wq, (uint32_t *)sink, N, K, empty != 0, st);
     if (nc <= 4) return launch_read_probe<2, 4>(wq, (uint32_t *)sink, N, K, empty != 0, st);
-    if (nc <= 6) return launch_read_probe<2, 6>(wq, (uint32_t *)sink, N, K, empty != 0, st);
-    if (nc <= 8) return launch_read_probe<2, 8>(wq, (uint32_t *)sink, N, K, empty != 0, st);
-    return launch_read_probe<2, 14>(wq, (uint32_t *)sink, N, K, empty != 0, st);
+    if (nc <= 6) return launch_read_probe<2, 6, 3>(wq, (uint32_t *)sink, N, K, empty != 0, st);
+    if (nc <= 8) return launch_read_probe<2, 8, 4>(wq, (uint32_t *)sink, N, K, empty != 0, st);
+    return launch_read_probe<2, 14, 5>(wq, (uint32_t *)sink, N, K, empty != 0, st);
 }

@@ -1,5 +1,6 @@
 """What the documented build lines need: the library hipcc alone, the Python module a target of its own."""
 import os
+import re
 import subprocess
 
 from conftest import ROOT
@@ -20,3 +21,15 @@ def test_the_library_is_built_without_python():
 def test_the_python_module_is_a_target_of_its_own():
     rc, commands = planned("host_ops")
     assert rc == 0 and "_host_ops.so" in commands and "hipcc" not in commands
+
+
+def test_every_launch_role_of_the_benchmark_is_a_kernel_of_the_library():
+    """(rocprofv3's figures of a launch are found by the pattern of its kernel's name)"""
+    import sys
+
+    sys.path.insert(0, ROOT)
+    import bench
+
+    lib = open(os.path.join(ROOT, "my-nn-engine_amd", "lib", "libmynn_hip.so"), "rb").read()
+    assert len(bench.ROLE_PATTERNS) >= 13
+    assert not [role for role, pattern in bench.ROLE_PATTERNS.items() if not re.search(pattern.encode(), lib)]
