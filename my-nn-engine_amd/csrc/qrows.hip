@@ -13,6 +13,7 @@
 
 #include "kernels.h"
 #include "mfma.h"
+#include "wave_ring.h"
 
 namespace mynn {
 
@@ -40,14 +41,11 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
     M = min(M - m0, A8 * 8);
     const int steps = K / 128, n = __builtin_amdgcn_readfirstlane((steps - kw + WAVES - 1) / WAVES);  // in all, of this wave
     char *ring = lds + kw * ND * S::STAGE;
-    // Row 8 * i + lane / 8 of an operand, and of its 8 chunks of 16 bytes the one that makes the fragment reads meet different banks;
-    // as load_group_to_lds takes them, from 4096 bytes in front of a step
     uint32_t aoff[A8], woff[2 * NB];
-    auto chunk = [&](int i, int last) { return (uint32_t)(min(8 * i + (lane >> 3), last) * K + (((lane & 7) ^ (lane >> 3)) << 4) + 4096 - 1024 * (i % 4)); };
 #pragma unroll
-    for (int i = 0; i < A8; i++) aoff[i] = chunk(i, M - 1);
+    for (int i = 0; i < A8; i++) aoff[i] = ring_chunk(lane, i, M - 1, K);
 #pragma unroll
-    for (int i = 0; i < 2 * NB; i++) woff[i] = chunk(i, N - 1 - n0);
+    for (int i = 0; i < 2 * NB; i++) woff[i] = ring_chunk(lane, i, N - 1 - n0, K);
     auto request = [&](int i, int slot) {
         const size_t k = (size_t)(i * WAVES + kw) * 128;
         const char *a = (const char *)lhs + k - 4096, *w = (const char *)rhs + (size_t)n0 * K + k - 4096;
@@ -55,12 +53,6 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
         load_group_to_lds<(NB < 2 ? 2 : 4), true>(w, woff, to);
         if constexpr (NB > 2) load_group_to_lds<2 * NB - 4, true>(w, woff + 4, to + 4096);
         load_group_to_lds<A8>(a, aoff, to + 2 * NB * 1024);
-    };
-    auto wait = [&](auto left) {  // until no more than `left` loads are in flight, and all LDS reads are through
-        constexpr int V = decltype(left)::value;
-        static_assert(V < 64, "a counter of six bits");
-        __builtin_amdgcn_s_waitcnt((V & 15) | (V >> 4) << 14 | 0x70);
-        asm volatile("" ::: "memory");
     };
     qi4_t acc[NB][MT];
 #pragma unroll
@@ -93,7 +85,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
     for (int d = 0; d < ND - 1; d++)
         if (d < n) request(d, d);
     for (; i + ND - 1 < n; i++) {
-        wait(std::integral_constant<int, (ND - 2) * C>{});
+        wait_for_loads<(ND - 2) * C>();
         use(slot);
         request(i + ND - 1, slot == 0 ? ND - 1 : slot - 1);  // (the stage that the step before was read from)
         multiply();
@@ -104,7 +96,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void qrows_gemm_kernel(const int8_t 
         constexpr int L = decltype(left)::value;
         if constexpr (L < ND) {
             if (n - i != L) return;
-            wait(std::integral_constant<int, (L - 1) * C>{});
+            wait_for_loads<(L - 1) * C>();
             use(slot);
             multiply();
             slot = slot + 1 == ND ? 0 : slot + 1;

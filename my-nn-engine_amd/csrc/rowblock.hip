@@ -27,6 +27,7 @@
 
 #include "kernels.h"
 #include "mfma.h"
+#include "wave_ring.h"
 
 namespace mynn {
 
@@ -81,8 +82,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
     }
     if constexpr (!PACKED) {
 #pragma unroll
-        for (int j = 0; j < NB * H; j++)
-            woff[j] = (uint32_t)(min(8 * j + (lane >> 3), N - 1 - b0 * 16) * K + (((lane & 7) ^ (lane >> 3)) << 4) + 4096 - 1024 * (j % 4));
+        for (int j = 0; j < NB * H; j++) woff[j] = ring_chunk(lane, j, N - 1 - b0 * 16, K);
     } else
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -112,12 +112,6 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             load_group_to_lds<(A8 < 4 ? A8 : 4)>(src, aoff, to);
             if constexpr (A8 > 4) load_group_to_lds<A8 - 4>(src, aoff + 4, to + 4096);
         }
-    };
-    auto wait = [&](auto left) {  // until no more than `left` loads are in flight, and all LDS reads are through
-        constexpr int V = decltype(left)::value;
-        static_assert(V < 64, "a counter of six bits");
-        __builtin_amdgcn_s_waitcnt((V & 15) | (V >> 4) << 14 | 0x70);
-        asm volatile("" ::: "memory");
     };
     // what the store of this thread's first output needs (mostly its only one), fetched in front of everything else
     constexpr int PR = EPI == GEMM_SWIGLU ? 8 : 16;  // outputs per row block and activation row
@@ -168,7 +162,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
         for (int i = 0; i < NA; i++)
 #pragma unroll
             for (int b = 0; b < NB; b++) wr[i][b] = __builtin_nontemporal_load((const U4 *)(step_w(i) + woff[b] + 1024 * (b % 4)));
-        wait(std::integral_constant<int, (NA * NB < 63 ? NA * NB : 63)>{});
+        wait_for_loads<(NA * NB < 63 ? NA * NB : 63)>();
         float ss[A8];
 #pragma unroll
         for (int g = 0; g < A8; g++) ss[g] = 0.f;
@@ -235,7 +229,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
         for (int d = 0; d < ND - 1; d++)
             if (d < n) request(d, d);
         for (; i + ND - 1 < n; i++) {
-            wait(std::integral_constant<int, (ND - 2) * C>{});
+            wait_for_loads<(ND - 2) * C>();
             use(0);
             request(i + ND - 1, slot == 0 ? ND - 1 : slot - 1);  // (the stage that the step before was read from)
             multiply();
@@ -250,7 +244,7 @@ __global__ __launch_bounds__(S::WAVES * 64) void rowblock_gemm_kernel(const T *a
             constexpr int L = decltype(left)::value;
             if constexpr (L < ND) {
                 if (n - i != L) return;
-                wait(std::integral_constant<int, (L - 1) * C>{});
+                wait_for_loads<(L - 1) * C>();
                 use(0);
                 multiply();
                 if constexpr (H > 1) {
