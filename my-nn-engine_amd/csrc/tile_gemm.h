@@ -32,8 +32,9 @@
 // order of the ranges -- the result does not depend on who was last -- and stores the output.  Nobody waits for anybody.
 // SEQ: one workgroup takes all ranges of its tile one after the other and adds them up in registers: the same bits without
 // scratch memory, for calls that are being captured (a graph may be replayed on any stream and outlive any block).
-// It costs the parallelism: bf16, 6 rows x 4096 x 14336 109 us against 25, 6 x 2048 x 2048 14.3 against 8.2, 100 x 4096 x 4096
-// 29 against 17.
+// It costs the parallelism (us, bf16, captured / not): 6 rows x 4096 x 14352 61 / 18, 6 x 2048 x 2064 13.6 / 8.1, 16 x 4096 x 14336 80 / 21, 100 x
+// 4096 x 4096 25 / 16, 300 x 2048 x 5632 32 / 23 (with the steps' loop called in two places, not inlined and its registers in
+// memory: 1045, 185, 1961, 588, 770).
 #pragma once
 #include <type_traits>
 
@@ -432,34 +433,32 @@ __global__ __launch_bounds__(G::THREADS, G::WPE) void tile_gemm_kernel(const voi
         if constexpr (G::WIDE) one_range_wide();
         else one_range_step();
     };
-    one_range();
     if constexpr (SEQ) {
+        // (one_range is called in one place, or it is no longer inlined and its registers are memory)
         acc_t sum[TI][TJ];
+        for (int z = 0; z < ks; z++) {
+            if (z) {
+                range(z);
 #pragma unroll
-        for (int i = 0; i < TI; i++)
+                for (int i = 0; i < TI; i++)
 #pragma unroll
-            for (int j = 0; j < TJ; j++) sum[i][j] = acc[i][j];
-        for (int z = 1; z < ks; z++) {
+                    for (int j = 0; j < TJ; j++)
 #pragma unroll
-            for (int i = 0; i < TI; i++)
-#pragma unroll
-                for (int j = 0; j < TJ; j++)
-#pragma unroll
-                    for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
-            range(z);
+                        for (int e = 0; e < 16; e++) acc[i][j][e] = 0;
+            }
             one_range();
 #pragma unroll
             for (int i = 0; i < TI; i++)
 #pragma unroll
                 for (int j = 0; j < TJ; j++)
 #pragma unroll
-                    for (int e = 0; e < 16; e++) sum[i][j][e] += acc[i][j][e];
+                    for (int e = 0; e < 16; e++) sum[i][j][e] = z ? sum[i][j][e] + acc[i][j][e] : acc[i][j][e];
         }
 #pragma unroll
         for (int i = 0; i < TI; i++)
 #pragma unroll
             for (int j = 0; j < TJ; j++) acc[i][j] = sum[i][j];
-    }
+    } else one_range();
 
     if (!SEQ && ks > 1) {
         // partial sums, two per word, [range][(i, j), pair][thread]

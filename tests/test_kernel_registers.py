@@ -42,3 +42,20 @@ def test_gemv_forms_use_no_scratch_memory(tmp_path):
             forms[name] = int(scratch)
     assert len(forms) >= 40  # (both types, row lengths of up to 14 chunks, with the norm inside and without)
     assert not {k: v for k, v in forms.items() if v}
+
+
+def test_tile_products_use_no_scratch_memory(tmp_path):
+    """(with the K ranges of a tile one after the other, for captured calls, the loop over the steps was called in two places and no longer
+    inlined: fragments and sums in memory, ten times as long)"""
+    if not (os.path.exists(READELF) and os.path.exists(LIB)):
+        pytest.skip("needs the built library and llvm-readelf")
+    forms = {}
+    for code in device_code(open(LIB, "rb").read()):
+        if b"tile_gemm_kernel" not in code:
+            continue
+        (tmp_path / "code").write_bytes(code)
+        notes = subprocess.check_output([READELF, "--notes", str(tmp_path / "code")], text=True)
+        for name, scratch in re.findall(r"\.name:\s+(\S*tile_gemm_kernel\S*)\n(?:(?!\.name:).)*?\.private_segment_fixed_size:\s+(\d+)", notes, re.S):
+            forms[name] = int(scratch)
+    assert len(forms) >= 200  # (every tile, store and row tail of three kinds, with and without ranges in sequence)
+    assert not {k: v for k, v in forms.items() if v}
