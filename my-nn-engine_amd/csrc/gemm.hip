@@ -630,8 +630,7 @@ int tile_gemm_on_stream(int kind, TgPlan plan, void *out, int32_t *acc_out, cons
 // over K ranges or by the GEMV / so: bf16, 2 rows, 2048 x 2048 5.8 / 4.0, 4096 x 14336 18.3 / 10.9; 6 rows, 5632 x 2048 9.3 / 4.7, 6144 x 4096
 // 12.1 / 7.0, 4096 x 14336 19.1 / 11.7, 28672 x 4096 29.2 / 22.9; 15 rows, 2048 x 5632 10.6 / 7.0, 4096 x 14336 20.6 / 15.3; fp16 the same.
 static bool takes_few_rows(const void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int act_dtype, int out_dtype) {
-    return act_dtype != MYNN_F32 && act_dtype == out_dtype && dtype_ok(act_dtype) && rowblock_rows_supported(out, act, wq, scale, M, N, K) &&
-           rowblock_rows_first(M, N, K);
+    return act_dtype != MYNN_F32 && act_dtype == out_dtype && dtype_ok(act_dtype) && rowblock_rows_supported(out, act, wq, scale, M, N, K);
 }
 
 // the reference's kernel choice (cuda.rs:1518-1652): matrix cores for M >= 16 with 16-bit operands
@@ -673,6 +672,8 @@ extern "C" int mynn_dequant_matmul_ws(void *out, const void *act, const int8_t *
         }
         return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, workspace, gemm_tile, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }
+    // (whether or not K ranges would be the faster form: fewer than 16 rows have no workspace for their sums.  us, by the GEMV or the plain
+    // kernel / so: bf16, 6 x 500 x 65536 254 / 31, 15 x 500 x 32768 141 / 21, 15 x 2048 x 32768 549 / 26, 15 x 18432 x 8192 1289 / 42)
     if (M > 1 && M < 16 && takes_few_rows(out, act, wq, scale, M, N, K, act_dtype, out_dtype)) return rowblock_rows_gemm(out, act, wq, scale, M, N, K, out_dtype, as_stream(s));
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));
 }
@@ -680,7 +681,8 @@ extern "C" int mynn_dequant_matmul_ws(void *out, const void *act, const int8_t *
 extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N,
                                    int K, int act_dtype, int out_dtype, mynn_stream s) {
     MYNN_REQUIRE(M >= 1, MYNN_ERR_INVALID, "dequant_matmul: M=%d", M);
-    if (M > 1 && M < 16 && takes_few_rows(out, act, wq, scale, M, N, K, act_dtype, out_dtype)) return rowblock_rows_gemm(out, act, wq, scale, M, N, K, out_dtype, as_stream(s));
+    const bool few = M > 1 && M < 16 && takes_few_rows(out, act, wq, scale, M, N, K, act_dtype, out_dtype);
+    if (few && rowblock_rows_first(M, N, K)) return rowblock_rows_gemm(out, act, wq, scale, M, N, K, out_dtype, as_stream(s));
     int kind = 0;
     const bool tiles = scale && takes_tiles(out, act, wq, M, N, K, act_dtype, out_dtype, &kind);
     if (tiles) {
@@ -700,6 +702,7 @@ extern "C" int mynn_dequant_matmul(void *out, const void *act, const int8_t *wq,
         if (rc) return rc;
         return dequant_gemm_mfma(out, act, wq, scale, M, N, K, out_dtype, ws.ptr + kWsCounterBytes, 0, as_stream(s), sum_ranges(M, N, K, out_dtype));
     }
+    if (few) return rowblock_rows_gemm(out, act, wq, scale, M, N, K, out_dtype, as_stream(s));  // (an output that the tiles refuse)
     return dequant_gemv_dispatch(out, act, wq, scale, M, N, K, act_dtype, out_dtype, as_stream(s));
 }
 

@@ -90,3 +90,28 @@ def test_odd_places(g, dt, M, N, K):
         assert torch.equal(run(shifts), want), shifts
     for shifts in ((4, 0, 0, 0), (0, 8, 0, 0), (4, 8, 1, 1)):
         assert np.all(np.abs(g.f32(g.to_host(run(shifts).contiguous()), dt).reshape(M, N) - exact) <= bound), shifts
+
+
+# Few weight rows with long rows, which K ranges do faster: with a caller's workspace (there is none for fewer than 16 rows) and for an output that the
+# tiles refuse it is the streams all the same, whose sums do not depend on how many weight rows there are
+@pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
+@pytest.mark.parametrize("M", [2, 15])
+def test_streams_where_k_ranges_cannot_be(g, dt, M):
+    import torch
+
+    N, wide, K = 500, 3100, 49152
+    first = g.mynn.lib().mynn_few_rows_first
+    assert first(0, M, wide, K) and not first(0, M, N, K)
+    gen = torch.Generator(device="cuda").manual_seed(M)
+    tdt = torch.float16 if dt == orc.F16 else torch.bfloat16
+    act = torch.randn((M, K), generator=gen, device="cuda").to(tdt)
+    w = torch.randint(-128, 128, (wide, K), generator=gen, device="cuda").to(torch.int8)
+    sc = (torch.rand((wide,), generator=gen, device="cuda") * 1e-3 + 1e-3).to(tdt)
+    want = g.mynn.dequant_matmul(act, w, sc)[:, :N]
+    assert torch.equal(g.mynn.dequant_matmul_ws(act, w[:N], sc[:N]), want)
+    flat = torch.full((M * N + 16,), 7.0, dtype=tdt, device="cuda")
+    g.mynn.check(g.mynn.lib().mynn_dequant_matmul(flat.data_ptr() + 2, act.data_ptr(), w.data_ptr(), sc.data_ptr(), M, N, K, dt, dt,
+                                                  torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert flat[0] == 7 and (flat[1 + M * N:] == 7).all()
+    assert torch.equal(flat[1:1 + M * N].view(M, N), want)

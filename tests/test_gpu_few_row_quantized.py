@@ -47,3 +47,25 @@ def test_few_rows_int8(g, dt, M, N, K):
 def test_rings_in_turn(g, M, N, K, blocks, groups, waves):
     assert K // 128 // waves >= 2 * min(8, 20 // (2 * blocks + groups)) and g.mynn.lib().mynn_few_rows_first(1, M, N, K)
     check(g, orc.F16, M, N, K)
+
+
+# (where K ranges are the faster form a captured call, whose tiles would take them as one, takes the streams)
+@pytest.mark.parametrize("M,N,K", [(3, 500, 32768), (32, 1024, 32768), (33, 160, 16384), (128, 1024, 8192)])
+def test_captured(g, M, N, K):
+    import torch
+
+    assert not g.mynn.lib().mynn_few_rows_first(1, M, N, K)
+    rng = np.random.default_rng(M)
+    a, w = (g.to_dev(rng.integers(-127, 128, sh).astype(np.int8)) for sh in ((M, K), (N, K)))
+    sa, sw = (g.to_dev(orc.to_storage(rng.uniform(1e-3, 1e-2, n), orc.F16), orc.F16) for n in (M, N))
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got, acc = g.mynn.quantized_matmul(a, sa, w, sw)
+    for _ in range(3):
+        got.zero_(), acc.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want, sums = g.mynn.quantized_matmul(a, sa, w, sw)
+        assert torch.equal(got, want) and torch.equal(acc, sums)
+        a.copy_(torch.roll(a, 1, 0))
