@@ -109,7 +109,7 @@ extern "C" int mynn_quantized_matmul(void *out, int32_t *acc_out, const int8_t *
         if (dtype != MYNN_F32 && qgemm_dma_us(M, N, K) < plan.us)
             return qgemm_dma(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, nullptr, M, N, K, dtype, GEMM_PLAIN, as_stream(s));
         // (captured, a product whose K ranges would be side by side takes them as one: the streams, which need no memory for the sums.  us
-        // captured, tiles / so: 8 x 500 x 32768 41.6 / 8.1, 32 x 1024 x 32768 41.9 / 25.7, 128 x 1024 x 8192 12.8 / 6.4, 64 x 4096 x 14336 21.2 / 18.8)
+        // captured, tiles / so: 8 x 500 x 32768 41.6 / 8.1, 32 x 1024 x 32768 41.9 / 25.7, 40 x 2048 x 14336 20.6 / 12.9, 64 x 4096 x 14336 21.2 / 18.8)
         if (plan.ks > 1 && qrows_supported(M, N, K) && stream_capturing(as_stream(s)))
             return qrows_gemm(out, acc_out, lhs, lhs_scale, rhs, rhs_scale, M, N, K, dtype, as_stream(s));
         return tile_gemm_on_stream(TG_I8, plan, out, acc_out, lhs, rhs, lhs_scale, rhs_scale, M, N, K, dtype, as_stream(s));

@@ -169,33 +169,36 @@ static int qr_go(const int8_t *lhs, const int8_t *rhs, const void *a_scale, cons
 }
 
 bool qrows_supported(int M, int N, int K) { return M >= 2 && M <= 128 && N >= 1 && K >= 128 && K % 128 == 0; }
-// Where it is the form to take (us, dot products (two rows) or tiles / so; profiles/few_row_times.csv has both over 2100 shapes).
-//   Two rows: up to 4096 weight rows (2048 x 5632 6.2 / 4.8, 4096 x 4096 5.9 / 5.3), beyond, not where rows of whole 8192 bytes (8192 x 8192 14.0 / 16.6;
-//   but three row blocks of 16: 10240 x 8192 1.09 times as fast), with two workgroups of streams per CU whole 4096, meet at the same channels of the
-//   memory (16384 x 16384 44.2 / 52.4).
+// Where it is the form to take (us a call with weights that are not cached, dot products (two rows) or tiles / so; profiles/few_row_times.csv has
+// both over 4000 shapes; a call of tiles costs the host some 5.4 us, of the streams 4.4).
+//   Two rows: up to 4096 weight rows (2048 x 5632 6.2 / 5.0, 4096 x 4096 6.1 / 5.3), beyond, not where rows of whole 8192 bytes (8192 x 8192 14.5 / 16.8;
+//   but three row blocks of 16: 10240 x 8192 16.7 / 15.6), with two workgroups of streams per CU whole 4096, meet at the same channels of the
+//   memory (16384 x 16384 44.9 / 52.5); more than 16384 weight rows where rows are short (28672 x 1024 8.8 / 6.8, x 4096 21.5 / 22.2).
 //   Few weight rows leave most CUs without a workgroup, and what one reads for itself, 16 weight rows and the lhs rows over all of K, outlasts K
-//   ranges over the device from some 500 KB on (8 rows, 500 x 14336 8.9 / 8.2, x 32768 11.6 / 14.8; 32 rows, 1024 x 6144 7.5 / 7.5, x 8192 8.1 / 8.6,
-//   x 32768 15.1 / 26.3); with 1536 weight rows and up to 16 of lhs 1000 KB; a workgroup on every CU, 32 rows, 4096 x 14336 16.7 / 15.6, x 32768 27.7 / 32.0.
-//   17 .. 32 rows otherwise: short K of wide matrices is stores, which tiles do better (10000 x 1024 4.9 / 5.6, x 4096 12.1 / 11.4); with 16384
-//   weight rows the device is full of tiles as well (14336 x 1024 5.6 / 6.3, x 7168 0.92 times as fast); beyond, 32000 x 4096 34.3 / 29.5, x 8192 58.2 / 68.8.
-//   More: groups of 32 rows where a narrow matrix leaves CUs for them (64 rows, 2048 x 4096 7.3 / 5.8, x 6144 8.3 / 7.6; 2560 x 4096 7.7 / 7.6, x 5632
-//   8.2 / 9.3; 128 rows, 1024 x 6144 8.3 / 7.0, 160 x 6144 7.2 / 8.4).
+//   ranges over the device from some 500 KB on (8 rows, 500 x 14336 9.8 / 8.5, x 32768 12.8 / 15.3; 32 rows, 1024 x 6144 8.8 / 7.8, x 32768 15.5 /
+//   26.6); with 1536 weight rows 650, and with up to 16 of lhs 1000 KB; a workgroup on every CU, 32 rows, 4096 x 14336 16.8 / 15.6, x 32768 32.1 / 32.0.
+//   17 .. 32 rows otherwise: 5120 x 14336 18.8 / 20.9; with three row blocks, and beyond 12288 weight rows where rows are below 8192 bytes (32 rows, 9216 x
+//   1024 6.3 / 5.6, 12288 x 4096 13.7 / 12.4, 14336 x 2048 8.6 / 8.9, 32000 x 4096 33.4 / 28.9, x 8192 56.6 / 65.6; ragged rows of the output cost the tiles
+//   more: 9219 x 1024 6.9 / 5.8).
+//   More: groups of 32 rows where a narrow matrix leaves CUs for them (64 rows, 2048 x 4096 8.1 / 6.0, x 6144 9.4 / 7.7, 2560 x 4096 8.6 / 7.7, x 5632
+//   9.3 / 9.4; 128 rows, 2048 x 5632 10.0 / 9.1, 1024 x 6144 9.1 / 7.3, but 160 x 6144 8.2 / 8.6; with weights that are still cached, 73 rows, 2048 x 5632 8.5 /
+//   6.3), or rows are so short that the host's time decides.
 bool qrows_first(int M, int N, int K) {
     if (!qrows_supported(M, N, K)) return false;
     const long reads = (16 + 2l * M) * K, cols = (long)N * ((M + 31) / 32);
-    if (M == 2) return N <= 256 * 16 || (N <= 256 * 32 ? K % 8192 != 0 : N <= 256 * 48 || (N <= 256 * 64 && K % 4096 != 0));
-    if (M <= 16) {
-        if (N < 2304) return reads <= (N < 1536 ? 525000 : 1000000);
-        return !(N > 256 * 56 && N <= 256 * 64 && K % 16384 == 8192);  // (16384 x 8192, 8 rows 21.6 / 25.5; 14336 x 8192 1.16 times as fast)
+    if (M == 2) {
+        if (N <= 256 * 32) return N <= 256 * 16 || K % 8192 != 0;
+        return N <= 256 * 48 || (N <= 256 * 64 ? K % 4096 != 0 : K <= 2560);
     }
+    if (M <= 16) return N >= 2304 || reads <= (N < 1536 ? 525000 : 1000000);
     if (M <= 32) {
-        if (N < 3072) return reads <= 525000;
+        if (N < 3072) return reads <= (N < 1536 ? 525000 : 650000);
         if (N <= 256 * 16) return reads <= 1700000;
-        if (N <= 256 * 32) return N > 256 * 22 || K <= 8192;  // (32 rows, 5120 x 14336 18.7 / 20.8)
-        if (N <= 256 * 48) return K >= 2560;
-        return K < 8192 && (N > 256 * 64 || (M <= 24 && K >= 2048));
+        if (N <= 256 * 32) return N > 256 * 22 || K <= 8192;
+        return N <= 256 * 48 || K < 8192;
     }
-    return cols <= 256 * 32 && K <= (cols <= 256 * 16 && N >= 256 ? 6144 : 4096);
+    if (cols <= 256 * 16) return K <= (N >= 256 ? 8192 : 4096);
+    return cols <= 256 * 32 ? K <= 6144 : cols <= 256 * 64 && K <= 640;
 }
 int qrows_gemm(void *out, int32_t *acc_out, const int8_t *lhs, const void *a_scale, const int8_t *rhs, const void *b_scale, int M, int N, int K, int dtype,
                hipStream_t s) {

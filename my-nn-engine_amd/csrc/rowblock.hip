@@ -432,17 +432,17 @@ template <typename F> static int rb_rows_shape(int M, int N, F &&f) {
 bool rowblock_rows_supported(const void *out, const void *act, const void *wq, const void *scale, int M, int N, int K) {
     return out && act && wq && scale && M >= 2 && M <= 15 && N >= 1 && K >= 128 && K % 128 == 0 && (long)K * 128 < (1l << 31) && aligned16(act) && aligned16(wq);
 }
-// ... and where it is the one to take (us, tiles over K ranges / so; profiles/few_row_times.csv has both over 900 shapes):
+// ... and where it is the one to take (us a call with weights that are not cached, tiles over K ranges / so; profiles/few_row_times.csv has both over
+// 1200 shapes):
 //   Few weight rows leave most CUs without a workgroup, and a workgroup's own share, 16 weight rows and all of the activations over the whole
-//   of K, outlasts K ranges over the device from some 800 KB on (15 rows: 500 x 14336 14.0 / 12.7, 1024 x 32768 20.1 / 25.8, 500 x 65536
-//   27.1 / 48.3; 8 rows, 500 x 65536 27.0 / 35.6), with 1536 weight rows from 1100 KB (9 rows, 2048 x 32768 23.4 / 23.5).
+//   of K, outlasts K ranges over the device from some 800 KB on (15 rows: 500 x 14336 14.2 / 13.0, 1024 x 32768 19.8 / 25.9, 500 x 65536
+//   26.8 / 48.9; 8 rows, 500 x 65536 26.7 / 35.7), with 1536 weight rows from 1100 KB (9 rows, 2048 x 32768 23.0 / 23.6).
 //   Rows of whole 8192 bytes begin at the same channels of the memory; workgroups of four waves, two per CU, ask for little of each at a time
-//   and meet there: 16384 x 8192, 6 rows 26.4 / 31.4, 15 rows 27.0 / 35.4; 18432 x 8192, 15 rows 35.4 / 50.2 (x 7168 34.5 / 33.8; 14336 x
-//   8192 31.7 / 27.3; 64 rows each, for up to 8 activation rows, 32000 x 8192 62.6 / 50.9).
+//   and meet there: 15 rows, 18432 x 8192 37.3 / 44.4 (x 7168 34.5 / 33.9), 32000 x 8192 61.0 / 64.5 (x 7168 46.3 / 42.0).  (16384 x 8192 with its 32 weight
+//   rows each by where the matrices lie: 6 rows 26.4 / 31.4 and 36.6 / 32.0.)
 bool rowblock_rows_first(int M, int N, int K) {
     if (N < 3072 && (16 + 2l * M) * K > (N < 1536 ? 790000 : 1100000)) return false;
-    if (N > 512 * 32 && M > 8) return K % 8192 != 0;
-    return !(N > 448 * 32 && N <= 512 * 32 && K % 16384 == 8192);
+    return N <= 512 * 32 || M <= 8 || K % 8192 != 0;
 }
 int rowblock_rows_gemm(void *out, const void *act, const int8_t *wq, const void *scale, int M, int N, int K, int dtype, hipStream_t s) {
     MYNN_REQUIRE(rowblock_rows_supported(out, act, wq, scale, M, N, K), MYNN_ERR_UNSUPPORTED, "rowblock_rows_gemm: M=%d N=%d K=%d", M, N, K);

@@ -34,3 +34,10 @@ def test_choice_against_measured_times(kind):
 def test_few_weight_rows(int8_lhs, M, most):
     """500 weight rows: the streams up to some length of a row, K ranges over the device beyond."""
     assert [bool(mynn.lib().mynn_few_rows_first(int8_lhs, M, 500, K)) for K in range(128, 131072, 128)] == [K <= most for K in range(128, 131072, 128)]
+
+
+@pytest.mark.parametrize("M,N,K,streams", [(2, 8192, 8192, 0), (2, 10240, 8192, 1), (2, 28672, 2560, 1), (2, 28672, 2688, 0), (16, 2304, 65536, 1), (17, 1536, 13056, 0), (17, 1536, 12928, 1),
+                                           (32, 5632, 8192, 1), (32, 5632, 8320, 0), (32, 9216, 1024, 1), (32, 12288, 32768, 1), (32, 14336, 8064, 1), (32, 14336, 8192, 0),
+                                           (64, 2048, 8192, 1), (64, 2560, 4096, 1), (64, 2560, 6144, 1), (64, 2560, 6272, 0), (97, 2048, 5632, 1), (128, 160, 4224, 0), (64, 8192, 640, 1), (64, 8192, 768, 0)])
+def test_edges_of_the_choice(M, N, K, streams):
+    assert mynn.lib().mynn_few_rows_first(1, M, N, K) == streams
