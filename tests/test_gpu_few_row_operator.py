@@ -17,26 +17,22 @@ def g():
     return gpu_util
 
 
-def operands(g, M, N, K, dt):
-    """activations, weights, scales, the sums in 64 bits, and what f32 sums of K exact products in any order and one rounding of the stored
-    value may be off"""
-    rng = np.random.default_rng(M + N + K)
-    act, sc = orc.to_storage(rng.standard_normal((M, K)), dt), orc.to_storage(rng.uniform(1e-3, 1e-2, N), dt)
-    W = rng.integers(-128, 128, (N, K)).astype(np.int8)
-    a, s, w = g.f32(act, dt).astype(np.float64).reshape(M, K), g.f32(sc, dt).astype(np.float64), W.astype(np.float64)
-    exact = (a @ w.T) * s
-    return act, W, sc, exact, (np.abs(a) @ np.abs(w).T) * s * K * 2.0 ** -24 + np.abs(exact) * (2.0 ** -8 if dt == orc.BF16 else 2.0 ** -11) * 1.01 + 1e-30
-
-
 @pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
 @pytest.mark.parametrize("M", [2, 8, 9, 15])
 @pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 2048), (4099, 384), (8193, 1024), (12290, 640), (16400, 1152), (700, 14336)])
 def test_few_rows_row_major(g, dt, M, N, K):
     import torch
 
-    act, W, sc, exact, bound = operands(g, M, N, K, dt)
+    rng = np.random.default_rng(M + N + K)
+    act, sc = orc.to_storage(rng.standard_normal((M, K)), dt), orc.to_storage(rng.uniform(1e-3, 1e-2, N), dt)
+    W = rng.integers(-128, 128, (N, K)).astype(np.int8)
     da, dw, ds = g.to_dev(act, dt), g.to_dev(W), g.to_dev(sc, dt)
     got = g.mynn.dequant_matmul(da, dw, ds)
+    a, s = g.f32(act, dt).astype(np.float64).reshape(M, K), g.f32(sc, dt).astype(np.float64)
+    w = W.astype(np.float64)
+    exact = (a @ w.T) * s
+    # f32 sums of K exact products in any order, one rounding of the stored value
+    bound = (np.abs(a) @ np.abs(w).T) * s * K * 2.0 ** -24 + np.abs(exact) * (2.0 ** -8 if dt == orc.BF16 else 2.0 ** -11) * 1.01 + 1e-30
     assert np.all(np.abs(g.f32(g.to_host(got), dt).reshape(M, N) - exact) <= bound)
     assert torch.equal(g.mynn.dequant_matmul_ws(da, dw, ds), got)
     side = torch.cuda.Stream()
@@ -49,6 +45,17 @@ def test_few_rows_row_major(g, dt, M, N, K):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, got)
+
+
+def operands(g, M, N, K, dt):
+    """activations, weights, scales, the sums in 64 bits, and what f32 sums of K exact products in any order and one rounding of the stored
+    value may be off"""
+    rng = np.random.default_rng(M + N + K)
+    act, sc = orc.to_storage(rng.standard_normal((M, K)), dt), orc.to_storage(rng.uniform(1e-3, 1e-2, N), dt)
+    W = rng.integers(-128, 128, (N, K)).astype(np.int8)
+    a, s, w = g.f32(act, dt).astype(np.float64).reshape(M, K), g.f32(sc, dt).astype(np.float64), W.astype(np.float64)
+    exact = (a @ w.T) * s
+    return act, W, sc, exact, (np.abs(a) @ np.abs(w).T) * s * K * 2.0 ** -24 + np.abs(exact) * (2.0 ** -8 if dt == orc.BF16 else 2.0 ** -11) * 1.01 + 1e-30
 
 
 # (1, 2 and 3 row blocks and eight waves, 2 and 4 and four waves: a ring has up to 5, 3, 2, 3 and 2 stages of 128 k)

@@ -16,7 +16,10 @@ def g():
     return gpu_util
 
 
-def check(g, dt, M, N, K):
+@pytest.mark.parametrize("dt", [orc.F32, orc.F16, orc.BF16])
+@pytest.mark.parametrize("M", [2, 8, 9, 17, 32, 33, 65, 128])
+@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336), (2050, 1152)])
+def test_few_rows_int8(g, dt, M, N, K):
     import torch
 
     rng = np.random.default_rng(M + N + K)
@@ -32,13 +35,6 @@ def check(g, dt, M, N, K):
     assert none is None and torch.equal(alone, out)
 
 
-@pytest.mark.parametrize("dt", [orc.F32, orc.F16, orc.BF16])
-@pytest.mark.parametrize("M", [2, 8, 9, 17, 32, 33, 65, 128])
-@pytest.mark.parametrize("N,K", [(1, 128), (15, 256), (33, 1152), (4096, 1024), (4099, 384), (8193, 640), (12290, 1152), (16385, 512), (700, 14336), (2050, 1152)])
-def test_few_rows_int8(g, dt, M, N, K):
-    check(g, dt, M, N, K)
-
-
 # (row blocks, groups of 8 lhs rows, waves: 20 / (2 blocks + groups) stages of 128 k, 8 at most)
 @pytest.mark.parametrize("M,N,K,blocks,groups,waves", [
     (8, 700, 12288, 1, 1, 8), (16, 700, 10240, 1, 2, 8), (32, 700, 6272, 1, 4, 8), (65, 300, 6144, 1, 4, 8), (8, 5700, 8320, 2, 1, 8), (9, 5700, 8320, 2, 2, 8),
@@ -46,7 +42,7 @@ def test_few_rows_int8(g, dt, M, N, K):
     (16, 12290, 4224, 4, 2, 8), (5, 16400, 2176, 4, 1, 4), (12, 16400, 2176, 4, 2, 4), (24, 12290, 2176, 2, 4, 4), (32, 16400, 3200, 2, 4, 4)])
 def test_rings_in_turn(g, M, N, K, blocks, groups, waves):
     assert K // 128 // waves >= 2 * min(8, 20 // (2 * blocks + groups)) and g.mynn.lib().mynn_few_rows_first(1, M, N, K)
-    check(g, orc.F16, M, N, K)
+    test_few_rows_int8(g, orc.F16, M, N, K)
 
 
 # (where K ranges are the faster form a captured call, whose tiles would take them as one, takes the streams)

@@ -58,7 +58,7 @@ def test_same_bits_from_every_form(g, dt, M, N, K, size):
 
 
 @pytest.mark.parametrize("dt", [orc.F16, orc.BF16])
-@pytest.mark.parametrize("M,N,K", [(3, 33, 96), (6, 4096, 14336), (6, 4096, 14352), (15, 500, 2064)])
+@pytest.mark.parametrize("M,N,K", [(3, 33, 96), (6, 4096, 14336), (15, 500, 2064)])
 def test_few_rows_captured(g, dt, M, N, K):
     """the same below 16 rows (scale after the sum)"""
     import torch

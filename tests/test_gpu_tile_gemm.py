@@ -18,7 +18,7 @@ def g():
 
 # rows one below, at and one above tiles of 32 / 64 / 128; N odd, below and above a tile; K of half a step, odd halves of a
 # step, long enough for several ranges
-SHAPES = [(3, 33, 96), (15, 500, 2048), (15, 500, 4112), (16, 1, 16), (31, 64, 544), (33, 65, 4112), (64, 129, 2080), (97, 700, 5632), (129, 127, 1056), (260, 2050, 4096),
+SHAPES = [(3, 33, 96), (15, 500, 2048), (16, 1, 16), (31, 64, 544), (33, 65, 4112), (64, 129, 2080), (97, 700, 5632), (129, 127, 1056), (260, 2050, 4096),
           (300, 20, 14336)]
 
 
